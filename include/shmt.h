@@ -118,8 +118,10 @@ int shmt_hashmap_create(shmt_hashmap_t **out, const void *keys,
 typedef struct shmt_hashmap_layout {
   int kind;            /* SHMT_MAP_*                                        */
   int slot_bytes;      /* buckets: 16 or 8; direct: 4; range: 0; rank: 16   */
-  int64_t lo, span;    /* flat forms: id range [lo, lo + span)              */
-  int64_t delta;       /* range: value = key + delta; rank: rank + delta    */
+  int64_t lo, span;    /* flat forms and packed 8-byte slots: id range
+                          [lo, lo + span); 0, 0: unpacked slots             */
+  int64_t delta;       /* range: value = key + delta; rank: rank + delta;
+                          packed slots: middle of the values                */
   int64_t table_bytes; /* device memory the build needs (128-byte aligned)  */
 } shmt_hashmap_layout;
 int64_t shmt_hashmap_plan_scratch_bytes(int64_t n);
@@ -133,6 +135,21 @@ int shmt_hashmap_create_planned(shmt_hashmap_t **out,
                                 int key_bytes, int val_bytes,
                                 double load_factor, void *table_mem,
                                 int64_t table_bytes, void *stream);
+/* The same with scratch memory (device, 16-byte aligned), which lets a large
+ * table of 8-byte slots be built without an atomic per key. The first
+ * function says how much a layout asks for (0: none); with less, or none,
+ * the build is shmt_hashmap_create_planned's. The scratch memory is free
+ * again when the work queued on the stream has run.                        */
+int64_t shmt_hashmap_build_scratch_bytes(const shmt_hashmap_layout *layout,
+                                         int64_t n, double load_factor);
+int shmt_hashmap_create_planned_scratch(shmt_hashmap_t **out,
+                                        const shmt_hashmap_layout *layout,
+                                        const void *keys, const void *vals,
+                                        int64_t n, int key_bytes,
+                                        int val_bytes, double load_factor,
+                                        void *table_mem, int64_t table_bytes,
+                                        void *scratch, int64_t scratch_bytes,
+                                        void *stream);
 /* SHMT_MAP_* of a built map, and the table bytes it actually uses.         */
 int shmt_hashmap_kind(const shmt_hashmap_t *map);
 int64_t shmt_hashmap_used_bytes(const shmt_hashmap_t *map);

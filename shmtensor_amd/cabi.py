@@ -23,6 +23,9 @@ SIGNATURES = {
     "shmt_hashmap_create": (_int, [_c.POINTER(_vp), _vp, _vp, _i64, _int, _int, _dbl, _vp, _i64, _vp]),
     "shmt_hashmap_plan_scratch_bytes": (_i64, [_i64]),
     "shmt_hashmap_plan": (_int, [_vp, _vp, _i64, _int, _int, _dbl, _vp, _i64, _vp, _vp]),
+    "shmt_hashmap_build_scratch_bytes": (_i64, [_vp, _i64, _dbl]),
+    "shmt_hashmap_create_planned_scratch": (_int, [_c.POINTER(_vp), _vp, _vp, _vp, _i64, _int, _int, _dbl, _vp, _i64,
+                                                   _vp, _i64, _vp]),
     "shmt_hashmap_create_planned": (_int, [_c.POINTER(_vp), _vp, _vp, _vp, _i64, _int, _int, _dbl, _vp, _i64, _vp]),
     "shmt_hashmap_kind": (_int, [_vp]),
     "shmt_hashmap_used_bytes": (_i64, [_vp]),

@@ -8,8 +8,15 @@
 //   wide   (kSlot16): 8 slots {int64 key, int64 value}; used whenever the key
 //                     or the value is 8 bytes wide (4-byte members are
 //                     sign-extended on insert).
-//   narrow (kSlot8) : 16 slots {int32 key, int32 value}; each lane sees two.
-// Empty slots hold key = value = -1 (all bits set). Keys probe buckets
+//   narrow (kSlot8) : 16 slots of one 64-bit word {key | value}, the key in the
+//                     high bits; each lane sees two. Two ways to fill it:
+//                     32 + 32 bits when every key and value fits 32 bits; or,
+//                     packed, the key's distance from the smallest key above
+//                     the value's distance from the middle of the values,
+//                     when both together need at most 64 bits (a cache's slot
+//                     numbers leave 40 bits and more to the keys). A table
+//                     half the size is cleared, written and probed for.
+// Empty slots hold all bits set; no key of either narrow form is stored so. Keys probe buckets
 // linearly from hash(key) and are always placed in the first bucket of their
 // probe sequence that still has a free slot, so a lookup stops at the first
 // bucket that contains either the key or an empty slot.
@@ -52,23 +59,44 @@ struct MapView {
   uint32_t nbuckets;
   int key32;              // 1: keys are int32 -> requests are narrowed before the lookup
   int kind;               // MapKind
-  int fits32;             // 1: 64-bit keys stored in narrow slots (they all fit): a request that
-                          //    does not fit 32 bits is absent
-  int64_t lo;             // flat forms: smallest key
-  int64_t span;           // flat forms: keys lie in [lo, lo + span)
-  int64_t delta;          // range form: value = key + delta; rank form: value = rank + delta
+  int fits32;             // narrow slots, 1: 64-bit keys that all fit 32 bits: a request that does not is
+                          //    absent; 2: packed, looked up by key - lo
+  int val_bits;           // narrow slots: low bits of a word that hold the value
+  int64_t lo;             // flat forms, packed slots: smallest key
+  int64_t span;           // flat forms, packed slots: keys lie in [lo, lo + span)
+  int64_t delta;          // range form: value = key + delta; rank form: value = rank + delta; narrow slots:
+                          //    value = stored signed field + delta
 };
 
-inline MapView empty_map_view() { return MapView{nullptr, 1, 0, kKindBuckets, 0, 0, 0, 0}; }
+inline MapView empty_map_view() { return MapView{nullptr, 1, 0, kKindBuckets, 0, 32, 0, 0, 0}; }
 
 // Normalise a request to the key domain of the map (what requests.to(key
 // dtype) does in the reference): int32-keyed maps see the low 32 bits,
-// sign-extended. A request that cannot be a key of a narrow-stored 64-bit
-// map becomes the empty sentinel, which every lookup resolves to -1.
+// sign-extended. A request that cannot be a key of a narrow-stored map
+// becomes the empty sentinel, which every lookup resolves to -1.
 __device__ __forceinline__ int64_t map_key(const MapView &m, int64_t req) {
-  if (m.key32) return static_cast<int64_t>(static_cast<int32_t>(req));
+  if (m.key32) req = static_cast<int64_t>(static_cast<int32_t>(req));
+  if (m.fits32 == 2) {
+    const uint64_t off = static_cast<uint64_t>(req) - static_cast<uint64_t>(m.lo);  // req < lo wraps around
+    return off < static_cast<uint64_t>(m.span) ? static_cast<int64_t>(off) : -1;
+  }
   if (m.fits32 && req != static_cast<int64_t>(static_cast<int32_t>(req))) return -1;
   return req;
+}
+
+// Narrow slots: the word of a normalised key (not -1) and its value, the key
+// of a word, and the value in a word's low bits.
+__device__ __forceinline__ uint64_t slot8_word(const MapView &m, int64_t key, int64_t val) {
+  return (static_cast<uint64_t>(key) << m.val_bits) |
+         (static_cast<uint64_t>(val - m.delta) & ((1ull << m.val_bits) - 1));
+}
+__device__ __forceinline__ int64_t slot8_key(const MapView &m, uint64_t word) {
+  if (m.fits32 == 2) return static_cast<int64_t>(word >> m.val_bits);
+  return static_cast<int64_t>(word) >> 32;
+}
+__device__ __forceinline__ int64_t slot8_value(const MapView &m, uint64_t word) {
+  const int s = 64 - m.val_bits;
+  return (static_cast<int64_t>(word << s) >> s) + m.delta;
 }
 
 // Table entries that will not be looked at again soon (the probe of a row
@@ -167,7 +195,7 @@ __device__ __forceinline__ uint32_t map_bucket(const MapView &m, int64_t key) {
 // done with this key (value written to *val: the mapped value, or -1 when the
 // bucket proved the key absent); false when the bucket was full of other keys.
 template <int FMT>
-__device__ __forceinline__ bool probe_step(const uint4 frag, int64_t key, int64_t *val) {
+__device__ __forceinline__ bool probe_step(const MapView &m, const uint4 frag, int64_t key, int64_t *val) {
   const int gbase = lane_id() & ~(kProbeGroup - 1);
   bool match, empty;
   int64_t v;
@@ -177,12 +205,15 @@ __device__ __forceinline__ bool probe_step(const uint4 frag, int64_t key, int64_
     match = (k == key);
     empty = (k == -1);
   } else {
-    int32_t k32 = static_cast<int32_t>(key);
-    bool m0 = static_cast<int32_t>(frag.x) == k32;
-    bool m1 = static_cast<int32_t>(frag.z) == k32;
+    const uint64_t w0 = (static_cast<uint64_t>(frag.y) << 32) | frag.x;
+    const uint64_t w1 = (static_cast<uint64_t>(frag.w) << 32) | frag.z;
+    const uint64_t want = static_cast<uint64_t>(key) << m.val_bits, field = 1ull << m.val_bits;
+    const bool e0 = w0 == ~0ull, e1 = w1 == ~0ull;
+    const bool m0 = !e0 && (w0 ^ want) < field;  // (the sentinel's bits equal an empty slot's: no match)
+    const bool m1 = !e1 && (w1 ^ want) < field;
     match = m0 || m1;
-    v = static_cast<int64_t>(static_cast<int32_t>(m0 ? frag.y : frag.w));
-    empty = (frag.x == 0xFFFFFFFFu) || (frag.z == 0xFFFFFFFFu);
+    empty = e0 || e1;
+    v = slot8_value(m, m0 ? w0 : w1);
   }
   uint64_t mm = group_ballot<kProbeGroup>(match);
   if (mm) {
@@ -208,7 +239,7 @@ __device__ __forceinline__ int64_t group_find(const MapView &m, int64_t key) {
   int64_t val = -1;
   for (uint32_t probes = 0; probes < m.nbuckets; ++probes) {
     uint4 frag = m.buckets[static_cast<size_t>(b) * kProbeGroup + sub];
-    if (probe_step<FMT>(frag, key, &val)) return val;
+    if (probe_step<FMT>(m, frag, key, &val)) return val;
     b = (b + 1 == m.nbuckets) ? 0 : b + 1;
   }
   return -1;
@@ -249,7 +280,7 @@ __device__ __forceinline__ int64_t wave_find(const MapView &m, int64_t mykey) {
       for (int j = 0; j < BATCH; ++j) {
         if (pending & (1u << j)) {
           int64_t val;
-          if (probe_step<FMT>(frag[j], shfl64(mykey, gbase + j0 + j), &val)) {
+          if (probe_step<FMT>(m, frag[j], shfl64(mykey, gbase + j0 + j), &val)) {
             pending &= ~(1u << j);
             if (sub == j0 + j) res = val;
           }
@@ -324,7 +355,7 @@ __device__ __forceinline__ int64_t half_wave_finish(const MapView &m, int64_t my
 #pragma unroll
   for (int j = 0; j < kHalfWaveKeys; ++j) {
     int64_t val;
-    if (probe_step<FMT>(p.frag[j], shfl64(mykey, grp * kHalfWaveKeys + j), &val)) {
+    if (probe_step<FMT>(m, p.frag[j], shfl64(mykey, grp * kHalfWaveKeys + j), &val)) {
       if (sub == j) res = val;
     } else {
       pending |= 1u << j;
@@ -339,7 +370,7 @@ __device__ __forceinline__ int64_t half_wave_finish(const MapView &m, int64_t my
         if (b >= m.nbuckets) b -= m.nbuckets;
         const uint4 frag = m.buckets[static_cast<size_t>(b) * kProbeGroup + sub];
         int64_t val;
-        if (probe_step<FMT>(frag, key, &val)) {
+        if (probe_step<FMT>(m, frag, key, &val)) {
           pending &= ~(1u << j);
           if (sub == j) res = val;
         }

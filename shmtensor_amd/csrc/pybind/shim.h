@@ -204,8 +204,13 @@ class StaticHashmap {
     table_ = device_bytes(layout.table_bytes);
     memory_usage_ = layout.kind == SHMT_MAP_RANGE ? 0 : layout.table_bytes;
     kind_ = layout.kind;
-    check(shmt_hashmap_create_planned(&handle_, &layout, keys.data_ptr(), values.data_ptr(), n, kb, vb,
-                                      load_factor, table_.data_ptr(), layout.table_bytes, current_stream()));
+    const int64_t build_bytes = shmt_hashmap_build_scratch_bytes(&layout, n, load_factor);
+    torch::Tensor build_scratch;
+    if (build_bytes > 0) build_scratch = device_bytes(build_bytes);
+    check(shmt_hashmap_create_planned_scratch(&handle_, &layout, keys.data_ptr(), values.data_ptr(), n, kb, vb,
+                                              load_factor, table_.data_ptr(), layout.table_bytes,
+                                              build_bytes > 0 ? build_scratch.data_ptr() : nullptr, build_bytes,
+                                              current_stream()));
   }
   ~StaticHashmap() { shmt_hashmap_destroy(handle_); }
   StaticHashmap(const StaticHashmap &) = delete;

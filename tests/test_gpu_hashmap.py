@@ -338,3 +338,60 @@ def test_planned_build_through_the_c_abi(cabi):
     small = torch.empty(1024, dtype=torch.uint8, device="cuda")
     assert lib.shmt_hashmap_plan(big.data_ptr(), vals.data_ptr(), n, 8, 8, 0.5, small.data_ptr(), 1024,
                                  ctypes.byref(lay), stream) == -4                     # scratch too small
+
+
+@pytest.mark.parametrize("case", ["unpacked", "packed", "one_key_many_times", "few_pairs", "eight_million", "int32"])
+def test_large_narrow_tables_are_built_by_partitions(capi, case):
+    """From 2^18 pairs on, tables of 8-byte slots are built partition by partition in LDS; keys beyond 32 bits are
+    stored as distances from the smallest key when those and the values share 64 bits. Members give their value,
+    everything else -1 (near misses around the key range, ids whose low bits equal a key's); a key given many times,
+    which outgrows the room of its partition, gives one of its values."""
+    g = torch.Generator(device="cuda").manual_seed(5)
+    n = {"few_pairs": (1 << 18) + 1, "eight_million": 8_300_001}.get(case, 700_003)
+    span = 1 << (29 if case in ("unpacked", "int32") else 41)
+    lo = 0 if case in ("unpacked", "int32") else (1 << 33) + 12_345
+    keys = torch.unique(torch.randint(0, span, (n + n // 8,), device="cuda", generator=g))
+    keys = (lo + keys[torch.randperm(keys.numel(), device="cuda", generator=g)][:n]).contiguous()
+    assert keys.numel() == n
+    # (packed: 41 bits of key leave 22 or 23 bits of value, which these use up, below zero and above)
+    vals = torch.arange(n, device="cuda") - (n // 2 if case == "packed" else 0)
+    if case == "one_key_many_times":
+        keys[: n // 2] = keys[0]
+    if case == "int32":
+        keys, vals = keys.int(), vals.int()
+    h = capi.CUCOStaticHashmap(keys, vals, 0.8)
+    assert h.layout() == "buckets" and h.memory_usage() <= 2 * n * 8 + 128
+    first = 0 if case != "one_key_many_times" else n // 2
+    assert torch.equal(h.query(keys[first:]), vals[first:])
+    if first:
+        won = h.query(keys[:1]).item()
+        assert 0 <= won < n // 2 and bool((h.query(keys[:1000]) == won).all())
+    wide = keys.long()
+    ordered = torch.sort(wide).values
+    for other in (wide + 1, wide - 1, ordered[:1] - torch.arange(1, 200, device="cuda"),
+                  ordered[-1:] + torch.arange(1, 200, device="cuda"), torch.tensor([-1, 0, 2**62, -2**62]).cuda()):
+        other = other.to(keys.dtype)
+        at = torch.searchsorted(ordered, other.long()).clamp(max=n - 1)
+        absent = ordered[at] != other.long()
+        assert bool((h.query(other)[absent] == -1).all())
+    if case != "int32":
+        assert bool((h.query(wide[:5000] + 2**63 - 2**62) == -1).all())
+        assert bool((h.query(wide[:5000] ^ (1 << 45)) == -1).all())
+
+
+@pytest.mark.parametrize("n,packs", [((4 << 20) // 32, False), ((4 << 20) // 32 + 1, True)])
+def test_values_and_spans_that_just_pack(capi, n, packs):
+    """The line of the packed form: more than 131,072 pairs, and key distances and values that share 64 bits. The
+    widest values that fit (and, one beyond them, the 16-byte slots) come back exactly."""
+    g = torch.Generator(device="cuda").manual_seed(6)
+    # 2^40 - 1 ids: 40 bits of key, 24 of value
+    keys = torch.unique(torch.cat([torch.randint(1, (1 << 40) - 2, (n + 2000,), device="cuda", generator=g)]))
+    keys = keys[torch.randperm(keys.numel(), device="cuda", generator=g)][:n].contiguous()
+    keys[0], keys[1] = 0, (1 << 40) - 2
+    for span, narrow in (((1 << 24) - 1, packs), (1 << 24, False)):
+        vals = torch.randint(0, span + 1, (n,), device="cuda", generator=g) - (1 << 35)
+        vals[0], vals[1] = -(1 << 35), span - (1 << 35)
+        h = capi.CUCOStaticHashmap(keys, vals, 0.5)
+        assert h.layout() == "buckets" and h.memory_usage() == (2 * n + (15 if narrow else 7)) // (16 if narrow else 8) * 128
+        assert torch.equal(h.query(keys), vals)
+        assert h.query(torch.tensor([-1, (1 << 40) - 1, 1 << 40]).cuda()).tolist() == [-1, -1, -1]
