@@ -596,6 +596,18 @@ int shmt_subcsr_copy(const void *indptr, const void *indices, int ptr_bytes,
                      int idx_bytes, const void *seeds, int seed_bytes,
                      int64_t C, const void *cache_indptr, int64_t nnz,
                      void *cache_indices, void *stream);
+/* The same, with the start of every chosen row in the source kept between
+ * the two calls: row_begins has room for C int64 (device memory; NULL: as
+ * above). The copy then reads no row offset over the host link.            */
+int shmt_subcsr_plan_rows(const void *indptr, int ptr_bytes, const void *seeds,
+                          int seed_bytes, int64_t C, void *cache_indptr,
+                          int64_t *row_begins, void *tmp, int64_t tmp_bytes,
+                          int64_t *nnz_out, void *stream);
+int shmt_subcsr_copy_rows(const void *indptr, const void *indices,
+                          int ptr_bytes, int idx_bytes, const void *seeds,
+                          int seed_bytes, int64_t C, const void *cache_indptr,
+                          const int64_t *row_begins, int64_t nnz,
+                          void *cache_indices, void *stream);
 
 #ifdef __cplusplus
 }

@@ -76,6 +76,8 @@ SIGNATURES = {
     "shmt_graph_destroy": (None, [_vp]),
     "shmt_stage_seeds": (_int, [_vp, _int, _i64, _vp, _int, _vp, _c.c_uint64, _vp, _vp]),
     "shmt_csr_rows": (_int, [_vp, _int, _i64, _i64, _vp, _int, _vp]),
+    "shmt_subcsr_plan_rows": (_int, [_vp, _int, _vp, _int, _i64, _vp, _vp, _vp, _i64, _vp, _vp]),
+    "shmt_subcsr_copy_rows": (_int, [_vp, _vp, _int, _int, _vp, _int, _i64, _vp, _vp, _i64, _vp, _vp]),
     "shmt_subcsr_plan": (_int, [_vp, _int, _vp, _int, _i64, _vp, _vp, _i64, _vp, _vp]),
     "shmt_subcsr_copy": (_int, [_vp, _vp, _int, _int, _vp, _int, _i64, _vp, _i64, _vp, _vp]),
 }

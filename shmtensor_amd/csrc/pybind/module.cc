@@ -327,13 +327,15 @@ std::tuple<torch::Tensor, torch::Tensor> create_subcsr(torch::Tensor uva_indptr,
   const Readback::Slot total = readback().acquire();
   void *stream = current_stream();
   void *indptr_dev = device_address(uva_indptr, "uva_indptr");
-  check(shmt_subcsr_plan(indptr_dev, pb, seeds.data_ptr(), static_cast<int>(seeds.element_size()), C,
-                         gpu_indptr.data_ptr(), tmp.data_ptr(), tmp_bytes, total.dev, stream));
+  torch::Tensor begins = torch::empty({C}, seeds.options().dtype(torch::kInt64));
+  check(shmt_subcsr_plan_rows(indptr_dev, pb, seeds.data_ptr(), static_cast<int>(seeds.element_size()), C,
+                              gpu_indptr.data_ptr(), begins.data_ptr<int64_t>(), tmp.data_ptr(), tmp_bytes, total.dev,
+                              stream));
   const int64_t nnz = Readback::wait(total);
   torch::Tensor gpu_indices = torch::empty({nnz}, uva_indices.options().device(torch::kCUDA));
-  check(shmt_subcsr_copy(indptr_dev, device_address(uva_indices, "uva_indices"), pb, ib,
-                         seeds.data_ptr(), static_cast<int>(seeds.element_size()), C,
-                         gpu_indptr.data_ptr(), nnz, gpu_indices.data_ptr(), stream));
+  check(shmt_subcsr_copy_rows(indptr_dev, device_address(uva_indices, "uva_indices"), pb, ib,
+                              seeds.data_ptr(), static_cast<int>(seeds.element_size()), C,
+                              gpu_indptr.data_ptr(), begins.data_ptr<int64_t>(), nnz, gpu_indices.data_ptr(), stream));
   return std::make_tuple(gpu_indptr, gpu_indices);
 }
 
