@@ -12,10 +12,12 @@
 // arithmetic), or the mask is loaded. Each lane ends up holding the source
 // (fetch) or destination (set) address of its row. A wave with several tiles
 // keeps phase 1 of the next tiles in flight while it moves rows.
-// Phase 2 (sub-wave group of L lanes per row): the row addresses are
-// broadcast with lane shuffles and the rows are moved with the widest vector
-// access the row size and base pointers allow (16 bytes per lane when
-// aligned). The dependent chain id -> bucket -> row is paid once per tile
+// Phase 2: the row addresses are broadcast with lane shuffles and the rows are
+// moved with the widest vector access the row size and base pointers allow (16
+// bytes per lane when aligned). Rows of 8, 16, 32 or 64 vectors (or nearly) take
+// a sub-wave group of as many lanes each; the vectors of rows of any other size
+// are dealt to the lanes one after the other, whatever row they belong to, so
+// that no lane is left over at the end of a row. The dependent chain id -> bucket -> row is paid once per tile
 // instead of once per row.
 //
 // A fetch can also go out as two launches (shmt_fetch_cached_part /
@@ -50,8 +52,10 @@ struct RowArgs {
   int64_t row_bytes;
   int idx_bytes;
   int mask_bytes;
-  int log2_lanes;      // lanes per row in phase 2 = 1 << log2_lanes, in [8, 64]
+  int log2_lanes;      // lanes per row in phase 2 = 1 << log2_lanes, in [8, 64] (ONE_VEC)
   int log2_tile;       // rows per wave tile = 1 << log2_tile, in [64 / lanes, 32]
+  uint32_t nvec;        // vectors per row (!ONE_VEC); 0: too many for a tile's to be counted in 32 bits
+  uint32_t nvec_magic;  // floor((2^32 - 1) / nvec): the high half of i * magic is i / nvec, or one less
   uint32_t *miss_bits;  // DEFER: bit (i & 31) of word i / 32 is set when row i missed the cache
 };
 
@@ -77,6 +81,15 @@ constexpr int kRowsWavesPerSimd = 8;  // register budget: 512 / 8 = 64 VGPRs
 // 256 B: 1 row in flight per group 92 us, 2 rows 96 us, 4 rows 94 us (eight resident waves per SIMD
 // already keep the memory system busy; shorter load/store bursts per wave mix reads and writes better).
 constexpr int kRowsInFlight = 1;
+// Vectors a lane moves concurrently when they are dealt out one by one, and the waves per SIMD the register
+// budget is set for. 262,144 rows, all hits, buffers not in the caches, one / two in flight (with lane groups
+// before): fetch of 33 floats 22.0 / 23.9 (27.9) us, 300 floats 123 / 137 (144), 300 halves 71 / 91 (107); set
+// of 33 floats 25.4 / 30.6 (35.8), 50 floats 27.5 / 30.6 (29.1), but 100 floats 45.8 / 43.9 (48.5) and 300 floats
+// 178 / 171 (171): a set of 16-byte vectors takes two, which need the registers of six waves. Four gain nothing.
+constexpr int vecs_in_flight(bool set, int vector_bytes) { return set && vector_bytes == 16 ? 2 : 1; }
+constexpr int rows_waves_per_simd(bool set, bool one_vec, int vector_bytes) {
+  return one_vec || vecs_in_flight(set, vector_bytes) == 1 ? kRowsWavesPerSimd : 6;
+}
 // Rows per wave tile, at most. 32 measured 2 % faster than 64 on all-hit rows (90 against 92 us) and the
 // same on mixed hit / miss batches; 16 gains nothing more and costs the bucket-table probe 15 %.
 constexpr int kMaxLog2Tile = 5;
@@ -87,7 +100,7 @@ constexpr int kMaxLog2Tile = 5;
 // miss the cache are not moved; every tile leaves one word of a bitmap that
 // marks them for rows_missed_kernel (no counter, no atomics, nothing to clear).
 template <typename VT, int MODE, bool SET, bool ONE_VEC, bool THROUGH = false, bool DEFER = false>
-__global__ __launch_bounds__(kRowsBlock, ONE_VEC ? kRowsWavesPerSimd : kRowsWavesPerSimd / 2) void rows_kernel(RowArgs a) {
+__global__ __launch_bounds__(kRowsBlock, rows_waves_per_simd(SET, ONE_VEC, sizeof(VT))) void rows_kernel(RowArgs a) {
   static_assert(!THROUGH || (SET && MODE != kDirect), "write-through is a cached set");
   static_assert(!DEFER || (!SET && MODE != kDirect), "only a cached fetch sets its misses aside");
   const int lane = lane_id();
@@ -100,7 +113,6 @@ __global__ __launch_bounds__(kRowsBlock, ONE_VEC ? kRowsWavesPerSimd : kRowsWave
   const int64_t wave = static_cast<int64_t>(blockIdx.x) * waves_per_block + threadIdx.x / kWave;
   const int64_t nwaves = static_cast<int64_t>(gridDim.x) * waves_per_block;
   const int64_t R = a.row_bytes;
-  const int64_t step = static_cast<int64_t>(L) * sizeof(VT);
   const int64_t my_off = static_cast<int64_t>(gl) * sizeof(VT);
   int64_t Q = a.Q;
   if (a.count) {
@@ -241,32 +253,63 @@ __global__ __launch_bounds__(kRowsBlock, ONE_VEC ? kRowsWavesPerSimd : kRowsWave
           }
         }
       }
-    } else {
-      for (int r0 = 0; r0 < nrows; r0 += rows_per_step) {
-        const int row = r0 + grp;
-        char *trow = reinterpret_cast<char *>(shfl64(my_table_row, row & (kWave - 1)));
-        char *second =
-            THROUGH ? reinterpret_cast<char *>(shfl64(my_second_row, row & (kWave - 1))) : nullptr;
-        if (row >= nrows || (DEFER && !trow)) continue;
-        char *drow = a.dense + (base + row) * R;
-        const char *src = SET ? drow : trow;
-        char *dst = SET ? trow : drow;
-        int64_t off = my_off;
-        for (; off + 3 * step < R; off += 4 * step) {
-          const VT v0 = gload<VT>(src + off);
-          const VT v1 = gload<VT>(src + off + step);
-          const VT v2 = gload<VT>(src + off + 2 * step);
-          const VT v3 = gload<VT>(src + off + 3 * step);
-          gstore<VT>(dst + off, v0);
-          gstore<VT>(dst + off + step, v1);
-          gstore<VT>(dst + off + 2 * step, v2);
-          gstore<VT>(dst + off + 3 * step, v3);
+    } else if (a.nvec == 0) {
+      for (int row = 0; row < nrows; ++row) {
+        char *const trow = reinterpret_cast<char *>(shfl64(my_table_row, row));
+        char *const second = THROUGH ? reinterpret_cast<char *>(shfl64(my_second_row, row)) : nullptr;
+        if (DEFER && !trow) continue;
+        char *const drow = a.dense + (base + row) * R;
+        for (int64_t off = lane * static_cast<int64_t>(sizeof(VT)); off < R; off += kWave * static_cast<int64_t>(sizeof(VT))) {
+          const VT v = gload<VT>((SET ? drow : trow) + off);
+          gstore<VT>((SET ? trow : drow) + off, v);
+          if (THROUGH && second) gstore<VT>(second + off, v);
         }
-        for (; off < R; off += step)
-          gstore<VT>(dst + off, gload<VT>(src + off));
-        if (THROUGH && second) {
-          for (off = my_off; off < R; off += step)
-            gstore<VT>(second + off, gload<VT>(src + off));
+      }
+    } else {
+      constexpr int kVecsInFlight = vecs_in_flight(SET, sizeof(VT));
+      const uint32_t total = static_cast<uint32_t>(nrows) * a.nvec;
+      char *const dense = a.dense + base * R;  // the tile's rows lie one behind the other
+      for (uint32_t v0 = 0; v0 < total; v0 += kVecsInFlight * kWave) {
+        VT v[kVecsInFlight];
+        char *at[kVecsInFlight];
+        char *second[kVecsInFlight];
+        bool on[kVecsInFlight];
+#pragma unroll
+        for (int u = 0; u < kVecsInFlight; ++u) {  // (every lane takes part in the shuffles)
+          const uint32_t i = v0 + u * kWave + lane;
+          uint32_t row = __umulhi(i, a.nvec_magic);
+          uint32_t vec = i - row * a.nvec;
+          if (vec >= a.nvec) {
+            ++row;
+            vec -= a.nvec;
+          }
+          const uint32_t off = vec * static_cast<uint32_t>(sizeof(VT));
+          char *const trow = reinterpret_cast<char *>(shfl64(my_table_row, row & (kWave - 1)));
+          on[u] = i < total && (!DEFER || trow);
+          at[u] = trow + off;
+          second[u] = nullptr;
+          if (THROUGH) {
+            char *const srow = reinterpret_cast<char *>(shfl64(my_second_row, row & (kWave - 1)));
+            second[u] = srow ? srow + off : nullptr;
+          }
+        }
+#pragma unroll
+        for (int u = 0; u < kVecsInFlight; ++u) {
+          if (!on[u]) continue;
+          if (SET)
+            v[u] = __builtin_nontemporal_load(reinterpret_cast<const VT *>(dense) + (v0 + u * kWave + lane));
+          else
+            v[u] = gload<VT>(at[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < kVecsInFlight; ++u) {
+          if (!on[u]) continue;
+          if (SET) {
+            gstore<VT>(at[u], v[u]);
+            if (THROUGH && second[u]) gstore<VT>(second[u], v[u]);
+          } else {
+            __builtin_nontemporal_store(v[u], reinterpret_cast<VT *>(dense) + (v0 + u * kWave + lane));
+          }
         }
       }
     }
@@ -514,15 +557,23 @@ static int move_rows(const char *who, void *miss, void *cache, const void *indic
   a.log2_lanes = log2_lanes;
   // Tile of 64 rows per wave when there are rows enough to occupy the chip
   // (256 CUs x 8 waves); fewer rows per wave otherwise, down to one phase-2 step.
+  // A lane group per row where the row fills it; a fetch of 16-byte vectors also where it fills three quarters
+  // (100 floats: 44.1 us, 45.8 with the vectors dealt out; with half of the lanes idle they are ahead).
+  const int64_t lanes = 1ll << log2_lanes;
+  const bool one_vec = nvec == lanes || (!SET && vb == 16 && nvec < lanes && 4 * nvec >= 3 * lanes);
+  a.nvec = nvec < (1ll << 26) ? static_cast<uint32_t>(nvec) : 0u;
+  a.nvec_magic = a.nvec ? 0xFFFFFFFFu / a.nvec : 0u;
   int log2_tile = kMaxLog2Tile;
-  while (log2_tile > 6 - log2_lanes && (Q >> log2_tile) < 2048) --log2_tile;
+  int log2_least = one_vec ? 6 - log2_lanes : 0;  // fewest rows per tile: a wave's worth of vectors
+  while (!one_vec && log2_least < kMaxLog2Tile && (nvec << log2_least) < kWave) ++log2_least;
+  while (log2_tile > log2_least && (Q >> log2_tile) < 2048) --log2_tile;
   if (miss_bits) log2_tile = 5;  // one bitmap word per tile
   a.log2_tile = log2_tile;
   // As many workgroups as the device holds at once (256 units x 8 waves per SIMD): beyond that a wave takes
   // several tiles and keeps the lookups of the next ones in flight while it moves rows.
-  const unsigned grid = grid_for(Q, static_cast<int64_t>(kRowsBlock / kWave) << log2_tile, 256 * 8);
+  const unsigned grid = grid_for(Q, static_cast<int64_t>(kRowsBlock / kWave) << log2_tile,
+                                 256 * rows_waves_per_simd(SET, one_vec, vb));
   hipStream_t s = as_stream(stream);
-  const bool one_vec = nvec <= (1ll << log2_lanes);
   if (miss_bits) {
     SHMT_REQUIRE(!SET && mode != kDirect, "%s: only a fetch through a hashmap or mask sets its misses aside", who);
     SHMT_REQUIRE(vb == 16, "%s: rows and tables must allow 16-byte accesses (row_bytes %lld)", who,

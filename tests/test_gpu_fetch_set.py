@@ -506,3 +506,41 @@ def test_fetch_and_set_through_tables_larger_than_the_caches(capi, layout):
     s = slot_of[uq]
     assert torch.equal(cache[s[s >= 0]], upd[s >= 0])
     assert torch.equal(table[uq[s < 0].cpu()], upd[s < 0].cpu())
+
+
+@pytest.mark.parametrize("dtype,D", [(torch.int8, d) for d in (1, 3, 7, 9, 31, 63, 65, 129, 1000)] +
+                         [(torch.float16, d) for d in (1, 33, 36, 75, 300)] +
+                         [(torch.float32, d) for d in (1, 2, 4, 33, 50, 72, 96, 100, 127, 260, 4100)] +
+                         [(torch.int64, d) for d in (1, 3, 25, 48, 130)])
+@pytest.mark.parametrize("layout", ["auto", "buckets"])
+def test_rows_that_fill_no_lane_group(capi, dtype, D, layout):
+    """Rows whose vectors are dealt to the lanes one by one (every vector width, rows shorter and longer than a wave,
+    tiles of 1 to 32 rows and a ragged last one, hits and misses): fetch, set and write-through give what
+    indexing gives, byte for byte, and touch nothing beside the rows."""
+    g = torch.Generator(device="cuda").manual_seed(D)
+    n = 3000
+    def rows(k):
+        return torch.randint(-100, 100, (k, D), device="cuda", generator=g).to(dtype)
+    full, hot = rows(n), torch.randperm(n, device="cuda", generator=g)[: n // 2]
+    host = torch.empty(n, D, dtype=dtype, pin_memory=True)
+    slots = torch.full((n,), -1, dtype=torch.int64, device="cuda")
+    slots[hot] = torch.arange(n // 2, device="cuda")
+    h = capi.CUCOStaticHashmap(hot, torch.arange(n // 2, device="cuda"), 0.8, layout=layout)
+    for q_len in (1, 2, 31, 33, 700, 70_001 if D < 1000 else 5001):
+        host.copy_(full)
+        cache = rows(n // 2)
+        q = torch.randint(0, n, (q_len,), device="cuda", generator=g)
+        s = slots[q]
+        want = torch.where((s >= 0)[:, None], cache[s.clamp(min=0)], full[q])
+        assert torch.equal(capi.cache_fetch(host, cache, q, h), want)
+        assert torch.equal(capi.uva_fetch(host, q), full[q])
+        w = torch.randperm(n, device="cuda", generator=g)[: min(q_len, n)]
+        upd, hit = rows(w.numel()), slots[w] >= 0
+        for through in (False, True):
+            host.copy_(full)
+            got, want_cache, want_host = cache.clone(), cache.clone(), full.clone()
+            capi.cache_set(host, got, w, upd, h, write_through=through)
+            torch.cuda.synchronize()
+            want_cache[slots[w][hit]] = upd[hit]
+            want_host[w if through else w[~hit]] = upd if through else upd[~hit]
+            assert torch.equal(got, want_cache) and torch.equal(host.cuda(), want_host)
