@@ -596,6 +596,22 @@ int shmt_subcsr_copy(const void *indptr, const void *indices, int ptr_bytes,
                      int idx_bytes, const void *seeds, int seed_bytes,
                      int64_t C, const void *cache_indptr, int64_t nnz,
                      void *cache_indices, void *stream);
+/* shmt_sample for row offsets in host memory: indptr has rows + 1 entries,
+ * which the call may copy to `stage` (device memory, 16-byte aligned, of
+ * shmt_sample_stage_bytes; that is 0 where so many seeds cannot pay for the
+ * copy) before the seeds' rows are looked up. Same results; stage NULL or
+ * too small: shmt_sample.                                                  */
+int64_t shmt_sample_stage_bytes(int64_t rows, int ptr_bytes, int64_t S);
+int shmt_sample_staged(const void *indptr, int ptr_bytes, int64_t rows,
+                       const void *indices, int idx_bytes,
+                       const void *cache_indptr, const void *cache_indices,
+                       const shmt_hashmap_t *map, const void *seeds,
+                       int seed_bytes, int64_t S, int64_t k, int replace,
+                       uint64_t rng_seed, uint32_t rng_stream,
+                       void *sub_indptr, void *sub_indices, void *plan,
+                       int64_t plan_bytes, void *stage, int64_t stage_bytes,
+                       int64_t *nnz_out, void *stream);
+
 /* The same, with the start of every chosen row in the source kept between
  * the two calls: row_begins has room for C int64 (device memory; NULL: as
  * above). The copy then reads no row offset over the host link.            */

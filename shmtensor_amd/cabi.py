@@ -63,6 +63,9 @@ SIGNATURES = {
                                 _c.c_uint64, _c.c_uint32, _vp]),
     "shmt_sample": (_int, [_vp, _int, _vp, _int, _vp, _vp, _vp, _vp, _int, _i64, _i64, _int, _c.c_uint64,
                            _c.c_uint32, _vp, _vp, _vp, _i64, _vp, _vp]),
+    "shmt_sample_stage_bytes": (_i64, [_i64, _int, _i64]),
+    "shmt_sample_staged": (_int, [_vp, _int, _i64, _vp, _int, _vp, _vp, _vp, _vp, _int, _i64, _i64, _int, _c.c_uint64, _c.c_uint32, _vp,
+                                  _vp, _vp, _i64, _vp, _i64, _vp, _vp]),
     "shmt_sample_hop": (_int, [_vp, _int, _vp, _int, _vp, _vp, _vp, _vp, _int, _i64, _i64, _int, _c.c_uint64,
                                _c.c_uint32, _vp, _vp, _vp, _i64, _int, _vp, _vp, _i64, _vp, _vp, _vp, _vp, _vp]),
     "shmt_sample_hop_chained": (_int, [_vp, _int, _vp, _int, _vp, _vp, _vp, _vp, _int, _i64, _vp, _i64, _int,

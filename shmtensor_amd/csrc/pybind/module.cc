@@ -275,11 +275,16 @@ std::tuple<torch::Tensor, torch::Tensor> sample_impl(const torch::Tensor &indptr
   torch::Tensor sub_indices;
   if (eager) {
     sub_indices = torch::empty({S * num_picks}, indices.options().device(dev));
-    check(shmt_sample(indptr_dev, pb, indices_dev, ib, map ? gpu_indptr->data_ptr() : nullptr,
-                      map ? gpu_indices->data_ptr() : nullptr, map ? map->handle() : nullptr, seeds.data_ptr(),
-                      sb, S, num_picks, replace, rng_seed, static_cast<uint32_t>(stream_id),
-                      sub_indptr.data_ptr(), sub_indices.data_ptr(), plan.data_ptr(), plan_bytes, total.dev,
-                      stream));
+    // many seeds on few rows of host memory: their offsets may be copied to the GPU first
+    const int64_t rows = indptr.numel() - 1;
+    const int64_t stage_bytes = indptr.is_cuda() || rows < 1 ? 0 : shmt_sample_stage_bytes(rows, pb, S);
+    torch::Tensor stage;
+    if (stage_bytes > 0) stage = device_bytes(stage_bytes);
+    check(shmt_sample_staged(indptr_dev, pb, rows, indices_dev, ib, map ? gpu_indptr->data_ptr() : nullptr,
+                             map ? gpu_indices->data_ptr() : nullptr, map ? map->handle() : nullptr, seeds.data_ptr(),
+                             sb, S, num_picks, replace, rng_seed, static_cast<uint32_t>(stream_id),
+                             sub_indptr.data_ptr(), sub_indices.data_ptr(), plan.data_ptr(), plan_bytes,
+                             stage_bytes > 0 ? stage.data_ptr() : nullptr, stage_bytes, total.dev, stream));
     const int64_t nnz = Readback::wait(total);
     // a view keeps the whole bound-sized buffer alive: hand back a copy when most of a large one is unused
     const bool mostly_unused = nnz < S * num_picks / 4 && S * num_picks * ib > (16ll << 20);

@@ -243,3 +243,37 @@ def test_config3_full_size_properties(capi):
         assert u.numel() == torch.unique(torch.cat([seeds, si.long()])).numel()
         seeds = u
     assert seeds.numel() > 100_000
+
+
+@pytest.mark.parametrize("ptr", [np.int32, np.int64])
+@pytest.mark.parametrize("rows,S,cached", [(40_000, 40_000, 0.0), (40_001, 9_000, 0.0), (3, 4_200, 0.0), (40_002, 40_000, 0.3),
+                                           (40_003, 40_000, 0.97), (40_003, 40_000, 1.0), (120_000, 4_000, 0.0)])
+def test_many_seeds_on_few_rows_of_host_memory(capi, ptr, rows, S, cached):
+    """Row offsets that are copied to the GPU before the plan (many cold seeds), that are not because hardly a seed is
+    cold, and that cannot pay (few seeds): all give what sampling the graph in device memory gives. The lengths
+    end 0, 4, 8 and 12 bytes into a 16-byte word."""
+    g = torch.Generator(device="cuda").manual_seed(rows + S)
+    deg = torch.randint(0, 40, (rows,), device="cuda", generator=g)
+    indptr = torch.zeros(rows + 1, dtype=torch.int64, device="cuda")
+    torch.cumsum(deg, 0, out=indptr[1:])
+    indices = torch.randint(0, rows, (int(indptr[-1]),), device="cuda", generator=g)
+    indptr = indptr.to(torch.int32 if ptr is np.int32 else torch.int64)
+    seeds = torch.randint(0, rows, (S,), device="cuda", generator=g)
+    want = capi.csr_sampling(indptr, indices, seeds, 5, False, seed=9)
+    hp, hi = indptr.cpu().pin_memory(), indices.cpu().pin_memory()
+    if cached == 0.0:
+        got = capi.csr_sampling(hp, hi, seeds, 5, False, seed=9)
+    else:
+        for hot in (torch.randperm(rows, device="cuda", generator=g)[: int(rows * cached)],
+                    torch.arange(int(rows * cached), device="cuda")):
+            sub = capi.create_subcsr(hp, hi, hot)
+            for layout in ("auto", "buckets"):
+                h = capi.CUCOStaticHashmap(hot, torch.arange(hot.numel(), device="cuda"), 0.8, layout=layout)
+                got = capi.csr_cache_sampling(hp, hi, sub[0], sub[1], h, seeds, 5, False, seed=9)
+                assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+    # offsets that start inside a 16-byte word are read where they are
+    shifted = torch.empty(rows + 2, dtype=indptr.dtype, pin_memory=True)
+    shifted[1:].copy_(indptr)
+    got = capi.csr_sampling(shifted[1:], hi, seeds, 5, False, seed=9)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
