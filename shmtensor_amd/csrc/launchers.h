@@ -25,8 +25,7 @@ enum StageKind : int {
   kStageRlSmall = 11,
   kStageRlInsert = 12,
   kStageRlFirst = 13,
-  kStageRlUnique = 14,
-  kStageRlLabels = 15,
+  kStageRlFinish = 14,
   kStageRpCount = 16,
   kStageRpRows = 17,
   kStageRpScatter = 18,
@@ -100,7 +99,7 @@ int launch_scan_partials(uint64_t *partials, int64_t nb, hipStream_t s);
 // Relabel as the tail of a fused launch sequence. relabel_table() names the
 // hash-table part of a relabel scratch buffer sized for N ids (n16 16-byte
 // words that must be all ones when the passes start); launch_relabel_passes()
-// runs insert -> first -> unique -> labels on `total`, which earlier kernels of
+// runs insert -> first -> finish on `total`, which earlier kernels of
 // the same stream have filled, for n_fixed + *n_extra_dev ids (at most n_bound;
 // with n_fixed_dev the first part is min(*n_fixed_dev, n_fixed), read on the
 // device); those kernels must also have stored `nonce` to *wide_mark if any id

@@ -7,13 +7,13 @@
 //   insert   per-workgroup de-duplication in LDS, then one global insert per
 //            distinct id of the tile (64-bit CAS on the key, atomicMin the index)
 //   first    first[i] = smallest index holding the same key (kept in the
-//            labels buffer); per-tile count of i with first[i] == i
+//            labels buffer); per 64 elements a bitmap of the first occurrences
+//            among them and their number before them within the tile
+//            (RlRanks); per tile their number
 //   partials exclusive scan of the per-tile counts (own launch only beyond 2 M ids)
-//   unique   rank of every first occurrence; unique[rank] = key; per 64
-//            elements a bitmap of the first occurrences among them and the
-//            number of first occurrences before them (RlRanks)
-//   labels   labels[i] = rank of element first[i], from that bitmap
-// The table is touched only by `insert` and `first`; the last two passes read
+//   finish   labels[i] = rank of element first[i], from that bitmap and the sum
+//            of the counts of the tiles before it; unique[rank] = key
+// The table is touched only by `insert` and `first`; the last pass reads
 // dense arrays. Slots are 16 bytes {int64 key, uint32 first, pad} at load
 // factor <= 0.5 with a mixed hash (the reference hashes with the low bits of
 // the id, src/tensor_relabel.cu:111-117); ids known to fit 32 bits use the
@@ -32,9 +32,9 @@
 namespace shmt {
 
 constexpr int kRlBlock = 256;
-constexpr int kRlItems = 2;
-constexpr int kRlTile = kRlBlock * kRlItems;
-constexpr int64_t kRlSelfPrefixTiles = 4096;  // up to 2 M ids the unique pass sums the tile counts itself
+constexpr int kRlTileLog2 = 9;
+constexpr int kRlTile = 1 << kRlTileLog2;
+constexpr int64_t kRlSelfPrefixTiles = 4096;  // up to 2 M ids the finish pass sums the tile counts itself
 
 // Number of input ids: a host-known part plus, optionally, a part that only
 // the device knows (the length of the last segment, e.g. the nnz a sampling
@@ -278,8 +278,8 @@ __global__ __launch_bounds__(kRlBlock) void rl_insert_jobs(Jobs<RlInsertArgs> j)
 }
 
 // First-occurrence index of every element: one id per thread, a workgroup of
-// kRlTile threads per tile (the tile whose count of first occurrences the
-// unique pass ranks). One id per thread keeps every value in registers and
+// kRlTile threads per tile (the tile within which first occurrences are
+// ranked here). One id per thread keeps every value in registers and
 // every probe chain in its own lane; with several ids per thread the chains of
 // a lane ran one after the other and a small input ran on a handful of
 // workgroups.
@@ -309,6 +309,20 @@ __device__ __forceinline__ uint32_t rl_first_of(const RlSlot *tbl, uint32_t cap,
   return 0xFFFFFFFFu;
 }
 
+// Ranks of the first occurrences, 16 bytes per 64 consecutive elements: bit b of `firsts` says that
+// element 64 w + b is the first occurrence of its id, `before` is the number of first occurrences in
+// front of element 64 w in its tile (kRlTile elements, or kRpTile where the partition passes work). The
+// rank of a first occurrence f is the sum of the counts of the tiles before + before + popcount(firsts below bit f & 63):
+// one 16-byte load from an array of N / 4 bytes, which stays in the L2s where an array of one rank per
+// element (4 N bytes, read at random positions by the finish pass) did not.
+struct RlRanks {
+  uint64_t firsts;
+  uint32_t before;
+  uint32_t pad;
+};
+static_assert(sizeof(RlRanks) == 16, "one 16-byte load per lookup");
+static_assert(kRlTile % kWave == 0, "a wave ranks whole 64-element words");
+
 struct RlFirstArgs {
   const RlSlot *tbl;
   uint32_t cap;
@@ -318,6 +332,7 @@ struct RlFirstArgs {
   void *labels;
   uint64_t *partials;
   RlPath path;
+  RlRanks *ranks;
 };
 
 __device__ __forceinline__ void rl_first_body(unsigned bx, const RlFirstArgs &a) {
@@ -334,7 +349,9 @@ __device__ __forceinline__ void rl_first_body(unsigned bx, const RlFirstArgs &a)
     cnt = (f == static_cast<uint32_t>(i));
   }
   uint64_t tile_total;
-  block_exclusive_scan<uint64_t, kRlTile>(cnt, lds, &tile_total);
+  const uint64_t before = block_exclusive_scan<uint64_t, kRlTile>(cnt, lds, &tile_total);
+  const uint64_t firsts = __builtin_amdgcn_ballot_w64(cnt != 0);
+  if (lane_id() == 0 && i < N) a.ranks[i / kWave] = RlRanks{firsts, static_cast<uint32_t>(before), 0u};
   if (threadIdx.x == 0) a.partials[bx] = tile_total;
 }
 
@@ -344,147 +361,83 @@ __global__ __launch_bounds__(kRlTile) void rl_first_jobs(Jobs<RlFirstArgs> j) {
   if (blockIdx.x < j.blocks[blockIdx.y]) rl_first_body(blockIdx.x, j.a[blockIdx.y]);
 }
 
-// Ranks of the first occurrences, 16 bytes per 64 consecutive elements: bit b of `firsts` says that
-// element 64 w + b is the first occurrence of its id, `before` is the number of first occurrences in
-// front of element 64 w. The rank of a first occurrence f is before + popcount(firsts below bit f & 63):
-// one 16-byte load from an array of N / 4 bytes, which stays in the L2s where an array of one rank per
-// element (4 N bytes, read at random positions by the labels pass) did not.
-struct RlRanks {
-  uint64_t firsts;
-  uint32_t before;
-  uint32_t pad;
-};
-static_assert(sizeof(RlRanks) == 16, "one 16-byte load per lookup");
-static_assert(kRlTile % kWave == 0 && kRlItems * kWave * (kRlBlock / kWave) == kRlTile, "a wave ranks whole 64-element words");
-
-struct RlUniqueArgs {
+struct RlFinishArgs {
   const void *total;
   int eb;
   RlCount n;
   const void *first;  // first-occurrence index of every element, fb bytes wide (the labels buffer, or an array of its own)
   int fb;
-  const uint64_t *partials;
+  const RlRanks *ranks;
+  const void *counts;  // first occurrences per tile, cb bytes wide; scanned: 8 bytes, those of the tiles before
+  int cb;
+  int log2_tile;       // elements per tile
+  int scanned;
   void *unique_out;
-  RlRanks *ranks;
+  void *labels;
   int64_t *count_out;
   int64_t *count_copy;
-  int scanned;             // 0: partials are raw tile counts, 1: scanned, 2: raw, with the sums of whole groups in `coarse`
-  const uint32_t *coarse;  // scanned == 2: coarse[g] = sum of the counts of tiles [g * group, (g + 1) * group)
-  int group;
 };
 
-__device__ __forceinline__ void rl_unique_body(unsigned bx, const RlUniqueArgs &a) {
-  const void *const total = a.total;
-  const int eb = a.eb;
-  const void *const labels = a.first;
-  const uint64_t *const partials = a.partials;
-  void *const unique_out = a.unique_out;
+// Every workgroup sums the tile counts for itself, in LDS (up to kRlSelfPrefixTiles of them, a fraction of the
+// N / 512 that a launch of its own would read), and then both lists the distinct ids and labels the elements:
+// what the ranks need of other workgroups is known before this pass starts. Bound by
+// random 16-byte reads of the ranks (in the L2s). 3.1 M ids: 15.3 us, where a launch that listed the distinct ids (12.1) and one
+// that labelled the elements (11.6) went before; 145,000 ids: 5.5 against 5.0 + 4.2.
+constexpr int kRlFinishBlocks = 2048;
+
+__device__ __forceinline__ void rl_finish_body(unsigned bx, unsigned gx, const RlFinishArgs &a) {
+  __shared__ uint32_t prefix[kRlSelfPrefixTiles];
+  __shared__ uint32_t lds[kRlBlock / kWave];
   const int64_t N = rl_count(a.n);
-  // launched for a bound of N: only the tiles that hold ids work (tile 0 reports N = 0)
-  if (bx > 0 && static_cast<int64_t>(bx) * kRlTile >= N) return;
-  __shared__ uint32_t wave_firsts[kRlBlock / kWave];
-  __shared__ uint64_t lds64[kRlBlock / kWave];
-  // Tile prefix: either already scanned by a separate launch, or (few tiles)
-  // summed here from the raw per-tile counts.
-  uint64_t tile_prefix;
-  if (a.scanned == 1) {
-    tile_prefix = partials[bx];
-  } else {
-    uint64_t part = 0;
-    int from = 0;
-    if (a.scanned == 2) {
-      const int groups = static_cast<int>(bx) / a.group;
-      for (int t = threadIdx.x; t < groups; t += kRlBlock) part += a.coarse[t];
-      from = groups * a.group;
+  // launched for a bound of N: only workgroups that have elements work (the first one reports N = 0)
+  if (bx > 0 && static_cast<int64_t>(bx) * kRlBlock >= N) return;
+  if (!a.scanned) {
+    const int tiles = static_cast<int>((N + (1ll << a.log2_tile) - 1) >> a.log2_tile);
+    const int per = (tiles + kRlBlock - 1) / kRlBlock;
+    const int t0 = static_cast<int>(threadIdx.x) * per, t1 = t0 + per < tiles ? t0 + per : tiles;
+    uint32_t sum = 0, all;
+    for (int t = t0; t < t1; ++t) sum += static_cast<uint32_t>(load_int(a.counts, t, a.cb));
+    uint32_t run = block_exclusive_scan<uint32_t, kRlBlock>(sum, lds, &all);
+    for (int t = t0; t < t1; ++t) {
+      prefix[t] = run;
+      run += static_cast<uint32_t>(load_int(a.counts, t, a.cb));
     }
-    for (int t = from + threadIdx.x; t < static_cast<int>(bx); t += kRlBlock) part += partials[t];
-    uint64_t below;
-    block_exclusive_scan<uint64_t, kRlBlock>(part, lds64, &below);
-    tile_prefix = below;
+    __syncthreads();
   }
-  // a wave takes kRlItems words of 64 consecutive elements: element = word start + lane
-  const int lane = lane_id(), wave = threadIdx.x / kWave;
-  const int64_t wave_first = static_cast<int64_t>(bx) * kRlTile + static_cast<int64_t>(wave) * (kRlItems * kWave);
-  bool win[kRlItems], ok[kRlItems];
-  int64_t idx[kRlItems], lab[kRlItems], val[kRlItems];
-#pragma unroll
-  for (int j = 0; j < kRlItems; ++j) {
-    idx[j] = wave_first + j * kWave + lane;
-    ok[j] = idx[j] < N;
-    lab[j] = -1;
-    val[j] = 0;
+  auto tiles_before = [&](int64_t i) -> uint32_t {
+    const int64_t tile = i >> a.log2_tile;
+    return a.scanned ? static_cast<uint32_t>(static_cast<const uint64_t *>(a.counts)[tile]) : prefix[tile];
+  };
+  if (bx == 0 && threadIdx.x == 0) {
+    int64_t count = 0;
+    if (N > 0) {
+      const RlRanks last = a.ranks[(N - 1) >> 6];
+      count = static_cast<int64_t>(tiles_before(N - 1)) + last.before + __builtin_popcountll(last.firsts);
+    }
+    if (a.count_copy) *a.count_copy = count;
+    publish_size(a.count_out, count);
   }
-  load_ints<kRlItems>(labels, idx, ok, a.fb, lab);
-  uint64_t firsts[kRlItems];
-  uint32_t mine = 0;  // first occurrences of this wave
-#pragma unroll
-  for (int j = 0; j < kRlItems; ++j) {
-    win[j] = ok[j] && lab[j] == idx[j];
-    firsts[j] = __builtin_amdgcn_ballot_w64(win[j]);
-    mine += static_cast<uint32_t>(__builtin_popcountll(firsts[j]));
-  }
-  load_ints<kRlItems>(total, idx, win, eb, val);
-  if (lane == 0) wave_firsts[wave] = mine;
-  __syncthreads();
-  uint32_t before_wave = 0, tile_total = 0;
-#pragma unroll
-  for (int w = 0; w < kRlBlock / kWave; ++w) {
-    const uint32_t c = wave_firsts[w];
-    if (w < wave) before_wave += c;
-    tile_total += c;
-  }
-  uint64_t word_rank = tile_prefix + before_wave;  // rank of the first first-occurrence of the word
-  const uint64_t below_lane = (1ull << lane) - 1ull;
-#pragma unroll
-  for (int j = 0; j < kRlItems; ++j) {
-    if (win[j])
-      store_int(unique_out, static_cast<int64_t>(word_rank + __builtin_popcountll(firsts[j] & below_lane)), eb, val[j]);
-    const int64_t word_start = wave_first + j * kWave;
-    if (lane == 0 && word_start < N) a.ranks[word_start / kWave] = RlRanks{firsts[j], static_cast<uint32_t>(word_rank), 0u};
-    word_rank += static_cast<uint64_t>(__builtin_popcountll(firsts[j]));
-  }
-  // the workgroup holding the last id reports the number of distinct ids
-  const int64_t last_tile = N > 0 ? (N - 1) / kRlTile : 0;
-  if (static_cast<int64_t>(bx) == last_tile && threadIdx.x == 0) {
-    if (a.count_copy) *a.count_copy = static_cast<int64_t>(tile_prefix + tile_total);
-    publish_size(a.count_out, static_cast<int64_t>(tile_prefix + tile_total));
-  }
-}
-
-__global__ __launch_bounds__(kRlBlock) void rl_unique_kernel(RlUniqueArgs a) { rl_unique_body(blockIdx.x, a); }
-
-__global__ __launch_bounds__(kRlBlock) void rl_unique_jobs(Jobs<RlUniqueArgs> j) {
-  if (blockIdx.x < j.blocks[blockIdx.y]) rl_unique_body(blockIdx.x, j.a[blockIdx.y]);
-}
-
-struct RlLabelsArgs {
-  void *labels;
-  int eb;
-  RlCount n;
-  const RlRanks *ranks;
-  const void *first;  // see RlUniqueArgs
-  int fb;
-};
-
-__device__ __forceinline__ void rl_labels_body(unsigned bx, unsigned gx, const RlLabelsArgs &a) {
-  const int64_t N = rl_count(a.n);
-  int64_t i = static_cast<int64_t>(bx) * blockDim.x + threadIdx.x;
-  const int64_t stride = static_cast<int64_t>(gx) * blockDim.x;
-  for (; i < N; i += stride) {
+  const int64_t stride = static_cast<int64_t>(gx) * kRlBlock;
+  for (int64_t i = static_cast<int64_t>(bx) * kRlBlock + threadIdx.x; i < N; i += stride) {
     const int64_t f = load_int(a.first, i, a.fb);
     const uint4 r = *reinterpret_cast<const uint4 *>(&a.ranks[f >> 6]);
+    const bool win = f == i;
+    int64_t id = 0;
+    if (win) id = load_int(a.total, i, a.eb);
     const uint64_t firsts = (static_cast<uint64_t>(r.y) << 32) | r.x;
-    const uint32_t rank = r.z + static_cast<uint32_t>(__builtin_popcountll(firsts & ((1ull << (f & 63)) - 1ull)));
-    store_int(a.labels, i, a.eb, static_cast<int64_t>(rank));
+    const int64_t rank = static_cast<int64_t>(
+        tiles_before(f) + r.z + static_cast<uint32_t>(__builtin_popcountll(firsts & ((1ull << (f & 63)) - 1ull))));
+    store_int(a.labels, i, a.eb, rank);
+    if (win) store_int(a.unique_out, rank, a.eb, id);
   }
 }
 
-__global__ __launch_bounds__(256) void rl_labels_kernel(RlLabelsArgs a) {
-  rl_labels_body(blockIdx.x, gridDim.x, a);
+__global__ __launch_bounds__(kRlBlock) void rl_finish_kernel(RlFinishArgs a) {
+  rl_finish_body(blockIdx.x, gridDim.x, a);
 }
 
-__global__ __launch_bounds__(256) void rl_labels_jobs(Jobs<RlLabelsArgs> j) {
-  if (blockIdx.x < j.blocks[blockIdx.y]) rl_labels_body(blockIdx.x, j.blocks[blockIdx.y], j.a[blockIdx.y]);
+__global__ __launch_bounds__(kRlBlock) void rl_finish_jobs(Jobs<RlFinishArgs> j) {
+  if (blockIdx.x < j.blocks[blockIdx.y]) rl_finish_body(blockIdx.x, j.blocks[blockIdx.y], j.a[blockIdx.y]);
 }
 
 struct RlSegments {
@@ -695,8 +648,8 @@ __global__ void rl_zero_count_kernel(int64_t *count_out, int64_t *count_copy) {
 // 50 G per second whatever the kernel does (3.1 M ids: 74 + 54 us, plus 22 us to
 // empty the table). From a million ids on (kRpExactMin; kRpDefaultMin for a
 // hop sized by a loose bound, kRpMergedMin for hops that share their launches)
-// the same two results -- the first-occurrence index of every element and the
-// number of first occurrences per tile of kRlTile ids -- come from five passes
+// the same results -- the first-occurrence index of every element, the ranks of
+// the first occurrences and their number per tile of kRpTile ids -- come from five passes
 // that read and write memory in runs instead:
 //   count    a workgroup per tile of kRpTile ids: histogram of the ids over P
 //            bins (bin = top bits of the id's hash), one column of the P x W
@@ -728,7 +681,8 @@ constexpr int kRpBlock = 1024;
 constexpr int kRpSlotsLog2 = 14;     // 16,384 slots of 4 + 4 bytes = 128 KB of LDS
 constexpr int kRpMinBinsLog2 = 8, kRpMaxBinsLog2 = 9;
 constexpr int64_t kRpBinIds = 14336; // ids per bin from which on the number of bins grows: 7/8 of the largest table
-constexpr int64_t kRpTile = 8192;    // ids per tile of the count / scatter / gather passes
+constexpr int kRpTileLog2 = 13;
+constexpr int64_t kRpTile = 1 << kRpTileLog2;  // ids per tile of the count / scatter / gather passes
 constexpr int kRpMaxRoundsLog2 = 10;
 constexpr int64_t kRpDefaultMin = kRlSelfPrefixTiles * kRlTile + 1;
 // Hops that share their launches with those of other batches (launchers.h) are sized for a bound of their
@@ -797,12 +751,12 @@ struct RpArgs {
   int log2P;
   uint32_t W;
   void *rec;
-  uint32_t *first;   // first-occurrence index of every element (what the unique and labels passes read)
+  uint32_t *first;   // first-occurrence index of every element (what the finish pass reads)
   uint32_t *firstp;  // the same per record, in the records' order
   uint32_t *hist, *bintot, *binstart, *coarse;
   uint16_t *local;  // position of every element's record among its tile's records in bin order
   uint32_t *tile_runs;  // per tile: where its run of every bin starts in memory (P words), then among its records (P + 1 words)
-  uint64_t *partials;
+  RlRanks *ranks;
   int slots_log2, max_rounds_log2;
 };
 
@@ -1371,7 +1325,7 @@ __global__ __launch_bounds__(rp_bins_threads(TABLE_LOG2)) void rp_bins_jobs(Jobs
 __device__ __forceinline__ void rp_gather_body(unsigned bx, const RpArgs &a) {
   extern __shared__ uint32_t words[];  // run start in memory (P), start among the tile's records (P + 1)
   __shared__ uint32_t result[kRpTile];
-  __shared__ uint32_t firsts[kRpTile / kRlTile];
+  __shared__ uint32_t before[kRpTile / kWave];  // first occurrences per 64 elements, then in front of them
   const int64_t N = rl_count(a.n);
   const int64_t lo = static_cast<int64_t>(bx) * kRpTile;
   if (lo >= N) return;
@@ -1379,8 +1333,6 @@ __device__ __forceinline__ void rp_gather_body(unsigned bx, const RpArgs &a) {
   const uint32_t P = 1u << a.log2P;
   const uint32_t *const runs = a.tile_runs + static_cast<size_t>(bx) * (2 * P + 1);
   for (uint32_t t = threadIdx.x; t < 2 * P + 1; t += kRpBlock) words[t] = runs[t];
-  const int sub_tiles = static_cast<int>(kRpTile / kRlTile);
-  for (int t = threadIdx.x; t < sub_tiles; t += kRpBlock) firsts[t] = 0;
   __syncthreads();
   const uint32_t *const run_at = words, *const lstart = words + P;
   const uint32_t records = lstart[P];
@@ -1392,6 +1344,8 @@ __device__ __forceinline__ void rp_gather_body(unsigned bx, const RpArgs &a) {
     result[q] = a.firstp[run_at[bin] + (q - lstart[bin])];
   }
   __syncthreads();
+  const int wave = threadIdx.x / kWave;
+  uint64_t wins[kRpItems];
   uint16_t at[kRpItems];
 #pragma unroll
   for (int j = 0; j < kRpItems; ++j) {
@@ -1403,23 +1357,24 @@ __device__ __forceinline__ void rp_gather_body(unsigned bx, const RpArgs &a) {
     const int64_t i = lo + j * kRpBlock + threadIdx.x;
     const uint32_t f = i < hi ? result[at[j]] : 0xFFFFFFFFu;
     if (i < hi) a.first[i] = f;
-    // a wave's 64 elements lie in one tile of kRlTile ids
-    const uint64_t wins = __builtin_amdgcn_ballot_w64(i < hi && f == static_cast<uint32_t>(i));
-    if (lane_id() == 0 && wins)
-      atomicAdd(&firsts[(i - lo) / kRlTile], static_cast<uint32_t>(__builtin_popcountll(wins)));
+    wins[j] = __builtin_amdgcn_ballot_w64(i < hi && f == static_cast<uint32_t>(i));
+    if (lane_id() == 0) before[j * (kRpBlock / kWave) + wave] = static_cast<uint32_t>(__builtin_popcountll(wins[j]));
   }
   __syncthreads();
-  uint32_t all = 0;
-  for (int t = threadIdx.x; t < sub_tiles; t += kRpBlock) {
-    const int64_t tile = lo / kRlTile + t;
-    if (tile * kRlTile < N) a.partials[tile] = firsts[t];
-    all += firsts[t];
-  }
-  // (one wave covers all sub-tiles) the tile's own total, so that the unique pass needs no scan of the counts
-  static_assert(kRpTile / kRlTile <= kWave, "the first wave sums a tile's counts");
+  // (the first wave) two neighbouring words per lane; the tile's total goes to the finish pass
+  static_assert(kRpTile / kWave == 2 * kWave, "the first wave scans a tile's counts");
   if (threadIdx.x < kWave) {
-    all = wave_last(wave_inclusive_scan(all));
-    if (threadIdx.x == 0) a.coarse[bx] = all;
+    const uint32_t c0 = before[2 * threadIdx.x], c1 = before[2 * threadIdx.x + 1];
+    const uint32_t inc = wave_inclusive_scan(c0 + c1);
+    before[2 * threadIdx.x] = inc - c0 - c1;
+    before[2 * threadIdx.x + 1] = inc - c1;
+    if (threadIdx.x == kWave - 1) a.coarse[bx] = inc;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < kRpItems; ++j) {
+    const int word = j * (kRpBlock / kWave) + wave;
+    if (lane_id() == 0 && lo + word * kWave < N) a.ranks[lo / kWave + word] = RlRanks{wins[j], before[word], 0u};
   }
 }
 
@@ -1688,6 +1643,7 @@ static int relabel_impl(const void *total, const RlSegments *segs, int64_t N, Rl
 
   int rc = SHMT_OK;
   const int scanned = nb > kRlSelfPrefixTiles;
+  const unsigned fin_blocks = grid_for(N, kRlBlock, kRlFinishBlocks);
   // a job among fewer merged ones than the partition passes pay for keeps the table (and stays mergeable)
   const RpPlan rp = rp_plan(N, defer ? (prepared ? defer->jobs : 1) : 0, n.fixed_dev != nullptr);
   if (!rp.ok && defer && rp_plan(N, 0, n.fixed_dev != nullptr).ok) {
@@ -1704,18 +1660,16 @@ static int relabel_impl(const void *total, const RlSegments *segs, int64_t N, Rl
              reinterpret_cast<uint32_t *>(base + rp.hist_off), reinterpret_cast<uint32_t *>(base + rp.bintot_off),
              reinterpret_cast<uint32_t *>(base + rp.binstart_off), reinterpret_cast<uint32_t *>(base + rp.coarse_off),
              reinterpret_cast<uint16_t *>(base + rp.local_off), reinterpret_cast<uint32_t *>(base + rp.tile_off),
-             partials, slots_log2, g_rp_tuning.max_rounds_log2};
-    const RlUniqueArgs unq{total, elem_bytes, n, a.first, 4, partials, unique_out, ranks, count_out, count_copy,
-                           2, a.coarse, static_cast<int>(kRpTile / kRlTile)};
-    const RlLabelsArgs lab{labels_out, elem_bytes, n, ranks, a.first, 4};
+             ranks, slots_log2, g_rp_tuning.max_rounds_log2};
+    const RlFinishArgs fin{total, elem_bytes, n, a.first, 4, ranks, a.coarse, 4, kRpTileLog2, 0, unique_out, labels_out,
+                           count_out, count_copy};
     if (defer) {
       stage_push(defer, kStageRpCount, rp.W, kRpBlock, a);
       stage_push(defer, kStageRpRows, (rp.P + 3) / 4, 256, a);
       stage_push(defer, kStageRpScatter, rp.W, kRpBlock, a);
       stage_push(defer, kStageRpBins + (kRpSlotsLog2 - rp.table_log2), rp.P, rp_bins_threads(rp.table_log2), a);
       stage_push(defer, kStageRpGather, rp.W, kRpBlock, a);
-      stage_push(defer, kStageRlUnique, static_cast<unsigned>(nb), kRlBlock, unq);
-      stage_push(defer, kStageRlLabels, grid_for(N, 256), 256, lab);
+      stage_push(defer, kStageRlFinish, fin_blocks, kRlBlock, fin);
       return SHMT_OK;
     }
     if (segs && !prepared)  // the count pass concatenates on the way: there is no table to empty
@@ -1736,22 +1690,19 @@ static int relabel_impl(const void *total, const RlSegments *segs, int64_t N, Rl
     SHMT_LAUNCH_CHECK();
     hipLaunchKernelGGL(rp_gather_kernel, dim3(rp.W), dim3(kRpBlock), (2 * rp.P + 1) * sizeof(uint32_t), s, a);
     SHMT_LAUNCH_CHECK();
-    hipLaunchKernelGGL(rl_unique_kernel, dim3(static_cast<unsigned>(nb)), dim3(kRlBlock), 0, s, unq);
-    SHMT_LAUNCH_CHECK();
-    hipLaunchKernelGGL(rl_labels_kernel, dim3(grid_for(N, 256)), dim3(256), 0, s, lab);
+    hipLaunchKernelGGL(rl_finish_kernel, dim3(fin_blocks), dim3(kRlBlock), 0, s, fin);
     SHMT_LAUNCH_CHECK();
     return SHMT_OK;
   }
   const RlInsertArgs ins{tbl, cap, total, elem_bytes, n, path};
-  const RlFirstArgs fst{tbl, cap, total, elem_bytes, n, labels_out, partials, path};
-  const RlUniqueArgs unq{total, elem_bytes, n, labels_out, elem_bytes, partials, unique_out, ranks, count_out,
-                         count_copy, scanned, nullptr, 1};
-  const RlLabelsArgs lab{labels_out, elem_bytes, n, ranks, labels_out, elem_bytes};
+  const RlFirstArgs fst{tbl, cap, total, elem_bytes, n, labels_out, partials, path, ranks};
+  const RlFinishArgs fin{total, elem_bytes, n, labels_out, elem_bytes, ranks, partials, 8, kRlTileLog2, scanned,
+                         unique_out, labels_out, count_out, count_copy};
   // At most 1,024 workgroups insert, each walking its tiles in turn: random global atomics run at 20-26 G/s on
   // this part whatever the grid (a third of the rate of plain stores), and a workgroup's later tiles then find
   // the ids of hub nodes already in the table with a smaller index and skip their atomics, where 8,192
   // workgroups starting together all miss them (8 batches per launch: 64.5 -> 62.3 us per batch).
-  const unsigned ins_blocks = grid_for(N, kRlInsertTile, 1024), lab_blocks = grid_for(N, 256);
+  const unsigned ins_blocks = grid_for(N, kRlInsertTile, 1024);
   if (defer) {
     if (!prepared || scanned) {
       defer->mergeable = false;
@@ -1759,8 +1710,7 @@ static int relabel_impl(const void *total, const RlSegments *segs, int64_t N, Rl
     }
     stage_push(defer, kStageRlInsert, ins_blocks, kRlBlock, ins);
     stage_push(defer, kStageRlFirst, static_cast<unsigned>(nb), kRlTile, fst);
-    stage_push(defer, kStageRlUnique, static_cast<unsigned>(nb), kRlBlock, unq);
-    stage_push(defer, kStageRlLabels, lab_blocks, 256, lab);
+    stage_push(defer, kStageRlFinish, fin_blocks, kRlBlock, fin);
     return SHMT_OK;
   }
   if (prepared) {
@@ -1783,9 +1733,7 @@ static int relabel_impl(const void *total, const RlSegments *segs, int64_t N, Rl
     rc = launch_scan_partials(partials, nb, s);
     if (rc) return rc;
   }
-  hipLaunchKernelGGL(rl_unique_kernel, dim3(static_cast<unsigned>(nb)), dim3(kRlBlock), 0, s, unq);
-  SHMT_LAUNCH_CHECK();
-  hipLaunchKernelGGL(rl_labels_kernel, dim3(lab_blocks), dim3(256), 0, s, lab);
+  hipLaunchKernelGGL(rl_finish_kernel, dim3(fin_blocks), dim3(kRlBlock), 0, s, fin);
   SHMT_LAUNCH_CHECK();
   return SHMT_OK;
 }
@@ -1847,16 +1795,10 @@ int launch_merged_relabel_stage(int n_jobs, const Stage *const *stages, hipStrea
       hipLaunchKernelGGL(rl_first_jobs, dim3(blocks, n_jobs), dim3(threads), 0, s, j);
       break;
     }
-    case kStageRlUnique: {
-      Jobs<RlUniqueArgs> j;
+    case kStageRlFinish: {
+      Jobs<RlFinishArgs> j;
       const unsigned blocks = jobs_from_stages(n_jobs, stages, &j);
-      hipLaunchKernelGGL(rl_unique_jobs, dim3(blocks, n_jobs), dim3(threads), 0, s, j);
-      break;
-    }
-    case kStageRlLabels: {
-      Jobs<RlLabelsArgs> j;
-      const unsigned blocks = jobs_from_stages(n_jobs, stages, &j);
-      hipLaunchKernelGGL(rl_labels_jobs, dim3(blocks, n_jobs), dim3(threads), 0, s, j);
+      hipLaunchKernelGGL(rl_finish_jobs, dim3(blocks, n_jobs), dim3(threads), 0, s, j);
       break;
     }
     case kStageRpCount:
