@@ -13,6 +13,7 @@ it is the DGLBlock the reference builds from either form
 (python/shmtensor/sampling.py:9-27)."""
 import collections
 import queue
+import sys
 import threading
 import weakref
 
@@ -29,11 +30,23 @@ CSCBlock = collections.namedtuple("CSCBlock", ["indptr", "indices", "num_src", "
 COOBlock = collections.namedtuple("COOBlock", ["row", "col", "num_src", "num_dst"])
 
 
-def _dgl():
+_dgl_missing = False
+
+
+def _dgl(look_again=False):
+    """The dgl module, or None. Python does not remember an import that failed: it searches the whole path anew,
+    20 to 50 us every time, which was half of the time of a prefetched epoch when every block of every batch
+    tried. A failure is kept here until the next loader is built (look_again); a dgl that anyone has
+    imported since is seen at once."""
+    global _dgl_missing
+    found = sys.modules.get("dgl")
+    if found is not None or (_dgl_missing and not look_again):
+        return found
     try:
-        import dgl  # noqa: F401
+        import dgl
         return dgl
     except Exception:
+        _dgl_missing = True
         return None
 
 
@@ -107,6 +120,7 @@ class GPUSamplingDataloader:
         if block_format not in ("csc", "coo"):
             raise ValueError("block_format must be 'csc' or 'coo'")
         self.block_format = block_format
+        _dgl(look_again=True)
 
         self.has_cache = False
         self.gpu_indptr = None
