@@ -557,15 +557,16 @@ static int move_rows(const char *who, void *miss, void *cache, const void *indic
   a.log2_lanes = log2_lanes;
   // Tile of 64 rows per wave when there are rows enough to occupy the chip
   // (256 CUs x 8 waves); fewer rows per wave otherwise, down to one phase-2 step.
-  // A lane group per row where the row fills it; a fetch of 16-byte vectors also where it fills three quarters
-  // (100 floats: 44.1 us, 45.8 with the vectors dealt out; with half of the lanes idle they are ahead).
+  // A lane group per row where the row fills it. A fetch of 16-byte vectors also where it fills three quarters of
+  // 8, 16 or 32 lanes: 262,144 rows of 100 floats 44.4 us, 45.7 with the vectors dealt out, 112 floats 45.0 / 45.7;
+  // but with 64 lanes 200 floats 92.0 / 81.4, 208 floats 82.6 / 81.0, 240 floats 97.2 / 95.5.
   const int64_t lanes = 1ll << log2_lanes;
-  const bool one_vec = nvec == lanes || (!SET && vb == 16 && nvec < lanes && 4 * nvec >= 3 * lanes);
+  const bool one_vec = nvec == lanes || (!SET && vb == 16 && lanes < kWave && nvec < lanes && 4 * nvec >= 3 * lanes);
   a.nvec = nvec < (1ll << 26) ? static_cast<uint32_t>(nvec) : 0u;
   a.nvec_magic = a.nvec ? 0xFFFFFFFFu / a.nvec : 0u;
   int log2_tile = kMaxLog2Tile;
-  int log2_least = one_vec ? 6 - log2_lanes : 0;  // fewest rows per tile: a wave's worth of vectors
-  while (!one_vec && log2_least < kMaxLog2Tile && (nvec << log2_least) < kWave) ++log2_least;
+  int log2_least = one_vec ? 6 - log2_lanes : 0;  // fewest rows per tile: a wave's worth of vectors, or eight
+  while (!one_vec && log2_least < 3 && (nvec << log2_least) < kWave) ++log2_least;
   while (log2_tile > log2_least && (Q >> log2_tile) < 2048) --log2_tile;
   if (miss_bits) log2_tile = 5;  // one bitmap word per tile
   a.log2_tile = log2_tile;
