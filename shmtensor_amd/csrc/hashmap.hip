@@ -167,7 +167,7 @@ __global__ __launch_bounds__(256) void hashmap_insert_kernel(
 //          pairs of one key) or in the last buckets of the partition: inserted
 //          one by one, as the general build does for all. Hardly ever any.
 // 4,194,304 pairs of 16 bytes: clear 23 + insert 212 us before (16-byte slots; 13 + 191 with packed words), deal 33 +
-// fill 40 + rest 11 us now. Deal reads 67 MB and writes 34, fill reads 34 and writes 67: 3 TB/s and 2.5 TB/s, with
+// fill 37 + rest 5 us now. Deal reads 67 MB and writes 34, fill reads 34 and writes 67: 3 TB/s and 2.7 TB/s, with
 // one and two workgroups per compute unit whose phases (load, count, order, write) hardly overlap.
 // A bucket is filled in any slot order and a key goes to the first bucket of
 // its probe sequence that has room, so lookups and `rest` see an ordinary table.
@@ -262,19 +262,23 @@ __global__ __launch_bounds__(kPartBlock) void part_fill_kernel(PartArgs a) {
   const uint32_t bucket0 = p << kPartLog2Buckets;
   const uint32_t nb = a.map.nbuckets - bucket0 < kPartBuckets ? a.map.nbuckets - bucket0 : kPartBuckets;
   const uint64_t field = 1ull << a.map.val_bits;
-  constexpr int kHeld = 4;  // words a thread has in flight
+  constexpr int kHeld = 5;  // words a thread has in flight: all of a partition at half load (4,096 and a reserve)
   const uint32_t cnt = a.filled[p] < a.room ? a.filled[p] : a.room;
   const uint64_t *const words = a.words + static_cast<size_t>(p) * a.room;
-  for (uint32_t i = threadIdx.x; i < kPartBuckets * kProbeGroup; i += kPartBlock)
-    slots4[i] = make_uint4(~0u, ~0u, ~0u, ~0u);
-  __syncthreads();
-  for (uint32_t e0 = 0; e0 < cnt; e0 += kHeld * kPartBlock) {
-    uint64_t held[kHeld];
+  uint64_t held[kHeld];
+  auto load = [&](uint32_t e0) {
 #pragma unroll
     for (int j = 0; j < kHeld; ++j) {
       const uint32_t e = e0 + j * kPartBlock + threadIdx.x;
       held[j] = e < cnt ? words[e] : ~0ull;
     }
+  };
+  load(0);  // on their way while the slots are cleared
+  for (uint32_t i = threadIdx.x; i < kPartBuckets * kProbeGroup; i += kPartBlock)
+    slots4[i] = make_uint4(~0u, ~0u, ~0u, ~0u);
+  __syncthreads();
+  for (uint32_t e0 = 0; e0 < cnt; e0 += kHeld * kPartBlock) {
+    if (e0 > 0) load(e0);
 #pragma unroll
     for (int j = 0; j < kHeld; ++j) {
       if (held[j] == ~0ull) continue;
@@ -301,18 +305,12 @@ __global__ __launch_bounds__(kPartBlock) void part_fill_kernel(PartArgs a) {
   for (uint32_t i = threadIdx.x; i < nb * kProbeGroup; i += kPartBlock) out[i] = slots4[i];
 }
 
+// One word per probe group at a time: as a rule there are a few dozen, and a wave that took 64 of them would
+// insert eight one after the other (11 us; 5 this way).
 __global__ __launch_bounds__(256) void part_rest_kernel(PartArgs a) {
   const uint32_t n = *a.rest_count;
-  const int lane = lane_id(), gbase = lane & ~(kProbeGroup - 1);
-  const uint32_t waves = gridDim.x * (256 / kWave);
-  for (uint32_t base = (blockIdx.x * (256 / kWave) + threadIdx.x / kWave) * kWave; base < n; base += waves * kWave) {
-    const uint64_t mine = base + lane < n ? a.rest[base + lane] : ~0ull;
-#pragma unroll 1
-    for (int j = 0; j < kProbeGroup; ++j) {
-      const uint64_t w = static_cast<uint64_t>(shfl64(static_cast<int64_t>(mine), gbase + j));
-      if (w != ~0ull) group_insert8(a.table, a.map, w);
-    }
-  }
+  const uint32_t groups = gridDim.x * (256 / kProbeGroup);
+  for (uint32_t e = (blockIdx.x * 256 + threadIdx.x) / kProbeGroup; e < n; e += groups) group_insert8(a.table, a.map, a.rest[e]);
 }
 
 // ---- what do the keys look like? ---------------------------------------------
