@@ -723,10 +723,11 @@ int shmt_hashmap_create_planned_scratch(shmt_hashmap_t **out, const shmt_hashmap
   if (layout->kind == SHMT_MAP_BUCKETS) {
     SHMT_REQUIRE(layout->slot_bytes == kSlot16 || layout->slot_bytes == kSlot8,
                  "shmt_hashmap_create_planned: bad slot size %d", layout->slot_bytes);
-    SHMT_REQUIRE(layout->span >= 0 && layout->span < (1ll << 62) && (layout->span == 0 || layout->slot_bytes == kSlot8),
+    // (16-byte slots have no use for an id range)
+    SHMT_REQUIRE(layout->slot_bytes == kSlot16 || (layout->span >= 0 && layout->span < (1ll << 62)),
                  "shmt_hashmap_create_planned: bad id range of packed slots");
     return build_buckets(out, layout->slot_bytes, keys, vals, n, key_bytes, val_bytes, load_factor, table_mem,
-                         table_bytes, stream, layout, scratch, scratch_bytes);
+                         table_bytes, stream, layout->slot_bytes == kSlot8 ? layout : nullptr, scratch, scratch_bytes);
   }
   SHMT_REQUIRE(layout->kind == SHMT_MAP_DIRECT || layout->kind == SHMT_MAP_RANGE || layout->kind == SHMT_MAP_RANK,
                "shmt_hashmap_create_planned: unknown layout kind %d", layout->kind);

@@ -395,3 +395,38 @@ def test_values_and_spans_that_just_pack(capi, n, packs):
         assert h.layout() == "buckets" and h.memory_usage() == (2 * n + (15 if narrow else 7)) // (16 if narrow else 8) * 128
         assert torch.equal(h.query(keys), vals)
         assert h.query(torch.tensor([-1, (1 << 40) - 1, 1 << 40]).cuda()).tolist() == [-1, -1, -1]
+
+
+def test_packed_layout_through_the_c_abi(cabi):
+    """A packed layout built without scratch memory (compare-and-swap) and with it (partitions) answers alike; with too
+    little the build is the one without; 16-byte slots do not look at the layout's id range."""
+    import ctypes
+    lib, stream = cabi.load(), cabi.current_stream()
+    n = (1 << 18) + 5
+    keys = (torch.randperm(1 << 22, device="cuda")[:n] * 1021 + (1 << 35)).contiguous()
+    vals = torch.arange(n, device="cuda")
+    sb = lib.shmt_hashmap_plan_scratch_bytes(n)
+    scratch = torch.empty(sb, dtype=torch.uint8, device="cuda")
+    lay = cabi.HashmapLayout()
+    cabi.check(lib.shmt_hashmap_plan(keys.data_ptr(), vals.data_ptr(), n, 8, 8, 0.5, scratch.data_ptr(), sb,
+                                     ctypes.byref(lay), stream))
+    assert (lay.kind, lay.slot_bytes, lay.lo) == (0, 8, int(keys.min()))
+    assert lay.span == int(keys.max()) - int(keys.min()) + 1
+    need = lib.shmt_hashmap_build_scratch_bytes(ctypes.byref(lay), n, 0.5)
+    assert need > 8 * n
+    build = torch.empty(need, dtype=torch.uint8, device="cuda")
+    req = torch.cat([keys, keys + 1, torch.tensor([-1, 0], device="cuda")])
+    want = torch.cat([vals, torch.full((n + 2,), -1, device="cuda")])
+    for given in (0, need - 1, need, None):
+        if given is None:
+            lay.slot_bytes, lay.span = 16, -7
+            lay.table_bytes = lib.shmt_hashmap_table_bytes(n, 0.5, 8, 8)
+        table = torch.empty(lay.table_bytes, dtype=torch.uint8, device="cuda")
+        handle = ctypes.c_void_p()
+        cabi.check(lib.shmt_hashmap_create_planned_scratch(
+            ctypes.byref(handle), ctypes.byref(lay), keys.data_ptr(), vals.data_ptr(), n, 8, 8, 0.5, table.data_ptr(),
+            table.numel(), build.data_ptr() if given else None, given or 0, stream))
+        out = torch.empty_like(req)
+        cabi.check(lib.shmt_hashmap_query(handle, req.data_ptr(), 8, req.numel(), out.data_ptr(), stream))
+        assert torch.equal(out, want)
+        lib.shmt_hashmap_destroy(handle)
