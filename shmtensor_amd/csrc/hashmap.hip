@@ -42,9 +42,10 @@ static int64_t buckets_for(int64_t n, double lf, int fmt) {
 // it is never all ones (the empty slot).
 static int packed_value_bits(int64_t key_span) {
   int key_bits = 1;
-  while ((1ll << key_bits) - 1 < key_span) ++key_bits;
+  while ((1ull << key_bits) - 1 < static_cast<uint64_t>(key_span)) ++key_bits;
   return 64 - key_bits;
 }
+constexpr int64_t kPackMaxSpan = 1ll << 62;  // 63 bits of key leave one of value
 constexpr int64_t kPackMinKeys = (4 << 20) / (2 * kSlot16);
 
 // ---- kernels ---------------------------------------------------------------
@@ -602,7 +603,7 @@ int shmt_hashmap_plan(const void *keys, const void *vals, int64_t n, int key_byt
   const int64_t flat_limit = 2 * buckets_for(n, load_factor, fmt) * kBucketBytes;  // of a rank or direct table
   // ... and, packed, when a key's distance from the smallest one and the span of the values share 64 bits.
   // Only for tables that outgrow an L2 (4 MiB) in 16-byte slots: below that a lookup costs the same either way.
-  if (fmt == kSlot16 && st.kmin >= 0 && st.kmax - st.kmin < (1ll << 62) && n > kPackMinKeys) {
+  if (fmt == kSlot16 && st.kmin >= 0 && st.kmax - st.kmin < kPackMaxSpan && n > kPackMinKeys) {
     const int64_t key_span = st.kmax - st.kmin + 1;
     const int val_bits = packed_value_bits(key_span);
     if (static_cast<uint64_t>(st.vmax) - static_cast<uint64_t>(st.vmin) < (1ull << val_bits)) {
@@ -724,7 +725,7 @@ int shmt_hashmap_create_planned_scratch(shmt_hashmap_t **out, const shmt_hashmap
     SHMT_REQUIRE(layout->slot_bytes == kSlot16 || layout->slot_bytes == kSlot8,
                  "shmt_hashmap_create_planned: bad slot size %d", layout->slot_bytes);
     // (16-byte slots have no use for an id range)
-    SHMT_REQUIRE(layout->slot_bytes == kSlot16 || (layout->span >= 0 && layout->span < (1ll << 62)),
+    SHMT_REQUIRE(layout->slot_bytes == kSlot16 || (layout->span >= 0 && layout->span <= kPackMaxSpan),
                  "shmt_hashmap_create_planned: bad id range of packed slots");
     return build_buckets(out, layout->slot_bytes, keys, vals, n, key_bytes, val_bytes, load_factor, table_mem,
                          table_bytes, stream, layout->slot_bytes == kSlot8 ? layout : nullptr, scratch, scratch_bytes);

@@ -397,6 +397,23 @@ def test_values_and_spans_that_just_pack(capi, n, packs):
         assert h.query(torch.tensor([-1, (1 << 40) - 1, 1 << 40]).cuda()).tolist() == [-1, -1, -1]
 
 
+@pytest.mark.parametrize("span,packs", [((1 << 62) - 1, True), (1 << 62, True), ((1 << 62) + 1, False)])
+def test_widest_span_that_packs(capi, span, packs):
+    """Keys that span 2^62 ids leave one bit to the values, which two neighbouring numbers share; one id more takes
+    16-byte slots."""
+    g = torch.Generator(device="cuda").manual_seed(7)
+    n = (4 << 20) // 32 + 1
+    keys = torch.unique(torch.randint(1, (1 << 62) - 2, (n + 2000,), device="cuda", generator=g))
+    keys = keys[torch.randperm(keys.numel(), device="cuda", generator=g)][:n].contiguous()
+    keys[0], keys[1] = 0, span - 1
+    vals = torch.randint(7, 9, (n,), device="cuda", generator=g)
+    vals[0], vals[1] = 7, 8
+    h = capi.CUCOStaticHashmap(keys, vals, 0.5)
+    assert h.layout() == "buckets" and h.memory_usage() == (2 * n + (15 if packs else 7)) // (16 if packs else 8) * 128
+    assert torch.equal(h.query(keys), vals)
+    assert h.query(torch.tensor([-1, span, 2**63 - 1, -2**63]).cuda()).tolist() == [-1, -1, -1, -1]
+
+
 def test_packed_layout_through_the_c_abi(cabi):
     """A packed layout built without scratch memory (compare-and-swap) and with it (partitions) answers alike; with too
     little the build is the one without; 16-byte slots do not look at the layout's id range."""
