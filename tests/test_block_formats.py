@@ -2,6 +2,7 @@
 import sys
 import types
 
+import pytest
 import torch
 
 
@@ -36,14 +37,39 @@ def test_blocks_with_and_without_dgl(monkeypatch):
     assert isinstance(sampling.create_block_from_coo(a, b, 2, 1), het.DGLBlock) and len(made) == 2
 
 
-def test_a_new_loader_looks_again(monkeypatch, tmp_path):
+@pytest.fixture
+def importable_dgl(tmp_path, monkeypatch):
+    """Writes a dgl module and puts it on the import path; what was imported of it is gone afterwards."""
+    before = {name: sys.modules.pop(name) for name in ("dgl", "dgl.heterograph") if name in sys.modules}
+
+    def make(source):
+        (tmp_path / "dgl.py").write_text(source)
+        monkeypatch.syspath_prepend(str(tmp_path))
+
+    yield make
+    for name in ("dgl", "dgl.heterograph"):
+        sys.modules.pop(name, None)
+    sys.modules.update(before)
+
+
+def _loader(sampling, monkeypatch):
+    """A loader built without a GPU (its tensors stay where they are)."""
+    monkeypatch.setattr(sampling.capi, "pin_memory", lambda t: None)
+    monkeypatch.setattr(sampling, "_unpin", lambda t: None)
+    monkeypatch.setattr(torch.Tensor, "cuda", lambda self: self)
+    return sampling.GPUSamplingDataloader(torch.tensor([0, 1, 2]), torch.tensor([1, 0]), torch.arange(2), 1, [1])
+
+
+def test_a_new_loader_looks_again(monkeypatch, importable_dgl):
     import shmtensor_amd
     shmtensor_amd.install_aliases()
     from shmtensor_amd.shmtensor import sampling
-    monkeypatch.delitem(sys.modules, "dgl", raising=False)
     monkeypatch.setattr(sampling, "_dgl_missing", True)
-    (tmp_path / "dgl.py").write_text("found = True\n")
-    monkeypatch.syspath_prepend(str(tmp_path))
+    importable_dgl("found = True\n")
     assert sampling._dgl() is None
-    assert sampling._dgl(look_again=True).found
-    monkeypatch.delitem(sys.modules, "dgl")
+    _loader(sampling, monkeypatch)
+    assert sampling._dgl().found
+
+
+def test_no_stub_is_left_behind():
+    assert not hasattr(sys.modules.get("dgl"), "found")
