@@ -30,23 +30,22 @@ CSCBlock = collections.namedtuple("CSCBlock", ["indptr", "indices", "num_src", "
 COOBlock = collections.namedtuple("COOBlock", ["row", "col", "num_src", "num_dst"])
 
 
-_dgl_missing = False
+class _Absent(threading.local):
+    """Set by a loader while it builds the blocks of a group: it looked for dgl before and did not find it."""
+    known = False
 
 
-def _dgl(look_again=False):
-    """The dgl module, or None. Python does not remember an import that failed: it searches the whole path anew,
-    20 to 50 us every time, which was half of the time of a prefetched epoch when every block of every batch
-    tried. A failure is kept here until the next loader is built (look_again); a dgl that anyone has
-    imported since is seen at once."""
-    global _dgl_missing
-    found = sys.modules.get("dgl")
-    if found is not None or (_dgl_missing and not look_again):
-        return found
+_absent = _Absent()
+
+
+def _dgl():
+    """The dgl module, or None. An import in progress in another thread is waited for."""
+    if _absent.known and "dgl" not in sys.modules:
+        return None
     try:
         import dgl
         return dgl
     except Exception:
-        _dgl_missing = True
         return None
 
 
@@ -120,7 +119,8 @@ class GPUSamplingDataloader:
         if block_format not in ("csc", "coo"):
             raise ValueError("block_format must be 'csc' or 'coo'")
         self.block_format = block_format
-        _dgl(look_again=True)
+        self._no_dgl_on = None     # where dgl was looked for and not found
+        self._dgl_known_absent()
 
         self.has_cache = False
         self.gpu_indptr = None
@@ -195,6 +195,15 @@ class GPUSamplingDataloader:
                                            self.hashmap, seeds, num_pick, self.replace, **extra)
         return capi.csr_sampling(self.indptr, self.indices, seeds, num_pick, self.replace, **extra)
 
+    def _dgl_known_absent(self):
+        """Python does not remember an import that failed: it searches the whole path anew, 20 to 50 us every time,
+        which was half of the time of a prefetched epoch when every block of every batch tried. A loader looks for
+        dgl once and again when the import path has changed; a dgl that someone has imported is seen in any case."""
+        path = (list(sys.path), list(sys.meta_path))
+        if self._no_dgl_on != path:
+            self._no_dgl_on = path if _dgl() is None else None
+        return self._no_dgl_on is not None
+
     def _sample_group(self, first_batch, count, batches_drawn):
         """Sample `count` consecutive batches starting at batch `first_batch`; returns one
         (input_nodes, output_nodes, blocks) per batch."""
@@ -220,18 +229,22 @@ class GPUSamplingDataloader:
             rows = [x for _, x in fetched]
             self._feature_rows = max([self._feature_rows] + [x.shape[0] for x in rows])
         out = []
-        for seeds, chain, x in zip(groups, chains, rows):
-            blocks, dst = [], seeds
-            for hop in chain:
-                sub_indptr, _, unique_tensor, relabel_indices = hop[:4]
-                if coo:
-                    blocks.insert(0, create_block_from_coo(relabel_indices, hop[4], unique_tensor.numel(),
-                                                           dst.numel()))
-                else:
-                    blocks.insert(0, create_block_from_csc(sub_indptr, relabel_indices, torch.Tensor(),
-                                                           unique_tensor.numel(), dst.numel()))
-                dst = unique_tensor
-            out.append((dst, seeds, blocks) if self.features is None else (dst, seeds, blocks, x))
+        _absent.known = self._dgl_known_absent()
+        try:
+            for seeds, chain, x in zip(groups, chains, rows):
+                blocks, dst = [], seeds
+                for hop in chain:
+                    sub_indptr, _, unique_tensor, relabel_indices = hop[:4]
+                    if coo:
+                        blocks.insert(0, create_block_from_coo(relabel_indices, hop[4], unique_tensor.numel(),
+                                                               dst.numel()))
+                    else:
+                        blocks.insert(0, create_block_from_csc(sub_indptr, relabel_indices, torch.Tensor(),
+                                                               unique_tensor.numel(), dst.numel()))
+                    dst = unique_tensor
+                out.append((dst, seeds, blocks) if self.features is None else (dst, seeds, blocks, x))
+        finally:
+            _absent.known = False
         return out
 
     def _produce(self, first_batch, batches_drawn, out_queue, stop):
