@@ -303,7 +303,8 @@ __device__ __forceinline__ void wave_probe_examine(const MapView &m, WaveProbe<F
   }
 }
 
-// One more bucket for the keys that are not resolved (their first one was full of other keys).
+// One more bucket for the keys that are not resolved (their first one was full of other keys). Only the groups
+// that have such a key read a line: it is the lines that lookups are bound by.
 template <int FMT>
 __device__ __forceinline__ void wave_probe_walk(const MapView &m, WaveProbe<FMT> *p, uint32_t round) {
   const int sub = lane_id() & (kProbeGroup - 1), gbase = lane_id() & ~(kProbeGroup - 1);
@@ -313,8 +314,11 @@ __device__ __forceinline__ void wave_probe_walk(const MapView &m, WaveProbe<FMT>
     uint32_t b = static_cast<uint32_t>(__shfl(static_cast<int>(p->home), gbase + j, kWave)) + round;
     if (b >= m.nbuckets) b -= m.nbuckets;
     const uint64_t want = static_cast<uint64_t>(shfl64(static_cast<int64_t>(p->want), gbase + j));
-    uint4 frag = m.buckets[static_cast<size_t>(b) * kProbeGroup + sub];
-    keep_loaded(&frag);
+    uint4 frag = make_uint4(0, 0, 0, 0);
+    if ((p->open >> (gbase + j)) & 1ull) {
+      frag = m.buckets[static_cast<size_t>(b) * kProbeGroup + sub];
+      keep_loaded(&frag);
+    }
     uint64_t raw;
     const uint64_t still = probe_buckets<FMT>(m, frag, want, &raw) << j;
     if (sub == j && ((p->open >> lane_id()) & 1ull)) p->res = raw;
