@@ -15,9 +15,11 @@
 // Phase 2: the row addresses are broadcast with lane shuffles and the rows are
 // moved with the widest vector access the row size and base pointers allow (16
 // bytes per lane when aligned). Rows of 8, 16, 32 or 64 vectors (or nearly) take
-// a sub-wave group of as many lanes each; the vectors of rows of any other size
+// a sub-wave group of as many lanes each; the vectors of other short rows
 // are dealt to the lanes one after the other, whatever row they belong to, so
-// that no lane is left over at the end of a row. The dependent chain id -> bucket -> row is paid once per tile
+// that no lane is left over at the end of a row; long rows (wide_from) are moved
+// one by one by the whole wave, with four vectors per lane in flight. The
+// dependent chain id -> bucket -> row is paid once per tile
 // instead of once per row.
 //
 // A fetch can also go out as two launches (shmt_fetch_cached_part /
@@ -52,10 +54,11 @@ struct RowArgs {
   int64_t row_bytes;
   int idx_bytes;
   int mask_bytes;
-  int log2_lanes;      // lanes per row in phase 2 = 1 << log2_lanes, in [8, 64] (ONE_VEC)
-  int log2_tile;       // rows per wave tile = 1 << log2_tile, in [64 / lanes, 32]
-  uint32_t nvec;        // vectors per row (!ONE_VEC); 0: too many for a tile's to be counted in 32 bits
+  int log2_lanes;      // lanes per row in phase 2 = 1 << log2_lanes, in [8, 64] (kOneVec)
+  int log2_tile;       // rows per wave tile = 1 << log2_tile, at most 32
+  uint32_t nvec;        // vectors per row (kDealt)
   uint32_t nvec_magic;  // floor((2^32 - 1) / nvec): the high half of i * magic is i / nvec, or one less
+  int stream_dense;     // kWide: `dense` is accessed past the caches
   uint32_t *miss_bits;  // DEFER: bit (i & 31) of word i / 32 is set when row i missed the cache
 };
 
@@ -87,20 +90,63 @@ constexpr int kRowsInFlight = 1;
 // of 33 floats 25.4 / 30.6 (35.8), 50 floats 27.5 / 30.6 (29.1), but 100 floats 45.8 / 43.9 (48.5) and 300 floats
 // 178 / 171 (171): a set of 16-byte vectors takes two, which need the registers of six waves. Four gain nothing.
 constexpr int vecs_in_flight(bool set, int vector_bytes) { return set && vector_bytes == 16 ? 2 : 1; }
-constexpr int rows_waves_per_simd(bool set, bool one_vec, int vector_bytes) {
-  return one_vec || vecs_in_flight(set, vector_bytes) == 1 ? kRowsWavesPerSimd : 6;
+// How the rows of a tile are moved: a lane group per row with one vector per lane, vectors dealt out one by one,
+// or one row after the other by the whole wave.
+enum RowRoute : int { kOneVec, kDealt, kWide };
+constexpr int rows_waves_per_simd(bool set, int route, int vector_bytes) {
+  return route == kOneVec || vector_bytes < 16 || (route == kDealt && vecs_in_flight(set, vector_bytes) == 1)
+             ? kRowsWavesPerSimd : 6;
+}
+
+// One row of more than 64 vectors, moved by the whole wave: a lane has kWideInFlight vectors in flight, also
+// where the row ends among them.
+constexpr int kWideInFlight = 4;
+constexpr bool may_stream(bool set, int vector_bytes) { return vector_bytes >= (set ? 4 : 16); }
+// (1- and 2-byte vectors are held in registers of their own: packed into one, each load would wait for the last)
+template <typename VT> struct Held { using type = VT; };
+template <> struct Held<uint8_t> { using type = uint32_t; };
+template <> struct Held<uint16_t> { using type = uint32_t; };
+template <typename VT, bool SET, bool STREAM>
+__device__ __forceinline__ void move_wide_row(char *dense, char *table, char *second, int64_t row_bytes) {
+  constexpr int64_t step = kWave * static_cast<int64_t>(sizeof(VT));
+  for (int64_t off = lane_id() * static_cast<int64_t>(sizeof(VT)); off < row_bytes; off += kWideInFlight * step) {
+    typename Held<VT>::type v[kWideInFlight];
+#pragma unroll
+    for (int u = 0; u < kWideInFlight; ++u) {
+      if (off + u * step >= row_bytes) continue;
+      if (SET && STREAM)
+        v[u] = __builtin_nontemporal_load(reinterpret_cast<const VT *>(dense + off + u * step));
+      else
+        v[u] = gload<VT>((SET ? dense : table) + off + u * step);
+    }
+#pragma unroll
+    for (int u = 0; u < kWideInFlight; ++u) {
+      if (off + u * step >= row_bytes) continue;
+      const VT x = static_cast<VT>(v[u]);
+      if (SET) {
+        gstore<VT>(table + off + u * step, x);
+        if (second) gstore<VT>(second + off + u * step, x);
+      } else if (STREAM) {
+        __builtin_nontemporal_store(x, reinterpret_cast<VT *>(dense + off + u * step));
+      } else {
+        gstore<VT>(dense + off + u * step, x);
+      }
+    }
+  }
 }
 // Rows per wave tile, at most. 32 measured 2 % faster than 64 on all-hit rows (90 against 92 us) and the
 // same on mixed hit / miss batches; 16 gains nothing more and costs the bucket-table probe 15 %.
 constexpr int kMaxLog2Tile = 5;
+constexpr int64_t kL2Bytes = 32ll << 20;      // the L2s together
+constexpr int64_t kCacheBytes = 256ll << 20;  // the memory-side cache
 
 // THROUGH (set only, with a map or mask): rows that hit the cache are written
 // to the id-addressed table as well, so that table never goes stale.
 // DEFER (fetch only, with a map or mask; tiles of exactly 32 rows): rows that
 // miss the cache are not moved; every tile leaves one word of a bitmap that
 // marks them for rows_missed_kernel (no counter, no atomics, nothing to clear).
-template <typename VT, int MODE, bool SET, bool ONE_VEC, bool THROUGH = false, bool DEFER = false>
-__global__ __launch_bounds__(kRowsBlock, rows_waves_per_simd(SET, ONE_VEC, sizeof(VT))) void rows_kernel(RowArgs a) {
+template <typename VT, int MODE, bool SET, int ROUTE, bool THROUGH = false, bool DEFER = false>
+__global__ __launch_bounds__(kRowsBlock, rows_waves_per_simd(SET, ROUTE, sizeof(VT))) void rows_kernel(RowArgs a) {
   static_assert(!THROUGH || (SET && MODE != kDirect), "write-through is a cached set");
   static_assert(!DEFER || (!SET && MODE != kDirect), "only a cached fetch sets its misses aside");
   const int lane = lane_id();
@@ -212,7 +258,7 @@ __global__ __launch_bounds__(kRowsBlock, rows_waves_per_simd(SET, ONE_VEC, sizeo
     const int nrows = static_cast<int>(Q - base < tile ? Q - base : tile);
 
     // ---- phase 2: move the rows ----
-    if (ONE_VEC) {
+    if (ROUTE == kOneVec) {
       // row_bytes <= L * sizeof(VT): one vector per lane per row
       const bool in = my_off < R;
       for (int r0 = 0; r0 < nrows; r0 += kRowsInFlight * rows_per_step) {
@@ -253,17 +299,16 @@ __global__ __launch_bounds__(kRowsBlock, rows_waves_per_simd(SET, ONE_VEC, sizeo
           }
         }
       }
-    } else if (a.nvec == 0) {
+    } else if (ROUTE == kWide) {
       for (int row = 0; row < nrows; ++row) {
-        char *const trow = reinterpret_cast<char *>(shfl64(my_table_row, row));
-        char *const second = THROUGH ? reinterpret_cast<char *>(shfl64(my_second_row, row)) : nullptr;
+        char *const trow = reinterpret_cast<char *>(lane64(my_table_row, row));
+        char *const second = THROUGH ? reinterpret_cast<char *>(lane64(my_second_row, row)) : nullptr;
         if (DEFER && !trow) continue;
         char *const drow = a.dense + (base + row) * R;
-        for (int64_t off = lane * static_cast<int64_t>(sizeof(VT)); off < R; off += kWave * static_cast<int64_t>(sizeof(VT))) {
-          const VT v = gload<VT>((SET ? drow : trow) + off);
-          gstore<VT>((SET ? trow : drow) + off, v);
-          if (THROUGH && second) gstore<VT>(second + off, v);
-        }
+        if (may_stream(SET, sizeof(VT)) && a.stream_dense)
+          move_wide_row<VT, SET, may_stream(SET, sizeof(VT))>(drow, trow, second, R);
+        else
+          move_wide_row<VT, SET, false>(drow, trow, second, R);
       }
     } else {
       constexpr int kVecsInFlight = vecs_in_flight(SET, sizeof(VT));
@@ -429,20 +474,20 @@ __global__ __launch_bounds__(kRowsBlock) void rows_missed_kernel(MissedArgs a) {
   }
 }
 
-template <bool ONE_VEC>
+template <int ROUTE>
 static void launch_defer(int mode, unsigned grid, hipStream_t s, const RowArgs &a) {
   switch (mode) {
     case kMap16:
-      hipLaunchKernelGGL((rows_kernel<u32x4, kMap16, false, ONE_VEC, false, true>), dim3(grid), dim3(kRowsBlock), 0, s, a);
+      hipLaunchKernelGGL((rows_kernel<u32x4, kMap16, false, ROUTE, false, true>), dim3(grid), dim3(kRowsBlock), 0, s, a);
       break;
     case kMap8:
-      hipLaunchKernelGGL((rows_kernel<u32x4, kMap8, false, ONE_VEC, false, true>), dim3(grid), dim3(kRowsBlock), 0, s, a);
+      hipLaunchKernelGGL((rows_kernel<u32x4, kMap8, false, ROUTE, false, true>), dim3(grid), dim3(kRowsBlock), 0, s, a);
       break;
     case kMapFlat:
-      hipLaunchKernelGGL((rows_kernel<u32x4, kMapFlat, false, ONE_VEC, false, true>), dim3(grid), dim3(kRowsBlock), 0, s, a);
+      hipLaunchKernelGGL((rows_kernel<u32x4, kMapFlat, false, ROUTE, false, true>), dim3(grid), dim3(kRowsBlock), 0, s, a);
       break;
     default:
-      hipLaunchKernelGGL((rows_kernel<u32x4, kMask, false, ONE_VEC, false, true>), dim3(grid), dim3(kRowsBlock), 0, s, a);
+      hipLaunchKernelGGL((rows_kernel<u32x4, kMask, false, ROUTE, false, true>), dim3(grid), dim3(kRowsBlock), 0, s, a);
       break;
   }
 }
@@ -456,59 +501,95 @@ static int pick_vector_bytes(int64_t row_bytes, const void *p0, const void *p1, 
   return v;
 }
 
-template <typename VT, bool ONE_VEC>
+template <typename VT, int ROUTE>
 static void launch_through(int mode, unsigned grid, hipStream_t s, const RowArgs &a) {
   switch (mode) {
     case kMap16:
-      hipLaunchKernelGGL((rows_kernel<VT, kMap16, true, ONE_VEC, true>), dim3(grid), dim3(kRowsBlock), 0, s, a);
+      hipLaunchKernelGGL((rows_kernel<VT, kMap16, true, ROUTE, true>), dim3(grid), dim3(kRowsBlock), 0, s, a);
       break;
     case kMap8:
-      hipLaunchKernelGGL((rows_kernel<VT, kMap8, true, ONE_VEC, true>), dim3(grid), dim3(kRowsBlock), 0, s, a);
+      hipLaunchKernelGGL((rows_kernel<VT, kMap8, true, ROUTE, true>), dim3(grid), dim3(kRowsBlock), 0, s, a);
       break;
     case kMapFlat:
-      hipLaunchKernelGGL((rows_kernel<VT, kMapFlat, true, ONE_VEC, true>), dim3(grid), dim3(kRowsBlock), 0, s, a);
+      hipLaunchKernelGGL((rows_kernel<VT, kMapFlat, true, ROUTE, true>), dim3(grid), dim3(kRowsBlock), 0, s, a);
       break;
     default:
-      hipLaunchKernelGGL((rows_kernel<VT, kMask, true, ONE_VEC, true>), dim3(grid), dim3(kRowsBlock), 0, s, a);
+      hipLaunchKernelGGL((rows_kernel<VT, kMask, true, ROUTE, true>), dim3(grid), dim3(kRowsBlock), 0, s, a);
       break;
   }
 }
 
-template <typename VT, bool SET, bool ONE_VEC>
+template <typename VT, bool SET, int ROUTE>
 static void launch_mode(int mode, unsigned grid, hipStream_t s, const RowArgs &a) {
   switch (mode) {
     case kDirect:
-      hipLaunchKernelGGL((rows_kernel<VT, kDirect, SET, ONE_VEC>), dim3(grid), dim3(kRowsBlock), 0, s, a);
+      hipLaunchKernelGGL((rows_kernel<VT, kDirect, SET, ROUTE>), dim3(grid), dim3(kRowsBlock), 0, s, a);
       break;
     case kMap16:
-      hipLaunchKernelGGL((rows_kernel<VT, kMap16, SET, ONE_VEC>), dim3(grid), dim3(kRowsBlock), 0, s, a);
+      hipLaunchKernelGGL((rows_kernel<VT, kMap16, SET, ROUTE>), dim3(grid), dim3(kRowsBlock), 0, s, a);
       break;
     case kMap8:
-      hipLaunchKernelGGL((rows_kernel<VT, kMap8, SET, ONE_VEC>), dim3(grid), dim3(kRowsBlock), 0, s, a);
+      hipLaunchKernelGGL((rows_kernel<VT, kMap8, SET, ROUTE>), dim3(grid), dim3(kRowsBlock), 0, s, a);
       break;
     case kMapFlat:
-      hipLaunchKernelGGL((rows_kernel<VT, kMapFlat, SET, ONE_VEC>), dim3(grid), dim3(kRowsBlock), 0, s, a);
+      hipLaunchKernelGGL((rows_kernel<VT, kMapFlat, SET, ROUTE>), dim3(grid), dim3(kRowsBlock), 0, s, a);
       break;
     default:
-      hipLaunchKernelGGL((rows_kernel<VT, kMask, SET, ONE_VEC>), dim3(grid), dim3(kRowsBlock), 0, s, a);
+      hipLaunchKernelGGL((rows_kernel<VT, kMask, SET, ROUTE>), dim3(grid), dim3(kRowsBlock), 0, s, a);
       break;
   }
 }
 
 template <typename VT, bool SET>
-static void launch_vec(bool one_vec, bool through, int mode, unsigned grid, hipStream_t s,
+static void launch_vec(int route, bool through, int mode, unsigned grid, hipStream_t s,
                        const RowArgs &a) {
   if (SET && through && mode != kDirect) {
-    if (one_vec)
-      launch_through<VT, true>(mode, grid, s, a);
+    if (route == kOneVec)
+      launch_through<VT, kOneVec>(mode, grid, s, a);
+    else if (route == kDealt)
+      launch_through<VT, kDealt>(mode, grid, s, a);
     else
-      launch_through<VT, false>(mode, grid, s, a);
+      launch_through<VT, kWide>(mode, grid, s, a);
     return;
   }
-  if (one_vec)
-    launch_mode<VT, SET, true>(mode, grid, s, a);
+  if (route == kOneVec)
+    launch_mode<VT, SET, kOneVec>(mode, grid, s, a);
+  else if (route == kDealt)
+    launch_mode<VT, SET, kDealt>(mode, grid, s, a);
   else
-    launch_mode<VT, SET, false>(mode, grid, s, a);
+    launch_mode<VT, SET, kWide>(mode, grid, s, a);
+}
+
+// Rows of more vectors than this go one by one (kWide), shorter ones that fill no lane group are dealt out. All hits,
+// us for 100 MB of output or update in all (for 400 MB), dealt out / one by one:
+//   fetch  16-byte vectors  65: 50 / 42 (156 / 190), 75: 54 / 41 (171 / 190), 88: 58 / 41 (187 / 164), 128: 46 / 36 (163 / 166)
+//          8-byte           65: 55 / 46 (186 / 194), 89: 63 / 43 (187 / 190), 145: 74 / 42 (201 / 191)
+//          4-byte           65: 30 / 38 (251 / 234), 89: 53 / 43 (243 / 200), 257: 122 / 55 (329 / 231)
+//          2-byte           65: 25 / 25 (231 / 249), 89: 32 / 25 (348 / 273), 257: 140 / 65 (538 / 255)
+//          1-byte           97: 27 / 24 (186 / 221), 113: 31 / 24 (257 / 237), 257: 91 / 57 (607 / 355)
+//   set    16-byte          65: 54 / 57 (240 / 234), 75: 51 / 51 (233 / 227), 128: 41 / 44 (195 / 180)
+//          8-byte           75: 53 / 57 (234 / 249), 89: 54 / 54 (242 / 240), 145: 69 / 53 (243 / 232)
+//          4-byte           97: 55 / 60 (236 / 261), 127: 67 / 68 (252 / 266), 145: 72 / 58 (249 / 251), 257: 112 / 81 (330 / 288)
+//          2-byte           75: 41 / 41 (291 / 291), 89: 47 / 42 (335 / 307), 257: 114 / 90 (398 / 334)
+//          1-byte           65: 41 / 25 (292 / 244), 257: 131 / 66 (793 / 381)
+// (With at most two loads in flight per lane, as dealt out, rows of 5 to 15 KB took up to 2.7 times as long.)
+static int64_t wide_from(bool set, int vector_bytes, int64_t dense_bytes) {
+  switch (vector_bytes) {
+    case 16: return !set && dense_bytes > kCacheBytes ? 87 : 64;
+    case 8: return set ? 80 : 64;
+    case 4: return set ? 128 : 80;
+    case 2: return set ? 80 : 64;
+    default: return set ? 64 : 112;
+  }
+}
+
+// Whether `dense` is accessed past the caches (kWide). A fetch does so when its output is larger than the
+// memory-side cache (rows of 128 16-byte vectors, 400 MB: 178 us plain, 164 streaming; 100 MB: 36 / 38). A set does
+// so with an update that would push the rows it writes out of that cache (100 MB: 49 plain, 44 streaming), but not
+// with one small enough to lie in the L2s (512 vectors, 16 MB: 7.0 / 8.5) or beyond both (400 MB: 188 / 191).
+static bool stream_dense(bool set, int vector_bytes, int64_t dense_bytes) {
+  if (!may_stream(set, vector_bytes)) return false;
+  return set ? dense_bytes > kL2Bytes && dense_bytes <= kCacheBytes : dense_bytes > kCacheBytes;
 }
 
 template <bool SET>
@@ -562,8 +643,11 @@ static int move_rows(const char *who, void *miss, void *cache, const void *indic
   // but with 64 lanes 200 floats 92.0 / 81.4, 208 floats 82.6 / 81.0, 240 floats 97.2 / 95.5.
   const int64_t lanes = 1ll << log2_lanes;
   const bool one_vec = nvec == lanes || (!SET && vb == 16 && lanes < kWave && nvec < lanes && 4 * nvec >= 3 * lanes);
-  a.nvec = nvec < (1ll << 26) ? static_cast<uint32_t>(nvec) : 0u;
-  a.nvec_magic = a.nvec ? 0xFFFFFFFFu / a.nvec : 0u;
+  const int64_t dense_bytes = Q * row_bytes;
+  const int route = one_vec ? kOneVec : nvec > wide_from(SET, vb, dense_bytes) ? kWide : kDealt;
+  a.stream_dense = stream_dense(SET, vb, dense_bytes);
+  a.nvec = route == kDealt ? static_cast<uint32_t>(nvec) : 0u;
+  a.nvec_magic = route == kDealt ? 0xFFFFFFFFu / a.nvec : 0u;
   int log2_tile = kMaxLog2Tile;
   int log2_least = one_vec ? 6 - log2_lanes : 0;  // fewest rows per tile: a wave's worth of vectors, or eight
   while (!one_vec && log2_least < 3 && (nvec << log2_least) < kWave) ++log2_least;
@@ -573,23 +657,28 @@ static int move_rows(const char *who, void *miss, void *cache, const void *indic
   // As many workgroups as the device holds at once (256 units x 8 waves per SIMD): beyond that a wave takes
   // several tiles and keeps the lookups of the next ones in flight while it moves rows.
   const unsigned grid = grid_for(Q, static_cast<int64_t>(kRowsBlock / kWave) << log2_tile,
-                                 256 * rows_waves_per_simd(SET, one_vec, vb));
+                                 256 * rows_waves_per_simd(SET, route, vb));
   hipStream_t s = as_stream(stream);
   if (miss_bits) {
     SHMT_REQUIRE(!SET && mode != kDirect, "%s: only a fetch through a hashmap or mask sets its misses aside", who);
     SHMT_REQUIRE(vb == 16, "%s: rows and tables must allow 16-byte accesses (row_bytes %lld)", who,
                  static_cast<long long>(row_bytes));
     SHMT_REQUIRE(Q < (1ll << 32), "%s: at most 2^32 - 1 rows", who);
-    if (one_vec) launch_defer<true>(mode, grid, s, a); else launch_defer<false>(mode, grid, s, a);
+    if (route == kOneVec)
+      launch_defer<kOneVec>(mode, grid, s, a);
+    else if (route == kDealt)
+      launch_defer<kDealt>(mode, grid, s, a);
+    else
+      launch_defer<kWide>(mode, grid, s, a);
     SHMT_LAUNCH_CHECK();
     return SHMT_OK;
   }
   switch (vb) {
-    case 16: launch_vec<u32x4, SET>(one_vec, through, mode, grid, s, a); break;
-    case 8: launch_vec<u32x2, SET>(one_vec, through, mode, grid, s, a); break;
-    case 4: launch_vec<uint32_t, SET>(one_vec, through, mode, grid, s, a); break;
-    case 2: launch_vec<uint16_t, SET>(one_vec, through, mode, grid, s, a); break;
-    default: launch_vec<uint8_t, SET>(one_vec, through, mode, grid, s, a); break;
+    case 16: launch_vec<u32x4, SET>(route, through, mode, grid, s, a); break;
+    case 8: launch_vec<u32x2, SET>(route, through, mode, grid, s, a); break;
+    case 4: launch_vec<uint32_t, SET>(route, through, mode, grid, s, a); break;
+    case 2: launch_vec<uint16_t, SET>(route, through, mode, grid, s, a); break;
+    default: launch_vec<uint8_t, SET>(route, through, mode, grid, s, a); break;
   }
   SHMT_LAUNCH_CHECK();
   return SHMT_OK;

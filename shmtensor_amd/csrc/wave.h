@@ -119,6 +119,13 @@ __device__ __forceinline__ int64_t shfl64(int64_t v, int src_lane) {
                               static_cast<uint32_t>(lo));
 }
 
+// Value held by lane `src`, the same for all lanes (src too).
+__device__ __forceinline__ int64_t lane64(int64_t v, int src) {
+  const uint32_t lo = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(static_cast<uint64_t>(v)), src));
+  const uint32_t hi = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(static_cast<uint64_t>(v) >> 32), src));
+  return static_cast<int64_t>((static_cast<uint64_t>(hi) << 32) | lo);
+}
+
 // ---- wavefront scans -----------------------------------------------------
 // Inclusive prefix sum across the 64 lanes with DPP row shifts and the two
 // gfx9 row broadcasts; lanes shifted in from outside a row read zero

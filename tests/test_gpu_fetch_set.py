@@ -544,3 +544,66 @@ def test_rows_that_fill_no_lane_group(capi, dtype, D, layout):
             want_cache[slots[w][hit]] = upd[hit]
             want_host[w if through else w[~hit]] = upd if through else upd[~hit]
             assert torch.equal(got, want_cache) and torch.equal(host.cuda(), want_host)
+
+
+def _check_moves(capi, full, cache, hot, q_len, layout="auto", seed=1):
+    """fetch, uva_fetch, set and write-through of q_len rows against indexing, byte for byte, whole tables compared."""
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    n = full.shape[0]
+    host = torch.empty(full.shape, dtype=full.dtype, pin_memory=True).copy_(full)
+    slots = torch.full((n,), -1, dtype=torch.int64, device="cuda")
+    slots[hot] = torch.arange(hot.numel(), device="cuda")
+    h = capi.CUCOStaticHashmap(hot, torch.arange(hot.numel(), device="cuda"), 0.8, layout=layout)
+    q = torch.randint(0, n, (q_len,), device="cuda", generator=g)
+    s = slots[q]
+    got = capi.cache_fetch(host, cache, q, h)
+    for at in range(0, q_len, 1 << 16):
+        part = slice(at, at + (1 << 16))
+        assert torch.equal(got[part], torch.where((s[part] >= 0)[:, None], cache[s[part].clamp(min=0)], full[q[part]]))
+    del got
+    few = q[:200]
+    assert torch.equal(capi.uva_fetch(host, few), full[few])
+    w = torch.randperm(n, device="cuda", generator=g)[: min(q_len, n)]
+    upd, hit = (full[w].flip(0) ^ 1 if not full.is_floating_point() else full[w].flip(0) + 1), slots[w] >= 0
+    for through in (False, True):
+        host.copy_(full)
+        after, want_cache, want_host = cache.clone(), cache.clone(), full.clone()
+        capi.cache_set(host, after, w, upd, h, write_through=through)
+        torch.cuda.synchronize()
+        want_cache[slots[w][hit]] = upd[hit]
+        want_host[w if through else w[~hit]] = upd if through else upd[~hit]
+        assert torch.equal(after, want_cache) and torch.equal(host.cuda(), want_host)
+
+
+@pytest.mark.parametrize("dtype,D", [(torch.float32, d) for d in (256, 260, 1024, 1028, 1276, 129, 191, 193, 257, 511)] +
+                         [(torch.float16, d) for d in (256 + 4, 320 + 4, 1024 + 4, 65, 81, 255, 257, 513)] +
+                         [(torch.uint8, d) for d in (64, 65, 112, 113, 255, 257, 1025)])
+@pytest.mark.parametrize("layout", ["auto", "buckets"])
+def test_rows_of_more_vectors_than_a_wave(capi, dtype, D, layout):
+    """Rows that the whole wave moves one by one, around the lengths from which it does (by vector width, for fetch and
+    set) and around multiples of the four vectors a lane has in flight."""
+    g = torch.Generator(device="cuda").manual_seed(D)
+    full, cache = (torch.randint(0, 100, (k, D), device="cuda", generator=g).to(dtype) for k in (2500, 1000))
+    hot = torch.randperm(2500, device="cuda", generator=g)[:1000]
+    for q_len in (1, 33, 2100):
+        _check_moves(capi, full, cache, hot, q_len, layout)
+
+
+@pytest.mark.parametrize("dtype,D,q_len", [(torch.float32, 348, 200_000), (torch.float32, 352, 200_000),   # 278 MB, 282 MB
+                                           (torch.float32, 1028, 70_000),                                # 288 MB
+                                           (torch.float32, 2056, 8_000),                                 # sets of 66 MB
+                                           (torch.float16, 1028, 20_000), (torch.float32, 401, 25_000)])  # 41 MB, 40 MB
+def test_moves_larger_than_the_caches(capi, dtype, D, q_len):
+    """Outputs beyond the memory-side cache (256 MiB) and updates beyond the L2s (32 MiB), which are accessed with the
+    streaming policy."""
+    g = torch.Generator(device="cuda").manual_seed(D)
+    full, cache = (torch.randint(0, 100, (k, D), device="cuda", generator=g).to(dtype) for k in (q_len, 1000))
+    _check_moves(capi, full, cache, torch.randperm(q_len, device="cuda", generator=g)[:1000], q_len)
+
+
+@pytest.mark.parametrize("D", [(1 << 26) - 1, (1 << 26) + 1])
+def test_rows_of_64_mib(capi, D):
+    """Byte rows of an odd length, on both sides of 2^26 vectors."""
+    g = torch.Generator(device="cuda").manual_seed(3)
+    full, cache = (torch.randint(0, 256, (k, D), device="cuda", generator=g, dtype=torch.uint8) for k in (3, 2))
+    _check_moves(capi, full, cache, torch.tensor([2, 0], device="cuda"), 3)
