@@ -93,9 +93,9 @@ constexpr int vecs_in_flight(bool set, int vector_bytes) { return set && vector_
 // How the rows of a tile are moved: a lane group per row with one vector per lane, vectors dealt out one by one,
 // or one row after the other by the whole wave.
 enum RowRoute : int { kOneVec, kDealt, kWide };
-constexpr int rows_waves_per_simd(bool set, int route, int vector_bytes) {
-  return route == kOneVec || vector_bytes < 16 || (route == kDealt && vecs_in_flight(set, vector_bytes) == 1)
-             ? kRowsWavesPerSimd : 6;
+constexpr int rows_waves_per_simd(bool set, bool through, int route, int vector_bytes) {
+  if (route == kWide) return vector_bytes == 16 || through ? 6 : kRowsWavesPerSimd;
+  return route == kOneVec || vecs_in_flight(set, vector_bytes) == 1 ? kRowsWavesPerSimd : 6;
 }
 
 // One row of more than 64 vectors, moved by the whole wave: a lane has kWideInFlight vectors in flight, also
@@ -139,6 +139,7 @@ __device__ __forceinline__ void move_wide_row(char *dense, char *table, char *se
 constexpr int kMaxLog2Tile = 5;
 constexpr int64_t kL2Bytes = 32ll << 20;      // the L2s together
 constexpr int64_t kCacheBytes = 256ll << 20;  // the memory-side cache
+constexpr int64_t kLargeOutput = 160ll << 20;  // an output that it does not hold beside the rows read
 
 // THROUGH (set only, with a map or mask): rows that hit the cache are written
 // to the id-addressed table as well, so that table never goes stale.
@@ -146,7 +147,7 @@ constexpr int64_t kCacheBytes = 256ll << 20;  // the memory-side cache
 // miss the cache are not moved; every tile leaves one word of a bitmap that
 // marks them for rows_missed_kernel (no counter, no atomics, nothing to clear).
 template <typename VT, int MODE, bool SET, int ROUTE, bool THROUGH = false, bool DEFER = false>
-__global__ __launch_bounds__(kRowsBlock, rows_waves_per_simd(SET, ROUTE, sizeof(VT))) void rows_kernel(RowArgs a) {
+__global__ __launch_bounds__(kRowsBlock, rows_waves_per_simd(SET, THROUGH, ROUTE, sizeof(VT))) void rows_kernel(RowArgs a) {
   static_assert(!THROUGH || (SET && MODE != kDirect), "write-through is a cached set");
   static_assert(!DEFER || (!SET && MODE != kDirect), "only a cached fetch sets its misses aside");
   const int lane = lane_id();
@@ -563,33 +564,35 @@ static void launch_vec(int route, bool through, int mode, unsigned grid, hipStre
 // Rows of more vectors than this go one by one (kWide), shorter ones that fill no lane group are dealt out. All hits,
 // us for 100 MB of output or update in all (for 400 MB), dealt out / one by one:
 //   fetch  16-byte vectors  65: 50 / 42 (156 / 190), 75: 54 / 41 (171 / 190), 88: 58 / 41 (187 / 164), 128: 46 / 36 (163 / 166)
-//          8-byte           65: 55 / 46 (186 / 194), 89: 63 / 43 (187 / 190), 145: 74 / 42 (201 / 191)
+//          8-byte           65: 55 / 46 (186 / 194), 75: 59 / 45 (185 / 192; 314 MB 140 / 158), 89: 63 / 43 (187 / 190), 145: 74 / 42 (201 / 191)
 //          4-byte           65: 30 / 38 (251 / 234), 89: 53 / 43 (243 / 200), 257: 122 / 55 (329 / 231)
-//          2-byte           65: 25 / 25 (231 / 249), 89: 32 / 25 (348 / 273), 257: 140 / 65 (538 / 255)
+//          2-byte           65: 25 / 25 (231 / 249; 160 MB 110 / 149), 89: 32 / 25 (348 / 273), 257: 140 / 65 (538 / 255)
 //          1-byte           97: 27 / 24 (186 / 221), 113: 31 / 24 (257 / 237), 257: 91 / 57 (607 / 355)
 //   set    16-byte          65: 54 / 57 (240 / 234), 75: 51 / 51 (233 / 227), 128: 41 / 44 (195 / 180)
-//          8-byte           75: 53 / 57 (234 / 249), 89: 54 / 54 (242 / 240), 145: 69 / 53 (243 / 232)
+//          8-byte           75: 53 / 57 (234 / 249), 97: 56 / 57 (254 / 244; 160 MB 90 / 98), 145: 69 / 53 (243 / 232)
 //          4-byte           97: 55 / 60 (236 / 261), 127: 67 / 68 (252 / 266), 145: 72 / 58 (249 / 251), 257: 112 / 81 (330 / 288)
 //          2-byte           75: 41 / 41 (291 / 291), 89: 47 / 42 (335 / 307), 257: 114 / 90 (398 / 334)
 //          1-byte           65: 41 / 25 (292 / 244), 257: 131 / 66 (793 / 381)
 // (With at most two loads in flight per lane, as dealt out, rows of 5 to 15 KB took up to 2.7 times as long.)
 static int64_t wide_from(bool set, int vector_bytes, int64_t dense_bytes) {
   switch (vector_bytes) {
-    case 16: return !set && dense_bytes > kCacheBytes ? 87 : 64;
-    case 8: return set ? 80 : 64;
+    case 16: return !set && dense_bytes > kLargeOutput ? 87 : 64;
+    case 8: return set ? 112 : dense_bytes > kLargeOutput ? 87 : 64;
     case 4: return set ? 128 : 80;
-    case 2: return set ? 80 : 64;
+    case 2: return 80;
     default: return set ? 64 : 112;
   }
 }
 
-// Whether `dense` is accessed past the caches (kWide). A fetch does so when its output is larger than the
-// memory-side cache (rows of 128 16-byte vectors, 400 MB: 178 us plain, 164 streaming; 100 MB: 36 / 38). A set does
-// so with an update that would push the rows it writes out of that cache (100 MB: 49 plain, 44 streaming), but not
-// with one small enough to lie in the L2s (512 vectors, 16 MB: 7.0 / 8.5) or beyond both (400 MB: 188 / 191).
-static bool stream_dense(bool set, int vector_bytes, int64_t dense_bytes) {
+// Whether `dense` is accessed past the caches (kWide). A fetch does so when the memory-side cache cannot hold its
+// output (rows of 128 16-byte vectors, 400 MB: 178 us plain, 164 streaming; 100 MB: 36 / 38). A set does so with an
+// update that would push the rows it writes out of that cache (100 MB: 49 plain, 44 streaming), but not with one
+// small enough to lie in the L2s (512 vectors, 16 MB: 7.0 / 8.5), nor, when it is larger than the cache, with rows
+// that do not end on a line (100 vectors, 400 MB: 193 / 213).
+static bool stream_dense(bool set, int vector_bytes, int64_t row_bytes, int64_t dense_bytes) {
   if (!may_stream(set, vector_bytes)) return false;
-  return set ? dense_bytes > kL2Bytes && dense_bytes <= kCacheBytes : dense_bytes > kCacheBytes;
+  if (!set) return dense_bytes > kLargeOutput;
+  return dense_bytes > kL2Bytes && (dense_bytes <= kCacheBytes || row_bytes % 128 == 0);
 }
 
 template <bool SET>
@@ -645,7 +648,7 @@ static int move_rows(const char *who, void *miss, void *cache, const void *indic
   const bool one_vec = nvec == lanes || (!SET && vb == 16 && lanes < kWave && nvec < lanes && 4 * nvec >= 3 * lanes);
   const int64_t dense_bytes = Q * row_bytes;
   const int route = one_vec ? kOneVec : nvec > wide_from(SET, vb, dense_bytes) ? kWide : kDealt;
-  a.stream_dense = stream_dense(SET, vb, dense_bytes);
+  a.stream_dense = stream_dense(SET, vb, row_bytes, dense_bytes);
   a.nvec = route == kDealt ? static_cast<uint32_t>(nvec) : 0u;
   a.nvec_magic = route == kDealt ? 0xFFFFFFFFu / a.nvec : 0u;
   int log2_tile = kMaxLog2Tile;
@@ -657,7 +660,7 @@ static int move_rows(const char *who, void *miss, void *cache, const void *indic
   // As many workgroups as the device holds at once (256 units x 8 waves per SIMD): beyond that a wave takes
   // several tiles and keeps the lookups of the next ones in flight while it moves rows.
   const unsigned grid = grid_for(Q, static_cast<int64_t>(kRowsBlock / kWave) << log2_tile,
-                                 256 * rows_waves_per_simd(SET, route, vb));
+                                 256 * rows_waves_per_simd(SET, through, route, vb));
   hipStream_t s = as_stream(stream);
   if (miss_bits) {
     SHMT_REQUIRE(!SET && mode != kDirect, "%s: only a fetch through a hashmap or mask sets its misses aside", who);
