@@ -409,15 +409,18 @@ __device__ __forceinline__ int64_t half_wave_finish(const MapView &m, int64_t my
     if (sub == j) res = raw;
   }
   for (uint32_t round = 1; open != 0 && round < m.nbuckets; ++round) {  // some bucket was full of other keys: walk on
-#pragma unroll
+#pragma unroll 1
     for (int j = 0; j < kHalfWaveKeys; ++j) {
       if (((open >> j) & kGroupBits) == 0) continue;
       const int64_t key = shfl64(mykey, grp * kHalfWaveKeys + j);
-      uint32_t b = map_bucket(m, key) + round;
-      if (b >= m.nbuckets) b -= m.nbuckets;
+      uint4 frag = make_uint4(0, 0, 0, 0);  // (a group whose key is resolved reads no line)
+      if ((open >> (grp * kProbeGroup + j)) & 1ull) {
+        uint32_t b = map_bucket(m, key) + round;
+        if (b >= m.nbuckets) b -= m.nbuckets;
+        frag = m.buckets[static_cast<size_t>(b) * kProbeGroup + sub];
+      }
       uint64_t raw;
-      const uint64_t still = probe_buckets<FMT>(m, m.buckets[static_cast<size_t>(b) * kProbeGroup + sub],
-                                                probe_want<FMT>(m, key), &raw) << j;
+      const uint64_t still = probe_buckets<FMT>(m, frag, probe_want<FMT>(m, key), &raw) << j;
       if (sub == j && ((open >> lane) & 1ull)) res = raw;
       open &= still | ~(kGroupBits << j);
     }
