@@ -166,7 +166,10 @@ __global__ __launch_bounds__(256) void hashmap_insert_kernel(
 //   fill   one workgroup per partition.
 //   rest   words that found no room in the reserve of their partition (many
 //          pairs of one key) or in the last buckets of the partition: inserted
-//          one by one, as the general build does for all. Hardly ever any.
+//          one by one, as the general build does for all. Hardly ever any when
+//          keys differ; of keys given many times, deal drops most repeats itself.
+// Repeats, 4,194,304 pairs, whole constructor in place / by partitions: half on one key 870 / 111 us, 64 keys 201 / 96,
+// 4,194 keys 111 / 127, 41,943 keys 118 / 121; 1,048,576 pairs of 10,486 keys 60 / 82, where hardly anything is inserted.
 // 4,194,304 pairs of 16 bytes: clear 23 + insert 212 us before (16-byte slots; 13 + 191 with packed words), deal 33 +
 // fill 37 + rest 5 us now. Deal reads 67 MB and writes 34, fill reads 34 and writes 67: 3 TB/s and 2.7 TB/s, with
 // one and two workgroups per compute unit whose phases (load, count, order, write) hardly overlap.
@@ -176,6 +179,8 @@ constexpr int kPartLog2Buckets = 9;
 constexpr int kPartBuckets = 1 << kPartLog2Buckets;  // 64 KB of LDS: two workgroups per compute unit
 constexpr int kPartMax = 2048;                       // partitions a dealing workgroup counts in LDS
 constexpr int kPartBlock = 1024;
+constexpr uint32_t kPartLookBack = 16;    // words in which a repeat of a key is looked for
+constexpr int kPartRestBlocks = 1024;     // (none to do: 4 us, as with 64)
 
 struct PartArgs {
   MapView map;
@@ -201,6 +206,8 @@ __global__ __launch_bounds__(kPartBlock) void part_deal_kernel(PartArgs a) {
   __shared__ uint32_t start[kPartMax];  // words per partition, then where they start in `staged`
   __shared__ uint32_t base[kPartMax];   // where they go in the partition, minus start
   __shared__ uint32_t lds[kPartBlock / kWave];
+  __shared__ uint32_t late_count, late_base;
+  if (threadIdx.x == 0) late_count = 0;
   for (uint32_t p = threadIdx.x; p < kPartMax; p += kPartBlock) start[p] = 0;
   __syncthreads();
   const int64_t first = static_cast<int64_t>(blockIdx.x) * (ITEMS * kPartBlock);
@@ -245,15 +252,34 @@ __global__ __launch_bounds__(kPartBlock) void part_deal_kernel(PartArgs a) {
   for (int j = 0; j < ITEMS; ++j)
     if (ok[j]) staged[start[place[j] >> 16] + (place[j] & 0xFFFFu)] = word[j];
   __syncthreads();
-  for (uint32_t e = threadIdx.x; e < total; e += kPartBlock) {
+  // Words without room. A partition that overflows holds few keys many times: a word whose key stands shortly before
+  // it is dropped. One reservation per workgroup (a counter that every wave asks takes 250 us of a 4 M-pair deal).
+  const uint64_t field = 1ull << a.map.val_bits;
+  uint32_t late[ITEMS];  // place among the workgroup's words without room, ~0: none
+#pragma unroll
+  for (int j = 0; j < ITEMS; ++j) {
+    const uint32_t e = j * kPartBlock + threadIdx.x;
+    late[j] = ~0u;
+    if (e >= total) continue;
     const uint64_t w = staged[e];
     const uint32_t p = part_of(a.map, w);
     const uint32_t to = base[p] + e;
-    if (to < a.room)
+    if (to < a.room) {
       a.words[static_cast<size_t>(p) * a.room + to] = w;
-    else
-      a.rest[atomicAdd(a.rest_count, 1u)] = w;
+    } else {
+      const uint32_t from = e - start[p] > kPartLookBack ? e - kPartLookBack : start[p];
+      bool again = false;
+      for (uint32_t b = e; b > from && !again; --b) again = (staged[b - 1] ^ w) < field;
+      if (!again) late[j] = atomicAdd(&late_count, 1u);
+    }
   }
+  __syncthreads();
+  if (late_count == 0) return;
+  if (threadIdx.x == 0) late_base = atomicAdd(a.rest_count, late_count);
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < ITEMS; ++j)
+    if (late[j] != ~0u) a.rest[late_base + late[j]] = staged[j * kPartBlock + threadIdx.x];
 }
 
 __global__ __launch_bounds__(kPartBlock) void part_fill_kernel(PartArgs a) {
@@ -867,7 +893,7 @@ static int build_buckets(shmt_hashmap_t **out, const int fmt, const void *keys, 
       hipLaunchKernelGGL(part_deal_kernel<4>, dim3(static_cast<unsigned>((n + 4 * kPartBlock - 1) / (4 * kPartBlock))),
                          dim3(kPartBlock), 0, s, a);
     hipLaunchKernelGGL(part_fill_kernel, dim3(parts.parts), dim3(kPartBlock), 0, s, a);
-    hipLaunchKernelGGL(part_rest_kernel, dim3(64), dim3(256), 0, s, a);
+    hipLaunchKernelGGL(part_rest_kernel, dim3(kPartRestBlocks), dim3(256), 0, s, a);
     SHMT_LAUNCH_CHECK();
   } else {
     int rc = launch_fill_ones(table_mem, nb * (kBucketBytes / 16), s);

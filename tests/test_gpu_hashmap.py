@@ -379,6 +379,35 @@ def test_large_narrow_tables_are_built_by_partitions(capi, case):
         assert bool((h.query(wide[:5000] ^ (1 << 45)) == -1).all())
 
 
+@pytest.mark.parametrize("n", [(1 << 18) + 77, (1 << 21) + 5])
+@pytest.mark.parametrize("repeats", ["half_on_one", "64_keys", "1000_each", "100_each", "runs_of_30", "17_in_turn"])
+@pytest.mark.parametrize("bits", [30, 41])
+def test_repeated_keys_in_tables_built_by_partitions(capi, n, repeats, bits):
+    """Keys given many times outgrow the room of their partitions: whatever the order in which the repeats come (more
+    or fewer keys between two of them than a dealing workgroup looks back), every key gives one of its values and
+    nothing else is in the table."""
+    g = torch.Generator(device="cuda").manual_seed(11)
+    pool = torch.unique(torch.randint(0, 1 << bits, (n + n // 8,), device="cuda", generator=g))
+    pool = pool[torch.randperm(pool.numel(), device="cuda", generator=g)][:n]
+    if repeats == "half_on_one":
+        keys = torch.where(torch.rand(n, device="cuda", generator=g) < 0.5, pool[:1], pool)
+    elif repeats == "runs_of_30":
+        keys = pool.repeat_interleave(30)[:n]
+    elif repeats == "17_in_turn":      # (17 keys one after the other, over and over, then others)
+        keys = torch.cat([pool[:17].repeat(n // 34), pool[: n - n // 34 * 17]])
+    else:
+        distinct = {"64_keys": 64, "1000_each": n // 1000, "100_each": n // 100}[repeats]
+        keys = pool[torch.randint(0, distinct, (n,), device="cuda", generator=g)]
+    keys = keys.contiguous()
+    keys[0], keys[1] = 0, (1 << bits) - 1          # (the table is neither an id range nor direct)
+    h = capi.CUCOStaticHashmap(keys, torch.arange(n, device="cuda"), 0.5)
+    assert h.layout() == "buckets"
+    got = h.query(keys)
+    assert bool(((got >= 0) & (got < n)).all()) and torch.equal(keys[got], keys)
+    others = pool[~torch.isin(pool, keys)]
+    assert bool((h.query(others) == -1).all())
+
+
 @pytest.mark.parametrize("n,packs", [((4 << 20) // 32, False), ((4 << 20) // 32 + 1, True)])
 def test_values_and_spans_that_just_pack(capi, n, packs):
     """The line of the packed form: more than 131,072 pairs, and key distances and values that share 64 bits. The
