@@ -224,16 +224,18 @@ __global__ __launch_bounds__(1024) void plan_totals_kernel(uint64_t *partials, i
 
 // Many seeds on a graph of not so many rows: a cold seed costs the plan a
 // 128-byte line over the host link for its two offsets (and lines are not
-// shared between the XCDs), so from some number of cold seeds on it is cheaper
+// shared between the XCDs), so from some number of lines on it is cheaper
 // to copy the row offsets to HBM first, in order and at the rate of a long
-// copy. How many seeds are cold only the map knows: every workgroup looks up
-// the same kStageSamples seeds, spread over all of them, and so all
-// come to the same answer without talking to each other; when too few are cold
-// nothing is copied and the plan reads as it always did. 100,000 seeds on
+// copy. How many seeds are cold only the map knows, and how many lines they
+// need depends on their order (seeds in id order share them): every workgroup
+// looks up the same kStageSamples seeds, runs of kStageRun in a row spread over
+// all of them, counts the lines each run needs, and so all
+// come to the same answer without talking to each other; when too few lines are needed
+// nothing is copied and the plan reads as it always did. 100,000 seeds in random order on
 // 400,000 rows of which 30 % are cached: plan 191 us, copy 66 + plan 6 now. Where 90 % of the seeds are cached
 // the launch and the lookups cost 122 -> 125 us (131 with 1,024 samples).
 constexpr int kStageBlock = 256, kStageBlocks = 64;  // 64 workgroups fill the link (4 MB: 53 GB/s; 512: 47)
-constexpr int kStageSamples = 256;
+constexpr int kStageSamples = 256, kStageRun = 16;
 constexpr int64_t kLinkLine = 128;
 constexpr int64_t kStageMargin = 512 << 10;  // what the link carries while the extra launch and the lookups run
 
@@ -243,6 +245,7 @@ struct StageArgs {
   int64_t bytes;
   const void *seeds;
   int seed_bytes;
+  int ptr_bytes;
   int64_t S;
   MapView map;
   uint32_t *ok;
@@ -250,27 +253,27 @@ struct StageArgs {
 
 template <int MODE>
 __global__ __launch_bounds__(kStageBlock) void stage_rows_kernel(StageArgs a) {
-  if (MODE != 0) {
-    __shared__ uint32_t cold_lds[kStageBlock / kWave];
-    const int64_t samples = a.S < kStageSamples ? a.S : kStageSamples;
-    uint32_t cold = 0;
-    for (int base = 0; base < kStageSamples; base += kStageBlock) {  // (whole waves: the lookups are cooperative)
-      const int64_t j = base + threadIdx.x;
-      int64_t key = -1;
-      if (j < samples) key = map_key(a.map, load_int(a.seeds, j * a.S / samples, a.seed_bytes));
-      const int64_t slot = MODE == 1 ? wave_find<kSlot16>(a.map, key) : wave_find<kSlot8>(a.map, key);
-      cold += static_cast<uint32_t>(__builtin_popcountll(__builtin_amdgcn_ballot_w64(j < samples && slot < 0)));
-    }
-    if (lane_id() == 0) cold_lds[threadIdx.x / kWave] = cold;
-    __syncthreads();
-    cold = 0;
-    for (int w = 0; w < kStageBlock / kWave; ++w) cold += cold_lds[w];
-    const bool worth = static_cast<int64_t>(cold) * a.S / samples * kLinkLine >= a.bytes + kStageMargin;
-    if (blockIdx.x == 0 && threadIdx.x == 0) *a.ok = worth ? 1u : 0u;
-    if (!worth) return;
-  } else if (blockIdx.x == 0 && threadIdx.x == 0) {
-    *a.ok = 1u;
+  __shared__ uint32_t lines_lds[kStageBlock / kWave];
+  static_assert(kStageSamples == kStageBlock && kWave % kStageRun == 0, "one sample per thread, runs within a wave");
+  const int run = threadIdx.x / kStageRun, in_run = threadIdx.x % kStageRun;
+  const int64_t first = run * (a.S - kStageRun) / (kStageSamples / kStageRun - 1);  // (S >= kStageRun)
+  const int64_t node = load_int(a.seeds, first + in_run, a.seed_bytes);
+  const int64_t slot = MODE == 0 ? -1 : MODE == 1 ? wave_find<kSlot16>(a.map, map_key(a.map, node))
+                                                  : wave_find<kSlot8>(a.map, map_key(a.map, node));
+  const int64_t line = slot < 0 ? node * a.ptr_bytes / kLinkLine : -1;
+  bool counts = slot < 0;
+  for (int d = 1; d < kStageRun; ++d) {
+    const int64_t other = shfl64(line, lane_id() - d);
+    counts = counts && !(in_run >= d && other == line);
   }
+  const uint64_t counted = __builtin_amdgcn_ballot_w64(counts);
+  if (lane_id() == 0) lines_lds[threadIdx.x / kWave] = static_cast<uint32_t>(__builtin_popcountll(counted));
+  __syncthreads();
+  uint32_t lines = 0;
+  for (int w = 0; w < kStageBlock / kWave; ++w) lines += lines_lds[w];
+  const bool worth = static_cast<int64_t>(lines) * a.S / kStageSamples * kLinkLine >= a.bytes + kStageMargin;
+  if (blockIdx.x == 0 && threadIdx.x == 0) *a.ok = worth ? 1u : 0u;
+  if (!worth) return;
   constexpr int kHeld = 4;  // 16-byte loads a lane has in flight
   const int64_t n16 = a.bytes / 16, stride = static_cast<int64_t>(gridDim.x) * kStageBlock;
   const uint4 *const src = reinterpret_cast<const uint4 *>(a.src);
@@ -1178,6 +1181,7 @@ int shmt_sample_staged(const void *indptr, int ptr_bytes, int64_t rows, const vo
     a.bytes = (rows + 1) * ptr_bytes;
     a.seeds = seeds;
     a.seed_bytes = seed_bytes;
+    a.ptr_bytes = ptr_bytes;
     a.S = S;
     if (map) a.map = map->view; else a.map = empty_map_view();
     a.ok = static_cast<uint32_t *>(stage);

@@ -277,3 +277,47 @@ def test_many_seeds_on_few_rows_of_host_memory(capi, ptr, rows, S, cached):
     shifted[1:].copy_(indptr)
     got = capi.csr_sampling(shifted[1:], hi, seeds, 5, False, seed=9)
     assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+
+
+@pytest.mark.parametrize("order,copied", [("random", 1), ("sorted", 0), ("consecutive", 0), ("descending", 0), ("one row", 0)])
+@pytest.mark.parametrize("mapped", [False, True])
+def test_row_offsets_are_copied_only_for_the_lines_they_save(cabi, order, copied, mapped):
+    """200,000 row offsets (1.6 MB) and 40,000 cold seeds: in random order each needs a line of its own (5 MB) and the
+    offsets are copied first; seeds in id order share lines and are read where they are. Same samples either way."""
+    import ctypes
+    lib, stream = cabi.load(), cabi.current_stream()
+    rows, S, k = 200_000, 40_000, 3
+    g = torch.Generator(device="cuda").manual_seed(4)
+    indptr = torch.zeros(rows + 1, dtype=torch.int64, device="cuda")
+    torch.cumsum(torch.randint(0, 9, (rows,), device="cuda", generator=g), 0, out=indptr[1:])
+    indices = torch.randint(0, rows, (int(indptr[-1]),), device="cuda", generator=g, dtype=torch.int32)
+    seeds = {"random": torch.randperm(rows, device="cuda", generator=g)[:S],
+             "sorted": torch.sort(torch.randperm(rows // 2, device="cuda", generator=g)[:S]).values,
+             "consecutive": torch.arange(70_000, 70_000 + S, device="cuda"),
+             "descending": torch.arange(S - 1, -1, -1, device="cuda"),
+             "one row": torch.full((S,), 123, device="cuda")}[order].contiguous()
+    handle, table = ctypes.c_void_p(), torch.empty(lib.shmt_hashmap_table_bytes(8, 0.5, 8, 8), dtype=torch.uint8, device="cuda")
+    none = torch.arange(rows, rows + 8, device="cuda")     # (a map that holds none of the seeds)
+    if mapped:
+        cabi.check(lib.shmt_hashmap_create(ctypes.byref(handle), none.data_ptr(), none.data_ptr(), 8, 8, 8, 0.5, table.data_ptr(),
+                                           table.numel(), stream))
+    graph = (indptr.data_ptr(), 8, rows, indices.data_ptr(), 4) + ((indptr.data_ptr(), indices.data_ptr(), handle) if mapped
+                                                                  else (None, None, None))
+    plan = torch.empty(lib.shmt_sample_plan_bytes(S), dtype=torch.uint8, device="cuda")
+    stage = torch.full((lib.shmt_sample_stage_bytes(rows, 8, S),), 255, dtype=torch.uint8, device="cuda")
+    results = []
+    for st in (stage, None):
+        sp, si = torch.empty(S + 1, dtype=torch.int64, device="cuda"), torch.zeros(S * k, dtype=torch.int32, device="cuda")
+        nnz = torch.zeros(1, dtype=torch.int64, pin_memory=True)
+        cabi.check(lib.shmt_sample_staged(*graph, seeds.data_ptr(), 8, S, k, 0, 7, 0, sp.data_ptr(), si.data_ptr(), plan.data_ptr(),
+                                          plan.numel(), st.data_ptr() if st is not None else None,
+                                          st.numel() if st is not None else 0, nnz.data_ptr(), stream))
+        torch.cuda.synchronize()
+        results.append((sp, si, int(nnz)))
+    assert torch.equal(results[0][0], results[1][0]) and torch.equal(results[0][1], results[1][1])
+    assert results[0][2] == results[1][2]
+    assert int(stage[:4].view(torch.int32)) == copied
+    if copied:
+        assert torch.equal(stage[128:128 + 8 * (rows + 1)].view(torch.int64), indptr)
+    if mapped:
+        lib.shmt_hashmap_destroy(handle)
