@@ -275,16 +275,18 @@ std::tuple<torch::Tensor, torch::Tensor> sample_impl(const torch::Tensor &indptr
   torch::Tensor sub_indices;
   if (eager) {
     sub_indices = torch::empty({S * num_picks}, indices.options().device(dev));
-    // many seeds on few rows of host memory: their offsets may be copied to the GPU first
-    const int64_t rows = indptr.numel() - 1;
-    const int64_t stage_bytes = indptr.is_cuda() || rows < 1 ? 0 : shmt_sample_stage_bytes(rows, pb, S);
-    torch::Tensor stage;
-    if (stage_bytes > 0) stage = device_bytes(stage_bytes);
-    check(shmt_sample_staged(indptr_dev, pb, rows, indices_dev, ib, map ? gpu_indptr->data_ptr() : nullptr,
-                             map ? gpu_indices->data_ptr() : nullptr, map ? map->handle() : nullptr, seeds.data_ptr(),
-                             sb, S, num_picks, replace, rng_seed, static_cast<uint32_t>(stream_id),
-                             sub_indptr.data_ptr(), sub_indices.data_ptr(), plan.data_ptr(), plan_bytes,
-                             stage_bytes > 0 ? stage.data_ptr() : nullptr, stage_bytes, total.dev, stream));
+    {
+      // many seeds on few rows of host memory: their offsets may be copied to the GPU first
+      const int64_t rows = indptr.numel() - 1;
+      const int64_t stage_bytes = indptr.is_cuda() || rows < 1 ? 0 : shmt_sample_stage_bytes(rows, pb, S);
+      const torch::Tensor stage = spare_device_bytes(stage_bytes);
+      check(shmt_sample_staged(indptr_dev, pb, rows, indices_dev, ib, map ? gpu_indptr->data_ptr() : nullptr,
+                               map ? gpu_indices->data_ptr() : nullptr, map ? map->handle() : nullptr, seeds.data_ptr(),
+                               sb, S, num_picks, replace, rng_seed, static_cast<uint32_t>(stream_id),
+                               sub_indptr.data_ptr(), sub_indices.data_ptr(), plan.data_ptr(), plan_bytes,
+                               stage.defined() ? stage.data_ptr() : nullptr, stage.defined() ? stage_bytes : 0, total.dev,
+                               stream));
+    }
     const int64_t nnz = Readback::wait(total);
     // a view keeps the whole bound-sized buffer alive: hand back a copy when most of a large one is unused
     const bool mostly_unused = nnz < S * num_picks / 4 && S * num_picks * ib > (16ll << 20);
@@ -332,15 +334,25 @@ std::tuple<torch::Tensor, torch::Tensor> create_subcsr(torch::Tensor uva_indptr,
   const Readback::Slot total = readback().acquire();
   void *stream = current_stream();
   void *indptr_dev = device_address(uva_indptr, "uva_indptr");
-  torch::Tensor begins = torch::empty({C}, seeds.options().dtype(torch::kInt64));
+  torch::Tensor begins = spare_device_bytes(C * 8);
+  int64_t *row_begins = begins.defined() ? static_cast<int64_t *>(begins.data_ptr()) : nullptr;
   check(shmt_subcsr_plan_rows(indptr_dev, pb, seeds.data_ptr(), static_cast<int>(seeds.element_size()), C,
-                              gpu_indptr.data_ptr(), begins.data_ptr<int64_t>(), tmp.data_ptr(), tmp_bytes, total.dev,
+                              gpu_indptr.data_ptr(), row_begins, tmp.data_ptr(), tmp_bytes, total.dev,
                               stream));
   const int64_t nnz = Readback::wait(total);
-  torch::Tensor gpu_indices = torch::empty({nnz}, uva_indices.options().device(torch::kCUDA));
+  torch::Tensor gpu_indices;
+  const auto index_options = uva_indices.options().device(torch::kCUDA);
+  try {
+    gpu_indices = torch::empty({nnz}, index_options);
+  } catch (const c10::OutOfMemoryError &) {
+    if (!begins.defined()) throw;
+    begins.reset();
+    row_begins = nullptr;
+    gpu_indices = torch::empty({nnz}, index_options);
+  }
   check(shmt_subcsr_copy_rows(indptr_dev, device_address(uva_indices, "uva_indices"), pb, ib,
                               seeds.data_ptr(), static_cast<int>(seeds.element_size()), C,
-                              gpu_indptr.data_ptr(), begins.data_ptr<int64_t>(), nnz, gpu_indices.data_ptr(), stream));
+                              gpu_indptr.data_ptr(), row_begins, nnz, gpu_indices.data_ptr(), stream));
   return std::make_tuple(gpu_indptr, gpu_indices);
 }
 

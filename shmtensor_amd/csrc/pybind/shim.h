@@ -163,6 +163,16 @@ inline torch::Tensor device_bytes(int64_t nbytes) {
                       torch::TensorOptions().dtype(torch::kUInt8).device(torch::kCUDA));
 }
 
+// Memory that makes a call faster but that it can do without: undefined when there is none left.
+inline torch::Tensor spare_device_bytes(int64_t nbytes) {
+  if (nbytes <= 0) return torch::Tensor();
+  try {
+    return device_bytes(nbytes);
+  } catch (const c10::OutOfMemoryError &) {
+    return torch::Tensor();
+  }
+}
+
 // ---- hashmap ---------------------------------------------------------------
 
 class StaticHashmap {
@@ -205,12 +215,11 @@ class StaticHashmap {
     memory_usage_ = layout.kind == SHMT_MAP_RANGE ? 0 : layout.table_bytes;
     kind_ = layout.kind;
     const int64_t build_bytes = shmt_hashmap_build_scratch_bytes(&layout, n, load_factor);
-    torch::Tensor build_scratch;
-    if (build_bytes > 0) build_scratch = device_bytes(build_bytes);
+    const torch::Tensor build_scratch = spare_device_bytes(build_bytes);
     check(shmt_hashmap_create_planned_scratch(&handle_, &layout, keys.data_ptr(), values.data_ptr(), n, kb, vb,
                                               load_factor, table_.data_ptr(), layout.table_bytes,
-                                              build_bytes > 0 ? build_scratch.data_ptr() : nullptr, build_bytes,
-                                              current_stream()));
+                                              build_scratch.defined() ? build_scratch.data_ptr() : nullptr,
+                                              build_scratch.defined() ? build_bytes : 0, current_stream()));
   }
   ~StaticHashmap() { shmt_hashmap_destroy(handle_); }
   StaticHashmap(const StaticHashmap &) = delete;

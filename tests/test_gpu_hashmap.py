@@ -476,3 +476,25 @@ def test_packed_layout_through_the_c_abi(cabi):
         cabi.check(lib.shmt_hashmap_query(handle, req.data_ptr(), 8, req.numel(), out.data_ptr(), stream))
         assert torch.equal(out, want)
         lib.shmt_hashmap_destroy(handle)
+
+
+def _leave_free(mib):
+    """Lets this process's allocator take `mib` MiB more than it holds now."""
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(0).total_memory
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (mib << 20)) / total)
+
+
+def test_map_without_memory_for_build_scratch(capi):
+    """A table that fits is built also where the 70 MB with which the build is faster do not."""
+    g = torch.Generator(device="cuda").manual_seed(9)
+    n = 1 << 22
+    keys = torch.unique(torch.randint(0, 1 << 40, (n + n // 8,), device="cuda", generator=g))
+    keys, vals = keys[torch.randperm(keys.numel(), device="cuda", generator=g)][:n].contiguous(), torch.arange(n, device="cuda")
+    try:
+        _leave_free(64 + 40)          # table 64 MiB, plan 4.5 MB
+        h = capi.CUCOStaticHashmap(keys, vals, 0.5)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert torch.equal(h.query(keys), vals) and bool((h.query(keys[:1000] + (1 << 41)) == -1).all())

@@ -321,3 +321,24 @@ def test_row_offsets_are_copied_only_for_the_lines_they_save(cabi, order, copied
         assert torch.equal(stage[128:128 + 8 * (rows + 1)].view(torch.int64), indptr)
     if mapped:
         lib.shmt_hashmap_destroy(handle)
+
+
+def test_sub_graph_without_memory_for_row_starts(capi):
+    """A sub-graph that fits is copied also where the 8 bytes per row that save host-link reads do not."""
+    rows = 4_000_000
+    indptr = torch.arange(0, 5 * rows + 1, 5, dtype=torch.int32)
+    indices = torch.arange(5 * rows, dtype=torch.int32)
+    seeds = torch.arange(rows, device="cuda")
+    hp, hi = indptr.pin_memory(), indices.pin_memory()
+    want = (5 * rows * 4 + (rows + 1) * 4) >> 20            # 80 MB + 16 MB
+    total = torch.cuda.get_device_properties(0).total_memory
+    for spare in (12, 40, 60):        # no room for the row starts (32 MB); for them alone; for all
+        torch.cuda.synchronize()
+        torch.cuda.empty_cache()
+        try:
+            torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + ((want + spare) << 20)) / total)
+            gp, gi = capi.create_subcsr(hp, hi, seeds)
+        finally:
+            torch.cuda.set_per_process_memory_fraction(1.0)
+        assert torch.equal(gp.cpu(), indptr) and torch.equal(gi.cpu(), indices)
+        del gp, gi
