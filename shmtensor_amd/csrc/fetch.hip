@@ -54,10 +54,11 @@ struct RowArgs {
   int64_t row_bytes;
   int idx_bytes;
   int mask_bytes;
-  int log2_lanes;      // lanes per row in phase 2 = 1 << log2_lanes, in [8, 64] (kOneVec)
+  int log2_lanes;      // lanes per row in phase 2 = 1 << log2_lanes, in [8, 64]
   int log2_tile;       // rows per wave tile = 1 << log2_tile, at most 32
   uint32_t nvec;        // vectors per row (kDealt)
   uint32_t nvec_magic;  // floor((2^32 - 1) / nvec): the high half of i * magic is i / nvec, or one less
+  uint32_t group_step;  // kDealt: vectors that a wave moves at a time with a lane group per row; 0: always dealt out
   int stream_dense;     // kWide: `dense` is accessed past the caches
   uint32_t *miss_bits;  // DEFER: bit (i & 31) of word i / 32 is set when row i missed the cache
 };
@@ -315,14 +316,25 @@ __global__ __launch_bounds__(kRowsBlock, rows_waves_per_simd(SET, THROUGH, ROUTE
       constexpr int kVecsInFlight = vecs_in_flight(SET, sizeof(VT));
       const uint32_t total = static_cast<uint32_t>(nrows) * a.nvec;
       char *const dense = a.dense + base * R;  // the tile's rows lie one behind the other
-      for (uint32_t v0 = 0; v0 < total; v0 += kVecsInFlight * kWave) {
+      // Rows that come over the host link get a lane group each after all: a row that is split between two steps, or
+      // whose vectors are shifted against the groups of four lanes that read a line together, costs link reads (16,384
+      // rows, 5 % hits, 50 floats: 95 us in lane groups, 101 dealt out; 20 floats: 66 / 67.5), unless a lane group would
+      // be half empty (33 floats: 78 / 81, with 90 % hits 15.0 / 13.7). From one row in 16 on the link is what the
+      // tile waits for.
+      uint32_t per_step = kVecsInFlight * kWave, my_vec = lane;
+      if (!SET && !DEFER && a.group_step &&
+          16 * __builtin_popcountll(__builtin_amdgcn_ballot_w64(live && slot < 0)) >= nrows) {
+        per_step = a.group_step;
+        my_vec = static_cast<uint32_t>(gl) < a.nvec ? static_cast<uint32_t>(grp) * a.nvec + gl : 1u << 31;  // (an idle lane)
+      }
+      for (uint32_t v0 = 0; v0 < total; v0 += per_step) {
         VT v[kVecsInFlight];
         char *at[kVecsInFlight];
         char *second[kVecsInFlight];
         bool on[kVecsInFlight];
 #pragma unroll
         for (int u = 0; u < kVecsInFlight; ++u) {  // (every lane takes part in the shuffles)
-          const uint32_t i = v0 + u * kWave + lane;
+          const uint32_t i = v0 + u * kWave + my_vec;
           uint32_t row = __umulhi(i, a.nvec_magic);
           uint32_t vec = i - row * a.nvec;
           if (vec >= a.nvec) {
@@ -343,7 +355,7 @@ __global__ __launch_bounds__(kRowsBlock, rows_waves_per_simd(SET, THROUGH, ROUTE
         for (int u = 0; u < kVecsInFlight; ++u) {
           if (!on[u]) continue;
           if (SET)
-            v[u] = __builtin_nontemporal_load(reinterpret_cast<const VT *>(dense) + (v0 + u * kWave + lane));
+            v[u] = __builtin_nontemporal_load(reinterpret_cast<const VT *>(dense) + (v0 + u * kWave + my_vec));
           else
             v[u] = gload<VT>(at[u]);
         }
@@ -354,7 +366,7 @@ __global__ __launch_bounds__(kRowsBlock, rows_waves_per_simd(SET, THROUGH, ROUTE
             gstore<VT>(at[u], v[u]);
             if (THROUGH && second[u]) gstore<VT>(second[u], v[u]);
           } else {
-            __builtin_nontemporal_store(v[u], reinterpret_cast<VT *>(dense) + (v0 + u * kWave + lane));
+            __builtin_nontemporal_store(v[u], reinterpret_cast<VT *>(dense) + (v0 + u * kWave + my_vec));
           }
         }
       }
@@ -595,6 +607,13 @@ static bool stream_dense(bool set, int vector_bytes, int64_t row_bytes, int64_t 
   return dense_bytes > kL2Bytes && (dense_bytes <= kCacheBytes || row_bytes % 128 == 0);
 }
 
+static bool in_host_memory(const void *p) {
+  hipPointerAttribute_t attr;
+  if (hipPointerGetAttributes(&attr, p) == hipSuccess) return attr.type == hipMemoryTypeHost;
+  (void)hipGetLastError();
+  return false;
+}
+
 template <bool SET>
 static int move_rows(const char *who, void *miss, void *cache, const void *indices, int idx_bytes,
                      const shmt_hashmap_t *map, const void *mask, int mask_bytes, void *dense,
@@ -647,10 +666,15 @@ static int move_rows(const char *who, void *miss, void *cache, const void *indic
   const int64_t lanes = 1ll << log2_lanes;
   const bool one_vec = nvec == lanes || (!SET && vb == 16 && lanes < kWave && nvec < lanes && 4 * nvec >= 3 * lanes);
   const int64_t dense_bytes = Q * row_bytes;
-  const int route = one_vec ? kOneVec : nvec > wide_from(SET, vb, dense_bytes) ? kWide : kDealt;
+  // (misses of a fetch: rows over the host link)
+  const bool link = !SET && !one_vec && in_host_memory(miss);
+  const int64_t dealt_most = link && mode == kDirect ? kWave : wide_from(SET, vb, dense_bytes);
+  const int route = one_vec ? kOneVec : nvec > dealt_most ? kWide : kDealt;
   a.stream_dense = stream_dense(SET, vb, row_bytes, dense_bytes);
   a.nvec = route == kDealt ? static_cast<uint32_t>(nvec) : 0u;
   a.nvec_magic = route == kDealt ? 0xFFFFFFFFu / a.nvec : 0u;
+  const bool by_group = route == kDealt && link && nvec <= lanes && (mode == kDirect || 16 * nvec >= 9 * lanes);
+  a.group_step = by_group ? (kWave >> log2_lanes) * a.nvec : 0u;
   int log2_tile = kMaxLog2Tile;
   int log2_least = one_vec ? 6 - log2_lanes : 0;  // fewest rows per tile: a wave's worth of vectors, or eight
   while (!one_vec && log2_least < 3 && (nvec << log2_least) < kWave) ++log2_least;

@@ -607,3 +607,29 @@ def test_rows_of_64_mib(capi, D):
     g = torch.Generator(device="cuda").manual_seed(3)
     full, cache = (torch.randint(0, 256, (k, D), device="cuda", generator=g, dtype=torch.uint8) for k in (3, 2))
     _check_moves(capi, full, cache, torch.tensor([2, 0], device="cuda"), 3)
+
+
+@pytest.mark.parametrize("dtype,D", [(torch.float32, d) for d in (3, 5, 8, 20, 33, 47, 50, 100, 200)] +
+                         [(torch.float16, d) for d in (25, 50, 75, 100)] + [(torch.uint8, d) for d in (5, 25, 33, 63)])
+@pytest.mark.parametrize("hits", [0, 1, 25, 93, 94, 97, 100])
+@pytest.mark.parametrize("host", [True, False])
+def test_ragged_rows_that_miss(capi, dtype, D, hits, host):
+    """Short ragged rows by the share of them that hit the cache (in per cent): tiles with no miss, few and many (from
+    two rows of 32 on a tile takes a lane group per row), with the missed rows in host memory and on the GPU."""
+    g = torch.Generator(device="cuda").manual_seed(D + hits)
+    n = 2000
+    full, cache = (torch.randint(0, 100, (k, D), device="cuda", generator=g).to(dtype) for k in (n, max(1, n * hits // 100)))
+    hot = torch.randperm(n, device="cuda", generator=g)[: n * hits // 100]
+    table = torch.empty(n, D, dtype=dtype, pin_memory=True).copy_(full) if host else full
+    slots = torch.full((n,), -1, dtype=torch.int64, device="cuda")
+    slots[hot] = torch.arange(hot.numel(), device="cuda")
+    for q_len in (1, 31, 4000):
+        q = torch.randint(0, n, (q_len,), device="cuda", generator=g)
+        s = slots[q]
+        want = torch.where((s >= 0)[:, None], cache[s.clamp(min=0)], full[q])
+        assert torch.equal(capi.cache_fetch_with_mask(table, cache, q, s), want)
+        assert torch.equal(capi.uva_fetch(table, q), full[q])
+        if hot.numel():
+            for layout in ("auto", "buckets"):
+                h = capi.CUCOStaticHashmap(hot, torch.arange(hot.numel(), device="cuda"), 0.8, layout=layout)
+                assert torch.equal(capi.cache_fetch(table, cache, q, h), want)

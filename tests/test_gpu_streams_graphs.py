@@ -67,6 +67,28 @@ def test_fetch_query_and_set_replay_in_a_hip_graph(capi, cache):
         assert float(static_out.abs().sum()) > 0
 
 
+@pytest.mark.parametrize("dtype,D", [(torch.float32, 50), (torch.float16, 25), (torch.float32, 300), (torch.uint8, 1025)])
+def test_ragged_fetches_replay_in_a_hip_graph(capi, dtype, D):
+    """Rows that fill no lane group (whether their table lies in host memory is asked for on the host) and long rows."""
+    full = torch.randint(0, 100, (5000, D), device="cuda").to(dtype)
+    host = torch.empty(5000, D, dtype=dtype, pin_memory=True).copy_(full)
+    ids = torch.randperm(5000, device="cuda")[:3000]
+    cache, h = full[ids], capi.CUCOStaticHashmap(ids, torch.arange(3000, device="cuda"), 0.8)
+    q = torch.randint(0, 5000, (3000,), device="cuda")
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out, missed = capi.cache_fetch(host, cache, q, h), capi.uva_fetch(host, q)
+    for _ in range(4):           # replays with eager work and synchronisations in between
+        q.copy_(torch.randint(0, 5000, (3000,), device="cuda"))
+        out.zero_()
+        missed.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, full[q]) and torch.equal(missed, full[q])
+        assert torch.equal(capi.cache_fetch(host, cache, q, h), out)
+
+
 def test_one_pass_scans_replay_in_a_hip_graph(capi, cabi):
     """thrust_scan (workspace from the shim), shmt_exclusive_scan with a caller's workspace and the form
     without a workspace, each over several tiles, recorded once and replayed on new data: the kernels clear
