@@ -368,3 +368,19 @@ def test_a_wait_that_gave_up_is_reported(capi, cabi):
     uniq, _ = capi.tensor_relabel([a])
     assert uniq.numel() == 977
     capi.raise_async_error()
+
+
+@pytest.mark.parametrize("tiles,past", [(1, 0), (64, -1), (64, 1), (255, 0), (256, 0), (256, 1), (257, 5), (512, 1), (1023, 3),
+                                        (1024, 0), (1025, 1), (2047, 511)])
+@pytest.mark.parametrize("spread", [0.3, 4.0])
+def test_relabel_around_whole_steps_of_tile_counts(capi, tiles, past, spread):
+    """The counts of tiles of 512 ids are summed by every workgroup, 64 to a wave's step and 256 to a workgroup's."""
+    n = tiles * 512 + past
+    g = torch.Generator(device="cuda").manual_seed(n)
+    ids = torch.randint(0, max(2, int(n * spread)), (n,), device="cuda", generator=g)
+    seeds = ids[: max(1, n // 9)].clone()
+    uniq, (seed_labels, labels) = capi.tensor_relabel([seeds, ids[seeds.numel():].contiguous()])
+    first = torch.full((int(ids.max()) + 1,), n, device="cuda").scatter_reduce_(0, ids, torch.arange(n, device="cuda"), "amin")
+    order = torch.sort(first[first < n]).values
+    assert torch.equal(uniq, ids[order])
+    assert torch.equal(uniq[torch.cat([seed_labels, labels])], ids)
