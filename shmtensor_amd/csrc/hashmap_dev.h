@@ -88,7 +88,7 @@ __device__ __forceinline__ int64_t map_key(const MapView &m, int64_t req) {
 // of a word, and the value in a word's low bits.
 __device__ __forceinline__ uint64_t slot8_word(const MapView &m, int64_t key, int64_t val) {
   return (static_cast<uint64_t>(key) << m.val_bits) |
-         (static_cast<uint64_t>(val - m.delta) & ((1ull << m.val_bits) - 1));
+         ((static_cast<uint64_t>(val) - static_cast<uint64_t>(m.delta)) & ((1ull << m.val_bits) - 1));
 }
 __device__ __forceinline__ int64_t slot8_key(const MapView &m, uint64_t word) {
   if (m.fits32 == 2) return static_cast<int64_t>(word >> m.val_bits);
@@ -96,7 +96,7 @@ __device__ __forceinline__ int64_t slot8_key(const MapView &m, uint64_t word) {
 }
 __device__ __forceinline__ int64_t slot8_value(const MapView &m, uint64_t word) {
   const int s = 64 - m.val_bits;
-  return (static_cast<int64_t>(word << s) >> s) + m.delta;
+  return static_cast<int64_t>(static_cast<uint64_t>(static_cast<int64_t>(word << s) >> s) + static_cast<uint64_t>(m.delta));
 }
 
 // Table entries that will not be looked at again soon (the probe of a row
@@ -428,14 +428,6 @@ __device__ __forceinline__ int64_t half_wave_finish(const MapView &m, int64_t my
   const uint64_t mine = static_cast<uint64_t>(
       shfl64(static_cast<int64_t>(res), (lane / kHalfWaveKeys) * kProbeGroup + (lane & (kHalfWaveKeys - 1))));
   return raw_value<FMT>(m, mine);
-}
-
-template <int FMT, bool STREAM>
-__device__ __forceinline__ int64_t half_wave_find(const MapView &m, int64_t mykey) {
-  if (m.kind != kKindBuckets) return lane_id() < 32 ? flat_find<STREAM>(m, mykey) : -1;
-  HalfWaveProbe p;
-  half_wave_issue<FMT, STREAM>(m, mykey, &p);
-  return half_wave_finish<FMT>(m, mykey, p);
 }
 
 }  // namespace shmt

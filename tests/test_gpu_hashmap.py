@@ -443,6 +443,19 @@ def test_widest_span_that_packs(capi, span, packs):
     assert h.query(torch.tensor([-1, span, 2**63 - 1, -2**63]).cuda()).tolist() == [-1, -1, -1, -1]
 
 
+@pytest.mark.parametrize("lowest", [-2**63, 2**63 - 1000_000, 2**62 - 5])
+@pytest.mark.parametrize("n", [(4 << 20) // 32 + 1, 1 << 18])
+def test_packed_values_at_the_ends_of_64_bits(capi, lowest, n):
+    """The middle of the values, from which packed words count, wraps around with them."""
+    g = torch.Generator(device="cuda").manual_seed(8)
+    keys = torch.unique(torch.randint(0, 1 << 40, (n + 2000,), device="cuda", generator=g))
+    keys = keys[torch.randperm(keys.numel(), device="cuda", generator=g)][:n].contiguous()
+    vals = lowest + torch.randint(0, 1000_000, (n,), device="cuda", generator=g)
+    h = capi.CUCOStaticHashmap(keys, vals, 0.5)
+    assert h.memory_usage() == (2 * n + 15) // 16 * 128
+    assert torch.equal(h.query(keys), vals) and bool((h.query(keys + (1 << 40)) == -1).all())
+
+
 def test_packed_layout_through_the_c_abi(cabi):
     """A packed layout built without scratch memory (compare-and-swap) and with it (partitions) answers alike; with too
     little the build is the one without; 16-byte slots do not look at the layout's id range."""
