@@ -261,9 +261,11 @@ def bench_fetch(capi, args, result):
     del m, kept, pos, req
     ids = torch.arange(C, device="cuda")
     slots = torch.randperm(C, device="cuda", generator=gq)
-    for name, keys_t, req in (("direct_table", ids, qh), ("bucket_table_8B_slots", ids * 11 + 1, qh * 11 + 1),
-                              ("bucket_table_16B_slots", ids * 37 + (1 << 33), qh * 37 + (1 << 33))):
-        m = capi.CUCOStaticHashmap(keys_t, slots, 0.8)
+    # (keys beyond 32 bits are packed into 8-byte slots where the constructor chooses; "buckets" keeps 16-byte slots)
+    for name, layout, keys_t, req in (("direct_table", "auto", ids, qh), ("bucket_table_8B_slots", "auto", ids * 11 + 1, qh * 11 + 1),
+                                      ("bucket_table_packed_slots", "auto", ids * 37 + (1 << 33), qh * 37 + (1 << 33)),
+                                      ("bucket_table_16B_slots", "buckets", ids * 37 + (1 << 33), qh * 37 + (1 << 33))):
+        m = capi.CUCOStaticHashmap(keys_t, slots, 0.8, layout=layout)
         assert torch.equal(capi.cache_fetch(host, cache, req[:4096], m), cache[slots[qh[:4096]]])
         tt = gpu_time_ms(lambda: capi.cache_fetch(host, cache, req, m), 30)
         a = algo_bytes / (tt["median"] * 1e-3) / 1e9
@@ -400,16 +402,17 @@ def bench_hashmap(capi, args, result):
     tb = gpu_time_ms(lambda: capi.CUCOStaticHashmap(keys, vals, 0.5), 10)
     h = capi.CUCOStaticHashmap(keys, vals, 0.5)
     assert torch.equal(h.query(req), expect)
+    in_range = int(((req >= keys.min()) & (req <= keys.max())).sum())
     tq = gpu_time_ms(lambda: h.query(req), 30)
     result["extra"]["hashmap_config2"] = {
         "build_ms": round(tb["median"], 4), "build_Mkeys_s": round(n / tb["median"] / 1e3, 1),
         "query_ms": round(tq["median"], 4), "query_Mkeys_s": round(nq / tq["median"] / 1e3, 1),
         "query_algorithmic_GBs": round(nq * 32 / tq["median"] / 1e6, 1),
         "query_frac_hbm_peak": round(nq * 32 / tq["median"] / 1e6 / HBM_PEAK_GBS, 4),
-        # what the memory system moves: a probe reads one whole 128-byte bucket line (FETCH_SIZE per launch in
-        # profiles/hashmap_sampling_kernels_pmc.md: 2,291 MB = nq x (128 + 8)), next to 8 B request + 8 B result
-        "query_line_traffic_GBs": round(nq * 144 / tq["median"] / 1e6, 1),
-        "query_line_traffic_frac_hbm_peak": round(nq * 144 / tq["median"] / 1e6 / HBM_PEAK_GBS, 4),
+        # a probe reads one whole 128-byte bucket line, next to 8 B request + 8 B result; requests outside the key range
+        # (here all that are not members) are answered by a packed table without a line of their own
+        "query_requests_in_key_range": in_range,
+        "query_line_traffic_GBs": round((in_range * 128 + nq * 16) / tq["median"] / 1e6, 1),
         "table_bytes": h.memory_usage(), "map_layout": h.layout()}
     if not args.no_cpu:
         from oracle import oracle as orc
@@ -435,7 +438,7 @@ def bench_hashmap_sweep(capi, args, result):
     for lg in range(14, 27):
         n = 1 << lg
         keys = (torch.randperm(1 << 27, device="cuda", generator=g)[:n] * 8191 + (1 << 34)).contiguous()
-        h = capi.CUCOStaticHashmap(keys, torch.arange(n, device="cuda"), 0.5)
+        h = capi.CUCOStaticHashmap(keys, torch.arange(n, device="cuda"), 0.5, layout="buckets")
         req = keys[torch.randint(0, n, (nq,), device="cuda", generator=g)]
         t = gpu_time_ms(lambda: h.query(req), 10)
         rows.append({"keys": n, "table_MiB": round(h.memory_usage() / 2**20, 1), "query_ms": round(t["median"], 4),
@@ -1104,7 +1107,7 @@ def main():
         summary["scan_frac_hbm_peak"] = {"exclusive_int64": extra["scan"]["exclusive_int64_16777216"]["frac_hbm_peak"],
                                          "inclusive_int32": extra["scan"]["thrust_scan_int32_16777216"]["frac_hbm_peak"]}
     if "hashmap_config2" in extra:
-        summary["hashmap_query_line_traffic_frac_hbm_peak"] = extra["hashmap_config2"]["query_line_traffic_frac_hbm_peak"]
+        summary["hashmap_query_Mkeys_s"] = extra["hashmap_config2"]["query_Mkeys_s"]
     if "sampling_config3" in extra:
         s3 = extra["sampling_config3"]
         summary["config3_ms_per_batch"] = {"operators": s3["ms_per_batch"], "fused_hop": s3["fused_hop_ms_per_batch"],

@@ -99,7 +99,8 @@ int shmt_hashmap_create(shmt_hashmap_t **out, const void *keys,
  *                    one 16-byte load per lookup from a table that stays in
  *                    the caches (span / 6 bytes);
  * and the bucket table uses 8-byte slots whenever all keys and values fit 32
- * bits, whatever their dtype. Every form answers exactly like the general
+ * bits, whatever their dtype, or (packed, large tables) when the keys' distances
+ * from the smallest and the span of the values share 64 bits. Every form answers exactly like the general
  * table (same contract as the constructor above: include/cuco_hashmap.cuh:
  * 57-87). shmt_hashmap_plan looks at the keys and values (one sweep, plus a
  * repeat check for range candidates), SYNCHRONISES the stream once (twice
@@ -430,6 +431,22 @@ int shmt_sample(const void *indptr, int ptr_bytes, const void *indices,
                 int replace, uint64_t rng_seed, uint32_t rng_stream,
                 void *sub_indptr, void *sub_indices, void *plan,
                 int64_t plan_bytes, int64_t *nnz_out, void *stream);
+/* shmt_sample for row offsets in host memory: indptr has rows + 1 entries,
+ * which the call may copy to `stage` (device memory, 16-byte aligned, of
+ * shmt_sample_stage_bytes; that is 0 where so many seeds cannot pay for the
+ * copy) before the seeds' rows are looked up; it does so where the seeds need
+ * enough lines of the array, which depends on the map and on their order.
+ * Same results; stage NULL or too small: shmt_sample.                      */
+int64_t shmt_sample_stage_bytes(int64_t rows, int ptr_bytes, int64_t S);
+int shmt_sample_staged(const void *indptr, int ptr_bytes, int64_t rows,
+                       const void *indices, int idx_bytes,
+                       const void *cache_indptr, const void *cache_indices,
+                       const shmt_hashmap_t *map, const void *seeds,
+                       int seed_bytes, int64_t S, int64_t k, int replace,
+                       uint64_t rng_seed, uint32_t rng_stream,
+                       void *sub_indptr, void *sub_indices, void *plan,
+                       int64_t plan_bytes, void *stage, int64_t stage_bytes,
+                       int64_t *nnz_out, void *stream);
 
 /* One hop of mini-batch sampling as one launch sequence: the body of the
  * dataloader's loop, python/shmtensor/sampling.py:128-143, i.e.
@@ -596,25 +613,10 @@ int shmt_subcsr_copy(const void *indptr, const void *indices, int ptr_bytes,
                      int idx_bytes, const void *seeds, int seed_bytes,
                      int64_t C, const void *cache_indptr, int64_t nnz,
                      void *cache_indices, void *stream);
-/* shmt_sample for row offsets in host memory: indptr has rows + 1 entries,
- * which the call may copy to `stage` (device memory, 16-byte aligned, of
- * shmt_sample_stage_bytes; that is 0 where so many seeds cannot pay for the
- * copy) before the seeds' rows are looked up. Same results; stage NULL or
- * too small: shmt_sample.                                                  */
-int64_t shmt_sample_stage_bytes(int64_t rows, int ptr_bytes, int64_t S);
-int shmt_sample_staged(const void *indptr, int ptr_bytes, int64_t rows,
-                       const void *indices, int idx_bytes,
-                       const void *cache_indptr, const void *cache_indices,
-                       const shmt_hashmap_t *map, const void *seeds,
-                       int seed_bytes, int64_t S, int64_t k, int replace,
-                       uint64_t rng_seed, uint32_t rng_stream,
-                       void *sub_indptr, void *sub_indices, void *plan,
-                       int64_t plan_bytes, void *stage, int64_t stage_bytes,
-                       int64_t *nnz_out, void *stream);
-
-/* The same, with the start of every chosen row in the source kept between
- * the two calls: row_begins has room for C int64 (device memory; NULL: as
- * above). The copy then reads no row offset over the host link.            */
+/* shmt_subcsr_plan and shmt_subcsr_copy with the start of every chosen row in
+ * the source kept between the two calls: row_begins has room for C int64
+ * (device memory; NULL: the plain calls). The copy then reads no row offset
+ * over the host link.                                                       */
 int shmt_subcsr_plan_rows(const void *indptr, int ptr_bytes, const void *seeds,
                           int seed_bytes, int64_t C, void *cache_indptr,
                           int64_t *row_begins, void *tmp, int64_t tmp_bytes,

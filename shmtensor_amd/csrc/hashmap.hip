@@ -539,12 +539,14 @@ __global__ __launch_bounds__(256) void rank_build_kernel(uint4 *table, int64_t n
 // Bulk query: a wave owns 64 consecutive requests; the first buckets of all
 // 64 are in flight before one is examined, the requests of the next step as
 // well, and results land in the lane that loaded the request, so request reads
-// and result writes are both fully coalesced. Bound by random 128-byte lines,
-// of which this part moves some 50 G a second: 16,777,216 requests to a table of
-// 4,194,304 40-bit keys (half of them members) take 344 us, 366 us when each
-// bucket load waited for the one before and every group hashed all of its keys
-// on all lanes. Eight waves per SIMD are asked for: the fragments alone are 32
-// registers.
+// and result writes are both fully coalesced. Bound by random 128-byte lines, one per
+// request and a few per cent of second buckets, of which this kernel gets some 50 G a second
+// from beyond the L2s: 16,777,216 requests to a packed table (64 MiB) of 4,194,304 40-bit
+// keys, half of them members, take 335 us, with the same requests again and again as well as
+// with changing ones; 8,388,608 requests in 16-byte slots (128 MiB) 187 us. (Requests outside the key
+// range of a packed table read no line of their own: half of them there, 204 us.) Each bucket load waiting for
+// the one before, and all lanes of a group hashing all of its keys: 366 us. Eight waves per SIMD
+// are asked for: the fragments alone are 32 registers.
 template <int FMT>
 __global__ __launch_bounds__(256, 8) void hashmap_query_kernel(
     MapView m, const void *req, int req_bytes, void *out, int out_bytes, int64_t n) {

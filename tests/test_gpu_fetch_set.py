@@ -354,7 +354,7 @@ def test_c_abi_fetch_with_the_row_count_in_device_memory(cabi, route, count):
 
 
 @pytest.mark.parametrize("route", ["map", "mask"])
-@pytest.mark.parametrize("D", [4, 48, 256, 1000])
+@pytest.mark.parametrize("D", [4, 36, 48, 256, 300, 1000])
 @pytest.mark.parametrize("count", [None, 0, 1, 700, 9000])
 def test_c_abi_fetch_in_two_launches_equals_fetch(cabi, route, D, count):
     """shmt_fetch_cached_part (hits now, the misses marked in a bitmap) followed by shmt_fetch_missed_part on
