@@ -342,3 +342,30 @@ def test_sub_graph_without_memory_for_row_starts(capi):
             torch.cuda.set_per_process_memory_fraction(1.0)
         assert torch.equal(gp.cpu(), indptr) and torch.equal(gi.cpu(), indices)
         del gp, gi
+
+
+@pytest.mark.parametrize("S,looked_at", [(5_000, False), (13_500, False), (13_600, True)])
+def test_few_seeds_beside_a_map_are_not_looked_at(cabi, S, looked_at):
+    """With a map the seeds are looked at only where a copy of the row offsets could save a good deal: 160,008 bytes
+    of offsets and 1.5 MiB are 13,539 lines. (The flag in front of the staged offsets stays as it was otherwise.)"""
+    import ctypes
+    lib, stream = cabi.load(), cabi.current_stream()
+    rows, k = 20_000, 3
+    indptr = torch.arange(0, 2 * rows + 1, 2, device="cuda")
+    indices = torch.arange(2 * rows, device="cuda", dtype=torch.int32)
+    seeds = torch.randint(0, rows, (S,), device="cuda")
+    handle, table = ctypes.c_void_p(), torch.empty(lib.shmt_hashmap_table_bytes(8, 0.5, 8, 8), dtype=torch.uint8, device="cuda")
+    none = torch.arange(rows, rows + 8, device="cuda")
+    cabi.check(lib.shmt_hashmap_create(ctypes.byref(handle), none.data_ptr(), none.data_ptr(), 8, 8, 8, 0.5, table.data_ptr(),
+                                       table.numel(), stream))
+    plan = torch.empty(lib.shmt_sample_plan_bytes(S), dtype=torch.uint8, device="cuda")
+    stage = torch.full((max(128, lib.shmt_sample_stage_bytes(rows, 8, S)),), 255, dtype=torch.uint8, device="cuda")
+    sp, si = torch.empty(S + 1, dtype=torch.int64, device="cuda"), torch.zeros(S * k, dtype=torch.int32, device="cuda")
+    nnz = torch.zeros(1, dtype=torch.int64, pin_memory=True)
+    cabi.check(lib.shmt_sample_staged(indptr.data_ptr(), 8, rows, indices.data_ptr(), 4, indptr.data_ptr(), indices.data_ptr(),
+                                      handle, seeds.data_ptr(), 8, S, k, 0, 7, 0, sp.data_ptr(), si.data_ptr(), plan.data_ptr(),
+                                      plan.numel(), stage.data_ptr(), stage.numel(), nnz.data_ptr(), stream))
+    torch.cuda.synchronize()
+    assert int(nnz) == 2 * S and torch.equal(si[: 2 * S].view(S, 2).long(), torch.stack([2 * seeds, 2 * seeds + 1], 1))
+    assert (int(stage[:4].view(torch.int32)) in (0, 1)) == looked_at
+    lib.shmt_hashmap_destroy(handle)
