@@ -409,6 +409,7 @@ __device__ __forceinline__ void rl_finish_body(unsigned bx, unsigned gx, const R
       }
 #pragma unroll
       for (int h = 0; h < kHeld; ++h) {
+        if (t0 + h * kWave >= last) continue;
         const uint32_t t = t0 + h * kWave + lane_id();
         const uint32_t inc = wave_inclusive_scan(c[h]);
         if (t < last) prefix[t] = run + inc - c[h];

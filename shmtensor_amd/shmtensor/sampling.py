@@ -199,9 +199,9 @@ class GPUSamplingDataloader:
         """Python does not remember an import that failed: it searches the whole path anew, 20 to 50 us every time,
         which was half of the time of a prefetched epoch when every block of every batch tried. A loader looks for
         dgl once and again when the import path has changed; a dgl that someone has imported is seen in any case."""
-        path = (list(sys.path), list(sys.meta_path))
-        if self._no_dgl_on != path:
-            self._no_dgl_on = path if _dgl() is None else None
+        seen = self._no_dgl_on
+        if seen is None or seen[0] != sys.path or seen[1] != sys.meta_path:
+            self._no_dgl_on = (list(sys.path), list(sys.meta_path)) if _dgl() is None else None
         return self._no_dgl_on is not None
 
     def _sample_group(self, first_batch, count, batches_drawn):
