@@ -60,6 +60,7 @@ struct RowArgs {
   uint32_t nvec_magic;  // floor((2^32 - 1) / nvec): the high half of i * magic is i / nvec, or one less
   uint32_t group_step;  // kDealt: vectors that a wave moves at a time with a lane group per row; 0: always dealt out
   int stream_dense;     // kWide: `dense` is accessed past the caches
+  int link_rows;        // kWide, fetch of 16-byte vectors: missed rows keep one vector per lane in flight
   uint32_t *miss_bits;  // DEFER: bit (i & 31) of word i / 32 is set when row i missed the cache
 };
 
@@ -100,20 +101,23 @@ constexpr int rows_waves_per_simd(bool set, bool through, int route, int vector_
 }
 
 // One row of more than 64 vectors, moved by the whole wave: a lane has kWideInFlight vectors in flight, also
-// where the row ends among them.
+// where the row ends among them. A row of 16-byte vectors that comes over the host link has one: the link is full
+// without more, and more cost it reads (16,384 rows of 512 floats 590 us with one, 615 with four, 1,024 floats
+// 1174 / 1230; 1,000 rows 78 / 97). Narrower vectors are faster with four (4,097 bytes 1740 / 1495, 1,001 halves
+// 806 / 648, 301 floats 403 / 394), and so are calls of few rows (below).
 constexpr int kWideInFlight = 4;
 constexpr bool may_stream(bool set, int vector_bytes) { return vector_bytes >= (set ? 4 : 16); }
 // (1- and 2-byte vectors are held in registers of their own: packed into one, each load would wait for the last)
 template <typename VT> struct Held { using type = VT; };
 template <> struct Held<uint8_t> { using type = uint32_t; };
 template <> struct Held<uint16_t> { using type = uint32_t; };
-template <typename VT, bool SET, bool STREAM>
+template <typename VT, bool SET, bool STREAM, int kInFlight = kWideInFlight>
 __device__ __forceinline__ void move_wide_row(char *dense, char *table, char *second, int64_t row_bytes) {
   constexpr int64_t step = kWave * static_cast<int64_t>(sizeof(VT));
-  for (int64_t off = lane_id() * static_cast<int64_t>(sizeof(VT)); off < row_bytes; off += kWideInFlight * step) {
-    typename Held<VT>::type v[kWideInFlight];
+  for (int64_t off = lane_id() * static_cast<int64_t>(sizeof(VT)); off < row_bytes; off += kInFlight * step) {
+    typename Held<VT>::type v[kInFlight];
 #pragma unroll
-    for (int u = 0; u < kWideInFlight; ++u) {
+    for (int u = 0; u < kInFlight; ++u) {
       if (off + u * step >= row_bytes) continue;
       if (SET && STREAM)
         v[u] = __builtin_nontemporal_load(reinterpret_cast<const VT *>(dense + off + u * step));
@@ -121,7 +125,7 @@ __device__ __forceinline__ void move_wide_row(char *dense, char *table, char *se
         v[u] = gload<VT>((SET ? dense : table) + off + u * step);
     }
 #pragma unroll
-    for (int u = 0; u < kWideInFlight; ++u) {
+    for (int u = 0; u < kInFlight; ++u) {
       if (off + u * step >= row_bytes) continue;
       const VT x = static_cast<VT>(v[u]);
       if (SET) {
@@ -307,7 +311,9 @@ __global__ __launch_bounds__(kRowsBlock, rows_waves_per_simd(SET, THROUGH, ROUTE
         char *const second = THROUGH ? reinterpret_cast<char *>(lane64(my_second_row, row)) : nullptr;
         if (DEFER && !trow) continue;
         char *const drow = a.dense + (base + row) * R;
-        if (may_stream(SET, sizeof(VT)) && a.stream_dense)
+        if (!SET && !DEFER && sizeof(VT) == 16 && a.link_rows && (MODE == kDirect || lane64(slot, row) < 0))
+          move_wide_row<VT, SET, false, 1>(drow, trow, second, R);
+        else if (may_stream(SET, sizeof(VT)) && a.stream_dense)
           move_wide_row<VT, SET, may_stream(SET, sizeof(VT))>(drow, trow, second, R);
         else
           move_wide_row<VT, SET, false>(drow, trow, second, R);
@@ -671,6 +677,10 @@ static int move_rows(const char *who, void *miss, void *cache, const void *indic
   const int64_t dealt_most = link && mode == kDirect ? kWave : wide_from(SET, vb, dense_bytes);
   const int route = one_vec ? kOneVec : nvec > dealt_most ? kWide : kDealt;
   a.stream_dense = stream_dense(SET, vb, row_bytes, dense_bytes);
+  // (256 waves fill the link: 256 rows of 2,048 floats 40.3 us with one vector in flight, 43.3 with four; 64 rows of
+  // 8,192 floats 45.9 / 40.2. Few missed rows among hits keep waves waiting that have long ones: 4,096 rows, 90 %
+  // hits, of 8,192 floats 257 / 239, of 1,024 floats, 16,384 rows, 130 / 127, but with 20 % hits 946 / 988)
+  a.link_rows = link && Q >= 256 && (mode == kDirect || nvec <= 1024);
   a.nvec = route == kDealt ? static_cast<uint32_t>(nvec) : 0u;
   a.nvec_magic = route == kDealt ? 0xFFFFFFFFu / a.nvec : 0u;
   const bool by_group = route == kDealt && link && nvec <= lanes && (mode == kDirect || 16 * nvec >= 9 * lanes);
