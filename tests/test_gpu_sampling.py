@@ -369,3 +369,23 @@ def test_few_seeds_beside_a_map_are_not_looked_at(cabi, S, looked_at):
     assert int(nnz) == 2 * S and torch.equal(si[: 2 * S].view(S, 2).long(), torch.stack([2 * seeds, 2 * seeds + 1], 1))
     assert (int(stage[:4].view(torch.int32)) in (0, 1)) == looked_at
     lib.shmt_hashmap_destroy(handle)
+
+
+@pytest.mark.parametrize("dtype", [torch.int32, torch.int64])
+@pytest.mark.parametrize("skew", [0, 3, 31])
+@pytest.mark.parametrize("longest", [150, 700, 40_000])
+def test_sub_graph_of_long_rows(capi, oracle, dtype, skew, longest):
+    """Rows of several lines are copied line by line: rows that begin and end anywhere in a line, that fill lines exactly,
+    empty ones, rows longer than a wave's chunk, and an index array that does not begin on a line."""
+    g = np.random.default_rng(longest + skew)
+    rows = 3000 if longest < 10_000 else 60
+    deg = g.integers(longest // 2, longest + 1, rows)
+    deg[g.integers(0, rows, rows // 10)] = 0
+    deg[: 12] = [0, 1, 15, 16, 17, 31, 32, 33, 64, longest, 128, 0]
+    indptr = np.concatenate([[0], np.cumsum(deg)]).astype(np.int64)
+    ids = torch.randint(0, 1 << 30, (int(indptr[-1]) + skew,), dtype=dtype).pin_memory()[skew:]
+    hp = torch.from_numpy(indptr).pin_memory()
+    for order in (np.arange(rows), g.permutation(rows)[: rows * 2 // 3], g.integers(0, rows, rows)):
+        gp, gi = capi.create_subcsr(hp, ids, torch.from_numpy(order.astype(np.int64)).cuda())
+        ep, ei = oracle.create_subcsr(indptr, ids.numpy(), order.astype(np.int64))
+        assert np.array_equal(gp.cpu().numpy(), ep) and np.array_equal(gi.cpu().numpy(), ei)
