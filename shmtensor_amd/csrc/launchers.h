@@ -23,14 +23,15 @@ enum StageKind : int {
   kStagePlanTile = 3,    // + map mode
   kStagePickNarrowHop = 6,  // + log2(lanes per seed) - 2, i.e. 6 .. 10
   kStageRlSmall = 11,
-  kStageRlInsert = 12,
-  kStageRlFirst = 13,
+  kStageRcBins = 12,  // + 1: the larger table
   kStageRlFinish = 14,
+  kStageRcRanks = 15,
   kStageRpCount = 16,
   kStageRpRows = 17,
   kStageRpScatter = 18,
   kStageRpGather = 19,
   kStageRpBins = 20,  // + (largest table - this launch's table), log2 of the slots: 20 .. 22
+  kStagePickClassifyHop = 24,  // + log2(lanes per seed) - 2, i.e. 24 .. 28
 };
 
 struct Stage {
@@ -105,11 +106,28 @@ int launch_scan_partials(uint64_t *partials, int64_t nb, hipStream_t s);
 // device); those kernels must also have stored `nonce` to *wide_mark if any id
 // lies outside [0, 2^32). n16 is 0 when the passes need no table in memory
 // (small inputs). count_copy, if set, receives the count as well (device memory).
+//
+// Inputs of the sizes between take classes instead of a table in memory (rc_*_kernel): classes.count != 0. Either the
+// earlier kernels classify the ids and say so (classified), or the passes begin with a launch that does.
+// Element i has class cls[i] = relabel_class(hash_id(id), count), or, when it is known to repeat the id of an
+// element in front of it that has its class, kRelabelNoClass, and stands_for[i] is the index of that element.
+constexpr uint8_t kRelabelNoClass = 255;
+struct RelabelClasses {
+  uint32_t count;  // at most 255; 0: no classes wanted
+  uint8_t *cls;
+  uint32_t *stands_for;
+};
+__device__ __forceinline__ uint8_t relabel_class(uint32_t hash, uint32_t classes) {
+  return static_cast<uint8_t>(__umulhi(hash, classes));
+}
+
 struct RelabelTable {
   void *slots;
   int64_t n16;
   uint64_t *wide_mark;  // where the earlier kernels store `nonce` when an id lies outside [0, 2^32)
   uint64_t nonce;
+  RelabelClasses classes;
+  bool classified;
 };
 int relabel_table(int64_t N, bool n_is_loose_bound, int merged_jobs, void *scratch, int64_t scratch_bytes,
                   RelabelTable *out);  // merged_jobs: 0 for a launch sequence of its own

@@ -19,9 +19,10 @@
 // the id, src/tensor_relabel.cu:111-117); ids known to fit 32 bits use the
 // same memory as packed 8-byte slots (see rl_packed_insert).
 // Up to 8,192 ids all of this is one launch of one workgroup with its table
-// in LDS (rl_small_kernel). Beyond 1 M ids (and up to 7.3 M) fill, insert and
-// first are replaced by passes that partition the ids by hash and give every
-// partition a table in LDS (rp_*_kernel, further down).
+// in LDS (rl_small_kernel). From there to 1 M ids (2 M where that is a bound) fill, insert and first
+// are replaced by passes in which a workgroup finds the ids of its class by scanning one byte per id
+// (rc_*_kernel), and up to 7.3 M by passes that partition the ids by hash
+// (rp_*_kernel); both give every class or partition a table in LDS.
 #include "common.h"
 #include "launchers.h"
 #include "scan_dev.h"
@@ -273,10 +274,6 @@ __global__ __launch_bounds__(kRlBlock) void rl_insert_kernel(RlInsertArgs a) {
   rl_insert_body(blockIdx.x, gridDim.x, a);
 }
 
-__global__ __launch_bounds__(kRlBlock) void rl_insert_jobs(Jobs<RlInsertArgs> j) {
-  if (blockIdx.x < j.blocks[blockIdx.y]) rl_insert_body(blockIdx.x, j.blocks[blockIdx.y], j.a[blockIdx.y]);
-}
-
 // First-occurrence index of every element: one id per thread, a workgroup of
 // kRlTile threads per tile (the tile within which first occurrences are
 // ranked here). One id per thread keeps every value in registers and
@@ -356,10 +353,6 @@ __device__ __forceinline__ void rl_first_body(unsigned bx, const RlFirstArgs &a)
 }
 
 __global__ __launch_bounds__(kRlTile) void rl_first_kernel(RlFirstArgs a) { rl_first_body(blockIdx.x, a); }
-
-__global__ __launch_bounds__(kRlTile) void rl_first_jobs(Jobs<RlFirstArgs> j) {
-  if (blockIdx.x < j.blocks[blockIdx.y]) rl_first_body(blockIdx.x, j.a[blockIdx.y]);
-}
 
 struct RlFinishArgs {
   const void *total;
@@ -465,6 +458,30 @@ struct RlSegments {
   int bytes[SHMT_RELABEL_MAX_SEGMENTS];
   int n;
 };
+
+// Elements idx[j] of a tile [lo, hi) of the segments' concatenation, where ok[j]. As a rule a tile lies within one
+// segment: one pointer and one width for all its loads.
+template <int ITEMS>
+__device__ __forceinline__ void rl_load_segments(const RlSegments &segs, int64_t lo, int64_t hi, const int64_t (&idx)[ITEMS],
+                                                 const bool (&ok)[ITEMS], int64_t (&key)[ITEMS]) {
+  int first_seg = 0, last_seg = 0;
+  while (first_seg + 1 < segs.n && lo >= segs.start[first_seg + 1]) ++first_seg;
+  while (last_seg + 1 < segs.n && hi - 1 >= segs.start[last_seg + 1]) ++last_seg;
+  if (first_seg == last_seg) {
+    int64_t at[ITEMS];
+#pragma unroll
+    for (int j = 0; j < ITEMS; ++j) at[j] = idx[j] - segs.start[first_seg];
+    load_ints<ITEMS>(segs.ptr[first_seg], at, ok, segs.bytes[first_seg], key);
+  } else {
+#pragma unroll
+    for (int j = 0; j < ITEMS; ++j) {
+      if (!ok[j]) continue;
+      int sgm = first_seg;
+      while (sgm < last_seg && idx[j] >= segs.start[sgm + 1]) ++sgm;
+      key[j] = load_int(segs.ptr[sgm], idx[j] - segs.start[sgm], segs.bytes[sgm]);
+    }
+  }
+}
 
 // First pass when the input arrives as segments: empties the table and writes
 // the concatenated, widened ids in one sweep (both are streaming stores).
@@ -848,30 +865,13 @@ __device__ __forceinline__ void rp_count_body(unsigned bx, const RpArgs &a, cons
   bool ok[kRpItems];
   uint32_t hash[kRpItems];
   if (SEGS) {
-    // as a rule a tile lies within one segment: one pointer and one width for all its loads
-    int first_seg = 0, last_seg = 0;
-    while (first_seg + 1 < segs.n && lo >= segs.start[first_seg + 1]) ++first_seg;
-    while (last_seg + 1 < segs.n && hi - 1 >= segs.start[last_seg + 1]) ++last_seg;
 #pragma unroll
     for (int j = 0; j < kRpItems; ++j) {
       idx[j] = lo + j * kRpBlock + threadIdx.x;
       ok[j] = idx[j] < hi;
       key[j] = 0;
     }
-    if (first_seg == last_seg) {
-      int64_t at[kRpItems];
-#pragma unroll
-      for (int j = 0; j < kRpItems; ++j) at[j] = idx[j] - segs.start[first_seg];
-      load_ints<kRpItems>(segs.ptr[first_seg], at, ok, segs.bytes[first_seg], key);
-    } else {
-#pragma unroll
-      for (int j = 0; j < kRpItems; ++j) {
-        if (!ok[j]) continue;
-        int sgm = first_seg;
-        while (sgm < last_seg && idx[j] >= segs.start[sgm + 1]) ++sgm;
-        key[j] = load_int(segs.ptr[sgm], idx[j] - segs.start[sgm], segs.bytes[sgm]);
-      }
-    }
+    rl_load_segments<kRpItems>(segs, lo, hi, idx, ok, key);
 #pragma unroll
     for (int j = 0; j < kRpItems; ++j)
       if (ok[j]) store_int(const_cast<void *>(a.total), idx[j], a.eb, key[j]);
@@ -1122,6 +1122,31 @@ struct RpTable {
       p = (p + step) & mask;
     }
     return false;
+  }
+
+  // One element from its home slot on.
+  __device__ __forceinline__ bool insert(Key key, uint32_t i, uint32_t hash) const {
+    if (key == kEmpty) {
+      atomicMin(all_ones, i);
+      return true;
+    }
+    const uint32_t home = hash & mask;
+    Key k;
+    uint32_t cur, slot;
+    look(home, &k, &cur);
+    if (k == kEmpty) k = atomicCAS(key_at(home), kEmpty, key);
+    if (k == kEmpty || k == key) {
+      if (cur > i) atomicMin(index_at(home), i);
+      return true;
+    }
+    return insert_from(key, i, hash, &slot);
+  }
+  __device__ __forceinline__ uint32_t first_of(Key key, uint32_t hash) const {
+    if (key == kEmpty) return *all_ones;
+    Key k;
+    uint32_t cur;
+    look(hash & mask, &k, &cur);
+    return k == key ? cur : first_from(key, hash);
   }
 
   __device__ __forceinline__ uint32_t first_from(Key key, uint32_t hash) const {
@@ -1403,6 +1428,329 @@ __global__ __launch_bounds__(kRpBlock) void rp_gather_jobs(Jobs<RpArgs> j) {
   if (blockIdx.x < j.blocks[blockIdx.y]) rp_gather_body(blockIdx.x, j.a[blockIdx.y]);
 }
 
+// ---- inputs of the sizes between: a class per workgroup, found by scanning one byte per id ------------
+// A table in memory costs a few hundred thousand ids one memory-side atomic each (17 - 26 G per second), a pass of
+// random reads and a table to empty first; the passes above are too many launches for them. Here whoever
+// writes the ids (the pick kernel of a hop; rc_classify_kernel) gives every id a class, one byte, and
+//   bins     a workgroup per class: reads the bytes of ALL ids, 64 per lane and step, compared four at a time in
+//            32-bit words (at most 2 MB, which the L2s hold: reading them a hundred times over costs less than
+//            dealing the ids out would), collects those of its class in LDS, and finds the smallest
+//            index per id through a table in LDS
+//   ranks    first occurrences per 64 elements and per tile, and the elements that another stands for
+//   finish   as everywhere
+// A class is 1 / classes of the distinct ids; one that does not fit its table is worked through in rounds over a second
+// hash, as a bin of the partition passes is. More elements than the list holds (an id that comes in
+// most waves of the pick kernel) go into the table as they are found, and are found a second time for their results.
+// Measured: third hop of 1,024 seeds at fanouts 15, 10, 5 (355,000 ids, launched for a bound of 1.08 M) insert 22 + first
+// 7.3 us before, bins 19 + ranks 4.8 now (launch 2.6, reading the bytes 3.6, matching 2, listing 3, ids and tables 4,
+// results 2.5); second hop (38,000 ids) 12 + 4.3 before, 6.5 + 2.5 now. tensor_relabel of 100,000 / 400,000 / 1 M ids
+// 37 / 58 / 86 us before, 32 / 47 / 68 now, all distinct 42 / 68 / 106 and 33 / 48 / 75; below 50,000 ids no difference
+// but for a hundred distinct ids (27.4 -> 30.4 at 9,000), where the table in memory needs hardly an atomic.
+constexpr int kRcThreads = 1024;
+constexpr int kRcSlotsLog2 = 12, kRcMaxSlotsLog2 = 13;  // table slots, and elements of a class that are listed
+constexpr int64_t kRcSmallTableMax = 512 * 1024;        // the smaller one: two thirds full when all ids differ
+constexpr int64_t kRcMax = kRlSelfPrefixTiles * kRlTile;
+constexpr int kRcClassifyItems = 4;
+
+struct RcArgs {
+  const void *total;
+  int eb;
+  RlCount n;
+  RelabelClasses classes;  // stands_for: the first-occurrence index of every element when the passes are through
+  int slots_log2, max_rounds_log2;
+  RlRanks *ranks;
+  uint64_t *partials;
+};
+
+static int rc_table_log2(int64_t N) { return N <= kRcSmallTableMax ? kRcSlotsLog2 : kRcMaxSlotsLog2; }
+
+static bool rc_plan(int64_t N, int merged_jobs, void *table_memory, RelabelClasses *out) {
+  if (N <= kRlSmallMax || N > kRcMax) return false;
+  // 16 * rl_capacity(N) >= 32 N bytes are there
+  out->cls = static_cast<uint8_t *>(table_memory);
+  out->stands_for = reinterpret_cast<uint32_t *>(out->cls + ((N + 255) & ~255ll));
+  // one workgroup per compute unit; eight jobs of 38,000 ids: 64 classes each 22.9 us, 128 24.5
+  out->count = merged_jobs >= kRpMergedMinJobs ? 64 : 255;
+  return true;
+}
+
+// For ids that no earlier kernel has classified; SEGS: as in the count pass. Repeats within a tile are found through a
+// direct-mapped table: a slot holds the smallest place in the tile of the ids that map there.
+template <bool SEGS>
+__global__ __launch_bounds__(kRlBlock) void rc_classify_kernel(RcArgs a, RlSegments segs) {
+  constexpr int kTile = kRcClassifyItems * kRlBlock;
+  __shared__ int64_t ids[kTile];
+  __shared__ uint32_t owner[kTile];
+  const int64_t N = rl_count(a.n);
+  const int64_t lo = static_cast<int64_t>(blockIdx.x) * kTile;
+  if (lo >= N) return;
+  const int64_t hi = lo + kTile < N ? lo + kTile : N;
+  int64_t idx[kRcClassifyItems], key[kRcClassifyItems];
+  bool ok[kRcClassifyItems];
+  uint32_t hash[kRcClassifyItems];
+#pragma unroll
+  for (int j = 0; j < kRcClassifyItems; ++j) {
+    idx[j] = lo + j * kRlBlock + threadIdx.x;
+    ok[j] = idx[j] < hi;
+    key[j] = 0;
+    owner[j * kRlBlock + threadIdx.x] = 0xFFFFFFFFu;
+  }
+  if (SEGS)
+    rl_load_segments<kRcClassifyItems>(segs, lo, hi, idx, ok, key);
+  else
+    load_ints<kRcClassifyItems>(a.total, idx, ok, a.eb, key);
+#pragma unroll
+  for (int j = 0; j < kRcClassifyItems; ++j) {
+    ids[j * kRlBlock + threadIdx.x] = key[j];
+    hash[j] = hash_id(key[j]);
+    if (SEGS && ok[j]) store_int(const_cast<void *>(a.total), idx[j], a.eb, key[j]);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < kRcClassifyItems; ++j)
+    if (ok[j]) atomicMin(&owner[hash[j] % kTile], static_cast<uint32_t>(j * kRlBlock + threadIdx.x));
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < kRcClassifyItems; ++j) {
+    if (!ok[j]) continue;
+    const uint32_t o = owner[hash[j] % kTile];
+    const bool covered = o != static_cast<uint32_t>(j * kRlBlock + threadIdx.x) && ids[o] == key[j];
+    a.classes.cls[idx[j]] = covered ? kRelabelNoClass : relabel_class(hash[j], a.classes.count);
+    if (covered) a.classes.stands_for[idx[j]] = static_cast<uint32_t>(lo) + o;
+  }
+}
+
+// The bytes of all elements, 128 per lane and step: step(words, element), the same number of times in all lanes of a wave.
+// Bit b of words[w] set: element(w, b) may have class c; every element that does is among them. (Others are where a byte
+// c ^ 1 lies above a byte c, and past the ids: three instructions find the zero bytes of four, five would find only them.)
+constexpr uint32_t kRcVecs = 8;
+constexpr uint32_t kRcWords = kRcVecs / 2;
+
+template <typename Step>
+__device__ __forceinline__ void rc_scan(const uint8_t *cls, uint32_t n, uint32_t c, Step step) {
+  const uint4 *const vec = reinterpret_cast<const uint4 *>(cls);
+  const uint32_t vecs = (n + 15) / 16, pattern = c * 0x01010101u;
+  uint4 next[kRcVecs];
+  auto load = [&](uint32_t v0) {
+#pragma unroll
+    for (uint32_t q = 0; q < kRcVecs; ++q) {
+      const uint32_t v = v0 + q * kRcThreads + threadIdx.x;
+      if (v < vecs) next[q] = vec[v]; else next[q] = make_uint4(~0u, ~0u, ~0u, ~0u);  // (kRelabelNoClass)
+    }
+  };
+  // bit 8 b + 7 - d: byte b of word d
+  auto matches = [&](const uint4 &w) -> uint32_t {
+    auto of = [&](uint32_t word) -> uint32_t {
+      const uint32_t x = word ^ pattern;
+      return (x - 0x01010101u) & ~x & 0x80808080u;
+    };
+    return of(w.x) | (of(w.y) >> 1) | (of(w.z) >> 2) | (of(w.w) >> 3);
+  };
+  load(0);
+  for (uint32_t v0 = 0; v0 < vecs; v0 += kRcVecs * kRcThreads) {
+    uint32_t words[kRcWords];
+#pragma unroll
+    for (uint32_t w = 0; w < kRcWords; ++w) words[w] = matches(next[2 * w]) | (matches(next[2 * w + 1]) >> 4);
+    load(v0 + kRcVecs * kRcThreads);
+    auto element = [&](uint32_t w, uint32_t b) -> uint32_t {
+      const uint32_t low = b & 7u, q = 2 * w + (low < 4u ? 1u : 0u);
+      return (v0 + q * kRcThreads + threadIdx.x) * 16 + (3u - (low & 3u)) * 4 + (b >> 3);
+    };
+    step(words, element);
+  }
+}
+
+// each(i) for every element that rc_scan shows this thread.
+template <typename Words, typename Element, typename Each>
+__device__ __forceinline__ void rc_each(Words &words, Element element, Each each) {
+  for (;;) {
+    uint32_t w = 0, bits = words[0];
+#pragma unroll
+    for (uint32_t o = 1; o < kRcWords; ++o) {
+      const bool take = bits == 0;
+      w = take ? o : w;
+      bits = take ? words[o] : bits;
+    }
+    if (bits == 0) break;
+    const uint32_t b = static_cast<uint32_t>(__builtin_ctz(bits));
+#pragma unroll
+    for (uint32_t o = 0; o < kRcWords; ++o) words[o] = o == w ? bits & (bits - 1) : words[o];
+    each(element(w, b));
+  }
+}
+
+template <bool PACKED, int SLOTS_LOG2>
+__device__ __forceinline__ void rc_bin_body(uint32_t c, const RcArgs &a, unsigned long long *mem, uint32_t *list,
+                                            uint32_t *shared_words) {
+  using Table = RpTable<PACKED>;
+  using Key = typename Table::Key;
+  constexpr uint32_t kRcList = 1u << SLOTS_LOG2;
+  constexpr int kRcHeld = kRcList / kRcThreads;
+  const uint32_t N = static_cast<uint32_t>(rl_count(a.n));
+  uint32_t *const overflow = &shared_words[0], *const found = &shared_words[2];
+  const Table tbl{mem, &shared_words[1], (1u << a.slots_log2) - 1};
+  uint32_t *const first = a.classes.stands_for;
+  for (int lg = 0; lg <= a.max_rounds_log2; ++lg) {
+    const uint32_t round_mask = (1u << lg) - 1u;
+    // an element that the scan showed: of this class and round? (One that another stands for passes if its class is
+    // this one: it then gets its first occurrence from here.)
+    auto theirs = [&](int64_t key, uint32_t round) {
+      return relabel_class(hash_id(key), a.classes.count) == c && rp_mine(key, round_mask, round);
+    };
+    bool done = true;
+    for (uint32_t r = 0; r <= round_mask && done; ++r) {
+      tbl.clear();
+      if (threadIdx.x == 0) {
+        *overflow = 0;
+        *found = 0;
+      }
+      __syncthreads();
+      bool fits = true;
+      rc_scan(a.classes.cls, N, c, [&](uint32_t (&words)[kRcWords], auto element) {
+        uint32_t mine = 0;
+#pragma unroll
+        for (uint32_t w = 0; w < kRcWords; ++w) mine += static_cast<uint32_t>(__builtin_popcount(words[w]));
+        const uint32_t upto = wave_inclusive_scan(mine), sum = wave_last(upto);
+        if (sum == 0) return;
+        uint32_t e = 0;
+        if (lane_id() == 0) e = atomicAdd(found, sum);  // one reservation per wave and step
+        e = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(e))) + upto - mine;
+        rc_each(words, element, [&](uint32_t i) {
+          if (e < kRcList) {
+            list[e] = i;
+          } else if (i < N) {
+            const int64_t key = load_int(a.total, i, a.eb);
+            if (theirs(key, r)) fits &= tbl.insert(static_cast<Key>(key), i, hash_id(key));
+          }
+          ++e;
+        });
+      });
+      __syncthreads();
+      const uint32_t listed = *found < kRcList ? *found : kRcList;
+      const bool all_listed = *found <= kRcList;
+      // the listed elements, up to kRcHeld a thread: loaded, looked up, claimed and lowered together
+      int64_t at[kRcHeld], key[kRcHeld];
+      uint32_t hash[kRcHeld], slot[kRcHeld], cur[kRcHeld];
+      bool on[kRcHeld];
+      Key k[kRcHeld];
+      constexpr uint32_t kNotMine = 0xFFFFFFFFu, kAllOnes = 0xFFFFFFFEu;
+#pragma unroll
+      for (int j = 0; j < kRcHeld; ++j) {
+        const uint32_t e = j * kRcThreads + threadIdx.x;
+        at[j] = e < listed ? list[e] : N;
+        on[j] = at[j] < N;
+        key[j] = 0;
+      }
+      load_ints<kRcHeld>(a.total, at, on, a.eb, key);
+#pragma unroll
+      for (int j = 0; j < kRcHeld; ++j) {
+        hash[j] = hash_id(key[j]);
+        on[j] = on[j] && theirs(key[j], r);
+        slot[j] = kNotMine;
+        if (on[j] && static_cast<Key>(key[j]) == Table::kEmpty) {
+          atomicMin(tbl.all_ones, static_cast<uint32_t>(at[j]));
+          on[j] = false;
+          slot[j] = kAllOnes;
+        }
+        k[j] = 0;
+        cur[j] = 0;
+        if (on[j]) tbl.look(hash[j] & tbl.mask, &k[j], &cur[j]);
+      }
+#pragma unroll
+      for (int j = 0; j < kRcHeld; ++j)
+        if (on[j] && k[j] == Table::kEmpty)
+          k[j] = atomicCAS(tbl.key_at(hash[j] & tbl.mask), Table::kEmpty, static_cast<Key>(key[j]));
+#pragma unroll
+      for (int j = 0; j < kRcHeld; ++j) {
+        if (!on[j]) continue;
+        if (k[j] == Table::kEmpty || k[j] == static_cast<Key>(key[j])) {
+          if (cur[j] > static_cast<uint32_t>(at[j])) atomicMin(tbl.index_at(hash[j] & tbl.mask), static_cast<uint32_t>(at[j]));
+          slot[j] = hash[j] & tbl.mask;
+        } else {
+          fits &= tbl.insert_from(static_cast<Key>(key[j]), static_cast<uint32_t>(at[j]), hash[j], &slot[j]);
+        }
+      }
+      if (!fits) *overflow = 1;
+      __syncthreads();
+      done = *overflow == 0;
+      if (done) {
+#pragma unroll
+        for (int j = 0; j < kRcHeld; ++j)
+          if (slot[j] != kNotMine) first[at[j]] = slot[j] == kAllOnes ? *tbl.all_ones : *tbl.index_at(slot[j]);
+        if (!all_listed)
+          rc_scan(a.classes.cls, N, c, [&](uint32_t (&words)[kRcWords], auto element) {
+            rc_each(words, element, [&](uint32_t i) {
+              if (i >= N) return;
+              const int64_t id = load_int(a.total, i, a.eb);
+              if (theirs(id, r)) first[i] = tbl.first_of(static_cast<Key>(id), hash_id(id));
+            });
+          });
+      }
+      __syncthreads();
+    }
+    if (done) return;
+  }
+  // every pair: the ids of this class defeat both hashes
+  rc_scan(a.classes.cls, N, c, [&](uint32_t (&words)[kRcWords], auto element) {
+    rc_each(words, element, [&](uint32_t i) {
+      if (i >= N || a.classes.cls[i] != c) return;
+      const int64_t id = load_int(a.total, i, a.eb);
+      uint32_t o = 0;
+      while (o < i && !(a.classes.cls[o] == c && load_int(a.total, o, a.eb) == id)) ++o;
+      first[i] = o;
+    });
+  });
+}
+
+template <int SLOTS_LOG2>
+__device__ __forceinline__ void rc_bins_body(unsigned bx, const RcArgs &a) {
+  __shared__ unsigned long long mem[(1 << SLOTS_LOG2) * 3 / 2];  // 8 bytes of id and 4 of index a slot
+  __shared__ uint32_t list[1 << SLOTS_LOG2];
+  __shared__ uint32_t shared_words[3];
+  if (a.eb == 4)
+    rc_bin_body<true, SLOTS_LOG2>(bx, a, mem, list, shared_words);
+  else
+    rc_bin_body<false, SLOTS_LOG2>(bx, a, mem, list, shared_words);
+}
+
+template <int SLOTS_LOG2>
+__global__ __launch_bounds__(kRcThreads) void rc_bins_kernel(RcArgs a) {
+  rc_bins_body<SLOTS_LOG2>(blockIdx.x, a);
+}
+
+template <int SLOTS_LOG2>
+__global__ __launch_bounds__(kRcThreads) void rc_bins_jobs(Jobs<RcArgs> j) {
+  if (blockIdx.x < j.blocks[blockIdx.y]) rc_bins_body<SLOTS_LOG2>(blockIdx.x, j.a[blockIdx.y]);
+}
+
+__device__ __forceinline__ void rc_ranks_body(unsigned bx, const RcArgs &a) {
+  const int64_t N = rl_count(a.n);
+  // launched for a bound of N: tiles past the ids have nothing to do, and nobody reads their count
+  if (static_cast<int64_t>(bx) * kRlTile >= N) return;
+  __shared__ uint32_t lds[kRlTile / kWave];
+  const int64_t i = static_cast<int64_t>(bx) * kRlTile + threadIdx.x;
+  uint32_t cnt = 0;
+  if (i < N) {
+    uint32_t f = a.classes.stands_for[i];
+    if (a.classes.cls[i] == kRelabelNoClass) {  // (the element that stands for this one has a class: nobody writes its entry here)
+      f = a.classes.stands_for[f];
+      a.classes.stands_for[i] = f;
+    }
+    cnt = f == static_cast<uint32_t>(i);
+  }
+  uint32_t tile_total;
+  const uint32_t before = block_exclusive_scan<uint32_t, kRlTile>(cnt, lds, &tile_total);
+  const uint64_t firsts = __builtin_amdgcn_ballot_w64(cnt != 0);
+  if (lane_id() == 0 && i < N) a.ranks[i / kWave] = RlRanks{firsts, before, 0u};
+  if (threadIdx.x == 0) a.partials[bx] = tile_total;
+}
+
+__global__ __launch_bounds__(kRlTile) void rc_ranks_kernel(RcArgs a) { rc_ranks_body(blockIdx.x, a); }
+
+__global__ __launch_bounds__(kRlTile) void rc_ranks_jobs(Jobs<RcArgs> j) {
+  if (blockIdx.x < j.blocks[blockIdx.y]) rc_ranks_body(blockIdx.x, j.a[blockIdx.y]);
+}
+
 // A value no earlier call has used (and that uninitialised memory is unlikely to hold).
 uint64_t relabel_nonce() {
   static std::atomic<uint64_t> counter{0x9E3779B97F4A7C15ull};
@@ -1601,7 +1949,7 @@ static int relabel_impl(const void *total, const RlSegments *segs, int64_t N, Rl
                         int elem_bytes, void *scratch, int64_t scratch_bytes, void *unique_out,
                         void *labels_out, int64_t *count_out, Launcher launcher, bool prepared = false,
                         uint64_t prepared_nonce = 0, int64_t *count_copy = nullptr,
-                        int64_t prepared_slots = 0) {
+                        int64_t prepared_slots = 0, bool classified = false) {
   SHMT_REQUIRE(N >= 0, "shmt_relabel: N must be >= 0");
   if (N >= (1ll << 31)) {
     // 64-bit positions: a plain call only (segments are concatenated by the caller, hops stay below 2^31)
@@ -1662,7 +2010,8 @@ static int relabel_impl(const void *total, const RlSegments *segs, int64_t N, Rl
 
   int rc = SHMT_OK;
   const int scanned = nb > kRlSelfPrefixTiles;
-  const unsigned fin_blocks = grid_for(N, kRlBlock, kRlFinishBlocks);
+  // (jobs that share the launch share its workgroups: every one of them sums the tile counts first)
+  const unsigned fin_blocks = grid_for(N, kRlBlock, kRlFinishBlocks / (defer && defer->jobs > 0 ? defer->jobs : 1));
   // a job among fewer merged ones than the partition passes pay for keeps the table (and stays mergeable)
   const RpPlan rp = rp_plan(N, defer ? (prepared ? defer->jobs : 1) : 0, n.fixed_dev != nullptr);
   if (!rp.ok && defer && rp_plan(N, 0, n.fixed_dev != nullptr).ok) {
@@ -1713,6 +2062,46 @@ static int relabel_impl(const void *total, const RlSegments *segs, int64_t N, Rl
     SHMT_LAUNCH_CHECK();
     return SHMT_OK;
   }
+  RelabelClasses classes;
+  if (rc_plan(N, defer ? defer->jobs : 0, tbl, &classes)) {
+    const int table_log2 = rc_table_log2(N);
+    const int slots_log2 = g_rp_tuning.slots_log2 < table_log2 ? g_rp_tuning.slots_log2 : table_log2;
+    const RcArgs a{total, elem_bytes, n, classes, slots_log2, g_rp_tuning.max_rounds_log2, ranks, partials};
+    const RlFinishArgs fin{total, elem_bytes, n, classes.stands_for, 4, ranks, partials, 8, kRlTileLog2, 0, unique_out,
+                           labels_out, count_out, count_copy};
+    if (defer) {
+      if (!classified) {
+        defer->mergeable = false;
+        return SHMT_OK;
+      }
+      stage_push(defer, kStageRcBins + (table_log2 - kRcSlotsLog2), classes.count, kRcThreads, a);
+      stage_push(defer, kStageRcRanks, static_cast<unsigned>(nb), kRlTile, a);
+      stage_push(defer, kStageRlFinish, fin_blocks, kRlBlock, fin);
+      return SHMT_OK;
+    }
+    if (!classified) {
+      const dim3 grid(grid_for(N, kRcClassifyItems * kRlBlock, kRcMax));
+      if (segs && !prepared)
+        hipLaunchKernelGGL(rc_classify_kernel<true>, grid, dim3(kRlBlock), 0, s, a, *segs);
+      else
+        hipLaunchKernelGGL(rc_classify_kernel<false>, grid, dim3(kRlBlock), 0, s, a, RlSegments{});
+      SHMT_LAUNCH_CHECK();
+    }
+    if (table_log2 == kRcSlotsLog2)
+      hipLaunchKernelGGL(rc_bins_kernel<kRcSlotsLog2>, dim3(classes.count), dim3(kRcThreads), 0, s, a);
+    else
+      hipLaunchKernelGGL(rc_bins_kernel<kRcMaxSlotsLog2>, dim3(classes.count), dim3(kRcThreads), 0, s, a);
+    SHMT_LAUNCH_CHECK();
+    hipLaunchKernelGGL(rc_ranks_kernel, dim3(static_cast<unsigned>(nb)), dim3(kRlTile), 0, s, a);
+    SHMT_LAUNCH_CHECK();
+    hipLaunchKernelGGL(rl_finish_kernel, dim3(fin_blocks), dim3(kRlBlock), 0, s, fin);
+    SHMT_LAUNCH_CHECK();
+    return SHMT_OK;
+  }
+  if (defer) {
+    defer->mergeable = false;
+    return SHMT_OK;
+  }
   const RlInsertArgs ins{tbl, cap, total, elem_bytes, n, path};
   const RlFirstArgs fst{tbl, cap, total, elem_bytes, n, labels_out, partials, path, ranks};
   const RlFinishArgs fin{total, elem_bytes, n, labels_out, elem_bytes, ranks, partials, 8, kRlTileLog2, scanned,
@@ -1722,16 +2111,6 @@ static int relabel_impl(const void *total, const RlSegments *segs, int64_t N, Rl
   // the ids of hub nodes already in the table with a smaller index and skip their atomics, where 8,192
   // workgroups starting together all miss them (8 batches per launch: 64.5 -> 62.3 us per batch).
   const unsigned ins_blocks = grid_for(N, kRlInsertTile, 1024);
-  if (defer) {
-    if (!prepared || scanned) {
-      defer->mergeable = false;
-      return SHMT_OK;
-    }
-    stage_push(defer, kStageRlInsert, ins_blocks, kRlBlock, ins);
-    stage_push(defer, kStageRlFirst, static_cast<unsigned>(nb), kRlTile, fst);
-    stage_push(defer, kStageRlFinish, fin_blocks, kRlBlock, fin);
-    return SHMT_OK;
-  }
   if (prepared) {
     // the caller's earlier kernels on this stream emptied the table and wrote `total`
   } else if (segs) {
@@ -1777,7 +2156,12 @@ int relabel_table(int64_t N, bool n_is_loose_bound, int merged_jobs, void *scrat
   // it did produce) half the slots are used: still one 16-byte slot per id in the worst case, and
   // half as much to empty.
   // Nor is there when the partition passes take the input (rp_plan).
-  out->n16 = (N <= kRlSmallMax || rp_plan(N, merged_jobs, n_is_loose_bound).ok) ? 0 : (n_is_loose_bound ? (l.cap / 2 + 7) & ~7ll : l.cap);
+  // Nor where the ids are told apart by class (rc_plan).
+  out->classes = RelabelClasses{};
+  out->classified = false;
+  const bool tableless = N <= kRlSmallMax || rp_plan(N, merged_jobs, n_is_loose_bound).ok ||
+                         rc_plan(N, merged_jobs, out->slots, &out->classes);
+  out->n16 = tableless ? 0 : (n_is_loose_bound ? (l.cap / 2 + 7) & ~7ll : l.cap);
   out->wide_mark = reinterpret_cast<uint64_t *>(static_cast<char *>(scratch) + l.flag_off);
   out->nonce = relabel_nonce();
   return SHMT_OK;
@@ -1790,7 +2174,7 @@ int launch_relabel_passes(const void *total, int64_t n_bound, int64_t n_fixed, c
   return relabel_impl(total, nullptr, n_bound,
                       RlCount{n_fixed, n_fixed_dev, n_extra_dev, n_extra_bytes, n_bound}, elem_bytes,
                       scratch, scratch_bytes, unique_out, labels_out, count_out, launcher, true, table.nonce,
-                      count_copy, table.n16);
+                      count_copy, table.n16, table.classified);
 }
 
 int launch_merged_relabel_stage(int n_jobs, const Stage *const *stages, hipStream_t s) {
@@ -1802,16 +2186,17 @@ int launch_merged_relabel_stage(int n_jobs, const Stage *const *stages, hipStrea
       hipLaunchKernelGGL(rl_small_jobs, dim3(1, n_jobs), dim3(threads), 0, s, j);
       break;
     }
-    case kStageRlInsert: {
-      Jobs<RlInsertArgs> j;
+    case kStageRcBins:
+    case kStageRcBins + 1:
+    case kStageRcRanks: {
+      Jobs<RcArgs> j;
       const unsigned blocks = jobs_from_stages(n_jobs, stages, &j);
-      hipLaunchKernelGGL(rl_insert_jobs, dim3(blocks, n_jobs), dim3(threads), 0, s, j);
-      break;
-    }
-    case kStageRlFirst: {
-      Jobs<RlFirstArgs> j;
-      const unsigned blocks = jobs_from_stages(n_jobs, stages, &j);
-      hipLaunchKernelGGL(rl_first_jobs, dim3(blocks, n_jobs), dim3(threads), 0, s, j);
+      if (stages[0]->kind == kStageRcBins)
+        hipLaunchKernelGGL(rc_bins_jobs<kRcSlotsLog2>, dim3(blocks, n_jobs), dim3(threads), 0, s, j);
+      else if (stages[0]->kind == kStageRcBins + 1)
+        hipLaunchKernelGGL(rc_bins_jobs<kRcMaxSlotsLog2>, dim3(blocks, n_jobs), dim3(threads), 0, s, j);
+      else
+        hipLaunchKernelGGL(rc_ranks_jobs, dim3(blocks, n_jobs), dim3(threads), 0, s, j);
       break;
     }
     case kStageRlFinish: {

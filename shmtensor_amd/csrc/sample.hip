@@ -328,6 +328,9 @@ struct PickArgs {
   uint64_t wide_nonce;
   void *coo_out;                // optional: position of the seed each sampled id belongs to (the destination
   int coo_bytes;                // side of the block's edges in coordinate form), coo_bytes wide
+  uint32_t classes;             // CLASSIFY kernels: class of every seed and sampled id among so many, and which
+  uint8_t *cls;                 // element stands for an id that repeats within a pass (see RelabelClasses)
+  uint32_t *stands_for;
 };
 
 __device__ __forceinline__ void note_wide_id(const PickArgs &a, int64_t id) {
@@ -544,6 +547,52 @@ __device__ __forceinline__ int64_t adj_value(const PickArgs &a, int64_t raw) {
 
 constexpr int kPickRounds = 4;  // seeds a lane group handles per pass, at most: that many adjacency loads in flight
 
+// Relabel classes of the wave's seeds and of the ids it picked, while they are in registers: one byte each. Of an id that
+// comes several times in a pass (hub nodes) only the occurrence with the smallest index keeps its class, the others name that
+// one: a direct-mapped table per wave, owned by the element with the smallest index that maps to a slot. Elements
+// are compared by 32 bits, so a pass with wider ids keeps its repeats. (Wave-private LDS, accesses in program order: no barrier.)
+constexpr int kPickDedupSlots = 256;
+
+__device__ __forceinline__ void pick_classify(const PickArgs &a, int64_t S, int64_t sl, bool seed_live, int64_t node,
+                                              const int64_t (&raw)[kPickRounds], const int64_t (&where)[kPickRounds]) {
+  __shared__ unsigned long long dedup_all[256 / kWave][kPickDedupSlots];
+  unsigned long long *const dedup = dedup_all[threadIdx.x / kWave];
+  if (seed_live) a.cls[sl] = relabel_class(hash_id(node), a.classes);
+  uint32_t hash[kPickRounds];
+  bool on[kPickRounds], wide = false;
+#pragma unroll
+  for (int r = 0; r < kPickRounds; ++r) {
+    const int64_t id = adj_value(a, raw[r]);
+    on[r] = where[r] >= 0;
+    hash[r] = on[r] ? hash_id(id) : 0;
+    wide |= on[r] && id != static_cast<int64_t>(static_cast<int32_t>(id));
+  }
+  const bool compare = __builtin_amdgcn_ballot_w64(wide) == 0;
+  if (compare) {
+#pragma unroll
+    for (int t = 0; t < kPickDedupSlots / kWave; ++t) dedup[t * kWave + lane_id()] = ~0ull;
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int r = 0; r < kPickRounds; ++r)
+      if (on[r])
+        atomicMin(&dedup[hash[r] % kPickDedupSlots],
+                  (static_cast<unsigned long long>(static_cast<uint32_t>(S + where[r])) << 32) | static_cast<uint32_t>(raw[r]));
+    __builtin_amdgcn_wave_barrier();
+  }
+#pragma unroll
+  for (int r = 0; r < kPickRounds; ++r) {
+    if (!on[r]) continue;
+    const uint32_t i = static_cast<uint32_t>(S + where[r]);
+    const unsigned long long owner =
+        compare ? __hip_atomic_load(&dedup[hash[r] % kPickDedupSlots], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT) : ~0ull;
+    const bool covered = compare && static_cast<uint32_t>(owner) == static_cast<uint32_t>(raw[r]) &&
+                         static_cast<uint32_t>(owner >> 32) != i;
+    a.cls[i] = covered ? kRelabelNoClass : relabel_class(hash[r], a.classes);
+    if (covered) a.stands_for[i] = static_cast<uint32_t>(owner >> 32);
+  }
+  __builtin_amdgcn_wave_barrier();
+}
+
 // k <= 64: group of G = 2^LG >= k lanes per seed. (bx, gx): this workgroup's
 // index and the number of workgroups of its job. A wave takes `rounds` x 64 / G
 // consecutive seeds per pass (a.rounds <= kPickRounds; they share a plan
@@ -557,7 +606,7 @@ constexpr int kPickRounds = 4;  // seeds a lane group handles per pass, at most:
 // and pass (four dependent chains per wave one after the other), 79 us so.
 // Capping the kernel at 64 registers for eight resident waves per SIMD spills
 // and measured 150 us; two rounds per pass instead of four measured the same.
-template <bool HOP, int LG>
+template <bool HOP, int LG, bool CLASSIFY = false>
 __device__ __forceinline__ void pick_narrow_body(unsigned bx, unsigned gx, const PickArgs &a) {
   pick_clear<HOP>(a, bx, gx);
   constexpr int G = 1 << LG;
@@ -643,17 +692,19 @@ __device__ __forceinline__ void pick_narrow_body(unsigned bx, unsigned gx, const
 #pragma unroll
     for (int r = 0; r < kPickRounds; ++r)
       if (where[r] >= 0) pick_store<HOP>(a, S, w0 + r * kGroups + grp, where[r], adj_value(a, raw[r]));
+    if constexpr (CLASSIFY) pick_classify(a, S, sl, seed_live, node_l, raw, where);
   }
 }
 
-template <bool HOP, int LG>
+template <bool HOP, int LG, bool CLASSIFY>
 __global__ __launch_bounds__(256) void pick_narrow_kernel(PickArgs a) {
-  pick_narrow_body<HOP, LG>(blockIdx.x, gridDim.x, a);
+  pick_narrow_body<HOP, LG, CLASSIFY>(blockIdx.x, gridDim.x, a);
 }
 
-template <int LG>
+template <int LG, bool CLASSIFY>
 __global__ __launch_bounds__(256) void pick_narrow_hop_jobs(Jobs<PickArgs> j) {
-  if (blockIdx.x < j.blocks[blockIdx.y]) pick_narrow_body<true, LG>(blockIdx.x, j.blocks[blockIdx.y], j.a[blockIdx.y]);
+  if (blockIdx.x < j.blocks[blockIdx.y])
+    pick_narrow_body<true, LG, CLASSIFY>(blockIdx.x, j.blocks[blockIdx.y], j.a[blockIdx.y]);
 }
 
 // k > 64: one wave (= one 64-thread workgroup) per seed. The chosen positions
@@ -1041,16 +1092,28 @@ struct PickHopExtras {
   uint64_t wide_nonce;
   void *coo_out;
   int coo_bytes;
+  RelabelClasses classes;
 };
 
-template <bool HOP>
+template <bool HOP, bool CLASSIFY>
 static void launch_pick_narrow(int lg, unsigned blocks, unsigned threads, hipStream_t s, const PickArgs &a) {
   switch (lg) {
-    case 2: hipLaunchKernelGGL((pick_narrow_kernel<HOP, 2>), dim3(blocks), dim3(threads), 0, s, a); break;
-    case 3: hipLaunchKernelGGL((pick_narrow_kernel<HOP, 3>), dim3(blocks), dim3(threads), 0, s, a); break;
-    case 4: hipLaunchKernelGGL((pick_narrow_kernel<HOP, 4>), dim3(blocks), dim3(threads), 0, s, a); break;
-    case 5: hipLaunchKernelGGL((pick_narrow_kernel<HOP, 5>), dim3(blocks), dim3(threads), 0, s, a); break;
-    default: hipLaunchKernelGGL((pick_narrow_kernel<HOP, 6>), dim3(blocks), dim3(threads), 0, s, a); break;
+    case 2: hipLaunchKernelGGL((pick_narrow_kernel<HOP, 2, CLASSIFY>), dim3(blocks), dim3(threads), 0, s, a); break;
+    case 3: hipLaunchKernelGGL((pick_narrow_kernel<HOP, 3, CLASSIFY>), dim3(blocks), dim3(threads), 0, s, a); break;
+    case 4: hipLaunchKernelGGL((pick_narrow_kernel<HOP, 4, CLASSIFY>), dim3(blocks), dim3(threads), 0, s, a); break;
+    case 5: hipLaunchKernelGGL((pick_narrow_kernel<HOP, 5, CLASSIFY>), dim3(blocks), dim3(threads), 0, s, a); break;
+    default: hipLaunchKernelGGL((pick_narrow_kernel<HOP, 6, CLASSIFY>), dim3(blocks), dim3(threads), 0, s, a); break;
+  }
+}
+
+template <bool CLASSIFY>
+static void launch_pick_narrow_jobs(int lg, dim3 grid, dim3 block, hipStream_t s, const Jobs<PickArgs> &j) {
+  switch (lg) {
+    case 2: hipLaunchKernelGGL((pick_narrow_hop_jobs<2, CLASSIFY>), grid, block, 0, s, j); break;
+    case 3: hipLaunchKernelGGL((pick_narrow_hop_jobs<3, CLASSIFY>), grid, block, 0, s, j); break;
+    case 4: hipLaunchKernelGGL((pick_narrow_hop_jobs<4, CLASSIFY>), grid, block, 0, s, j); break;
+    case 5: hipLaunchKernelGGL((pick_narrow_hop_jobs<5, CLASSIFY>), grid, block, 0, s, j); break;
+    default: hipLaunchKernelGGL((pick_narrow_hop_jobs<6, CLASSIFY>), grid, block, 0, s, j); break;
   }
 }
 
@@ -1083,12 +1146,16 @@ static int pick_launch(PickArgs a, Launcher launcher) {
     }
     if (defer) {
       if (HOP)
-        stage_push(defer, kStagePickNarrowHop + a.log2_group - 2, grid_for(blocks, 1), threads, a);
+        stage_push(defer, (a.cls ? kStagePickClassifyHop : kStagePickNarrowHop) + a.log2_group - 2, grid_for(blocks, 1),
+                   threads, a);
       else
         defer->mergeable = false;
       return SHMT_OK;
     }
-    launch_pick_narrow<HOP>(a.log2_group, grid_for(blocks, 1), threads, s, a);
+    if (HOP && a.cls)
+      launch_pick_narrow<true, true>(a.log2_group, grid_for(blocks, 1), threads, s, a);
+    else
+      launch_pick_narrow<HOP, false>(a.log2_group, grid_for(blocks, 1), threads, s, a);
   } else if (defer) {
     defer->mergeable = false;  // the one-wave-per-seed forms have no merged launch
     return SHMT_OK;
@@ -1112,13 +1179,11 @@ int launch_merged_sampling_stage(int n_jobs, const Stage *const *stages, hipStre
     Jobs<PickArgs> j;
     const unsigned blocks = jobs_from_stages(n_jobs, stages, &j);
     const dim3 grid(blocks, n_jobs), block(threads);
-    switch (kind - kStagePickNarrowHop + 2) {
-      case 2: hipLaunchKernelGGL(pick_narrow_hop_jobs<2>, grid, block, 0, s, j); break;
-      case 3: hipLaunchKernelGGL(pick_narrow_hop_jobs<3>, grid, block, 0, s, j); break;
-      case 4: hipLaunchKernelGGL(pick_narrow_hop_jobs<4>, grid, block, 0, s, j); break;
-      case 5: hipLaunchKernelGGL(pick_narrow_hop_jobs<5>, grid, block, 0, s, j); break;
-      default: hipLaunchKernelGGL(pick_narrow_hop_jobs<6>, grid, block, 0, s, j); break;
-    }
+    launch_pick_narrow_jobs<false>(kind - kStagePickNarrowHop + 2, grid, block, s, j);
+  } else if (kind >= kStagePickClassifyHop && kind < kStagePickClassifyHop + 5) {
+    Jobs<PickArgs> j;
+    const unsigned blocks = jobs_from_stages(n_jobs, stages, &j);
+    launch_pick_narrow_jobs<true>(kind - kStagePickClassifyHop + 2, dim3(blocks, n_jobs), dim3(threads), s, j);
   } else if (kind >= kStagePlanSingle && kind < kStagePlanTile + 3) {
     Jobs<PlanArgs> j;
     const unsigned blocks = jobs_from_stages(n_jobs, stages, &j);
@@ -1190,6 +1255,9 @@ static int pick_impl(const void *indices, const void *cache_indices, int idx_byt
   a.wide_nonce = 0;
   a.coo_out = nullptr;
   a.coo_bytes = 8;
+  a.classes = 0;
+  a.cls = nullptr;
+  a.stands_for = nullptr;
   if (!hop) return pick_launch<false>(a, launcher);
   a.sub_indptr_rw = hop->sub_indptr_rw;
   a.tile_prefix = hop->tile_prefix;
@@ -1206,6 +1274,9 @@ static int pick_impl(const void *indices, const void *cache_indices, int idx_byt
   a.wide_nonce = hop->wide_nonce;
   a.coo_out = hop->coo_out;
   a.coo_bytes = hop->coo_bytes;
+  a.classes = hop->classes.count;
+  a.cls = hop->classes.cls;
+  a.stands_for = hop->classes.stands_for;
   return pick_launch<true>(a, launcher);
 }
 
@@ -1277,7 +1348,7 @@ int shmt_sample_staged(const void *indptr, int ptr_bytes, int64_t rows, const vo
   if (rc) return rc;
   const PickHopExtras pick_hop{sub_indptr, plan_hop.tile_prefix_out, plan_hop.raw_tiles_out, nnz_out,
                                const_cast<uint64_t *>(plan_hop.total_out), nullptr, nullptr, nullptr, 8,
-                               nullptr, 0, nullptr, 0, nullptr, 8};
+                               nullptr, 0, nullptr, 0, nullptr, 8, RelabelClasses{}};
   return pick_impl(indices, cache_indices, idx_bytes, seeds, seed_bytes, S, k, replace, sub_indptr, ptr_bytes,
                    plan, sub_indices, rng_seed, rng_stream, launcher, &pick_hop);
 }
@@ -1305,6 +1376,7 @@ static int hop_impl(const void *indptr, int ptr_bytes, const void *indices, int 
   int rc = relabel_table(n_max, S_len != nullptr, launcher.defer ? launcher.defer->jobs : 0, scratch, scratch_bytes,
                          &table);
   if (rc) return rc;
+  table.classified = table.classes.count > 0 && k <= kWave;  // (the form of one wave per seed leaves it to the relabel)
   PlanHopExtras plan_hop{total_out, elem_bytes, S_len, nullptr, nullptr, nullptr, nullptr, 0};
   rc = plan_impl(indptr, ptr_bytes, cache_indptr, map, seeds, seed_bytes, S, k, replace, sub_indptr, plan,
                  plan_bytes, nnz_out, launcher, &plan_hop);
@@ -1312,7 +1384,7 @@ static int hop_impl(const void *indptr, int ptr_bytes, const void *indices, int 
   const PickHopExtras pick_hop{sub_indptr, plan_hop.tile_prefix_out, plan_hop.raw_tiles_out, nnz_out,
                                const_cast<uint64_t *>(plan_hop.total_out), S_len, rng_seed_dev, total_out, elem_bytes,
                                static_cast<uint4 *>(table.slots), table.n16, table.wide_mark, table.nonce,
-                               coo_dst, coo_bytes};
+                               coo_dst, coo_bytes, table.classified ? table.classes : RelabelClasses{}};
   rc = pick_impl(indices, cache_indices, idx_bytes, seeds, seed_bytes, S, k, replace, sub_indptr, ptr_bytes,
                  plan, sub_indices, rng_seed, rng_stream, launcher, &pick_hop);
   if (rc) return rc;
@@ -1387,8 +1459,9 @@ int shmt_sample_hops_chained(const shmt_hop_job *jobs, int n_jobs, void *stream)
     for (int i = 0; i < lists[0].n; ++i) {
       const Stage *stages[kMaxJobs];
       for (int j = 0; j < n; ++j) stages[j] = &lists[j].stage[i];
-      const int rc = stages[0]->kind >= kStageRlSmall ? launch_merged_relabel_stage(n, stages, s)
-                                                      : launch_merged_sampling_stage(n, stages, s);
+      const int kind = stages[0]->kind;
+      const int rc = kind >= kStageRlSmall && kind < kStagePickClassifyHop ? launch_merged_relabel_stage(n, stages, s)
+                                                                           : launch_merged_sampling_stage(n, stages, s);
       if (rc) return rc;
     }
   }
