@@ -110,6 +110,11 @@ int shmt_hashmap_create(shmt_hashmap_t **out, const void *keys,
  * layout must come from shmt_hashmap_plan on the same, unchanged keys and
  * values: the build trusts it (a rank layout is only re-checked for
  * n < 2^32, the width of its running counts).
+ * Large tables of 8-byte slots ask for some memory more than their buckets
+ * need: shmt_hashmap_create_planned_scratch puts a presence filter there, with
+ * which lookups of absent keys are cheaper. With a layout or table memory that
+ * holds the buckets alone (shmt_hashmap_table_bytes of 4-byte keys and values)
+ * the table has none.
  * `scratch` is device memory of shmt_hashmap_plan_scratch_bytes(n) bytes,
  * 16-byte aligned, free again when plan returns.                            */
 #define SHMT_MAP_BUCKETS 0

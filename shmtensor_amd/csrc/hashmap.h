@@ -12,4 +12,6 @@ struct shmt_hashmap {
   int val_bytes;
   int64_t n;              // number of (key, value) pairs given to the build
   int64_t table_bytes;
+  const uint32_t *filter; // presence filter (see filter_bits), or null
+  int filter_shift;
 };

@@ -182,6 +182,24 @@ constexpr int kPartBlock = 1024;
 constexpr uint32_t kPartLookBack = 16;    // words in which a repeat of a key is looked for
 constexpr int kPartRestBlocks = 1024;     // (none to do: 4 us, as with 64)
 
+// Presence filter of a table of `nb` buckets (see filter_bits). What a lookup costs is the line it reads from beyond the
+// L2s, which deliver some 52 G lines a second whether all of a line is asked for or 16 bytes of it; a request that is
+// not a key needs none if a filter that the L2s hold says so. One word per bucket: 8 keys on average at half load, of which
+// 1 absent request in 6 gets past; tables of more than 2^19 buckets share words, as 2 MiB is what an L2 of 4 MiB
+// keeps beside the lines that stream through it (stand-alone probe, half of 16.8 M requests let through to a table
+// of 64 MiB: no filter 320 us, 1 MiB 227, 2 MiB 239, 4 MiB 300).
+constexpr int64_t kFilterMaxWords = 1 << 19;
+// From 2^19 pairs on, where the table no longer fits the L2s: 16.8 M requests, half of them keys, 16 slots of 128 bytes for
+// 5 keys (load 0.3) 247 us without, 205 with; for 8 keys 206 and 204, all absent 208 and 187.
+constexpr int64_t kFilterMinKeys = 1 << 19;
+
+static int filter_shift(int64_t nb) {
+  int shift = 0;
+  while ((nb >> shift) > kFilterMaxWords) ++shift;
+  return shift;
+}
+__host__ __device__ __forceinline__ uint32_t filter_words(uint32_t nb, int shift) { return (nb + (1u << shift) - 1) >> shift; }
+
 struct PartArgs {
   MapView map;
   uint64_t *table;
@@ -194,6 +212,8 @@ struct PartArgs {
   uint64_t *rest;       // n
   uint32_t *rest_count;
   uint32_t *filled;     // per partition: words dealt to it (may exceed room)
+  uint32_t *filter;     // presence filter to be written, or null
+  int filter_shift;
 };
 
 __device__ __forceinline__ uint32_t part_of(const MapView &m, uint64_t word) {
@@ -284,6 +304,7 @@ __global__ __launch_bounds__(kPartBlock) void part_deal_kernel(PartArgs a) {
 
 __global__ __launch_bounds__(kPartBlock) void part_fill_kernel(PartArgs a) {
   __shared__ alignas(16) unsigned long long slots[kPartBuckets * 16];
+  __shared__ uint32_t present[kPartBuckets];  // this partition's words of the presence filter
   uint4 *const slots4 = reinterpret_cast<uint4 *>(slots);
   const uint32_t p = blockIdx.x;
   const uint32_t bucket0 = p << kPartLog2Buckets;
@@ -303,6 +324,7 @@ __global__ __launch_bounds__(kPartBlock) void part_fill_kernel(PartArgs a) {
   load(0);  // on their way while the slots are cleared
   for (uint32_t i = threadIdx.x; i < kPartBuckets * kProbeGroup; i += kPartBlock)
     slots4[i] = make_uint4(~0u, ~0u, ~0u, ~0u);
+  if (threadIdx.x < kPartBuckets) present[threadIdx.x] = 0;
   __syncthreads();
   for (uint32_t e0 = 0; e0 < cnt; e0 += kHeld * kPartBlock) {
     if (e0 > 0) load(e0);
@@ -311,6 +333,7 @@ __global__ __launch_bounds__(kPartBlock) void part_fill_kernel(PartArgs a) {
       if (held[j] == ~0ull) continue;
       const uint32_t h = hash_id(slot8_key(a.map, held[j]));
       const uint32_t home = reduce_range(h, a.map.nbuckets) - bucket0;
+      if (a.filter) atomicOr(&present[home >> a.filter_shift], filter_bits(h));
       bool placed = false;
       for (uint32_t b = home; b < nb && !placed; ++b) {
         // any order of the slots will do: threads that meet in a bucket start at different ones
@@ -330,6 +353,8 @@ __global__ __launch_bounds__(kPartBlock) void part_fill_kernel(PartArgs a) {
   __syncthreads();
   uint4 *const out = reinterpret_cast<uint4 *>(a.table) + static_cast<size_t>(bucket0) * kProbeGroup;
   for (uint32_t i = threadIdx.x; i < nb * kProbeGroup; i += kPartBlock) out[i] = slots4[i];
+  if (a.filter && threadIdx.x < filter_words(nb, a.filter_shift))
+    a.filter[(bucket0 >> a.filter_shift) + threadIdx.x] = present[threadIdx.x];
 }
 
 // One word per probe group at a time: as a rule there are a few dozen, and a wave that took 64 of them would
@@ -337,7 +362,14 @@ __global__ __launch_bounds__(kPartBlock) void part_fill_kernel(PartArgs a) {
 __global__ __launch_bounds__(256) void part_rest_kernel(PartArgs a) {
   const uint32_t n = *a.rest_count;
   const uint32_t groups = gridDim.x * (256 / kProbeGroup);
-  for (uint32_t e = (blockIdx.x * 256 + threadIdx.x) / kProbeGroup; e < n; e += groups) group_insert8(a.table, a.map, a.rest[e]);
+  for (uint32_t e = (blockIdx.x * 256 + threadIdx.x) / kProbeGroup; e < n; e += groups) {
+    const uint64_t word = a.rest[e];
+    if (a.filter && (lane_id() & (kProbeGroup - 1)) == 0) {  // (words that found no room in `deal` never got to `fill`)
+      const uint32_t h = hash_id(slot8_key(a.map, word));
+      atomicOr(&a.filter[reduce_range(h, a.map.nbuckets) >> a.filter_shift], filter_bits(h));
+    }
+    group_insert8(a.table, a.map, word);
+  }
 }
 
 // ---- what do the keys look like? ---------------------------------------------
@@ -547,20 +579,39 @@ __global__ __launch_bounds__(256) void rank_build_kernel(uint4 *table, int64_t n
 // range of a packed table read no line of their own: half of them there, 204 us.) Each bucket load waiting for
 // the one before, and all lanes of a group hashing all of its keys: 366 us. Eight waves per SIMD
 // are asked for: the fragments alone are 32 registers.
-template <int FMT>
+// FILTER: the filter is asked first while that pays. It costs an access to the L2s per request and saves a line per
+// request that it turns away: a wave looks up its first 64 requests without it, turns to it when kFilterOn of 64
+// requests were absent, and away again when fewer than kFilterOff of 64 were turned away. (Stand-alone probe as
+// above, filter of 2 MiB: everything let through 393 us, 5/8 268, half 239, without filter 320: even at 15 of 64.)
+// 16,777,216 requests as above, all / 3/4 / half / none of them keys: 330 / 331 / 335 / 338 us without filter,
+// 328 / 335 / 274 / 209 with it; to a table of 2,097,152 keys 306 / 306 / 312 / 312 and 299 / 311 / 236 / 206.
+constexpr int kFilterOn = 28, kFilterOff = 16;
+
+template <int FMT, bool FILTER>
 __global__ __launch_bounds__(256, 8) void hashmap_query_kernel(
-    MapView m, const void *req, int req_bytes, void *out, int out_bytes, int64_t n) {
+    MapView m, const void *req, int req_bytes, void *out, int out_bytes, int64_t n, const uint32_t *filter, int filter_shift) {
   const int lane = lane_id();
   const int64_t waves_per_block = blockDim.x / kWave;
   int64_t wave = static_cast<int64_t>(blockIdx.x) * waves_per_block + threadIdx.x / kWave;
   const int64_t nwaves = static_cast<int64_t>(gridDim.x) * waves_per_block;
   int64_t i = wave * kWave + lane;
   int64_t next = i < n ? load_int(req, i, req_bytes) : -1;  // the requests stay one step ahead of the probes
+  bool ask = false;
   for (; i - lane < n; i += nwaves * kWave) {
     const int64_t mykey = i < n ? map_key(m, next) : -1;  // tail lanes look up the sentinel, which resolves to -1
     const int64_t ahead = i + nwaves * kWave;
     if (ahead < n) next = load_int(req, ahead, req_bytes);
-    const int64_t myres = wave_find<FMT>(m, mykey);
+    uint64_t wanted = ~0ull;
+    if (FILTER && ask) {
+      const uint32_t h = hash_id(mykey), bits = filter_bits(h);
+      wanted = __builtin_amdgcn_ballot_w64(mykey != -1 &&
+                                           (filter[reduce_range(h, m.nbuckets) >> filter_shift] & bits) == bits);
+    }
+    const int64_t myres = wave_find<FMT, FILTER>(m, mykey, wanted);
+    if (FILTER) {
+      const uint64_t away = ask ? ~wanted : __builtin_amdgcn_ballot_w64(myres == -1);
+      ask = __builtin_popcountll(away) >= (ask ? kFilterOff : kFilterOn);
+    }
     if (i < n) store_int(out, i, out_bytes, myres);
   }
 }
@@ -570,6 +621,8 @@ __global__ __launch_bounds__(256, 8) void hashmap_query_kernel(
 using namespace shmt;
 
 extern "C" {
+
+static int64_t filter_bytes(int64_t n, int64_t nbuckets);
 
 int64_t shmt_hashmap_capacity(int64_t n, double load_factor) {
   if (n < 0 || !(load_factor > 0.0)) return -1;
@@ -643,6 +696,7 @@ int shmt_hashmap_plan(const void *keys, const void *vals, int64_t n, int key_byt
   }
   layout->slot_bytes = fmt;
   layout->table_bytes = buckets_for(n, load_factor, fmt) * kBucketBytes;
+  if (fmt == kSlot8) layout->table_bytes += filter_bytes(n, layout->table_bytes / kBucketBytes);
   // flat forms need non-negative ids (-1 is the empty key) and a span that can be indexed
   if (st.kmin < 0 || st.kmax - st.kmin >= (1ll << 40)) return SHMT_OK;
   const int64_t span = st.kmax - st.kmin + 1;
@@ -722,6 +776,13 @@ static PartPlan part_plan(int fmt, int64_t n, int64_t nbuckets) {
   p.rest_off = p.words_off + static_cast<int64_t>(p.parts) * p.room * 8;
   p.bytes = p.rest_off + n * 8;
   return p;
+}
+
+// Bytes of the presence filter behind the buckets, of tables that are built by partitions.
+static int64_t filter_bytes(int64_t n, int64_t nbuckets) {
+  if (n < kFilterMinKeys || part_plan(kSlot8, n, nbuckets).parts == 0) return 0;
+  return (static_cast<int64_t>(filter_words(static_cast<uint32_t>(nbuckets), filter_shift(nbuckets))) * 4 + kBucketBytes - 1) /
+         kBucketBytes * kBucketBytes;
 }
 
 int64_t shmt_hashmap_build_scratch_bytes(const shmt_hashmap_layout *layout, int64_t n, double load_factor) {
@@ -868,6 +929,7 @@ static int build_buckets(shmt_hashmap_t **out, const int fmt, const void *keys, 
 
   hipStream_t s = as_stream(stream);
   const PartPlan parts = part_plan(fmt, n, nb);
+  uint32_t *filter = nullptr;  // in the memory that the plan asked for behind the buckets
   if (parts.parts > 0 && scratch != nullptr && scratch_bytes >= parts.bytes) {
     SHMT_REQUIRE((reinterpret_cast<uintptr_t>(scratch) & 15) == 0, "shmt_hashmap_create: scratch must be 16-byte aligned");
     char *const mem = static_cast<char *>(scratch);
@@ -885,6 +947,11 @@ static int build_buckets(shmt_hashmap_t **out, const int fmt, const void *keys, 
     a.rest_count = a.filled + kPartMax;
     a.words = reinterpret_cast<uint64_t *>(mem + parts.words_off);
     a.rest = reinterpret_cast<uint64_t *>(mem + parts.rest_off);
+    const int64_t with_filter = nb * kBucketBytes + filter_bytes(n, nb);
+    if (with_filter > nb * kBucketBytes && layout != nullptr && layout->table_bytes >= with_filter && table_bytes >= with_filter)
+      filter = reinterpret_cast<uint32_t *>(static_cast<char *>(table_mem) + nb * kBucketBytes);
+    a.filter = filter;
+    a.filter_shift = filter_shift(nb);
     hipLaunchKernelGGL(fill_zero_kernel, dim3(1), dim3(256), 0, s, a.filled, static_cast<int64_t>(kPartMax) + 1);
     // tiles of 16,384 pairs write longer runs: 4,189,304 pairs 130 us against 146 with tiles of 4,096, 2^21 98
     // against 102, 2^20 (64 tiles) the same
@@ -924,6 +991,8 @@ static int build_buckets(shmt_hashmap_t **out, const int fmt, const void *keys, 
   h->val_bytes = val_bytes;
   h->n = n;
   h->table_bytes = nb * kBucketBytes;
+  h->filter = filter;
+  h->filter_shift = filter_shift(nb);
   *out = h;
   return SHMT_OK;
 }
@@ -937,12 +1006,11 @@ int shmt_hashmap_query(const shmt_hashmap_t *map, const void *requests, int req_
   SHMT_REQUIRE(requests != nullptr && out != nullptr, "shmt_hashmap_query: null buffer");
   unsigned grid = grid_for(n, 256);
   hipStream_t s = as_stream(stream);
-  if (map->fmt == kSlot16)
-    hipLaunchKernelGGL(hashmap_query_kernel<kSlot16>, dim3(grid), dim3(256), 0, s, map->view,
-                       requests, req_bytes, out, map->val_bytes, n);
-  else
-    hipLaunchKernelGGL(hashmap_query_kernel<kSlot8>, dim3(grid), dim3(256), 0, s, map->view,
-                       requests, req_bytes, out, map->val_bytes, n);
+  const auto kernel = map->fmt == kSlot16 ? hashmap_query_kernel<kSlot16, false>
+                      : map->filter       ? hashmap_query_kernel<kSlot8, true>
+                                          : hashmap_query_kernel<kSlot8, false>;
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), 0, s, map->view, requests, req_bytes, out, map->val_bytes, n,
+                     map->filter, map->filter_shift);
   SHMT_LAUNCH_CHECK();
   return SHMT_OK;
 }

@@ -233,8 +233,8 @@ constexpr uint64_t kGroupBits = 0x0101010101010101ull;  // bit 8g: probe group g
 // found reaches every lane through three AND steps: against finding the
 // matching lane with a ballot per group and asking it for the value, this
 // takes a third of the vector instructions.
-template <int FMT>
-__device__ __forceinline__ uint64_t probe_buckets(const MapView &m, const uint4 frag, uint64_t want, uint64_t *raw) {
+template <int FMT, typename Frag>
+__device__ __forceinline__ uint64_t probe_buckets(const MapView &m, const Frag frag, uint64_t want, uint64_t *raw) {
   bool hit, empty;
   uint64_t mine;
   if (FMT == kSlot16) {
@@ -266,6 +266,12 @@ __device__ __forceinline__ uint64_t probe_buckets(const MapView &m, const uint4 
 __device__ __forceinline__ void keep_loaded(uint4 *frag) {
   asm volatile("" : "+v"(frag->x), "+v"(frag->y), "+v"(frag->z), "+v"(frag->w));
 }
+// (as one operand: of four the compiler may make copies, each with a wait for its load)
+__device__ __forceinline__ void keep_loaded(probe_u32x4 *frag) { asm volatile("" : "+v"(*frag)); }
+
+// Presence filter of a large narrow table: one word per 1 << shift home buckets, two bits of it set for every key. A
+// key whose bits are not both set is absent. The bucket number uses the top bits of the hash, these use the low ones.
+__device__ __forceinline__ uint32_t filter_bits(uint32_t hash) { return (1u << (hash & 31u)) | (1u << ((hash >> 5) & 31u)); }
 
 // Whole-wave find: every lane brings its own (already normalised) key; the
 // wave's eight probe groups resolve the 64 keys, eight keys per group. The
@@ -278,18 +284,29 @@ __device__ __forceinline__ void keep_loaded(uint4 *frag) {
 // every lane for itself.
 template <int FMT>
 struct WaveProbe {
-  uint4 frag[kProbeGroup];
+  probe_u32x4 frag[kProbeGroup];
   uint64_t want, res;
   uint64_t open;  // bit l: the key of lane l is not resolved (uniform)
   uint32_t home;
 };
 
-template <int FMT, int J>
-__device__ __forceinline__ void wave_probe_load(const MapView &m, WaveProbe<FMT> *p) {
+// SKIP: keys that are not in `wanted` (bit l: the key of lane l) are known to be absent and read no line. Their lanes ask
+// for an address behind the table, which a buffer load answers with zeros without a request: loads under a lane mask
+// would each end in a wait (the table must be below 4 GiB, see table_resource).
+constexpr uint32_t kNoBucket = ~0u;
+
+template <int FMT, int J, bool SKIP = false>
+__device__ __forceinline__ void wave_probe_load(const MapView &m, WaveProbe<FMT> *p, __amdgpu_buffer_rsrc_t table) {
   if constexpr (J < kProbeGroup) {
-    const int sub = lane_id() & (kProbeGroup - 1);
-    p->frag[J] = m.buckets[static_cast<size_t>(group_bcast<J>(p->home)) * kProbeGroup + sub];
-    wave_probe_load<FMT, J + 1>(m, p);
+    const uint32_t sub = lane_id() & (kProbeGroup - 1);
+    const uint32_t home = group_bcast<J>(p->home);
+    if constexpr (SKIP) {
+      p->frag[J] = __builtin_amdgcn_raw_buffer_load_b128(
+          table, home == kNoBucket ? kNoBucket : (home * kProbeGroup + sub) * 16u, 0, 0);
+    } else {
+      p->frag[J] = reinterpret_cast<const probe_u32x4 *>(m.buckets)[static_cast<size_t>(home) * kProbeGroup + sub];
+    }
+    wave_probe_load<FMT, J + 1, SKIP>(m, p, table);
   }
 }
 
@@ -326,17 +343,25 @@ __device__ __forceinline__ void wave_probe_walk(const MapView &m, WaveProbe<FMT>
   }
 }
 
-template <int FMT>
-__device__ __forceinline__ int64_t wave_find(const MapView &m, int64_t mykey) {
-  if (m.kind != kKindBuckets) return flat_find(m, mykey);  // uniform across the launch
+template <int FMT, bool SKIP = false>
+__device__ __forceinline__ int64_t wave_find(const MapView &m, int64_t mykey, uint64_t wanted = ~0ull) {
+  if (!SKIP && m.kind != kKindBuckets) return flat_find(m, mykey);  // uniform across the launch
   WaveProbe<FMT> p;
   p.want = probe_want<FMT>(m, mykey);
   p.home = map_bucket(m, mykey);
   p.open = 0;
-  wave_probe_load<FMT, 0>(m, &p);
+  // (used where SKIP: ends with the table, words as in table_resource)
+  const __amdgpu_buffer_rsrc_t table = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint4 *>(m.buckets), 0, static_cast<int>(m.nbuckets * static_cast<uint32_t>(kBucketBytes)), 0x00020000);
+  if (SKIP && !__builtin_amdgcn_inverse_ballot_w64(wanted)) p.home = kNoBucket;
+  wave_probe_load<FMT, 0, SKIP>(m, &p, table);
 #pragma unroll
   for (int j = 0; j < kProbeGroup; ++j) keep_loaded(&p.frag[j]);
   wave_probe_examine<FMT, 0>(m, &p);
+  if constexpr (SKIP) {
+    p.open &= wanted;
+    if (!__builtin_amdgcn_inverse_ballot_w64(wanted)) p.res = ~0ull;
+  }
   for (uint32_t round = 1; p.open != 0 && round < m.nbuckets; ++round) wave_probe_walk<FMT>(m, &p, round);
   return raw_value<FMT>(m, p.res);
 }

@@ -211,8 +211,12 @@ class StaticHashmap {
       check(shmt_hashmap_plan(keys.data_ptr(), values.data_ptr(), n, kb, vb, load_factor, scratch.data_ptr(),
                               scratch_bytes, &layout, current_stream()));
     }
-    table_ = device_bytes(layout.table_bytes);
-    memory_usage_ = layout.kind == SHMT_MAP_RANGE ? 0 : layout.table_bytes;
+    if (layout.kind == SHMT_MAP_BUCKETS && layout.slot_bytes == 8) {
+      // (a large one has a presence filter behind its buckets; where only the buckets fit, lookups go without it)
+      table_ = spare_device_bytes(layout.table_bytes);
+      if (!table_.defined()) layout.table_bytes = shmt_hashmap_table_bytes(n, load_factor, 4, 4);
+    }
+    if (!table_.defined()) table_ = device_bytes(layout.table_bytes);
     kind_ = layout.kind;
     const int64_t build_bytes = shmt_hashmap_build_scratch_bytes(&layout, n, load_factor);
     const torch::Tensor build_scratch = spare_device_bytes(build_bytes);
@@ -220,6 +224,7 @@ class StaticHashmap {
                                               load_factor, table_.data_ptr(), layout.table_bytes,
                                               build_scratch.defined() ? build_scratch.data_ptr() : nullptr,
                                               build_scratch.defined() ? build_bytes : 0, current_stream()));
+    memory_usage_ = shmt_hashmap_used_bytes(handle_);
   }
   ~StaticHashmap() { shmt_hashmap_destroy(handle_); }
   StaticHashmap(const StaticHashmap &) = delete;
