@@ -382,9 +382,9 @@ struct KeyStats {
   unsigned long long not_ranked;  // != 0: keys do not ascend strictly, or value i is not value 0 + i
 };
 
-constexpr int kStatBlocks = 1024;          // workgroups of a sweep, each leaving one partial result
-constexpr int64_t kStatPartialsOff = 256;  // scratch layout: header, partials, then one mark byte per id
-constexpr int64_t kStatMarksOff = kStatPartialsOff + ((kStatBlocks * sizeof(KeyStats) + 255) & ~255ll);
+constexpr int kStatThreads = 1024;
+constexpr int kStatBlocks = 256;           // workgroups of a sweep, one per compute unit, each leaving one partial result
+constexpr int64_t kStatMarksOff = 57600;   // scratch layout: one mark byte per id from here on (what lies before is spare)
 
 __device__ __forceinline__ int64_t wave_min64(int64_t v) {
 #pragma unroll
@@ -403,11 +403,21 @@ __device__ __forceinline__ int64_t wave_max64(int64_t v) {
   return v;
 }
 
+__device__ __host__ __forceinline__ void add_stats(KeyStats *to, const KeyStats &o) {
+  to->kmin = o.kmin < to->kmin ? o.kmin : to->kmin;
+  to->kmax = o.kmax > to->kmax ? o.kmax : to->kmax;
+  to->vmin = o.vmin < to->vmin ? o.vmin : to->vmin;
+  to->vmax = o.vmax > to->vmax ? o.vmax : to->vmax;
+  to->not_affine |= o.not_affine;
+  to->not_ranked |= o.not_ranked;
+  to->distinct += o.distinct;
+}
+
 // Combines the calling workgroup's per-thread values into one KeyStats, valid
 // in thread 0 (no atomics: thousands of them on a handful of addresses would
 // cost more than the sweep).
 __device__ __forceinline__ KeyStats block_combine(KeyStats mine) {
-  __shared__ KeyStats per_wave[256 / kWave];
+  __shared__ KeyStats per_wave[kStatThreads / kWave];
   mine.kmin = wave_min64(mine.kmin);
   mine.kmax = wave_max64(mine.kmax);
   mine.vmin = wave_min64(mine.vmin);
@@ -419,16 +429,7 @@ __device__ __forceinline__ KeyStats block_combine(KeyStats mine) {
   __syncthreads();
   KeyStats all = per_wave[0];
   if (threadIdx.x == 0) {
-    for (unsigned w = 1; w < blockDim.x / kWave; ++w) {
-      const KeyStats o = per_wave[w];
-      all.kmin = o.kmin < all.kmin ? o.kmin : all.kmin;
-      all.kmax = o.kmax > all.kmax ? o.kmax : all.kmax;
-      all.vmin = o.vmin < all.vmin ? o.vmin : all.vmin;
-      all.vmax = o.vmax > all.vmax ? o.vmax : all.vmax;
-      all.not_affine |= o.not_affine;
-      all.not_ranked |= o.not_ranked;
-      all.distinct += o.distinct;
-    }
+    for (unsigned w = 1; w < blockDim.x / kWave; ++w) add_stats(&all, per_wave[w]);
   }
   return all;
 }
@@ -437,65 +438,68 @@ __device__ __forceinline__ KeyStats neutral_stats() {
   return KeyStats{INT64_MAX, INT64_MIN, INT64_MAX, INT64_MIN, 0, 0, 0};
 }
 
-__global__ __launch_bounds__(256) void key_stats_kernel(const void *keys, const void *vals, int64_t n,
-                                                        int key_bytes, int val_bytes, KeyStats *partials) {
+// The sweep over all pairs. Bound by HBM: four pairs per thread are in flight, and the key before a pair's own comes from the
+// lane next door: 4,194,304 pairs of 16 bytes 15.9 us, 4.2 TB/s (with one pair, and that key loaded again, 19.8).
+constexpr int kStatItems = 4;
+__global__ __launch_bounds__(kStatThreads) void key_stats_kernel(const void *keys, const void *vals, int64_t n,
+                                                                 int key_bytes, int val_bytes, KeyStats *partials) {
   const int64_t v0 = load_int(vals, 0, val_bytes);
   const int64_t delta0 = v0 - load_int(keys, 0, key_bytes);
   KeyStats mine = neutral_stats();
-  const int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
-  for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += stride) {
-    const int64_t k = load_int(keys, i, key_bytes), v = load_int(vals, i, val_bytes);
-    mine.kmin = k < mine.kmin ? k : mine.kmin;
-    mine.kmax = k > mine.kmax ? k : mine.kmax;
-    mine.vmin = v < mine.vmin ? v : mine.vmin;
-    mine.vmax = v > mine.vmax ? v : mine.vmax;
-    mine.not_affine |= (v - k != delta0);
-    // the neighbour's key is the load of the thread next door: served by the caches
-    mine.not_ranked |= (v != v0 + i) || (i > 0 && load_int(keys, i - 1, key_bytes) >= k);
+  constexpr int64_t kSpan = kStatThreads * kStatItems;
+  for (int64_t base = blockIdx.x * kSpan; base < n; base += gridDim.x * kSpan) {
+    int64_t idx[kStatItems], before_idx[kStatItems], key[kStatItems], val[kStatItems], before[kStatItems];
+    bool ok[kStatItems], first[kStatItems];
+#pragma unroll
+    for (int j = 0; j < kStatItems; ++j) {
+      idx[j] = base + j * kStatThreads + threadIdx.x;
+      before_idx[j] = idx[j] - 1;
+      ok[j] = idx[j] < n;
+      first[j] = ok[j] && lane_id() == 0 && idx[j] > 0;
+      key[j] = val[j] = before[j] = 0;
+    }
+    load_ints<kStatItems>(keys, idx, ok, key_bytes, key);
+    load_ints<kStatItems>(vals, idx, ok, val_bytes, val);
+    load_ints<kStatItems>(keys, before_idx, first, key_bytes, before);
+#pragma unroll
+    for (int j = 0; j < kStatItems; ++j) {
+      const int64_t next_door = shfl64(key[j], lane_id() - 1);
+      if (!ok[j]) continue;
+      const int64_t k = key[j], v = val[j], b = lane_id() == 0 ? before[j] : next_door;
+      mine.kmin = k < mine.kmin ? k : mine.kmin;
+      mine.kmax = k > mine.kmax ? k : mine.kmax;
+      mine.vmin = v < mine.vmin ? v : mine.vmin;
+      mine.vmax = v > mine.vmax ? v : mine.vmax;
+      mine.not_affine |= (v - k != delta0);
+      mine.not_ranked |= (v != v0 + idx[j]) || (idx[j] > 0 && b >= k);
+    }
   }
   const KeyStats all = block_combine(mine);
   if (threadIdx.x == 0) partials[blockIdx.x] = all;
 }
 
-// One workgroup merges the partial results of a sweep and hands the outcome to
-// the host through a slot of pinned host memory (a device-to-host copy into
-// pageable memory would go through the runtime's staging path).
-__global__ __launch_bounds__(256) void stats_merge_kernel(const KeyStats *partials, int nb, KeyStats *host_slot) {
-  KeyStats mine = neutral_stats();
-  for (int b = threadIdx.x; b < nb; b += blockDim.x) {
-    const KeyStats o = partials[b];
-    mine.kmin = o.kmin < mine.kmin ? o.kmin : mine.kmin;
-    mine.kmax = o.kmax > mine.kmax ? o.kmax : mine.kmax;
-    mine.vmin = o.vmin < mine.vmin ? o.vmin : mine.vmin;
-    mine.vmax = o.vmax > mine.vmax ? o.vmax : mine.vmax;
-    mine.not_affine |= o.not_affine;
-    mine.not_ranked |= o.not_ranked;
-    mine.distinct += o.distinct;
-  }
-  const KeyStats all = block_combine(mine);
-  if (threadIdx.x == 0) *host_slot = all;
-}
-
-// One slot of pinned host memory per process, allocated on first use; map
-// builds that run at the same time take turns at it.
+// The partial results of a sweep go straight to pinned host memory, one set per process, allocated on first use (a
+// launch that merged them on the device took 4 us); map builds that run at the same time take turns at it.
 static std::mutex g_stat_mutex;
-static KeyStats *g_stat_slot = nullptr;      // pinned host memory
-static KeyStats *g_stat_slot_dev = nullptr;  // its device alias
+static KeyStats *g_stat_slots = nullptr;      // pinned host memory, kStatBlocks
+static KeyStats *g_stat_slots_dev = nullptr;  // its device alias
 
-// Merge the partial results of a sweep, hand them to the host and wait for them.
-static int read_stats(const KeyStats *partials, int nb, KeyStats *out, hipStream_t s) {
+// Launch a sweep of nb <= kStatBlocks workgroups (`launch` is given where their results go) and wait for what it finds.
+template <typename Launch>
+static int read_stats(int nb, KeyStats *out, hipStream_t s, Launch launch) {
   std::lock_guard<std::mutex> lock(g_stat_mutex);
-  if (g_stat_slot == nullptr) {
+  if (g_stat_slots == nullptr) {
     void *p = nullptr, *d = nullptr;
-    SHMT_HIP(hipHostMalloc(&p, 256, hipHostMallocMapped));
+    SHMT_HIP(hipHostMalloc(&p, kStatBlocks * sizeof(KeyStats), hipHostMallocMapped));
     SHMT_HIP(hipHostGetDevicePointer(&d, p, 0));
-    g_stat_slot = static_cast<KeyStats *>(p);
-    g_stat_slot_dev = static_cast<KeyStats *>(d);
+    g_stat_slots = static_cast<KeyStats *>(p);
+    g_stat_slots_dev = static_cast<KeyStats *>(d);
   }
-  hipLaunchKernelGGL(stats_merge_kernel, dim3(1), dim3(256), 0, s, partials, nb, g_stat_slot_dev);
+  launch(g_stat_slots_dev);
   SHMT_LAUNCH_CHECK();
   SHMT_HIP(hipStreamSynchronize(s));
-  *out = *g_stat_slot;
+  *out = g_stat_slots[0];
+  for (int b = 1; b < nb; ++b) add_stats(out, g_stat_slots[b]);
   return SHMT_OK;
 }
 
@@ -668,13 +672,12 @@ int shmt_hashmap_plan(const void *keys, const void *vals, int64_t n, int key_byt
   }
   SHMT_REQUIRE((reinterpret_cast<uintptr_t>(scratch) & 15) == 0, "shmt_hashmap_plan: scratch must be 16-byte aligned");
   hipStream_t s = as_stream(stream);
-  KeyStats *partials = reinterpret_cast<KeyStats *>(static_cast<char *>(scratch) + kStatPartialsOff);
   uint32_t *marks = reinterpret_cast<uint32_t *>(static_cast<char *>(scratch) + kStatMarksOff);  // one byte per id
-  const unsigned nb = grid_for(n, 256 * 8, kStatBlocks);
-  hipLaunchKernelGGL(key_stats_kernel, dim3(nb), dim3(256), 0, s, keys, vals, n, key_bytes, val_bytes, partials);
-  SHMT_LAUNCH_CHECK();
+  const unsigned nb = grid_for(n, kStatThreads * kStatItems, kStatBlocks);
   KeyStats st;
-  int rc = read_stats(partials, static_cast<int>(nb), &st, s);
+  int rc = read_stats(static_cast<int>(nb), &st, s, [&](KeyStats *partials) {
+    hipLaunchKernelGGL(key_stats_kernel, dim3(nb), dim3(kStatThreads), 0, s, keys, vals, n, key_bytes, val_bytes, partials);
+  });
   if (rc) return rc;
 
   const bool keys32 = st.kmin >= INT32_MIN && st.kmax <= INT32_MAX;
@@ -707,10 +710,11 @@ int shmt_hashmap_plan(const void *keys, const void *vals, int64_t n, int key_byt
     hipLaunchKernelGGL(key_mark_kernel, dim3(grid_for(n, 256 * 8, 256 * 8)), dim3(256), 0, s, keys, n, key_bytes,
                        static_cast<int64_t>(st.kmin), reinterpret_cast<uint8_t *>(marks));
     const unsigned nbc = grid_for(words, 256 * 8, kStatBlocks);
-    hipLaunchKernelGGL(key_count_marks_kernel, dim3(nbc), dim3(256), 0, s, marks, words, partials);
     SHMT_LAUNCH_CHECK();
     KeyStats counted;
-    rc = read_stats(partials, static_cast<int>(nbc), &counted, s);
+    rc = read_stats(static_cast<int>(nbc), &counted, s, [&](KeyStats *partials) {
+      hipLaunchKernelGGL(key_count_marks_kernel, dim3(nbc), dim3(256), 0, s, marks, words, partials);
+    });
     if (rc) return rc;
     if (counted.distinct == static_cast<unsigned long long>(n)) {
       layout->kind = SHMT_MAP_RANGE;
@@ -953,14 +957,11 @@ static int build_buckets(shmt_hashmap_t **out, const int fmt, const void *keys, 
     a.filter = filter;
     a.filter_shift = filter_shift(nb);
     hipLaunchKernelGGL(fill_zero_kernel, dim3(1), dim3(256), 0, s, a.filled, static_cast<int64_t>(kPartMax) + 1);
-    // tiles of 16,384 pairs write longer runs: 4,189,304 pairs 130 us against 146 with tiles of 4,096, 2^21 98
-    // against 102, 2^20 (64 tiles) the same
-    if (n >= (1ll << 20))
-      hipLaunchKernelGGL(part_deal_kernel<16>, dim3(static_cast<unsigned>((n + 16 * kPartBlock - 1) / (16 * kPartBlock))),
-                         dim3(kPartBlock), 0, s, a);
-    else
-      hipLaunchKernelGGL(part_deal_kernel<4>, dim3(static_cast<unsigned>((n + 4 * kPartBlock - 1) / (4 * kPartBlock))),
-                         dim3(kPartBlock), 0, s, a);
+    // tiles of 16,384 pairs write longer runs, but there are to be enough of them: 4,194,304 pairs, whole constructor, 104 us
+    // against 110 with tiles of 8,192 (deal 32 and 40), 2^21 75 both, 2^20 62 against 58
+    const auto deal = n >= (1ll << 21) ? part_deal_kernel<16> : n >= (1ll << 20) ? part_deal_kernel<8> : part_deal_kernel<4>;
+    const int64_t tile = (n >= (1ll << 21) ? 16 : n >= (1ll << 20) ? 8 : 4) * kPartBlock;
+    hipLaunchKernelGGL(deal, dim3(static_cast<unsigned>((n + tile - 1) / tile)), dim3(kPartBlock), 0, s, a);
     hipLaunchKernelGGL(part_fill_kernel, dim3(parts.parts), dim3(kPartBlock), 0, s, a);
     hipLaunchKernelGGL(part_rest_kernel, dim3(kPartRestBlocks), dim3(256), 0, s, a);
     SHMT_LAUNCH_CHECK();
