@@ -26,8 +26,6 @@ enum StageKind : int {
   kStageRcBins = 12,  // + 1: the larger table
   kStageRlFinish = 14,
   kStageRcRanks = 15,
-  kStageRpCount = 16,
-  kStageRpRows = 17,
   kStageRpScatter = 18,
   kStageRpGather = 19,
   kStageRpBins = 20,  // + (largest table - this launch's table), log2 of the slots: 20 .. 22

@@ -685,24 +685,21 @@ __global__ void rl_zero_count_kernel(int64_t *count_out, int64_t *count_copy) {
 // empty the table). From a million ids on (kRpExactMin; kRpDefaultMin for a
 // hop sized by a loose bound, kRpMergedMin for hops that share their launches)
 // the same results -- the first-occurrence index of every element, the ranks of
-// the first occurrences and their number per tile of kRpTile ids -- come from five passes
+// the first occurrences and their number per tile of kRpTile ids -- come from three passes
 // that read and write memory in runs instead:
-//   count    a workgroup per tile of kRpTile ids: histogram of the ids over P
-//            bins (bin = top bits of the id's hash), one column of the P x W
-//            matrix; ids that repeat within the tile are counted once
-//   rows     exclusive prefix along every row of the matrix, bin totals
-//   scatter  a workgroup per tile again: record {id, index} of every element
-//            to its bin's run for this tile (bins are contiguous, runs in tile
-//            order), through LDS so that a run is written by consecutive
-//            lanes; per element the place of its record among the tile's
-//   bins     a workgroup per bin: smallest index per id through a table in
+//   scatter  a workgroup per tile of kRpTile ids: records {id, index} of its elements, ordered by
+//            bin (top bits of the id's hash) and written in one piece; ids that repeat within the tile
+//            make one record; per tile where the run of every bin starts, per element the
+//            place of its record among the tile's
+//   bins     a workgroup per bin: the bin's runs of all tiles, smallest index per id through a table in
 //            LDS (the low bits of the hash address it), written per record
-//   gather   a workgroup per tile: the results of its runs, read through LDS
-//            the same way, handed to the elements: first[i], 4 bytes each
-// Few, large bins: a tile's run for a bin should span whole lines (8,192 ids
-// over 256 bins: 32 records; measured on 3.1 M ids, scatter / gather 24 / 14 us
-// with 256 bins, 31 / 17 us with 1,024, and 42 / 29 us before the runs went
-// through LDS).
+//   gather   a workgroup per tile: the results of its records, read in one piece, handed to the
+//            elements: first[i], 4 bytes each
+// 3.1 M ids of 4 bytes: scatter 18.4 us, bins 34, gather 9.6. Bins that lie in one piece instead cost two more passes in
+// front, a histogram per tile and a prefix over tiles, and runs to be found again in gather: 15 + 4 us, scatter 22, bins 25,
+// gather 15. Eight merged hops of up to 350,000 ids: 13.6 + 5 + 27.4 + 21.8 + 18.2 before, 18.2 + 28.8 + 11.4 now. (With room
+// reserved in every bin by an atomic per tile a bin overflows when few ids come often.)
+// Few, large bins: a tile's run for a bin should span whole lines (8,192 ids over 256 bins: 32 records).
 // P = 256 up to 3.67 M ids, 512 up to 7.34 M (a bin's table is at most 7/8 full
 // when every id of the input is distinct); larger inputs keep the table in memory.
 // A bin's table has 4,096 to 16,384 slots (half for ids beyond 32 bits), two
@@ -718,11 +715,13 @@ constexpr int kRpSlotsLog2 = 14;     // 16,384 slots of 4 + 4 bytes = 128 KB of 
 constexpr int kRpMinBinsLog2 = 8, kRpMaxBinsLog2 = 9;
 constexpr int64_t kRpBinIds = 14336; // ids per bin from which on the number of bins grows: 7/8 of the largest table
 constexpr int kRpTileLog2 = 13;
-constexpr int64_t kRpTile = 1 << kRpTileLog2;  // ids per tile of the count / scatter / gather passes
+constexpr int64_t kRpTile = 1 << kRpTileLog2;  // ids per tile of the scatter / gather passes
 constexpr int kRpMaxRoundsLog2 = 10;
+constexpr uint32_t kRpMaxTiles = static_cast<uint32_t>((kRpBinIds << kRpMaxBinsLog2) / kRpTile);
+static_assert((kRpBinIds << kRpMaxBinsLog2) % kRpTile == 0, "no tile beyond the last whole one");
 constexpr int64_t kRpDefaultMin = kRlSelfPrefixTiles * kRlTile + 1;
 // Hops that share their launches with those of other batches (launchers.h) are sized for a bound of their
-// ids, and the five passes' fixed costs are paid once for all of them: from this bound and this many jobs on
+// ids, and the passes' fixed costs are paid once for all of them: from this bound and this many jobs on
 // they take the partition passes as well.
 constexpr int64_t kRpMergedMin = 512 * 1024;
 // A call that knows its number of ids (not merely a loose bound of it) gains from about a million on.
@@ -741,7 +740,7 @@ struct RpPlan {
   int log2P;
   int table_log2;  // which compiled table size the bin pass uses (the tuning may use less of it)
   uint32_t P, W;
-  int64_t rec_off, first_off, firstp_off, local_off, hist_off, bintot_off, binstart_off, coarse_off, tile_off, end;
+  int64_t rec_off, first_off, firstp_off, local_off, runs_off, coarse_off, end;
 };
 
 // Where the partition passes keep their arrays inside the table memory (16 * cap bytes) of a
@@ -768,12 +767,9 @@ static RpPlan rp_plan(int64_t N, int merged_jobs = 0, bool loose = false) {
   p.first_off = up(16 * N);
   p.firstp_off = p.first_off + up(4 * N);
   p.local_off = p.firstp_off + up(4 * N);
-  p.hist_off = p.local_off + up(2 * N);
-  p.bintot_off = p.hist_off + up(4ll * p.P * p.W);
-  p.binstart_off = p.bintot_off + up(4ll * p.P);
-  p.coarse_off = p.binstart_off + up(4ll * (p.P + 1));
-  p.tile_off = p.coarse_off + up(4ll * p.W);
-  p.end = p.tile_off + up(8ll * p.W * (p.P + 1));
+  p.runs_off = p.local_off + up(2 * N);
+  p.coarse_off = p.runs_off + up(2ll * p.W * (p.P + 1));
+  p.end = p.coarse_off + up(4ll * p.W);
   p.ok = p.end <= rl_capacity(N) * 16;
   return p;
 }
@@ -783,15 +779,13 @@ struct RpArgs {
   int eb;
   RlCount n;
   RlPath path;
-  uint64_t *wide_mark;  // == path.wide_mark, writable: the count pass sets it itself
   int log2P;
-  uint32_t W;
-  void *rec;
+  void *rec;         // record j of tile t at kRpTile * t + j
   uint32_t *first;   // first-occurrence index of every element (what the finish pass reads)
   uint32_t *firstp;  // the same per record, in the records' order
-  uint32_t *hist, *bintot, *binstart, *coarse;
-  uint16_t *local;  // position of every element's record among its tile's records in bin order
-  uint32_t *tile_runs;  // per tile: where its run of every bin starts in memory (P words), then among its records (P + 1 words)
+  uint16_t *local;   // position of every element's record among its tile's records
+  uint16_t *runs;    // per tile: where the run of every bin starts among the tile's records (P + 1)
+  uint32_t *coarse;
   RlRanks *ranks;
   int slots_log2, max_rounds_log2;
 };
@@ -804,16 +798,24 @@ __device__ __forceinline__ uint32_t rp_class(int64_t key) {
 constexpr int kRpItems = static_cast<int>(kRpTile / kRpBlock);  // ids a thread keeps in flight
 static_assert(kRpItems * kRpBlock == kRpTile && kRpTile % kRlTile == 0, "tiles are whole chunks of kRpTile ids");
 
-// The ids of one chunk of kRpTile, element j * kRpBlock + t for thread t: all loads issued before any is used.
-__device__ __forceinline__ void rp_load_chunk(const RpArgs &a, int64_t base, int64_t hi, int64_t (&idx)[kRpItems],
-                                              bool (&ok)[kRpItems], int64_t (&key)[kRpItems]) {
+// The ids of one chunk of `count` <= kRpTile elements, element j * kRpBlock + t for thread t: all loads issued before any is used.
+__device__ __forceinline__ void rp_load_chunk(const void *chunk, uint32_t count, int eb, int64_t (&key)[kRpItems]) {
+  if (eb == 8) {
 #pragma unroll
-  for (int j = 0; j < kRpItems; ++j) {
-    idx[j] = base + j * kRpBlock + threadIdx.x;
-    ok[j] = idx[j] < hi;
-    key[j] = 0;
+    for (int j = 0; j < kRpItems; ++j) {
+      const uint32_t e = j * kRpBlock + threadIdx.x;
+      key[j] = e < count ? static_cast<const int64_t *>(chunk)[e] : 0;
+    }
+  } else {
+    int32_t narrow[kRpItems];
+#pragma unroll
+    for (int j = 0; j < kRpItems; ++j) {
+      const uint32_t e = j * kRpBlock + threadIdx.x;
+      narrow[j] = e < count ? static_cast<const int32_t *>(chunk)[e] : 0;
+    }
+#pragma unroll
+    for (int j = 0; j < kRpItems; ++j) key[j] = narrow[j];
   }
-  load_ints<kRpItems>(a.total, idx, ok, a.eb, key);
 }
 
 // Repeats within a tile. Ids of hub nodes come thousands of times in a sampled batch and would all land in
@@ -822,12 +824,11 @@ __device__ __forceinline__ void rp_load_chunk(const RpArgs &a, int64_t base, int
 // slot = low bits of the hash, value = {index | low 32 bits of the id} of the element with the smallest index
 // that maps there, so an id that comes often is the likely owner of its slot. An element is covered when
 // the slot names an earlier element of the same id; an id that shares its slot with an earlier one of
-// another id is simply not de-duplicated. The table's final content depends on the tile alone, so the
-// count and the scatter pass decide alike.
+// another id is simply not de-duplicated.
 constexpr int kRpDedupSlots = 2048;
 
-__device__ __forceinline__ unsigned long long rp_dedup_word(int64_t key, int64_t idx) {
-  return (static_cast<unsigned long long>(static_cast<uint32_t>(idx)) << 32) | static_cast<uint32_t>(key);
+__device__ __forceinline__ unsigned long long rp_dedup_word(int64_t key, uint32_t i) {
+  return (static_cast<unsigned long long>(i) << 32) | static_cast<uint32_t>(key);
 }
 
 __device__ __forceinline__ void rp_dedup_clear(unsigned long long *dedup) {
@@ -835,221 +836,170 @@ __device__ __forceinline__ void rp_dedup_clear(unsigned long long *dedup) {
 }
 
 __device__ __forceinline__ bool rp_covered(const RpArgs &a, const unsigned long long *dedup, int64_t key,
-                                           int64_t idx, uint32_t hash) {
+                                           uint32_t i, uint32_t hash) {
   const unsigned long long v = dedup[hash & (kRpDedupSlots - 1)];
-  if (static_cast<uint32_t>(v) != static_cast<uint32_t>(key) || static_cast<uint32_t>(v >> 32) == static_cast<uint32_t>(idx))
+  if (static_cast<uint32_t>(v) != static_cast<uint32_t>(key) || static_cast<uint32_t>(v >> 32) == i)
     return false;
   // same low half: 4-byte ids are then equal, 8-byte ids are compared in full
   return a.eb == 4 || static_cast<const int64_t *>(a.total)[static_cast<uint32_t>(v >> 32)] == key;
 }
 
-// SEGS: the ids are still in the caller's segments; the pass also writes their concatenation (`total`), so
-// that no launch of its own reads and writes every id just for that.
+// 8-byte ids that no earlier kernel has seen: whether one of them needs more than 32 bits has to be known before records
+// are written. This pass looks at all of them and writes the concatenation of the caller's segments on the way. (4-byte ids
+// need none: scatter concatenates.)
+constexpr int kRpLookItems = 4;
+
 template <bool SEGS>
-__device__ __forceinline__ void rp_count_body(unsigned bx, const RpArgs &a, const RlSegments &segs) {
-  extern __shared__ uint32_t hist[];  // P counters
-  __shared__ unsigned long long dedup[kRpDedupSlots];
+__global__ __launch_bounds__(256) void rp_look_kernel(RpArgs a, RlSegments segs, uint64_t *wide_mark) {
   const int64_t N = rl_count(a.n);
-  const uint32_t P = 1u << a.log2P;
-  const int64_t lo = static_cast<int64_t>(bx) * kRpTile;
-  if (lo >= N) {
-    // launched for a bound of N: a tile past the ids has an empty column
-    for (uint32_t b = threadIdx.x; b < P; b += kRpBlock) a.hist[static_cast<size_t>(b) * a.W + bx] = 0;
-    return;
-  }
-  for (uint32_t b = threadIdx.x; b < P; b += kRpBlock) hist[b] = 0;
-  rp_dedup_clear(dedup);
-  __syncthreads();
-  const int64_t hi = lo + kRpTile < N ? lo + kRpTile : N;
-  int64_t idx[kRpItems], key[kRpItems];
-  bool ok[kRpItems];
-  uint32_t hash[kRpItems];
-  if (SEGS) {
+  bool wide = false;
+  constexpr int64_t kSpan = 256 * kRpLookItems;
+  for (int64_t lo = static_cast<int64_t>(blockIdx.x) * kSpan; lo < N; lo += static_cast<int64_t>(gridDim.x) * kSpan) {
+    const int64_t hi = lo + kSpan < N ? lo + kSpan : N;
+    int64_t idx[kRpLookItems], key[kRpLookItems];
+    bool ok[kRpLookItems];
 #pragma unroll
-    for (int j = 0; j < kRpItems; ++j) {
-      idx[j] = lo + j * kRpBlock + threadIdx.x;
+    for (int j = 0; j < kRpLookItems; ++j) {
+      idx[j] = lo + j * 256 + threadIdx.x;
       ok[j] = idx[j] < hi;
       key[j] = 0;
     }
-    rl_load_segments<kRpItems>(segs, lo, hi, idx, ok, key);
+    if (SEGS)
+      rl_load_segments<kRpLookItems>(segs, lo, hi, idx, ok, key);
+    else
+      load_ints<kRpLookItems>(a.total, idx, ok, a.eb, key);
 #pragma unroll
-    for (int j = 0; j < kRpItems; ++j)
-      if (ok[j]) store_int(const_cast<void *>(a.total), idx[j], a.eb, key[j]);
-    // the repeats test below reads ids of this tile back from `total`
-    __syncthreads();
-  } else {
-    rp_load_chunk(a, lo, hi, idx, ok, key);
-  }
-  bool wide = false;
-#pragma unroll
-  for (int j = 0; j < kRpItems; ++j) {
-    hash[j] = hash_id(key[j]);
-    if (ok[j]) {
+    for (int j = 0; j < kRpLookItems; ++j) {
+      if (SEGS && ok[j]) store_int(const_cast<void *>(a.total), idx[j], a.eb, key[j]);
       wide |= (static_cast<uint64_t>(key[j]) >> 32) != 0;
-      atomicMin(&dedup[hash[j] & (kRpDedupSlots - 1)], rp_dedup_word(key[j], idx[j]));
     }
   }
-  if (wide && a.path.mode == 2) *a.wide_mark = a.path.nonce;
-  __syncthreads();
-#pragma unroll
-  for (int j = 0; j < kRpItems; ++j)
-    if (ok[j] && !rp_covered(a, dedup, key[j], idx[j], hash[j])) atomicAdd(&hist[hash[j] >> (32 - a.log2P)], 1u);
-  __syncthreads();
-  for (uint32_t b = threadIdx.x; b < P; b += kRpBlock) a.hist[static_cast<size_t>(b) * a.W + bx] = hist[b];
+  if (wide) *wide_mark = a.path.nonce;
 }
 
-__global__ __launch_bounds__(kRpBlock) void rp_count_kernel(RpArgs a) {
-  rp_count_body<false>(blockIdx.x, a, RlSegments{});
-}
-
-__global__ __launch_bounds__(kRpBlock) void rp_count_segments_kernel(RpArgs a, RlSegments segs) {
-  rp_count_body<true>(blockIdx.x, a, segs);
-}
-
-__global__ __launch_bounds__(kRpBlock) void rp_count_jobs(Jobs<RpArgs> j) {
-  if (blockIdx.x < j.blocks[blockIdx.y]) rp_count_body<false>(blockIdx.x, j.a[blockIdx.y], RlSegments{});
-}
-
-// One wave per bin: the row's counts become the offsets of the tiles' runs inside the bin.
-__device__ __forceinline__ void rp_rows_body(unsigned bx, const RpArgs &a) {
-  const uint32_t b = bx * (256 / kWave) + threadIdx.x / kWave;
-  if (b >= (1u << a.log2P)) return;
-  uint32_t *const row = a.hist + static_cast<size_t>(b) * a.W;
-  const uint32_t lane = lane_id();
-  uint32_t carry = 0;
-  for (uint32_t w0 = 0; w0 < a.W; w0 += kWave) {
-    const uint32_t w = w0 + lane;
-    const uint32_t v = w < a.W ? row[w] : 0u;
-    const uint32_t inc = wave_inclusive_scan(v);
-    if (w < a.W) row[w] = carry + inc - v;
-    carry += wave_last(inc);
-  }
-  if (lane == 0) a.bintot[b] = carry;
-}
-
-__global__ __launch_bounds__(256) void rp_rows_kernel(RpArgs a) { rp_rows_body(blockIdx.x, a); }
-
-__global__ __launch_bounds__(256) void rp_rows_jobs(Jobs<RpArgs> j) {
-  if (blockIdx.x < j.blocks[blockIdx.y]) rp_rows_body(blockIdx.x, j.a[blockIdx.y]);
-}
-
-// The id a packed record stands for, as the count pass hashed it (4-byte ids are signed).
-__device__ __forceinline__ int64_t rp_packed_key(unsigned long long rec, int eb) {
-  const uint32_t k = static_cast<uint32_t>(rec >> 32);
-  return eb == 4 ? static_cast<int64_t>(static_cast<int32_t>(k)) : static_cast<int64_t>(k);
-}
-
-// Scattered 8-byte stores cost one L2 transaction each and leave half-filled lines behind; the records of a
-// tile are therefore put in bin order in LDS first (position = start of the bin among the tile's records +
-// rank within the bin) and written out from there, consecutive lanes to consecutive addresses of a run.
-// 16-byte records (ids beyond 32 bits) do not fit the LDS and are stored directly.
-__device__ __forceinline__ void rp_scatter_body(unsigned bx, const RpArgs &a) {
-  extern __shared__ uint32_t words[];  // run start in memory, record count, start among the tile's records: P (+ 1) each
+// The records of a tile are put in bin order in LDS first (position = start of the bin among the tile's records +
+// rank within the bin) and written out from there. 16-byte records (ids beyond 32 bits) do not fit the LDS and are stored
+// directly.
+// SEGS: the ids are 4 bytes wide and still in the caller's segments; the pass also writes their concatenation (`total`).
+template <bool SEGS>
+__device__ __forceinline__ void rp_scatter_body(unsigned bx, const RpArgs &a, const RlSegments &segs) {
+  extern __shared__ uint32_t words[];  // per bin: record count, start among the tile's records: P (+ 1) each
   __shared__ unsigned long long stage[kRpTile];  // first the de-duplication table and the ranks of its owners
   __shared__ uint32_t scan_lds[kRpBlock / kWave];
   const int64_t N = rl_count(a.n);
   const uint32_t P = 1u << a.log2P;
-  // launched for a bound of N: a tile past the ids has nothing to scatter (tile 0 also publishes the bin starts)
-  if (bx > 0 && static_cast<int64_t>(bx) * kRpTile >= N) return;
-  uint32_t *const run_at = words, *const cnt = words + P, *const lstart = words + 2 * P;
+  const int64_t lo = static_cast<int64_t>(bx) * kRpTile;
+  if (lo >= N) return;  // launched for a bound of N: a tile past the ids has nothing to scatter
+  uint32_t *const cnt = words, *const lstart = words + P;
   unsigned long long *const dedup = stage;
   uint32_t *const rep_rank = reinterpret_cast<uint32_t *>(stage + kRpDedupSlots);
   static_assert(kRpDedupSlots * 12 <= kRpTile * 8, "table and ranks fit the staging memory");
   rp_dedup_clear(dedup);
-  // where every bin starts: thread t sums `per` consecutive bin totals
-  const uint32_t per = P > kRpBlock ? P / kRpBlock : 1u;
-  const uint32_t b0 = threadIdx.x * per;
-  uint32_t sum = 0;
-  for (uint32_t j = 0; j < per; ++j)
-    if (b0 + j < P) sum += a.bintot[b0 + j];
-  uint32_t all;
-  uint32_t run = block_exclusive_scan<uint32_t, kRpBlock>(sum, scan_lds, &all);
-  for (uint32_t j = 0; j < per; ++j) {
-    const uint32_t b = b0 + j;
-    if (b < P) {
-      run_at[b] = run + a.hist[static_cast<size_t>(b) * a.W + bx];
-      cnt[b] = 0;
-      if (bx == 0) a.binstart[b] = run;
-      run += a.bintot[b];
-    }
-  }
-  if (bx == 0 && threadIdx.x == 0) a.binstart[P] = all;
+  static_assert((1 << kRpMaxBinsLog2) <= kRpBlock, "a thread per bin");
+  if (threadIdx.x < P) cnt[threadIdx.x] = 0;
   __syncthreads();
   const bool packed = rl_packed(a.path);
-  const int64_t lo = static_cast<int64_t>(bx) * kRpTile;
-  const int64_t hi = lo + kRpTile < N ? lo + kRpTile : N;
-  int64_t idx[kRpItems], key[kRpItems];
-  bool ok[kRpItems];
+  // element j * kRpBlock + threadIdx.x of the tile; what lives through the whole pass is kept in 32 bits where it can be: two
+  // workgroups share a compute unit if a thread has at most 64 registers (with 86 one had the unit to itself: 27 -> 20 us for eight merged hops)
+  const uint32_t count = static_cast<uint32_t>(N - lo < kRpTile ? N - lo : kRpTile);
+  const uint32_t i0 = static_cast<uint32_t>(lo) + threadIdx.x;
+  auto here = [&](int j) { return j * kRpBlock + threadIdx.x < count; };
+  int64_t key[kRpItems];
   uint32_t hash[kRpItems], rank[kRpItems];
-  rp_load_chunk(a, lo, hi, idx, ok, key);
+  // (between phases: what one of them derived from the hashes is not worth its registers in the next)
+  auto forget = [&]() {
+#pragma unroll
+    for (int j = 0; j < kRpItems; ++j) asm volatile("" : "+v"(hash[j]));
+  };
+  if (SEGS) {
+    int64_t idx[kRpItems];
+    bool ok[kRpItems];
+#pragma unroll
+    for (int j = 0; j < kRpItems; ++j) {
+      idx[j] = lo + j * kRpBlock + threadIdx.x;
+      ok[j] = here(j);
+      key[j] = 0;
+    }
+    rl_load_segments<kRpItems>(segs, lo, lo + count, idx, ok, key);
+    int32_t *const total = static_cast<int32_t *>(const_cast<void *>(a.total)) + lo;
+#pragma unroll
+    for (int j = 0; j < kRpItems; ++j)
+      if (here(j)) total[j * kRpBlock + threadIdx.x] = static_cast<int32_t>(key[j]);
+  } else {
+    rp_load_chunk(static_cast<const char *>(a.total) + lo * a.eb, count, a.eb, key);
+  }
 #pragma unroll
   for (int j = 0; j < kRpItems; ++j) {
     hash[j] = hash_id(key[j]);
-    if (ok[j]) atomicMin(&dedup[hash[j] & (kRpDedupSlots - 1)], rp_dedup_word(key[j], idx[j]));
+    if (here(j)) atomicMin(&dedup[hash[j] & (kRpDedupSlots - 1)], rp_dedup_word(key[j], i0 + j * kRpBlock));
   }
   __syncthreads();
-  bool covered[kRpItems];
+  forget();
+  constexpr uint32_t kCovered = 1u << 31;  // (ranks are below kRpTile)
 #pragma unroll
   for (int j = 0; j < kRpItems; ++j) {
-    covered[j] = ok[j] && rp_covered(a, dedup, key[j], idx[j], hash[j]);
-    rank[j] = 0;
-    if (ok[j] && !covered[j]) {
+    rank[j] = kCovered;
+    if (here(j) && !rp_covered(a, dedup, key[j], i0 + j * kRpBlock, hash[j])) {
       rank[j] = atomicAdd(&cnt[hash[j] >> (32 - a.log2P)], 1u);
       // the element a slot names tells the ones it covers (same id, so same bin) where its record goes
-      if (dedup[hash[j] & (kRpDedupSlots - 1)] == rp_dedup_word(key[j], idx[j])) rep_rank[hash[j] & (kRpDedupSlots - 1)] = rank[j];
+      if (dedup[hash[j] & (kRpDedupSlots - 1)] == rp_dedup_word(key[j], i0 + j * kRpBlock))
+        rep_rank[hash[j] & (kRpDedupSlots - 1)] = rank[j];
     }
   }
   __syncthreads();
+  forget();
 #pragma unroll
   for (int j = 0; j < kRpItems; ++j)
-    if (covered[j]) rank[j] = rep_rank[hash[j] & (kRpDedupSlots - 1)];
+    if (here(j) && rank[j] == kCovered) rank[j] |= rep_rank[hash[j] & (kRpDedupSlots - 1)];
   // start of every bin among the tile's records (the scan's barriers also end the use of the table)
   {
-    uint32_t part = 0;
-    for (uint32_t j = 0; j < per; ++j)
-      if (b0 + j < P) part += cnt[b0 + j];
-    uint32_t records;
-    uint32_t at = block_exclusive_scan<uint32_t, kRpBlock>(part, scan_lds, &records);
-    for (uint32_t j = 0; j < per; ++j) {
-      const uint32_t b = b0 + j;
-      if (b < P) {
-        lstart[b] = at;
-        at += cnt[b];
-      }
+    const uint32_t part = threadIdx.x < P ? cnt[threadIdx.x] : 0;
+    // (the scan of common use keeps the totals of all 16 waves in registers, twice)
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x / kWave));
+    const uint32_t upto = wave_inclusive_scan(part);
+    if (lane_id() == kWave - 1) scan_lds[wave] = upto;
+    __syncthreads();
+    if (threadIdx.x < P) {
+      uint32_t at = upto - part;
+#pragma unroll 1
+      for (int w = 0; w < wave; ++w) at += scan_lds[w];
+      lstart[threadIdx.x] = at;
+      if (threadIdx.x == P - 1) lstart[P] = at + part;
     }
-    if (threadIdx.x == 0) lstart[P] = records;
   }
   __syncthreads();
-  uint32_t *const runs = a.tile_runs + static_cast<size_t>(bx) * (2 * P + 1);
-  for (uint32_t t = threadIdx.x; t < 2 * P + 1; t += kRpBlock) runs[t] = t < P ? run_at[t] : lstart[t - P];
+  forget();
+  uint16_t *const runs = a.runs + static_cast<size_t>(bx) * (P + 1);
+  for (uint32_t t = threadIdx.x; t < P + 1; t += kRpBlock) runs[t] = static_cast<uint16_t>(lstart[t]);  // (at most kRpTile)
 #pragma unroll
   for (int j = 0; j < kRpItems; ++j) {
-    if (!ok[j]) continue;
-    const uint32_t bin = hash[j] >> (32 - a.log2P);
-    const uint32_t at = lstart[bin] + rank[j];
-    a.local[idx[j]] = static_cast<uint16_t>(at);
-    if (covered[j]) continue;
+    if (!here(j)) continue;
+    const uint32_t at = lstart[hash[j] >> (32 - a.log2P)] + (rank[j] & ~kCovered);
+    a.local[lo + j * kRpBlock + threadIdx.x] = static_cast<uint16_t>(at);
+    if (rank[j] & kCovered) continue;
     if (packed)
-      stage[at] = (static_cast<unsigned long long>(static_cast<uint32_t>(key[j])) << 32) | static_cast<uint32_t>(idx[j]);
+      stage[at] = (static_cast<unsigned long long>(static_cast<uint32_t>(key[j])) << 32) | (i0 + j * kRpBlock);
     else
-      static_cast<uint4 *>(a.rec)[run_at[bin] + rank[j]] =
-          make_uint4(static_cast<uint32_t>(static_cast<uint64_t>(key[j])),
-                     static_cast<uint32_t>(static_cast<uint64_t>(key[j]) >> 32), static_cast<uint32_t>(idx[j]), 0u);
+      static_cast<uint4 *>(a.rec)[lo + at] = make_uint4(static_cast<uint32_t>(static_cast<uint64_t>(key[j])),
+                                                        static_cast<uint32_t>(static_cast<uint64_t>(key[j]) >> 32),
+                                                        i0 + j * kRpBlock, 0u);
   }
   if (!packed) return;
   __syncthreads();
   const uint32_t records = lstart[P];
-  for (uint32_t q = threadIdx.x; q < records; q += kRpBlock) {
-    const unsigned long long rec = stage[q];
-    const uint32_t bin = hash_id(rp_packed_key(rec, a.eb)) >> (32 - a.log2P);
-    static_cast<unsigned long long *>(a.rec)[run_at[bin] + (q - lstart[bin])] = rec;
-  }
+  for (uint32_t q = threadIdx.x; q < records; q += kRpBlock) static_cast<unsigned long long *>(a.rec)[lo + q] = stage[q];
 }
 
-__global__ __launch_bounds__(kRpBlock) void rp_scatter_kernel(RpArgs a) { rp_scatter_body(blockIdx.x, a); }
+__global__ __launch_bounds__(kRpBlock) void rp_scatter_kernel(RpArgs a) {
+  rp_scatter_body<false>(blockIdx.x, a, RlSegments{});
+}
+
+__global__ __launch_bounds__(kRpBlock) void rp_scatter_segments_kernel(RpArgs a, RlSegments segs) {
+  rp_scatter_body<true>(blockIdx.x, a, segs);
+}
 
 __global__ __launch_bounds__(kRpBlock) void rp_scatter_jobs(Jobs<RpArgs> j) {
-  if (blockIdx.x < j.blocks[blockIdx.y]) rp_scatter_body(blockIdx.x, j.a[blockIdx.y]);
+  if (blockIdx.x < j.blocks[blockIdx.y]) rp_scatter_body<false>(blockIdx.x, j.a[blockIdx.y], RlSegments{});
 }
 
 // The table of a bin: per slot an id, claimed by a compare-and-swap, and the smallest index seen for it,
@@ -1190,18 +1140,90 @@ __device__ __forceinline__ bool rp_mine(int64_t key, uint32_t round_mask, uint32
   return round_mask == 0 || (rp_class(key) & round_mask) == round;
 }
 
+// The runs of a bin, in LDS: records pre[t] .. pre[t + 1] - 1 of the bin come from tile t, and record e of them is record
+// base[t] + e of all. (base wraps around; tiles without a record have the pre of the next one.)
+struct RpRuns {
+  const uint32_t *pre, *base;
+  uint32_t tiles, top;  // top: the largest power of two up to tiles
+  uint32_t stride, coarse;  // tiles / 64, rounded up; pre[lane * stride]
+
+  __device__ __forceinline__ RpRuns(const uint32_t *pre_, const uint32_t *base_, uint32_t tiles_)
+      : pre(pre_), base(base_), tiles(tiles_), top(1u << (31 - __builtin_clz(tiles_))), stride((tiles_ + kWave - 1) / kWave) {
+    const uint32_t t = lane_id() * stride;
+    coarse = t < tiles ? pre[t] : ~0u;
+  }
+
+  __device__ __forceinline__ uint32_t tile_of(uint32_t e) const {
+    uint32_t t = 0;
+    for (uint32_t step = top; step > 0; step >>= 1)
+      if (t + step < tiles && pre[t + step] <= e) t += step;
+    return t;
+  }
+
+  // The same for 64 consecutive records, one per lane (all lanes active): the run of the first one by two ballots, the
+  // few that begin behind it one by one. (With a search per record the pass took 42 us at 3.1 M ids, 34 so.)
+  __device__ __forceinline__ uint32_t tile_of_wave(uint32_t e) const {
+    const uint32_t e_first = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(e)));
+    const uint32_t t0 = (__builtin_popcountll(__builtin_amdgcn_ballot_w64(coarse <= e_first)) - 1) * stride;
+    const uint32_t t = t0 + lane_id();
+    const uint32_t starts_at = t < tiles ? pre[t] : ~0u;
+    const uint64_t in_reach = __builtin_amdgcn_ballot_w64(starts_at <= e_first + (kWave - 1));
+    if (in_reach >> (kWave - 1)) return tile_of(e);  // (more runs than lanes)
+    const uint64_t before = __builtin_amdgcn_ballot_w64(starts_at <= e_first);
+    uint32_t mine = t0 + __builtin_popcountll(before) - 1;
+    for (uint64_t rest = in_reach & ~before; rest != 0; rest &= rest - 1)
+      mine += e >= static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(starts_at), __builtin_ctzll(rest)));
+    return mine;
+  }
+};
+
+// Fills pre and base (W words each) for bin bx and returns the number of its records. All threads of the workgroup.
+__device__ __forceinline__ uint32_t rp_find_runs(unsigned bx, const RpArgs &a, uint32_t tiles, uint32_t *pre, uint32_t *base,
+                                                 uint32_t *wave_sums) {
+  const uint32_t stride = (1u << a.log2P) + 1u;
+  uint32_t carry = 0;
+  for (uint32_t t0 = 0; t0 < tiles; t0 += blockDim.x) {
+    const uint32_t t = t0 + threadIdx.x;
+    uint32_t from = 0, len = 0;
+    if (t < tiles) {
+      from = a.runs[static_cast<size_t>(t) * stride + bx];
+      len = a.runs[static_cast<size_t>(t) * stride + bx + 1] - from;
+    }
+    const uint32_t upto = wave_inclusive_scan(len);
+    if (lane_id() == kWave - 1) wave_sums[threadIdx.x / kWave] = upto;
+    __syncthreads();
+    uint32_t before = carry;
+#pragma unroll 1
+    for (uint32_t w = 0; w < blockDim.x / kWave; ++w) {
+      const uint32_t sum = wave_sums[w];
+      if (w < threadIdx.x / kWave) before += sum;
+      carry += sum;
+    }
+    if (t < tiles) {
+      pre[t] = before + upto - len;
+      base[t] = static_cast<uint32_t>(t * kRpTile) + from - (before + upto - len);
+    }
+    __syncthreads();
+  }
+  return carry;
+}
+
 // kRpBinItems records of a bin, element e0 + j * (threads of the workgroup) for j = 0 .., all loads in flight together.
+// Whole waves.
 template <bool PACKED>
-__device__ __forceinline__ void rp_load_records(const RpArgs &a, uint32_t start, uint32_t cnt, uint32_t e0,
+__device__ __forceinline__ void rp_load_records(const RpArgs &a, const RpRuns &runs, uint32_t cnt, uint32_t e0,
                                                 uint32_t round_mask, uint32_t round,
                                                 RpRecord<PACKED> (&rec)[kRpBinItems], uint32_t (&hash)[kRpBinItems],
                                                 bool (&on)[kRpBinItems]) {
+  uint32_t tile[kRpBinItems];
+#pragma unroll
+  for (int j = 0; j < kRpBinItems; ++j) tile[j] = runs.tile_of_wave(e0 + j * blockDim.x);
 #pragma unroll
   for (int j = 0; j < kRpBinItems; ++j) {
     rec[j].key = 0;
     rec[j].i = 0;
     on[j] = e0 + j * blockDim.x < cnt;
-    if (on[j]) rec[j].load(a.rec, start + e0 + j * blockDim.x);
+    if (on[j]) rec[j].load(a.rec, runs.base[tile[j]] + e0 + j * blockDim.x);
   }
 #pragma unroll
   for (int j = 0; j < kRpBinItems; ++j) {
@@ -1211,19 +1233,17 @@ __device__ __forceinline__ void rp_load_records(const RpArgs &a, uint32_t start,
 }
 
 template <bool PACKED>
-__device__ __forceinline__ void rp_bin_body(unsigned bx, const RpArgs &a, unsigned long long *mem,
+__device__ __forceinline__ void rp_bin_body(const RpArgs &a, const RpRuns &runs, uint32_t cnt, unsigned long long *mem,
                                             uint32_t *shared_words) {
   using Table = RpTable<PACKED>;
   using Key = typename Table::Key;
-  const uint32_t start = a.binstart[bx];
-  const uint32_t cnt = a.binstart[bx + 1] - start;
-  if (cnt == 0) return;
   uint32_t *const overflow = &shared_words[0];
   const uint32_t slots = PACKED ? (1u << a.slots_log2) : (1u << (a.slots_log2 - 1));
   const Table tbl{mem, &shared_words[1], slots - 1};
-  // Where the records of the first kRpHeldPasses passes over the bin went (a slot, or one of the two marks):
-  // their results are then one LDS read each, without reading, hashing and probing a second time.
-  constexpr uint32_t kNotMine = 0xFFFFFFFFu, kAllOnes = 0xFFFFFFFEu;
+  // Where the records of the first kRpHeldPasses passes over the bin went (a slot, or one of the two marks, under the
+  // record's tile): their results are then one LDS read each, without reading, hashing and probing a second time.
+  constexpr uint32_t kNotMine = 0xFFFFu, kAllOnes = 0xFFFEu;
+  static_assert(kRpSlotsLog2 < 15, "slots and marks share 16 bits");
   uint32_t where[kRpHeldPasses][kRpBinItems];
   for (int lg = 0; lg <= a.max_rounds_log2; ++lg) {
     const uint32_t round_mask = (1u << lg) - 1u;
@@ -1238,7 +1258,7 @@ __device__ __forceinline__ void rp_bin_body(unsigned bx, const RpArgs &a, unsign
         RpRecord<PACKED> rec[kRpBinItems];
         uint32_t hash[kRpBinItems];
         bool on[kRpBinItems];
-        rp_load_records<PACKED>(a, start, cnt, e0, round_mask, r, rec, hash, on);
+        rp_load_records<PACKED>(a, runs, cnt, e0, round_mask, r, rec, hash, on);
         // the home slots of all records are looked at together, then claimed together, then their indices
         // lowered together; only a record that met another id goes on along its probe sequence
         Key k[kRpBinItems];
@@ -1272,7 +1292,7 @@ __device__ __forceinline__ void rp_bin_body(unsigned bx, const RpArgs &a, unsign
         }
         if (slot_out) {
 #pragma unroll
-          for (int j = 0; j < kRpBinItems; ++j) slot_out[j] = slot[j];
+          for (int j = 0; j < kRpBinItems; ++j) slot_out[j] = ((rec[j].i >> kRpTileLog2) << 16) | slot[j];
         }
       };
       const uint32_t pass_records = kRpBinItems * blockDim.x;
@@ -1282,7 +1302,7 @@ __device__ __forceinline__ void rp_bin_body(unsigned bx, const RpArgs &a, unsign
         for (int j = 0; j < kRpBinItems; ++j) where[pass][j] = kNotMine;
         if (pass * pass_records < cnt) insert_pass(threadIdx.x + pass * pass_records, where[pass]);
       }
-      for (uint32_t e0 = threadIdx.x + kRpHeldPasses * pass_records; e0 < cnt; e0 += pass_records) insert_pass(e0, nullptr);
+      for (uint32_t e0 = threadIdx.x + kRpHeldPasses * pass_records; e0 - lane_id() < cnt; e0 += pass_records) insert_pass(e0, nullptr);
       if (!fits) *overflow = 1;
       __syncthreads();
       done = *overflow == 0;
@@ -1291,17 +1311,17 @@ __device__ __forceinline__ void rp_bin_body(unsigned bx, const RpArgs &a, unsign
         for (int pass = 0; pass < kRpHeldPasses; ++pass) {
 #pragma unroll
           for (int j = 0; j < kRpBinItems; ++j) {
-            const uint32_t w = where[pass][j];
+            const uint32_t w = where[pass][j] & 0xFFFFu;
             if (w != kNotMine)
-              a.firstp[start + threadIdx.x + pass * pass_records + j * blockDim.x] =
+              a.firstp[runs.base[where[pass][j] >> 16] + threadIdx.x + pass * pass_records + j * blockDim.x] =
                   w == kAllOnes ? *tbl.all_ones : *tbl.index_at(w);
           }
         }
-        for (uint32_t e0 = threadIdx.x + kRpHeldPasses * pass_records; e0 < cnt; e0 += pass_records) {
+        for (uint32_t e0 = threadIdx.x + kRpHeldPasses * pass_records; e0 - lane_id() < cnt; e0 += pass_records) {
           RpRecord<PACKED> rec[kRpBinItems];
           uint32_t hash[kRpBinItems];
           bool on[kRpBinItems];
-          rp_load_records<PACKED>(a, start, cnt, e0, round_mask, r, rec, hash, on);
+          rp_load_records<PACKED>(a, runs, cnt, e0, round_mask, r, rec, hash, on);
           Key k[kRpBinItems];
           uint32_t f[kRpBinItems];
 #pragma unroll
@@ -1318,7 +1338,7 @@ __device__ __forceinline__ void rp_bin_body(unsigned bx, const RpArgs &a, unsign
               f[j] = *tbl.all_ones;
             else if (k[j] != key)
               f[j] = tbl.first_from(key, hash[j]);
-            a.firstp[start + e0 + j * blockDim.x] = f[j];
+            a.firstp[runs.base[rec[j].i >> kRpTileLog2] + e0 + j * blockDim.x] = f[j];
           }
         }
       }
@@ -1329,14 +1349,15 @@ __device__ __forceinline__ void rp_bin_body(unsigned bx, const RpArgs &a, unsign
   // every pair: the ids of this bin defeat both hashes
   for (uint32_t e = threadIdx.x; e < cnt; e += blockDim.x) {
     RpRecord<PACKED> mine;
-    mine.load(a.rec, start + e);
+    const uint32_t at = runs.base[runs.tile_of(e)] + e;
+    mine.load(a.rec, at);
     uint32_t first = mine.i;
     for (uint32_t o = 0; o < cnt; ++o) {
       RpRecord<PACKED> other;
-      other.load(a.rec, start + o);
+      other.load(a.rec, runs.base[runs.tile_of(o)] + o);
       if (other.key == mine.key && other.i < first) first = other.i;
     }
-    a.firstp[start + e] = first;
+    a.firstp[at] = first;
   }
 }
 
@@ -1347,11 +1368,17 @@ constexpr int rp_bins_threads(int table_log2) { return table_log2 >= 14 ? 1024 :
 template <int TABLE_LOG2>
 __device__ __forceinline__ void rp_bins_body(unsigned bx, const RpArgs &a) {
   __shared__ unsigned long long mem[1 << TABLE_LOG2];
+  __shared__ uint32_t pre[kRpMaxTiles], base[kRpMaxTiles];
+  __shared__ uint32_t wave_sums[rp_bins_threads(TABLE_LOG2) / kWave];
   __shared__ uint32_t shared_words[2];
+  const uint32_t tiles = static_cast<uint32_t>((rl_count(a.n) + kRpTile - 1) / kRpTile);
+  const uint32_t cnt = rp_find_runs(bx, a, tiles, pre, base, wave_sums);
+  if (cnt == 0) return;
+  const RpRuns runs(pre, base, tiles);
   if (rl_packed(a.path))
-    rp_bin_body<true>(bx, a, mem, shared_words);
+    rp_bin_body<true>(a, runs, cnt, mem, shared_words);
   else
-    rp_bin_body<false>(bx, a, mem, shared_words);
+    rp_bin_body<false>(a, runs, cnt, mem, shared_words);
 }
 
 template <int TABLE_LOG2>
@@ -1364,10 +1391,8 @@ __global__ __launch_bounds__(rp_bins_threads(TABLE_LOG2)) void rp_bins_jobs(Jobs
   if (blockIdx.x < j.blocks[blockIdx.y]) rp_bins_body<TABLE_LOG2>(blockIdx.x, j.a[blockIdx.y]);
 }
 
-// The results of the tile's records are read run by run, consecutive lanes from consecutive addresses, into
-// LDS in the tile's bin order; every element then picks the one of its record there.
+// The results of the tile's records are read into LDS; every element then picks the one of its record there.
 __device__ __forceinline__ void rp_gather_body(unsigned bx, const RpArgs &a) {
-  extern __shared__ uint32_t words[];  // run start in memory (P), start among the tile's records (P + 1)
   __shared__ uint32_t result[kRpTile];
   __shared__ uint32_t before[kRpTile / kWave];  // first occurrences per 64 elements, then in front of them
   const int64_t N = rl_count(a.n);
@@ -1375,18 +1400,15 @@ __device__ __forceinline__ void rp_gather_body(unsigned bx, const RpArgs &a) {
   if (lo >= N) return;
   const int64_t hi = lo + kRpTile < N ? lo + kRpTile : N;
   const uint32_t P = 1u << a.log2P;
-  const uint32_t *const runs = a.tile_runs + static_cast<size_t>(bx) * (2 * P + 1);
-  for (uint32_t t = threadIdx.x; t < 2 * P + 1; t += kRpBlock) words[t] = runs[t];
-  __syncthreads();
-  const uint32_t *const run_at = words, *const lstart = words + P;
-  const uint32_t records = lstart[P];
-  for (uint32_t q = threadIdx.x; q < records; q += kRpBlock) {
-    // the bin whose records include the q-th: the last one that starts at or before q
-    uint32_t bin = 0;
-    for (uint32_t step = P >> 1; step > 0; step >>= 1)
-      if (lstart[bin + step] <= q) bin += step;
-    result[q] = a.firstp[run_at[bin] + (q - lstart[bin])];
+  const uint32_t records = a.runs[static_cast<size_t>(bx) * (P + 1) + P];
+  uint32_t held[kRpItems];
+#pragma unroll
+  for (int j = 0; j < kRpItems; ++j) {
+    const uint32_t q = j * kRpBlock + threadIdx.x;
+    held[j] = q < records ? a.firstp[lo + q] : 0;
   }
+#pragma unroll
+  for (int j = 0; j < kRpItems; ++j) result[j * kRpBlock + threadIdx.x] = held[j];
   __syncthreads();
   const int wave = threadIdx.x / kWave;
   uint64_t wins[kRpItems];
@@ -1474,8 +1496,9 @@ static bool rc_plan(int64_t N, int merged_jobs, void *table_memory, RelabelClass
   return true;
 }
 
-// For ids that no earlier kernel has classified; SEGS: as in the count pass. Repeats within a tile are found through a
-// direct-mapped table: a slot holds the smallest place in the tile of the ids that map there.
+// For ids that no earlier kernel has classified; SEGS: the ids are still in the caller's segments, whose concatenation
+// the pass writes. Repeats within a tile are found through a direct-mapped table: a slot holds the smallest place in the
+// tile of the ids that map there.
 template <bool SEGS>
 __global__ __launch_bounds__(kRlBlock) void rc_classify_kernel(RcArgs a, RlSegments segs) {
   constexpr int kTile = kRcClassifyItems * kRlBlock;
@@ -2019,35 +2042,36 @@ static int relabel_impl(const void *total, const RlSegments *segs, int64_t N, Rl
     return SHMT_OK;
   }
   if (rp.ok) {
-    // 8-byte ids: the count pass looks at every id itself, so it can vouch for them like the kernels of a
-    // fused hop do (and an earlier kernel that stored the mark already is just as good)
+    // 8-byte ids: a pass of its own looks at every id, so it can vouch for them like the kernels of a fused hop do
     if (path.mode == 0) path.mode = 2;
     const int slots_log2 = g_rp_tuning.slots_log2 < rp.table_log2 ? g_rp_tuning.slots_log2 : rp.table_log2;
-    RpArgs a{total, elem_bytes, n, path, wide_mark, rp.log2P, rp.W, base + rp.rec_off,
-             reinterpret_cast<uint32_t *>(base + rp.first_off), reinterpret_cast<uint32_t *>(base + rp.firstp_off),
-             reinterpret_cast<uint32_t *>(base + rp.hist_off), reinterpret_cast<uint32_t *>(base + rp.bintot_off),
-             reinterpret_cast<uint32_t *>(base + rp.binstart_off), reinterpret_cast<uint32_t *>(base + rp.coarse_off),
-             reinterpret_cast<uint16_t *>(base + rp.local_off), reinterpret_cast<uint32_t *>(base + rp.tile_off),
-             ranks, slots_log2, g_rp_tuning.max_rounds_log2};
+    RpArgs a{total, elem_bytes, n, path, rp.log2P, base + rp.rec_off, reinterpret_cast<uint32_t *>(base + rp.first_off),
+             reinterpret_cast<uint32_t *>(base + rp.firstp_off), reinterpret_cast<uint16_t *>(base + rp.local_off),
+             reinterpret_cast<uint16_t *>(base + rp.runs_off), reinterpret_cast<uint32_t *>(base + rp.coarse_off), ranks,
+             slots_log2, g_rp_tuning.max_rounds_log2};
     const RlFinishArgs fin{total, elem_bytes, n, a.first, 4, ranks, a.coarse, 4, kRpTileLog2, 0, unique_out, labels_out,
                            count_out, count_copy};
     if (defer) {
-      stage_push(defer, kStageRpCount, rp.W, kRpBlock, a);
-      stage_push(defer, kStageRpRows, (rp.P + 3) / 4, 256, a);
       stage_push(defer, kStageRpScatter, rp.W, kRpBlock, a);
       stage_push(defer, kStageRpBins + (kRpSlotsLog2 - rp.table_log2), rp.P, rp_bins_threads(rp.table_log2), a);
       stage_push(defer, kStageRpGather, rp.W, kRpBlock, a);
       stage_push(defer, kStageRlFinish, fin_blocks, kRlBlock, fin);
       return SHMT_OK;
     }
-    if (segs && !prepared)  // the count pass concatenates on the way: there is no table to empty
-      hipLaunchKernelGGL(rp_count_segments_kernel, dim3(rp.W), dim3(kRpBlock), rp.P * sizeof(uint32_t), s, a, *segs);
+    const size_t scatter_lds = (2 * rp.P + 1) * sizeof(uint32_t);
+    const bool concat = segs && !prepared;
+    if (!prepared && elem_bytes == 8) {  // (the earlier kernels of a prepared input have marked wide ids)
+      const dim3 grid(grid_for(N, 256 * kRpLookItems));
+      if (concat)
+        hipLaunchKernelGGL(rp_look_kernel<true>, grid, dim3(256), 0, s, a, *segs, wide_mark);
+      else
+        hipLaunchKernelGGL(rp_look_kernel<false>, grid, dim3(256), 0, s, a, RlSegments{}, wide_mark);
+      SHMT_LAUNCH_CHECK();
+    }
+    if (concat && elem_bytes == 4)
+      hipLaunchKernelGGL(rp_scatter_segments_kernel, dim3(rp.W), dim3(kRpBlock), scatter_lds, s, a, *segs);
     else
-      hipLaunchKernelGGL(rp_count_kernel, dim3(rp.W), dim3(kRpBlock), rp.P * sizeof(uint32_t), s, a);
-    SHMT_LAUNCH_CHECK();
-    hipLaunchKernelGGL(rp_rows_kernel, dim3((rp.P + 3) / 4), dim3(256), 0, s, a);
-    SHMT_LAUNCH_CHECK();
-    hipLaunchKernelGGL(rp_scatter_kernel, dim3(rp.W), dim3(kRpBlock), (3 * rp.P + 1) * sizeof(uint32_t), s, a);
+      hipLaunchKernelGGL(rp_scatter_kernel, dim3(rp.W), dim3(kRpBlock), scatter_lds, s, a);
     SHMT_LAUNCH_CHECK();
     if (rp.table_log2 >= 14)
       hipLaunchKernelGGL(rp_bins_kernel<14>, dim3(rp.P), dim3(rp_bins_threads(14)), 0, s, a);
@@ -2056,7 +2080,7 @@ static int relabel_impl(const void *total, const RlSegments *segs, int64_t N, Rl
     else
       hipLaunchKernelGGL(rp_bins_kernel<12>, dim3(rp.P), dim3(rp_bins_threads(12)), 0, s, a);
     SHMT_LAUNCH_CHECK();
-    hipLaunchKernelGGL(rp_gather_kernel, dim3(rp.W), dim3(kRpBlock), (2 * rp.P + 1) * sizeof(uint32_t), s, a);
+    hipLaunchKernelGGL(rp_gather_kernel, dim3(rp.W), dim3(kRpBlock), 0, s, a);
     SHMT_LAUNCH_CHECK();
     hipLaunchKernelGGL(rl_finish_kernel, dim3(fin_blocks), dim3(kRlBlock), 0, s, fin);
     SHMT_LAUNCH_CHECK();
@@ -2205,8 +2229,6 @@ int launch_merged_relabel_stage(int n_jobs, const Stage *const *stages, hipStrea
       hipLaunchKernelGGL(rl_finish_jobs, dim3(blocks, n_jobs), dim3(threads), 0, s, j);
       break;
     }
-    case kStageRpCount:
-    case kStageRpRows:
     case kStageRpScatter:
     case kStageRpGather:
     case kStageRpBins:
@@ -2219,10 +2241,8 @@ int launch_merged_relabel_stage(int n_jobs, const Stage *const *stages, hipStrea
       const size_t P = static_cast<size_t>(1) << log2P;
       const dim3 grid(blocks, n_jobs), wg(threads);
       switch (stages[0]->kind) {
-        case kStageRpCount: hipLaunchKernelGGL(rp_count_jobs, grid, wg, P * sizeof(uint32_t), s, j); break;
-        case kStageRpRows: hipLaunchKernelGGL(rp_rows_jobs, grid, wg, 0, s, j); break;
-        case kStageRpScatter: hipLaunchKernelGGL(rp_scatter_jobs, grid, wg, (3 * P + 1) * sizeof(uint32_t), s, j); break;
-        case kStageRpGather: hipLaunchKernelGGL(rp_gather_jobs, grid, wg, (2 * P + 1) * sizeof(uint32_t), s, j); break;
+        case kStageRpScatter: hipLaunchKernelGGL(rp_scatter_jobs, grid, wg, (2 * P + 1) * sizeof(uint32_t), s, j); break;
+        case kStageRpGather: hipLaunchKernelGGL(rp_gather_jobs, grid, wg, 0, s, j); break;
         case kStageRpBins: hipLaunchKernelGGL(rp_bins_jobs<14>, grid, wg, 0, s, j); break;
         case kStageRpBins + 1: hipLaunchKernelGGL(rp_bins_jobs<13>, grid, wg, 0, s, j); break;
         default: hipLaunchKernelGGL(rp_bins_jobs<12>, grid, wg, 0, s, j); break;
