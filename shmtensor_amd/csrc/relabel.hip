@@ -19,7 +19,7 @@
 // the id, src/tensor_relabel.cu:111-117); ids known to fit 32 bits use the
 // same memory as packed 8-byte slots (see rl_packed_insert).
 // Up to 8,192 ids all of this is one launch of one workgroup with its table
-// in LDS (rl_small_kernel). From there to 1 M ids (2 M where that is a bound) fill, insert and first
+// in LDS (rl_small_kernel). From there to half a million ids (a bound of 2 M; 192 K for merged hops) fill, insert and first
 // are replaced by passes in which a workgroup finds the ids of its class by scanning one byte per id
 // (rc_*_kernel), and up to 7.3 M by passes that partition the ids by hash
 // (rp_*_kernel); both give every class or partition a table in LDS.
@@ -682,7 +682,7 @@ __global__ void rl_zero_count_kernel(int64_t *count_out, int64_t *count_copy) {
 // The insert and first-occurrence passes above touch a random line of a table
 // that no cache holds once per id and pass, and the part moves such lines at
 // 50 G per second whatever the kernel does (3.1 M ids: 74 + 54 us, plus 22 us to
-// empty the table). From a million ids on (kRpExactMin; kRpDefaultMin for a
+// empty the table). From half a million ids on (kRpExactMin; kRpDefaultMin for a
 // hop sized by a loose bound, kRpMergedMin for hops that share their launches)
 // the same results -- the first-occurrence index of every element, the ranks of
 // the first occurrences and their number per tile of kRpTile ids -- come from three passes
@@ -722,10 +722,14 @@ static_assert((kRpBinIds << kRpMaxBinsLog2) % kRpTile == 0, "no tile beyond the 
 constexpr int64_t kRpDefaultMin = kRlSelfPrefixTiles * kRlTile + 1;
 // Hops that share their launches with those of other batches (launchers.h) are sized for a bound of their
 // ids, and the passes' fixed costs are paid once for all of them: from this bound and this many jobs on
-// they take the partition passes as well.
-constexpr int64_t kRpMergedMin = 512 * 1024;
-// A call that knows its number of ids (not merely a loose bound of it) gains from about a million on.
-constexpr int64_t kRpExactMin = 1024 * 1024;
+// they take the partition passes as well. (Epoch of 8 batches of 1,024 seeds at fanouts 20, 15, 10 merged, from a bound of
+// 512 K / 400,000 / 200,000 / 50,000 on: 1,245 / 1,130 / 1,108 / 1,077 us; of 600 seeds, four merged: 1,154 / 1,072 / 1,060 /
+// 1,072; of 1,024 at 15, 10, 5: 418 / 418 / 417 / 425.)
+constexpr int64_t kRpMergedMin = 192 * 1024;
+// A call that knows its number of ids (not merely a loose bound of it): classes against partitions 42 / 43 us for 400,000
+// ids of 4 bytes, 52 / 44 for 600,000, 66 / 54 for a million; a hundred distinct ids, which the classes share out badly,
+// 61 / 45 and 55 / 44 and 120 / 52.
+constexpr int64_t kRpExactMin = 512 * 1024;
 constexpr int kRpMergedMinJobs = 4;
 constexpr int kRpMinSlotsLog2 = 12;  // smallest table a bin pass is compiled for
 
