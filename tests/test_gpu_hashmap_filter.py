@@ -92,3 +92,21 @@ def test_table_memory_decides_on_the_filter(cabi):
         assert torch.equal(out, want) and lib.shmt_hashmap_used_bytes(handle) == buckets
         assert bool((memory[used:] == 0x5A).all())
         lib.shmt_hashmap_destroy(handle)
+
+
+def test_map_whose_buckets_alone_fit(capi):
+    """Where there is memory for the buckets (64 MiB) but none for the filter behind them, the map is built without one."""
+    g = torch.Generator(device="cuda").manual_seed(8)
+    n = 1 << 22
+    pool = _keys(n + 100_000, 40, g)
+    keys, vals = pool[:n].contiguous(), torch.arange(n, device="cuda")
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(0).total_memory
+    try:
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (65 << 20)) / total)
+        h = capi.CUCOStaticHashmap(keys, vals, 0.5)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert h.memory_usage() == 64 << 20
+    _check(h, keys, pool[n:], 2_000_000, 0.5, g)
