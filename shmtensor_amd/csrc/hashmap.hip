@@ -605,7 +605,9 @@ __global__ __launch_bounds__(256, 8) void hashmap_query_kernel(
     const int64_t mykey = i < n ? map_key(m, next) : -1;  // tail lanes look up the sentinel, which resolves to -1
     const int64_t ahead = i + nwaves * kWave;
     if (ahead < n) next = load_int(req, ahead, req_bytes);
-    uint64_t wanted = ~0ull;
+    // (requests outside the key range read no line either way, and do not speak for the filter)
+    const uint64_t inside = FILTER ? __builtin_amdgcn_ballot_w64(mykey != -1) : ~0ull;
+    uint64_t wanted = inside;
     if (FILTER && ask) {
       const uint32_t h = hash_id(mykey), bits = filter_bits(h);
       wanted = __builtin_amdgcn_ballot_w64(mykey != -1 &&
@@ -613,7 +615,7 @@ __global__ __launch_bounds__(256, 8) void hashmap_query_kernel(
     }
     const int64_t myres = wave_find<FMT, FILTER>(m, mykey, wanted);
     if (FILTER) {
-      const uint64_t away = ask ? ~wanted : __builtin_amdgcn_ballot_w64(myres == -1);
+      const uint64_t away = inside & (ask ? ~wanted : __builtin_amdgcn_ballot_w64(myres == -1));
       ask = __builtin_popcountll(away) >= (ask ? kFilterOff : kFilterOn);
     }
     if (i < n) store_int(out, i, out_bytes, myres);
