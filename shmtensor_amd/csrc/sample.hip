@@ -867,11 +867,13 @@ __global__ __launch_bounds__(256) void subcsr_copy_aligned_kernel(const void *in
     return wave_uniform(row_begins ? row_begins[r] : load_int(indptr, load_int(seeds, r, seed_bytes), ptr_bytes));
   };
   // Where the border meant for output element e is, e lying in the row of outputs [o, o1) read from `begin` on: the
-  // next line of the source, at most the row's end; nowhere else if the row starts there.
+  // next line of the source, at most the row's end (and nnz, which may be less than the rows hold); nowhere else if
+  // the row starts there.
   auto border = [&](int64_t e, int64_t o, int64_t o1, int64_t begin) {
     const int64_t lead = (begin + (e - o) + skew) % kLine;
     if (lead == 0 || e == o) return e;
-    return e + (kLine - lead) < o1 ? e + (kLine - lead) : o1;
+    const int64_t most = o1 < nnz ? o1 : nnz;
+    return e + (kLine - lead) < most ? e + (kLine - lead) : most;
   };
   for (int64_t c = wave; c * chunk < nnz; c += nwaves) {
     int64_t e = c * chunk;

@@ -389,3 +389,20 @@ def test_sub_graph_of_long_rows(capi, oracle, dtype, skew, longest):
         gp, gi = capi.create_subcsr(hp, ids, torch.from_numpy(order.astype(np.int64)).cuda())
         ep, ei = oracle.create_subcsr(indptr, ids.numpy(), order.astype(np.int64))
         assert np.array_equal(gp.cpu().numpy(), ep) and np.array_equal(gi.cpu().numpy(), ei)
+
+
+@pytest.mark.parametrize("dtype", [torch.int32, torch.int64])
+def test_sub_graph_copy_stops_at_the_count_it_is_given(cabi, dtype):
+    """A count below what the rows hold: that many elements are written and none behind them, also where the chunk in front of
+    the last one ends within a few elements of the count (chunks start at multiples of 512 elements here)."""
+    lib, size = cabi.load(), torch.empty(0, dtype=dtype).element_size()
+    deg = torch.tensor([301, 0, 700, 333, 1500, 10])
+    indptr = torch.cat([torch.zeros(1, dtype=torch.int64), deg.cumsum(0)])
+    indices = torch.randint(0, 1 << 30, (int(indptr[-1]) + 3,), dtype=dtype).cuda()[3:]     # (borders move off the multiples)
+    rows, offsets, starts = torch.arange(6).cuda(), indptr.cuda(), indptr[:-1].contiguous().cuda()
+    for nnz in (400, 1001, 1025, 1026, 1540, 1567, 2049, 2078, 2560, 2561, int(indptr[-1])):
+        for begins in (None, starts.data_ptr()):
+            out = torch.full((int(indptr[-1]) + 64,), -1, dtype=dtype, device="cuda")
+            cabi.check(lib.shmt_subcsr_copy_rows(offsets.data_ptr(), indices.data_ptr(), 8, size, rows.data_ptr(), 8, 6,
+                                                 offsets.data_ptr(), begins, nnz, out.data_ptr(), cabi.current_stream()))
+            assert torch.equal(out[:nnz], indices[:nnz]) and bool((out[nnz:] == -1).all())
