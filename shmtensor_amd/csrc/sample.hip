@@ -841,16 +841,25 @@ __global__ __launch_bounds__(256) void subcsr_copy_kernel(const void *indptr, co
   }
 }
 
-// The same copy for rows of several lines: a wave per chunk of the output, which walks through the rows of its chunk and
-// reads their lines aligned, each once and whole. Lanes that follow the output element by element start
+// The same copy where rows have several lines on average: a wave per chunk of the output, which reads the lines of its rows
+// aligned, each once and whole. Lanes that follow the output element by element start
 // anywhere in a line of the source, and as nothing caches host memory, a line that two waves share crosses the link
 // twice. A chunk therefore also ends where a line of the source does: both neighbours move the border between them to the same element.
-// 102 M edges of 4 bytes in 120,000 rows 7.74 -> 7.38 ms (52.7 -> 55.3 GB/s), 30.5 M 2.48 -> 2.37, 10.1 M (338 bytes a row)
-// 0.97 -> 0.93; 2 M (66 bytes a row) 0.27 -> 0.33, where a wave's row is one line and half of its lanes idle (kAlignedRowBytes).
+// Rows may be of any lengths all the same (hubs beside rows of a few ids, runs of empty rows), so a chunk decides for itself: up to
+// kWave - 1 rows of kAlignedRowBytes on average are walked through one after the other, their offsets and begins held one row
+// per lane; in a chunk with more or shorter rows the elements find their rows each for itself, as above, but in LDS: what bounds
+// that form is the chain of loads, each of which waits behind those of the host link (the search in memory, with
+// eight loads side by side, 0.86 and 1.79 ms where this takes 0.79 and 1.57; it is left for steps of more than kAlignedRows rows).
+// Element-parallel kernel -> this one, ms: 60,000 rows of up to 1,000 ids of 4 bytes 2.25 -> 2.20; 120,000 rows of up to 170
+// 0.78 -> 0.79, of up to 130 0.61 both; 500 hubs and 250,000 rows of up to 8 ids 1.59 -> 1.57; 150,000 empty rows between
+// 50 M ids 3.70 -> 3.59; R-MAT of scale 20, the 30 % of rows with the highest degree, 4.38 -> 4.21. 8-byte ids the same within
+// 1 %. Below kAlignedRowBytes a row on average all chunks would be of the second form: the kernel above (2 M ids, 66 bytes
+// a row, 0.27 against 0.33 where a wave walked through them).
 constexpr int kAlignedHeld = 8;                             // loads a lane has in flight
 constexpr int64_t kAlignedChunk = 4096, kAlignedChunkMin = 512;
 constexpr int64_t kAlignedWaves = 4096;                     // 1,024 workgroups; smaller chunks before fewer waves
 constexpr int64_t kAlignedRowBytes = 256;
+constexpr int kAlignedRows = 256;                           // rows of a step that are searched in LDS
 
 template <typename T>
 __global__ __launch_bounds__(256) void subcsr_copy_aligned_kernel(const void *indptr, const T *indices, int ptr_bytes,
@@ -858,13 +867,15 @@ __global__ __launch_bounds__(256) void subcsr_copy_aligned_kernel(const void *in
                                                                   const void *cache_indptr, int64_t nnz, T *out,
                                                                   const int64_t *row_begins, int64_t chunk) {
   constexpr int64_t kLine = kLinkLine / static_cast<int64_t>(sizeof(T));  // elements
+  __shared__ int64_t starts_all[256 / kWave][kAlignedRows], shifts_all[256 / kWave][kAlignedRows];  // (private to a wave)
+  int64_t *const starts = starts_all[threadIdx.x / kWave], *const shifts = shifts_all[threadIdx.x / kWave];
   const int lane = lane_id();
   const int64_t wave = wave_uniform(static_cast<int64_t>(blockIdx.x) * (256 / kWave) + threadIdx.x / kWave);
   const int64_t nwaves = static_cast<int64_t>(gridDim.x) * (256 / kWave);
   const int64_t skew = static_cast<int64_t>((reinterpret_cast<uintptr_t>(indices) % kLinkLine) / sizeof(T));
-  auto offset = [&](int64_t r) { return wave_uniform(load_int(cache_indptr, r, ptr_bytes)); };
+  auto offset = [&](int64_t r) { return load_int(cache_indptr, r, ptr_bytes); };
   auto source = [&](int64_t r) {
-    return wave_uniform(row_begins ? row_begins[r] : load_int(indptr, load_int(seeds, r, seed_bytes), ptr_bytes));
+    return row_begins ? row_begins[r] : load_int(indptr, load_int(seeds, r, seed_bytes), ptr_bytes);
   };
   // Where the border meant for output element e is, e lying in the row of outputs [o, o1) read from `begin` on: the
   // next line of the source, at most the row's end (and nnz, which may be less than the rows hold); nowhere else if
@@ -875,43 +886,120 @@ __global__ __launch_bounds__(256) void subcsr_copy_aligned_kernel(const void *in
     const int64_t most = o1 < nnz ? o1 : nnz;
     return e + (kLine - lead) < most ? e + (kLine - lead) : most;
   };
-  for (int64_t c = wave; c * chunk < nnz; c += nwaves) {
-    int64_t e = c * chunk;
-    const int64_t e1 = e + chunk < nnz ? e + chunk : nnz;
-    int64_t r = 0, last = C - 1;  // the last row with offset(r) <= e, 64 candidates a step
-    while (r < last) {
-      const int64_t step = (last - r + kWave - 1) / kWave;
+  // The last row from r on that starts at element e or before (row r does): among the next 64, or 64 candidates a step.
+  auto row_at = [&](int64_t r, int64_t e) {
+    int64_t last = C - 1, step = 1;
+    for (;;) {
       const int64_t at = r + (lane + 1) * step;
-      const uint64_t below = __builtin_amdgcn_ballot_w64(at <= last && load_int(cache_indptr, at, ptr_bytes) <= e);
-      r += __builtin_popcountll(below) * step;
-      if (r + step - 1 < last) last = r + step - 1;
+      const int before = __builtin_popcountll(__builtin_amdgcn_ballot_w64(at <= last && offset(at) <= e));
+      r += before * step;
+      if (step == 1 && before < kWave) return r;
+      if (step > 1 && r + step - 1 < last) last = r + step - 1;
+      if (r >= last) return r;
+      step = (last - r + kWave - 1) / kWave;
     }
-    int64_t o = offset(r), o1 = offset(r + 1), begin = source(r);
-    if (c > 0) e = border(e, o, o1, begin);
-    while (e < e1) {
-      while (e >= o1 && r + 1 < C) {
-        ++r;
-        o = o1;
-        o1 = offset(r + 1);
-        if (e < o1) begin = source(r);
-      }
-      if (e >= o1) break;  // (nnz is more than the rows hold)
-      int64_t end = o1;
-      if (o1 > e1) end = e1 < nnz ? border(e1, o, o1, begin) : nnz;
-      const int64_t lead = (begin + (e - o) + skew) % kLine;
-      const T *const src = indices + begin + (e - o) - lead;
-      T *const dst = out + e - lead;
-      const int64_t n = end - e + lead;
-      for (int64_t t = lane; t < n; t += kAlignedHeld * kWave) {
-        T held[kAlignedHeld];
+  };
+  auto settle = [] {  // between the wave's writes to its LDS and its reads
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
+  for (int64_t c = wave; c * chunk < nnz; c += nwaves) {
+    int64_t e = c * chunk, end = e + chunk < nnz ? e + chunk : nnz;
+    const int64_t first = row_at(0, e), last = row_at(first, end - 1);
+    const int64_t rows = last - first + 1;
+    // lane l: the offset and the begin of row first + l (the lane behind the last row: the end of it); where there are more rows,
+    // lanes 0 to 3 have those of the first and the last one and of the rows behind them
+    const bool few = rows < kWave && rows * kAlignedRowBytes <= (end - e) * static_cast<int64_t>(sizeof(T));
+    int64_t row = first + lane;
+    if (!few && lane >= 2) row = last + (lane - 2);
+    const int held_rows = few ? static_cast<int>(rows) : 3;
+    const int64_t my_offset = lane <= held_rows ? offset(row) : 0;
+    const int64_t my_begin = lane <= held_rows && row <= last ? source(row) : 0;
+    const int at_last = few ? held_rows - 1 : 2;
+    const int64_t last_end = lane64(my_offset, at_last + 1);
+    if (c > 0) e = border(e, lane64(my_offset, 0), lane64(my_offset, 1), lane64(my_begin, 0));
+    if (last_end < end)
+      end = last_end;  // (nnz is more than the rows hold)
+    else if (end < nnz && last_end > end)
+      end = border(end, lane64(my_offset, at_last), last_end, lane64(my_begin, at_last));
+    if (few) {
+      for (int i = 0; i < held_rows; ++i) {
+        const int64_t o = lane64(my_offset, i), o1 = lane64(my_offset, i + 1);
+        const int64_t from = e > o ? e : o, to = end < o1 ? end : o1;
+        if (from >= to) continue;
+        const int64_t at = lane64(my_begin, i) + (from - o);
+        const int64_t lead = (at + skew) % kLine;
+        const T *const src = indices + at - lead;
+        T *const dst = out + from - lead;
+        const int64_t n = to - from + lead;
+        for (int64_t t = lane; t < n; t += kAlignedHeld * kWave) {
+          T held[kAlignedHeld];
 #pragma unroll
-        for (int h = 0; h < kAlignedHeld; ++h)
-          if (t + h * kWave >= lead && t + h * kWave < n) held[h] = src[t + h * kWave];
+          for (int h = 0; h < kAlignedHeld; ++h)
+            if (t + h * kWave >= lead && t + h * kWave < n) held[h] = src[t + h * kWave];
 #pragma unroll
-        for (int h = 0; h < kAlignedHeld; ++h)
-          if (t + h * kWave >= lead && t + h * kWave < n) dst[t + h * kWave] = held[h];
+          for (int h = 0; h < kAlignedHeld; ++h)
+            if (t + h * kWave >= lead && t + h * kWave < n) dst[t + h * kWave] = held[h];
+        }
       }
-      e = end;
+      continue;
+    }
+    // element by element
+    int64_t base = first;  // the row of element e
+    for (; e < end; e += kAlignedHeld * kWave) {
+      const int64_t e_last = (e + kAlignedHeld * kWave < end ? e + kAlignedHeld * kWave : end) - 1;
+      const int64_t top = row_at(base, e_last);
+      int64_t at[kAlignedHeld];
+      if (top - base < kAlignedRows) {
+        // the step's rows go through LDS: a search in memory is a chain of loads that queue behind those of the host link
+        const int n = static_cast<int>(top - base) + 1;
+        int64_t o[kAlignedRows / kWave], begin[kAlignedRows / kWave];
+#pragma unroll
+        for (int q = 0; q < kAlignedRows / kWave; ++q) {
+          const int64_t row = base + q * kWave + lane <= top ? base + q * kWave + lane : top;
+          o[q] = offset(row);
+          begin[q] = source(row);
+        }
+#pragma unroll
+        for (int q = 0; q < kAlignedRows / kWave; ++q) {
+          starts[q * kWave + lane] = q * kWave + lane < n ? o[q] : INT64_MAX;
+          shifts[q * kWave + lane] = begin[q] - o[q];
+        }
+        settle();
+#pragma unroll
+        for (int h = 0; h < kAlignedHeld; ++h) {
+          int r = 0;
+#pragma unroll
+          for (int step = kAlignedRows / 2; step > 0; step /= 2)
+            if (starts[r + step] <= e + h * kWave + lane) r += step;
+          at[h] = shifts[r] + e + h * kWave + lane;
+        }
+        settle();
+      } else {
+        int64_t r[kAlignedHeld];
+#pragma unroll
+        for (int h = 0; h < kAlignedHeld; ++h) r[h] = base;
+        int64_t step = 1;
+        while (step <= top - base) step *= 2;
+        for (step /= 2; step > 0; step /= 2) {
+#pragma unroll
+          for (int h = 0; h < kAlignedHeld; ++h) {
+            const int64_t next = r[h] + step <= top ? r[h] + step : top;
+            if (offset(next) <= e + h * kWave + lane) r[h] = next;
+          }
+        }
+#pragma unroll
+        for (int h = 0; h < kAlignedHeld; ++h) at[h] = source(r[h]) + (e + h * kWave + lane - offset(r[h]));
+      }
+      T held[kAlignedHeld];
+#pragma unroll
+      for (int h = 0; h < kAlignedHeld; ++h)
+        if (e + h * kWave + lane <= e_last) held[h] = indices[at[h]];
+#pragma unroll
+      for (int h = 0; h < kAlignedHeld; ++h)
+        if (e + h * kWave + lane <= e_last) out[e + h * kWave + lane] = held[h];
+      base = top;
     }
   }
 }

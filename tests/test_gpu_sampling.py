@@ -406,3 +406,60 @@ def test_sub_graph_copy_stops_at_the_count_it_is_given(cabi, dtype):
             cabi.check(lib.shmt_subcsr_copy_rows(offsets.data_ptr(), indices.data_ptr(), 8, size, rows.data_ptr(), 8, 6,
                                                  offsets.data_ptr(), begins, nnz, out.data_ptr(), cabi.current_stream()))
             assert torch.equal(out[:nnz], indices[:nnz]) and bool((out[nnz:] == -1).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.int32, torch.int64])
+@pytest.mark.parametrize("shape", ["empty runs", "hubs, then short rows", "hubs among short rows", "just few rows a chunk"])
+def test_sub_graph_of_rows_of_any_lengths(capi, cabi, oracle, dtype, shape):
+    """Long rows on average, but hubs beside rows of a few ids and runs of up to 9,000 empty rows (more rows than one look at 64
+    of them, or at 64 * 64, covers): chunks that walk through their rows and chunks whose elements look for theirs, side by side."""
+    g = np.random.default_rng(len(shape))
+    hubs = lambda n: g.integers(3000, 9000, n)
+    if shape == "empty runs":
+        parts = [g.integers(0, 900, 40), np.zeros(9000), [1], np.zeros(62), [5], np.zeros(63), [700], np.zeros(64), hubs(180), np.zeros(4095),
+                 [33], np.zeros(4097), hubs(20), np.zeros(300)]
+    elif shape == "hubs, then short rows":
+        parts = [hubs(200), g.integers(0, 8, 9000), hubs(1), g.integers(0, 3, 1000)]
+    elif shape == "hubs among short rows":
+        parts = [np.concatenate([hubs(1), g.integers(0, 9, int(g.integers(1, 90)))]) for _ in range(150)]
+    else:   # (62 to 65 rows in a chunk of 512 to 4,096 elements, and the fewest bytes a row that are walked through)
+        parts = [np.concatenate([np.full(int(g.integers(7, 66)), 64), hubs(1)]) for _ in range(60)]
+    deg = np.concatenate(parts).astype(np.int64)
+    indptr = np.concatenate([[0], np.cumsum(deg)]).astype(np.int64)
+    assert indptr[-1] * 4 >= deg.size * 256
+    ids = torch.randint(0, 1 << 30, (int(indptr[-1]) + 5,), dtype=dtype).pin_memory()[5:]
+    hp = torch.from_numpy(indptr).pin_memory()
+    for order in (np.arange(deg.size), g.permutation(deg.size)):
+        at = torch.from_numpy(order).cuda()
+        gp, gi = capi.create_subcsr(hp, ids, at)
+        ep, ei = oracle.create_subcsr(indptr, ids.numpy(), order)
+        assert np.array_equal(gp.cpu().numpy(), ep) and np.array_equal(gi.cpu().numpy(), ei)
+        # (where nothing tells the rows' begins, they come from the row offsets)
+        out, source, begins = torch.zeros_like(gi), ids.cuda(), hp.cuda()
+        cabi.check(cabi.load().shmt_subcsr_copy(begins.data_ptr(), source.data_ptr(), 8, gi.element_size(), at.data_ptr(), 8, deg.size,
+                                                gp.data_ptr(), gi.numel(), out.data_ptr(), cabi.current_stream()))
+        assert torch.equal(out, gi)
+
+
+def test_sub_graph_with_a_long_run_of_empty_rows_costs_what_its_ids_cost(capi):
+    """200,000 empty rows in the middle of 13 M ids, and the same ids without them: a wave that stepped through them one by one
+    took 20 times as long for the whole copy."""
+    indices = torch.arange(13_000_000, dtype=torch.int32).pin_memory()
+
+    def best_ms(empty):
+        deg = torch.full((26_000,), 500)
+        deg = torch.cat([deg[:13_000], torch.zeros(empty, dtype=torch.int64), deg[13_000:]])
+        indptr = torch.cat([torch.zeros(1, dtype=torch.int64), deg.cumsum(0)])
+        hp, rows = indptr.pin_memory(), torch.arange(deg.numel()).cuda()
+        times = []
+        for _ in range(5):
+            start, stop = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            gp, gi = capi.create_subcsr(hp, indices, rows)
+            stop.record()
+            stop.synchronize()
+            times.append(start.elapsed_time(stop))
+            assert torch.equal(gp.cpu(), indptr) and torch.equal(gi.cpu(), indices)
+        return min(times)
+
+    assert best_ms(200_000) < 4 * best_ms(0)
