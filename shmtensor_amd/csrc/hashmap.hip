@@ -189,9 +189,10 @@ constexpr int kPartRestBlocks = 1024;     // (none to do: 4 us, as with 64)
 // keeps beside the lines that stream through it (stand-alone probe, half of 16.8 M requests let through to a table
 // of 64 MiB: no filter 320 us, 1 MiB 227, 2 MiB 239, 4 MiB 300).
 constexpr int64_t kFilterMaxWords = 1 << 19;
-// From 2^19 pairs on, where the table no longer fits the L2s: 16.8 M requests, half of them keys, 16 slots of 128 bytes for
-// 5 keys (load 0.3) 247 us without, 205 with; for 8 keys 206 and 204, all absent 208 and 187.
-constexpr int64_t kFilterMinKeys = 1 << 19;
+// From 2^20 pairs on, where the table is four times the size of an L2. Below, many a line comes from the L2s all the same: 4.2 M
+// requests to 600,000 keys, none / half / 70 per cent / all of them keys, 58 / 57 / 56 / 54 us without, 51 / 54 / 59 / 57 with a
+// filter; to 1,048,576 keys 70 / 70 / 68 / 68 and 52 / 58 / 71 / 70.
+constexpr int64_t kFilterMinKeys = 1 << 20;
 
 static int filter_shift(int64_t nb) {
   int shift = 0;
@@ -583,13 +584,20 @@ __global__ __launch_bounds__(256) void rank_build_kernel(uint4 *table, int64_t n
 // range of a packed table read no line of their own: half of them there, 204 us.) Each bucket load waiting for
 // the one before, and all lanes of a group hashing all of its keys: 366 us. Eight waves per SIMD
 // are asked for: the fragments alone are 32 registers.
-// FILTER: the filter is asked first while that pays. It costs an access to the L2s per request and saves a line per
-// request that it turns away: a wave looks up its first 64 requests without it, turns to it when kFilterOn of 64
-// requests were absent, and away again when fewer than kFilterOff of 64 were turned away. (Stand-alone probe as
-// above, filter of 2 MiB: everything let through 393 us, 5/8 268, half 239, without filter 320: even at 15 of 64.)
-// 16,777,216 requests as above, all / 3/4 / half / none of them keys: 330 / 331 / 335 / 338 us without filter,
-// 328 / 335 / 274 / 209 with it; to a table of 2,097,152 keys 306 / 306 / 312 / 312 and 299 / 311 / 236 / 206.
-constexpr int kFilterOn = 28, kFilterOff = 16;
+// FILTER: the filter is asked first where that pays. It costs an access to the L2s per request and saves a line per
+// request that it turns away. All waves of a launch have to do the same, for beside waves that read a line for every
+// request the filter loses its place in the L2s: 16,777,216 requests to 4,194,304 keys (2 MiB of filter), 65 per cent of them keys,
+// take 331 us without it, 311 with it, and 359 where every wave judged by its last 64 requests. So every wave asks the filter for the
+// same 64 requests of the call while the lines of its own first ones are under way, and from then on uses it if kFilterAway of those were
+// turned away. (Always asked, the filter meets the time without it at 13 of 64 turned away for 4 M keys and 8 M, at 5 for 2 M; the
+// fewer steps a wave has, the more it takes.) Difference to lookups without filter at none / half / 60 / 70 / 80 per cent / all keys:
+//   16.8 M requests to 4,194,304 keys at half load  -37 / -19 / -10 /   0 / +0.5 / +0.5 %  (337 / 333 / 331 / 331 / 330 / 328 us without)
+//   to 8,000,000 keys (16 keys a word)              -32 /  -9 /   0 /  +1 / 0 / +0.5 %
+//   to 1,048,576 keys                               -26 / -14 / -13 / +1.5 / +1 / +2 %
+//   4.2 M requests to 4,194,304 keys                -34 / -10 /  +1 /  +3 / +1 / +1 %      (88 / 87 / 86 / 86 / 86 / 85 us without)
+// Where waves have hardly a step after the first the sample costs more than it can give: half keys of 1.6 M requests +2 %, 2.6 M -3 %.
+constexpr int kFilterAway = 18;
+constexpr int64_t kFilterMinRequests = 1 << 21;
 
 template <int FMT, bool FILTER>
 __global__ __launch_bounds__(256, 8) void hashmap_query_kernel(
@@ -600,23 +608,34 @@ __global__ __launch_bounds__(256, 8) void hashmap_query_kernel(
   const int64_t nwaves = static_cast<int64_t>(gridDim.x) * waves_per_block;
   int64_t i = wave * kWave + lane;
   int64_t next = i < n ? load_int(req, i, req_bytes) : -1;  // the requests stay one step ahead of the probes
-  bool ask = false;
+  bool ask = false, sample_inside = false;
+  uint32_t sample_bits = 0, sample_word = 0;
+  if (FILTER) {
+    // (anywhere in each 64th of the requests: they may alternate)
+    const int64_t share = n / kWave;
+    const int64_t at = lane * share + reduce_range(hash_id(lane), static_cast<uint32_t>(share < UINT32_MAX ? share : UINT32_MAX));
+    const int64_t key = map_key(m, load_int(req, at, req_bytes));
+    const uint32_t h = hash_id(key);
+    sample_inside = key != -1;  // (requests outside the key range read no line either way, and do not speak for the filter)
+    sample_bits = filter_bits(h);
+    sample_word = filter[reduce_range(h, m.nbuckets) >> filter_shift];
+  }
+  const int64_t first = i;
   for (; i - lane < n; i += nwaves * kWave) {
     const int64_t mykey = i < n ? map_key(m, next) : -1;  // tail lanes look up the sentinel, which resolves to -1
     const int64_t ahead = i + nwaves * kWave;
     if (ahead < n) next = load_int(req, ahead, req_bytes);
-    // (requests outside the key range read no line either way, and do not speak for the filter)
-    const uint64_t inside = FILTER ? __builtin_amdgcn_ballot_w64(mykey != -1) : ~0ull;
-    uint64_t wanted = inside;
+    uint64_t wanted = FILTER ? __builtin_amdgcn_ballot_w64(mykey != -1) : ~0ull;
     if (FILTER && ask) {
       const uint32_t h = hash_id(mykey), bits = filter_bits(h);
       wanted = __builtin_amdgcn_ballot_w64(mykey != -1 &&
                                            (filter[reduce_range(h, m.nbuckets) >> filter_shift] & bits) == bits);
     }
     const int64_t myres = wave_find<FMT, FILTER>(m, mykey, wanted);
-    if (FILTER) {
-      const uint64_t away = inside & (ask ? ~wanted : __builtin_amdgcn_ballot_w64(myres == -1));
-      ask = __builtin_popcountll(away) >= (ask ? kFilterOff : kFilterOn);
+    if (FILTER && i == first) {
+      const uint64_t inside = __builtin_amdgcn_ballot_w64(sample_inside);
+      const uint64_t away = inside & __builtin_amdgcn_ballot_w64((sample_word & sample_bits) != sample_bits);
+      ask = __builtin_popcountll(away) * kWave >= __builtin_popcountll(inside) * kFilterAway;
     }
     if (i < n) store_int(out, i, out_bytes, myres);
   }
@@ -1007,10 +1026,11 @@ int shmt_hashmap_query(const shmt_hashmap_t *map, const void *requests, int req_
   SHMT_REQUIRE(width_ok(req_bytes), "shmt_hashmap_query: ID can only be int32 or int64");
   if (n == 0) return SHMT_OK;
   SHMT_REQUIRE(requests != nullptr && out != nullptr, "shmt_hashmap_query: null buffer");
-  unsigned grid = grid_for(n, 256);
+  const bool filtered = map->filter != nullptr && n >= kFilterMinRequests;
+  const unsigned grid = grid_for(n, 256);
   hipStream_t s = as_stream(stream);
   const auto kernel = map->fmt == kSlot16 ? hashmap_query_kernel<kSlot16, false>
-                      : map->filter       ? hashmap_query_kernel<kSlot8, true>
+                      : filtered          ? hashmap_query_kernel<kSlot8, true>
                                           : hashmap_query_kernel<kSlot8, false>;
   hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), 0, s, map->view, requests, req_bytes, out, map->val_bytes, n,
                      map->filter, map->filter_shift);
