@@ -156,7 +156,9 @@ int shmt_hashmap_create_planned_scratch(shmt_hashmap_t **out,
                                         void *table_mem, int64_t table_bytes,
                                         void *scratch, int64_t scratch_bytes,
                                         void *stream);
-/* SHMT_MAP_* of a built map, and the table bytes it actually uses.         */
+/* SHMT_MAP_* of a built map, and the bytes of its table. Of a bucket table
+ * those are its buckets (shmt_hashmap_table_bytes); a presence filter behind
+ * them, at most 2 MiB, is not counted: layout.table_bytes has it in.        */
 int shmt_hashmap_kind(const shmt_hashmap_t *map);
 int64_t shmt_hashmap_used_bytes(const shmt_hashmap_t *map);
 
