@@ -385,7 +385,7 @@ struct KeyStats {
 
 constexpr int kStatThreads = 1024;
 constexpr int kStatBlocks = 256;           // workgroups of a sweep, one per compute unit, each leaving one partial result
-constexpr int64_t kStatMarksOff = 57600;   // scratch layout: one mark byte per id from here on (what lies before is spare)
+constexpr int64_t kStatMarksOff = 256;     // scratch: one mark byte per id from here on (callers know it as more than a byte per id)
 
 __device__ __forceinline__ int64_t wave_min64(int64_t v) {
 #pragma unroll
