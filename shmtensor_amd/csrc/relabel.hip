@@ -1465,8 +1465,10 @@ __global__ __launch_bounds__(kRpBlock) void rp_gather_jobs(Jobs<RpArgs> j) {
 //   ranks    first occurrences per 64 elements and per tile, and the elements that another stands for
 //   finish   as everywhere
 // A class is 1 / classes of the distinct ids; one that does not fit its table is worked through in rounds over a second
-// hash, as a bin of the partition passes is. More elements than the list holds (an id that comes in
-// most waves of the pick kernel) go into the table as they are found, and are found a second time for their results.
+// hash, as a bin of the partition passes is. Ids that come in most tiles, or in most waves of the pick kernel, make a class
+// of far more elements than distinct ids, so the list is longer than the table, as long as the LDS has room (520,000
+// ids, 1,000 of them distinct: bins 46 us where it was as long as the table, 24 now). More elements than it holds go into
+// the table as they are found, and are found a second time for their results.
 // Measured: third hop of 1,024 seeds at fanouts 15, 10, 5 (355,000 ids, launched for a bound of 1.08 M) insert 22 + first
 // 7.3 us before, bins 19 + ranks 4.8 now (launch 2.6, reading the bytes 3.6, matching 2, listing 3, ids and tables 4,
 // results 2.5); second hop (38,000 ids) 12 + 4.3 before, 6.5 + 2.5 now. tensor_relabel of 100,000 / 400,000 / 1 M ids
@@ -1487,6 +1489,10 @@ struct RcArgs {
   RlRanks *ranks;
   uint64_t *partials;
 };
+
+// Elements of a class that are listed: what the LDS of a compute unit holds beside the table.
+constexpr uint32_t rc_list(int slots_log2) { return slots_log2 == kRcSlotsLog2 ? 16384 : 12288; }
+constexpr int kRcBeyond = 2;
 
 static int rc_table_log2(int64_t N) { return N <= kRcSmallTableMax ? kRcSlotsLog2 : kRcMaxSlotsLog2; }
 
@@ -1611,8 +1617,8 @@ __device__ __forceinline__ void rc_bin_body(uint32_t c, const RcArgs &a, unsigne
                                             uint32_t *shared_words) {
   using Table = RpTable<PACKED>;
   using Key = typename Table::Key;
-  constexpr uint32_t kRcList = 1u << SLOTS_LOG2;
-  constexpr int kRcHeld = kRcList / kRcThreads;
+  constexpr uint32_t kRcList = rc_list(SLOTS_LOG2);
+  constexpr int kRcHeld = (1 << SLOTS_LOG2) / kRcThreads;  // listed elements whose slot a thread keeps
   const uint32_t N = static_cast<uint32_t>(rl_count(a.n));
   uint32_t *const overflow = &shared_words[0], *const found = &shared_words[2];
   const Table tbl{mem, &shared_words[1], (1u << a.slots_log2) - 1};
@@ -1697,10 +1703,30 @@ __device__ __forceinline__ void rc_bin_body(uint32_t c, const RcArgs &a, unsigne
           fits &= tbl.insert_from(static_cast<Key>(key[j]), static_cast<uint32_t>(at[j]), hash[j], &slot[j]);
         }
       }
+      // ids that come in many tiles: those beyond are looked up again for their results
+      auto beyond = [&](auto each) {
+        for (uint32_t e0 = kRcHeld * kRcThreads + threadIdx.x; e0 < listed; e0 += kRcBeyond * kRcThreads) {
+          int64_t i[kRcBeyond], id[kRcBeyond];
+          bool mine[kRcBeyond];
+#pragma unroll
+          for (int j = 0; j < kRcBeyond; ++j) {
+            const uint32_t e = e0 + j * kRcThreads;
+            i[j] = e < listed ? list[e] : N;
+            mine[j] = i[j] < N;
+            id[j] = 0;
+          }
+          load_ints<kRcBeyond>(a.total, i, mine, a.eb, id);
+#pragma unroll
+          for (int j = 0; j < kRcBeyond; ++j)
+            if (mine[j] && theirs(id[j], r)) each(static_cast<Key>(id[j]), static_cast<uint32_t>(i[j]), hash_id(id[j]));
+        }
+      };
+      beyond([&](Key id, uint32_t i, uint32_t h) { fits &= tbl.insert(id, i, h); });
       if (!fits) *overflow = 1;
       __syncthreads();
       done = *overflow == 0;
       if (done) {
+        beyond([&](Key id, uint32_t i, uint32_t h) { first[i] = tbl.first_of(id, h); });
 #pragma unroll
         for (int j = 0; j < kRcHeld; ++j)
           if (slot[j] != kNotMine) first[at[j]] = slot[j] == kAllOnes ? *tbl.all_ones : *tbl.index_at(slot[j]);
@@ -1732,7 +1758,7 @@ __device__ __forceinline__ void rc_bin_body(uint32_t c, const RcArgs &a, unsigne
 template <int SLOTS_LOG2>
 __device__ __forceinline__ void rc_bins_body(unsigned bx, const RcArgs &a) {
   __shared__ unsigned long long mem[(1 << SLOTS_LOG2) * 3 / 2];  // 8 bytes of id and 4 of index a slot
-  __shared__ uint32_t list[1 << SLOTS_LOG2];
+  __shared__ uint32_t list[rc_list(SLOTS_LOG2)];
   __shared__ uint32_t shared_words[3];
   if (a.eb == 4)
     rc_bin_body<true, SLOTS_LOG2>(bx, a, mem, list, shared_words);

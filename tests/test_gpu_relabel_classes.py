@@ -34,6 +34,33 @@ def test_more_elements_of_a_class_than_its_list_holds(capi, oracle, n, distinct)
     _check(capi, oracle, [np.random.default_rng(distinct).integers(0, distinct, n).astype(np.int64) * 7919])
 
 
+def test_ids_that_come_in_every_tile_are_no_slower(cabi):
+    """A thousand ids put up to 5,000 elements into a class, ten thousand about 2,000: the list has room for either. (Where the
+    elements beyond 4,096 went into the table one by one: 61 us against 37.)"""
+    lib, n = cabi.load(), 520_000
+    g = torch.Generator(device="cuda").manual_seed(1)
+    sbytes = lib.shmt_relabel_scratch_bytes(n)
+    scratch = torch.empty(sbytes, dtype=torch.uint8, device="cuda")
+    unique, labels = (torch.empty(n, dtype=torch.int32, device="cuda") for _ in range(2))
+    count = torch.zeros(1, dtype=torch.int64, device="cuda")
+    took = []
+    for distinct in (1_000, 10_000):
+        ids = (torch.randint(0, distinct, (n,), device="cuda", generator=g) * 7919).to(torch.int32)
+        runs = []
+        for _ in range(12):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            for _ in range(20):
+                cabi.check(lib.shmt_relabel(ids.data_ptr(), n, 4, scratch.data_ptr(), sbytes, unique.data_ptr(), labels.data_ptr(),
+                                            count.data_ptr(), cabi.current_stream()))
+            b.record()
+            torch.cuda.synchronize()
+            runs.append(a.elapsed_time(b))
+        assert int(count.item()) == distinct
+        took.append(min(runs))
+    assert took[0] < 1.3 * took[1]
+
+
 @pytest.mark.parametrize("slots_log2,rounds_log2", [(6, -1), (3, -1), (4, 2), (2, 0)])
 @pytest.mark.parametrize("kind", ["spread32", "wide", "minus_one", "hub"])
 def test_class_that_does_not_fit_its_table(capi, oracle, tuning, slots_log2, rounds_log2, kind):  # noqa: F811
