@@ -76,7 +76,8 @@ def test_crowded_partition_that_does_not_fit_its_table(cabi, oracle, tuning, slo
 
 @pytest.mark.parametrize("n_batches", [1, 5])
 def test_crowded_partitions_in_hops(capi, oracle, tuning, n_batches):
-    """Fused hops, alone and merged, on a graph whose neighbours all lie in two partitions: the same as by default."""
+    """Fused hops, alone and merged, on a graph whose neighbours all lie in two partitions: the same as by default, which goes
+    by classes (the last hops are sized for 188,100 ids)."""
     rng = np.random.default_rng(3)
     n = 1 << 15
     nodes = np.arange(n, dtype=np.int64)
@@ -84,7 +85,7 @@ def test_crowded_partitions_in_hops(capi, oracle, tuning, n_batches):
     deg = rng.integers(0, 40, size=n)
     indptr = torch.from_numpy(np.concatenate([[0], np.cumsum(deg)]).astype(np.int64)).cuda()
     indices = torch.from_numpy(rng.choice(few, size=int(deg.sum())).astype(np.int32)).cuda()
-    batches = [torch.from_numpy(rng.permutation(n)[:3000]).cuda() for _ in range(n_batches)]
+    batches = [torch.from_numpy(rng.permutation(n)[:1900]).cuda() for _ in range(n_batches)]
     got = []
     for min_ids in (0, 8193):
         tuning(min_ids)
