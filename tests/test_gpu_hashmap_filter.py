@@ -1,5 +1,5 @@
-"""Bulk lookups in tables with a presence filter (narrow tables built by partitions, from 2^20 pairs on): every share of absent
-requests, with which a wave uses the filter, leaves it and comes back to it, answers as the pairs say."""
+"""Bulk lookups in tables with a presence filter (narrow tables built by partitions, from 2^20 pairs on), asked by calls of 2^21
+requests and more: at every share of absent requests, with which the filter is used or not, they answer as the pairs say."""
 import ctypes
 
 import pytest
@@ -144,10 +144,15 @@ def test_map_whose_buckets_alone_fit(capi):
     torch.cuda.synchronize()
     torch.cuda.empty_cache()
     total = torch.cuda.get_device_properties(0).total_memory
+    before = torch.cuda.memory_allocated()
     try:
         torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (65 << 20)) / total)
         h = capi.CUCOStaticHashmap(keys, vals, 0.5)
     finally:
         torch.cuda.set_per_process_memory_fraction(1.0)
-    assert h.memory_usage() == 64 << 20
-    _check(h, keys, pool[n:], 2_000_000, 0.5, g)
+    assert torch.cuda.memory_allocated() - before == 64 << 20      # (no filter)
+    filtered = capi.CUCOStaticHashmap(keys, vals, 0.5)
+    assert torch.cuda.memory_allocated() - before == (64 + 66) << 20
+    for each in (h, filtered):
+        assert each.memory_usage() == 64 << 20
+        _check(each, keys, pool[n:], 2_500_000, 0.5, g)
