@@ -359,9 +359,9 @@ int shmt_relabel_wide(const void *total, int64_t N, void *scratch,
  * of touching one random line per id and pass; results are identical.
  * partition_min_ids <= 0 restores the defaults: 2,097,153 for a hop whose size
  * is only a loose bound of its ids (the chained hops of shmt_sample_hop_chained),
- * 524,288 for calls that know their size, 196,608 for hops that share their
- * launches with those of three or more other batches
- * (shmt_sample_hops_chained); a value given lowers all three to it.
+ * 393,217 for calls that know their size, 524,288 for hops that do, 196,608 for
+ * hops that share their launches with those of three or more other batches
+ * (shmt_sample_hops_chained); a value given lowers all of them to it.
  * lds_slots_log2 (0 = default, 14) and max_rounds_log2 (-1 = default, 10)
  * shrink a partition's table and the
  * number of rounds a partition may take before all pairs of its ids are

@@ -19,7 +19,7 @@
 // the id, src/tensor_relabel.cu:111-117); ids known to fit 32 bits use the
 // same memory as packed 8-byte slots (see rl_packed_insert).
 // Up to 8,192 ids all of this is one launch of one workgroup with its table
-// in LDS (rl_small_kernel). From there to half a million ids (a bound of 2 M; 192 K for merged hops) fill, insert and first
+// in LDS (rl_small_kernel). From there to 384 K ids (hops 512 K, sized by a loose bound 2 M; merged hops 192 K) fill, insert and first
 // are replaced by passes in which a workgroup finds the ids of its class by scanning one byte per id
 // (rc_*_kernel), and up to 7.3 M by passes that partition the ids by hash
 // (rp_*_kernel); both give every class or partition a table in LDS.
@@ -682,8 +682,8 @@ __global__ void rl_zero_count_kernel(int64_t *count_out, int64_t *count_copy) {
 // The insert and first-occurrence passes above touch a random line of a table
 // that no cache holds once per id and pass, and the part moves such lines at
 // 50 G per second whatever the kernel does (3.1 M ids: 74 + 54 us, plus 22 us to
-// empty the table). From half a million ids on (kRpExactMin; kRpDefaultMin for a
-// hop sized by a loose bound, kRpMergedMin for hops that share their launches)
+// empty the table). From 384 K ids on (kRpExactMin; kRpHopMin for a fused hop, kRpDefaultMin for one
+// sized by a loose bound, kRpMergedMin for hops that share their launches)
 // the same results -- the first-occurrence index of every element, the ranks of
 // the first occurrences and their number per tile of kRpTile ids -- come from three passes
 // that read and write memory in runs instead:
@@ -726,10 +726,16 @@ constexpr int64_t kRpDefaultMin = kRlSelfPrefixTiles * kRlTile + 1;
 // 512 K / 400,000 / 200,000 / 50,000 on: 1,245 / 1,130 / 1,108 / 1,077 us; of 600 seeds, four merged: 1,154 / 1,072 / 1,060 /
 // 1,072; of 1,024 at 15, 10, 5: 418 / 418 / 417 / 425.)
 constexpr int64_t kRpMergedMin = 192 * 1024;
-// A call that knows its number of ids (not merely a loose bound of it): classes against partitions 42 / 43 us for 400,000
-// ids of 4 bytes, 52 / 44 for 600,000, 66 / 54 for a million; a hundred distinct ids, which the classes share out badly,
-// 61 / 45 and 55 / 44 and 120 / 52.
-constexpr int64_t kRpExactMin = 512 * 1024;
+// A call that knows its number of ids (not merely a loose bound of it). 4-byte ids, all distinct / 10,000 / 1,000 / 100
+// distinct: classes against partitions 29 / 28 / 30 / 28 us and 31 / 31 / 29 / 31 for 300,000 ids, 34 / 33 / 35 / 33 and 33 / 31 / 30
+// / 32 for 400,000, 38 / 37 / 41 / 37 and 35 / 33 / 31 / 33 for 520,000, 60 / 58 / 67 / 62 and 48 / 44 / 41 / 45 for a million; of 393,216
+// ids, where the class scan is through in three steps, 31.7 / 31.0 / 33.0 / 31.8 and 32.6 / 31.2 / 30.0 / 31.8. Only where all ids are
+// one are the partitions behind (400,000: 32.5 and 33.5).
+constexpr int64_t kRpExactMin = 384 * 1024 + 1;
+// A fused hop: the pick kernel classifies on the way, which saves the classes a launch that partitions do not need. Hops of
+// 416,000 ids 58 / 58 / 60 / 68 us by classes and 59 / 58 / 57 / 59, of 494,000 65 / 64 / 66 / 74 and 64 / 63 / 61 / 63; with a
+// single id for all neighbours, which the seeds in front of it in its first tile may hide from the repeats test, 60 and 82.
+constexpr int64_t kRpHopMin = 512 * 1024;
 constexpr int kRpMergedMinJobs = 4;
 constexpr int kRpMinSlotsLog2 = 12;  // smallest table a bin pass is compiled for
 
@@ -749,11 +755,12 @@ struct RpPlan {
 
 // Where the partition passes keep their arrays inside the table memory (16 * cap bytes) of a
 // scratch buffer sized for N ids; ok = false when N is outside the range this path serves.
-static RpPlan rp_plan(int64_t N, int merged_jobs = 0, bool loose = false) {
+static RpPlan rp_plan(int64_t N, int merged_jobs, bool loose, bool hop) {
   RpPlan p{};
   const bool merged = merged_jobs >= kRpMergedMinJobs;
   if (merged_jobs > 0 && !merged) return p;
-  const int64_t exact_min = g_rp_tuning.min_ids < kRpExactMin ? g_rp_tuning.min_ids : kRpExactMin;
+  const int64_t known_min = hop ? kRpHopMin : kRpExactMin;
+  const int64_t exact_min = g_rp_tuning.min_ids < known_min ? g_rp_tuning.min_ids : known_min;
   if (N < (merged ? g_rp_tuning.min_ids_merged : (loose ? g_rp_tuning.min_ids : exact_min)) || N <= kRlSmallMax) return p;
   int lg = kRpMinBinsLog2;
   while ((kRpBinIds << lg) < N) ++lg;
@@ -764,7 +771,8 @@ static RpPlan rp_plan(int64_t N, int merged_jobs = 0, bool loose = false) {
   // two slots per id the bin may hold if every id of the input is distinct, as far as the largest table goes;
   // when N is a loose bound of the id count (a chained hop: typically three times what turns up) a quarter of
   // that, a bin that does get more taking two rounds
-  p.table_log2 = kRpMinSlotsLog2;
+  // (a bin pass of the smallest table has 256 threads: 520,000 ids 46 us, where the next one takes 35)
+  p.table_log2 = merged || loose ? kRpMinSlotsLog2 : kRpMinSlotsLog2 + 1;
   while (p.table_log2 < kRpSlotsLog2 && (static_cast<int64_t>(p.P) << p.table_log2) < (loose ? N / 2 : 2 * N)) ++p.table_log2;
   auto up = [](int64_t x) { return (x + 255) & ~255ll; };
   p.rec_off = 0;
@@ -1466,14 +1474,15 @@ __global__ __launch_bounds__(kRpBlock) void rp_gather_jobs(Jobs<RpArgs> j) {
 //   finish   as everywhere
 // A class is 1 / classes of the distinct ids; one that does not fit its table is worked through in rounds over a second
 // hash, as a bin of the partition passes is. Ids that come in most tiles, or in most waves of the pick kernel, make a class
-// of far more elements than distinct ids, so the list is longer than the table, as long as the LDS has room (520,000
-// ids, 1,000 of them distinct: bins 46 us where it was as long as the table, 24 now). More elements than it holds go into
+// of far more elements than distinct ids, so the list is longer than the table, as long as the LDS has room (hop of
+// 494,000 ids, 100 of them its neighbours: 98 us where it was as long as the table, 74 now). More elements than it holds go into
 // the table as they are found, and are found a second time for their results.
 // Measured: third hop of 1,024 seeds at fanouts 15, 10, 5 (355,000 ids, launched for a bound of 1.08 M) insert 22 + first
 // 7.3 us before, bins 19 + ranks 4.8 now (launch 2.6, reading the bytes 3.6, matching 2, listing 3, ids and tables 4,
-// results 2.5); second hop (38,000 ids) 12 + 4.3 before, 6.5 + 2.5 now. tensor_relabel of 100,000 / 400,000 / 1 M ids
-// 37 / 58 / 86 us before, 32 / 47 / 68 now, all distinct 42 / 68 / 106 and 33 / 48 / 75; below 50,000 ids no difference
-// but for a hundred distinct ids (27.4 -> 30.4 at 9,000), where the table in memory needs hardly an atomic.
+// results 2.5); second hop (38,000 ids) 12 + 4.3 before, 6.5 + 2.5 now. Table in memory -> classes, us a call, all distinct /
+// 10,000 / 1,000 / 100 distinct ids: 20,000 ids 24 / 21 / 21 / 17.5 -> 18 / 18 / 18 / 18; 100,000 30 / 23 / 25 / 27 -> 20 / 20 / 20 / 20;
+// 300,000 52 / 32 / 38 / 50 -> 29 / 28 / 30 / 28. Where hardly an id is new the table in memory needs hardly an atomic, and
+// classes are slower: 9,000 ids, 100 distinct 14.9 -> 16.9 us of kernels; 300,000 times the same id 27 -> 28.
 constexpr int kRcThreads = 1024;
 constexpr int kRcSlotsLog2 = 12, kRcMaxSlotsLog2 = 13;  // table slots, and elements of a class that are listed
 constexpr int64_t kRcSmallTableMax = 512 * 1024;        // the smaller one: two thirds full when all ids differ
@@ -2066,8 +2075,8 @@ static int relabel_impl(const void *total, const RlSegments *segs, int64_t N, Rl
   // (jobs that share the launch share its workgroups: every one of them sums the tile counts first)
   const unsigned fin_blocks = grid_for(N, kRlBlock, kRlFinishBlocks / (defer && defer->jobs > 0 ? defer->jobs : 1));
   // a job among fewer merged ones than the partition passes pay for keeps the table (and stays mergeable)
-  const RpPlan rp = rp_plan(N, defer ? (prepared ? defer->jobs : 1) : 0, n.fixed_dev != nullptr);
-  if (!rp.ok && defer && rp_plan(N, 0, n.fixed_dev != nullptr).ok) {
+  const RpPlan rp = rp_plan(N, defer ? (prepared ? defer->jobs : 1) : 0, n.fixed_dev != nullptr, prepared);
+  if (!rp.ok && defer && rp_plan(N, 0, n.fixed_dev != nullptr, prepared).ok) {
     defer->mergeable = false;  // a hop of this size on its own takes the partition passes: one by one then
     return SHMT_OK;
   }
@@ -2213,7 +2222,7 @@ int relabel_table(int64_t N, bool n_is_loose_bound, int merged_jobs, void *scrat
   // Nor where the ids are told apart by class (rc_plan).
   out->classes = RelabelClasses{};
   out->classified = false;
-  const bool tableless = N <= kRlSmallMax || rp_plan(N, merged_jobs, n_is_loose_bound).ok ||
+  const bool tableless = N <= kRlSmallMax || rp_plan(N, merged_jobs, n_is_loose_bound, true).ok ||
                          rc_plan(N, merged_jobs, out->slots, &out->classes);
   out->n16 = tableless ? 0 : (n_is_loose_bound ? (l.cap / 2 + 7) & ~7ll : l.cap);
   out->wide_mark = reinterpret_cast<uint64_t *>(static_cast<char *>(scratch) + l.flag_off);

@@ -1,4 +1,4 @@
-"""Relabel of 8,193 to 524,287 ids (for a hop sized by a loose bound up to 2,097,152), told apart by one class byte per id:
+"""Relabel of 8,193 to 393,216 ids (for a hop up to 524,287, sized by a loose bound up to 2,097,152), told apart by one class byte per id:
 against the oracle over what decides the path inside (repeats that another element stands for, lists that overflow, tables
 that do not hold their class), for ids that a separate launch classifies and for those that the pick kernel does."""
 import numpy as np
@@ -19,7 +19,7 @@ def _check(capi, oracle, parts):
         assert np.array_equal(got.cpu().numpy(), want)
 
 
-@pytest.mark.parametrize("n", [8193, 70_001, 524_287])
+@pytest.mark.parametrize("n", [8193, 70_001, 393_216, 393_217])      # (the last one: the first that takes partitions)
 @pytest.mark.parametrize("dt,kind", [(np.int64, k) for k in KINDS64] + [(np.int32, k) for k in KINDS32])
 def test_relabel_by_class_matches_oracle(capi, oracle, n, dt, kind):
     rng = np.random.default_rng(n)
@@ -29,36 +29,34 @@ def test_relabel_by_class_matches_oracle(capi, oracle, n, dt, kind):
 
 
 @pytest.mark.parametrize("distinct", [1, 100, 3000, 9000])
-@pytest.mark.parametrize("n", [500_000, 524_287])
+@pytest.mark.parametrize("n", [200_000, 393_216])
 def test_more_elements_of_a_class_than_its_list_holds(capi, oracle, n, distinct):
     """A few ids, each in every tile: a class has up to a hundred times the elements that its share of distinct ids suggests."""
     _check(capi, oracle, [np.random.default_rng(distinct).integers(0, distinct, n).astype(np.int64) * 7919])
 
 
-def test_ids_that_come_in_every_tile_are_no_slower(cabi):
-    """A thousand ids put up to 5,000 elements into a class, ten thousand about 2,000: the list has room for either. (Where the
-    elements beyond 4,096 went into the table one by one: 61 us against 37.)"""
-    lib, n = cabi.load(), 520_000
+def test_few_neighbours_are_hardly_slower_than_many(capi, oracle):
+    """A hundred ids that come in every wave of the pick kernel put up to 8,000 elements into a class, ten thousand about
+    2,000: the list has room for either. (Where those beyond 4,096 went into the table one by one: 98 us against 65.)"""
+    n, n_seeds = 200_000, 19_000
     g = torch.Generator(device="cuda").manual_seed(1)
-    sbytes = lib.shmt_relabel_scratch_bytes(n)
-    scratch = torch.empty(sbytes, dtype=torch.uint8, device="cuda")
-    unique, labels = (torch.empty(n, dtype=torch.int32, device="cuda") for _ in range(2))
-    count = torch.zeros(1, dtype=torch.int64, device="cuda")
+    indptr = torch.arange(0, 30 * n + 1, 30, device="cuda")
+    seeds = torch.randperm(n, device="cuda", generator=g)[:n_seeds].to(torch.int32)
     took = []
-    for distinct in (1_000, 10_000):
-        ids = (torch.randint(0, distinct, (n,), device="cuda", generator=g) * 7919).to(torch.int32)
+    for distinct in (100, 10_000):
+        indices = torch.randint(0, distinct, (30 * n,), device="cuda", generator=g).to(torch.int32)
         runs = []
         for _ in range(12):
             a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
             a.record()
             for _ in range(20):
-                cabi.check(lib.shmt_relabel(ids.data_ptr(), n, 4, scratch.data_ptr(), sbytes, unique.data_ptr(), labels.data_ptr(),
-                                            count.data_ptr(), cabi.current_stream()))
+                hop = capi.sample_hop(indptr, indices, None, None, None, seeds, 25, False, seed=11)
             b.record()
             torch.cuda.synchronize()
             runs.append(a.elapsed_time(b))
-        assert int(count.item()) == distinct
         took.append(min(runs))
+        eu, (_, el) = oracle.relabel([seeds.cpu().numpy(), hop[1].cpu().numpy()])
+        assert np.array_equal(hop[2].cpu().numpy(), eu) and np.array_equal(hop[3].cpu().numpy(), el)
     assert took[0] < 1.3 * took[1]
 
 
