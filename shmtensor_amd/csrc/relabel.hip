@@ -192,9 +192,7 @@ struct RlInsertArgs {
   RlPath path;
 };
 
-// (bx, gx): this workgroup's index and the number of workgroups of its job:
-// blockIdx.x / gridDim.x of a plain launch, the job's share of a merged one.
-__device__ __forceinline__ void rl_insert_body(unsigned bx, unsigned gx, const RlInsertArgs &a) {
+__global__ __launch_bounds__(kRlBlock) void rl_insert_kernel(RlInsertArgs a) {
   RlSlot *const tbl = a.tbl;
   const uint32_t cap = a.cap;
   const void *const total = a.total;
@@ -211,7 +209,7 @@ __device__ __forceinline__ void rl_insert_body(unsigned bx, unsigned gx, const R
   // tile (a batch without hub nodes: 99.4 % of the ids of the benchmark's largest hop are alone in their
   // tile) sends the ids of its later tiles straight to the table.
   bool staging = true;
-  for (int64_t tile = bx; tile < ntiles; tile += gx) {
+  for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
     if (!staging) {
       const int64_t i = tile * kRlInsertTile + threadIdx.x;
       if (i < N) {
@@ -256,7 +254,7 @@ __device__ __forceinline__ void rl_insert_body(unsigned bx, unsigned gx, const R
     }
     // (also the barrier between staging and reading it back) ids of this tile that another thread inserts
     const int repeats = __syncthreads_count(i < N && staged && lfirst[pos] != static_cast<uint32_t>(i));
-    if (tile == static_cast<int64_t>(bx)) staging = repeats * 32 > kRlInsertTile;  // more than 3 % repeats
+    if (tile == static_cast<int64_t>(blockIdx.x)) staging = repeats * 32 > kRlInsertTile;  // more than 3 % repeats
     // the thread holding the smallest index of an id inserts it for the whole tile:
     // one global probe chain per thread at most
     if (i < N && (!staged || lfirst[pos] == static_cast<uint32_t>(i))) {
@@ -268,10 +266,6 @@ __device__ __forceinline__ void rl_insert_body(unsigned bx, unsigned gx, const R
     }
     __syncthreads();
   }
-}
-
-__global__ __launch_bounds__(kRlBlock) void rl_insert_kernel(RlInsertArgs a) {
-  rl_insert_body(blockIdx.x, gridDim.x, a);
 }
 
 // First-occurrence index of every element: one id per thread, a workgroup of
@@ -332,12 +326,12 @@ struct RlFirstArgs {
   RlRanks *ranks;
 };
 
-__device__ __forceinline__ void rl_first_body(unsigned bx, const RlFirstArgs &a) {
+__global__ __launch_bounds__(kRlTile) void rl_first_kernel(RlFirstArgs a) {
   const int64_t N = rl_count(a.n);
   // launched for a bound of N: tiles past the ids have nothing to do, and nobody reads their count
-  if (static_cast<int64_t>(bx) * kRlTile >= N) return;
+  if (static_cast<int64_t>(blockIdx.x) * kRlTile >= N) return;
   __shared__ uint64_t lds[kRlTile / kWave];
-  const int64_t i = static_cast<int64_t>(bx) * kRlTile + threadIdx.x;
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * kRlTile + threadIdx.x;
   uint64_t cnt = 0;
   if (i < N) {
     const int64_t key = load_int(a.total, i, a.eb);
@@ -349,10 +343,8 @@ __device__ __forceinline__ void rl_first_body(unsigned bx, const RlFirstArgs &a)
   const uint64_t before = block_exclusive_scan<uint64_t, kRlTile>(cnt, lds, &tile_total);
   const uint64_t firsts = __builtin_amdgcn_ballot_w64(cnt != 0);
   if (lane_id() == 0 && i < N) a.ranks[i / kWave] = RlRanks{firsts, static_cast<uint32_t>(before), 0u};
-  if (threadIdx.x == 0) a.partials[bx] = tile_total;
+  if (threadIdx.x == 0) a.partials[blockIdx.x] = tile_total;
 }
-
-__global__ __launch_bounds__(kRlTile) void rl_first_kernel(RlFirstArgs a) { rl_first_body(blockIdx.x, a); }
 
 struct RlFinishArgs {
   const void *total;
@@ -2172,7 +2164,7 @@ static int relabel_impl(const void *total, const RlSegments *segs, int64_t N, Rl
   // At most 1,024 workgroups insert, each walking its tiles in turn: random global atomics run at 20-26 G/s on
   // this part whatever the grid (a third of the rate of plain stores), and a workgroup's later tiles then find
   // the ids of hub nodes already in the table with a smaller index and skip their atomics, where 8,192
-  // workgroups starting together all miss them (8 batches per launch: 64.5 -> 62.3 us per batch).
+  // workgroups starting together all miss them.
   const unsigned ins_blocks = grid_for(N, kRlInsertTile, 1024);
   if (prepared) {
     // the caller's earlier kernels on this stream emptied the table and wrote `total`
