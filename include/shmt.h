@@ -465,8 +465,8 @@ int shmt_sample_staged(const void *indptr, int ptr_bytes, int64_t rows,
  * learn nnz before the relabel is queued and so that no separate
  * concatenation, table-fill or offset pass is launched: the plan kernel also
  * writes the seeds to total_out[0..S), the pick kernel also writes every
- * sampled id to total_out[S + offset], adds the tile offsets and empties the
- * relabel table, and the relabel passes read the sampled count from
+ * sampled id to total_out[S + offset], adds the tile offsets and prepares the
+ * relabel (in scratch), and the relabel passes read the sampled count from
  * device memory (a word of the plan buffer).
  * Requires S >= 1, k >= 1 and S * (k + 1) < 2^31. Buffers: sub_indptr S + 1
  * entries (ptr_bytes); sub_indices S * k entries (idx_bytes; the first nnz are

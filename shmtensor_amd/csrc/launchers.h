@@ -98,12 +98,12 @@ int launch_scan_partials(uint64_t *partials, int64_t nb, hipStream_t s);
 // Relabel as the tail of a fused launch sequence. relabel_table() names the
 // hash-table part of a relabel scratch buffer sized for N ids (n16 16-byte
 // words that must be all ones when the passes start); launch_relabel_passes()
-// runs insert -> first -> finish on `total`, which earlier kernels of
+// runs the passes on `total`, which earlier kernels of
 // the same stream have filled, for n_fixed + *n_extra_dev ids (at most n_bound;
 // with n_fixed_dev the first part is min(*n_fixed_dev, n_fixed), read on the
 // device); those kernels must also have stored `nonce` to *wide_mark if any id
 // lies outside [0, 2^32). n16 is 0 when the passes need no table in memory
-// (small inputs). count_copy, if set, receives the count as well (device memory).
+// (one workgroup, classes, partitions: all inputs up to 7.34 M ids). count_copy, if set, receives the count as well (device memory).
 //
 // Inputs of the sizes between take classes instead of a table in memory (rc_*_kernel): classes.count != 0. Either the
 // earlier kernels classify the ids and say so (classified), or the passes begin with a launch that does.

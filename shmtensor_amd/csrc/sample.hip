@@ -24,7 +24,8 @@
 //        the relabel input, pick adds the tile offsets itself (every wave sums
 //        the tile totals below its tile; a totals kernel only beyond 1,024
 //        tiles) and publishes the total, writes every
-//        sampled id into the relabel input too, empties the relabel table and
+//        sampled id into the relabel input too, gives all ids their relabel
+//        class (or empties the relabel table, where the passes need one) and
 //        marks whether any id falls outside 32 bits. The number of seeds may
 //        itself live in device memory (the count a previous hop produced):
 //        launches and buffers are then sized for a bound and every kernel
